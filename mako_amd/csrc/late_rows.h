@@ -120,7 +120,7 @@ __device__ MAKO_RARE_CALL void finish_late_row(const mako_sample_desc& d, const 
         return;
     }
     CandSlots pre;
-    const bool prefetched = cls == kTopK && !d.draft && slots_cover(slices); // uniform
+    const bool prefetched = cls == kTopK && slots_cover(slices); // uniform
     if (prefetched)
         fetch_candidate_slots(sc, row, slices, pre);
     float m;

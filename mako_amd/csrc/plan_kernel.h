@@ -67,7 +67,7 @@ __global__ __launch_bounds__(kThreads) void plan_kernel(mako_sample_desc d_arg, 
             return;
         }
     }
-    const bool prefetched = covered && cls == kTopK && !d.draft; // uniform
+    const bool prefetched = covered && cls == kTopK; // uniform
     float m;
     uint32_t argidx, n_cands, any_overflow;
     row_summary_of(lane_stat, slices, m, argidx, n_cands, any_overflow);

@@ -484,7 +484,29 @@ __device__ __forceinline__ float ror_add(float v, float x)
                                                                  0xf, 0xf, false)) + x;
 }
 
-// S plus the entries of one span (len in 1..256), added one by one in fp32 (src/gen/sampler.cpp:80-82).  One wave.
+// S plus the entries of one span (n in 1..256, in registers as load_span_lanes() leaves them), added one by one in fp32
+// (src/gen/sampler.cpp:80-82).  One wave.
+__device__ __forceinline__ float lanes_sum(const float (&x)[4], uint32_t n, float S)
+{
+    float y[4] = {x[0], x[1], x[2], x[3]};
+    float v = S; // uniform
+    for (uint32_t base = 0; base < n; base += kWave) {
+        const float cur = y[0];
+        for (uint32_t b = 0; b < kWave && base + b < n; b += 16u) {
+#pragma unroll
+            for (uint32_t k = 0; k < 16; ++k)
+                v = ror_add(v, cur);
+        }
+        y[0] = y[1];
+        y[1] = y[2];
+        y[2] = y[3];
+    }
+    // entries past the end added 0.0f: the lane of the last step holds the sum
+    const uint32_t steps = (n + 15u) & ~15u;
+    return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), (steps - 1u) & 63u));
+}
+
+// The same for a span in memory.
 template <typename Keys>
 __device__ float exact_span_sum(Keys kf, uint32_t start, uint32_t len, float S)
 {
@@ -493,21 +515,7 @@ __device__ float exact_span_sum(Keys kf, uint32_t start, uint32_t len, float S)
     if (n == 0)
         return S;
     load_span_lanes(kf, uniform_u32(start), n, x);
-    float v = S; // uniform
-    for (uint32_t base = 0; base < n; base += kWave) {
-        const float cur = x[0];
-        for (uint32_t b = 0; b < kWave && base + b < n; b += 16u) {
-#pragma unroll
-            for (uint32_t k = 0; k < 16; ++k)
-                v = ror_add(v, cur);
-        }
-        x[0] = x[1];
-        x[1] = x[2];
-        x[2] = x[3];
-    }
-    // entries past the end added 0.0f: the lane of the last step holds the sum
-    const uint32_t steps = (n + 15u) & ~15u;
-    return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), (steps - 1u) & 63u));
+    return lanes_sum(x, n, S);
 }
 
 // The entries of one span (n in 1..256, in registers as load_span_lanes() leaves them; the span starts at entry
@@ -925,8 +933,8 @@ __device__ bool sorted_tail(const mako_sample_desc& d, uint32_t row, const mako_
     const bool topp_active = P.top_p < 1.0f;
     constexpr uint32_t kEpochBits = UNSORTED ? 0xffu : ~0u; // (of a pack's upper half)
     // (UNORDERED: verification takes the running sum's chain below and, only if the draft is rejected, the generic walk)
-    if ((d.draft && !UNORDERED) || (!PLANNED && n1 > kGroup * kMaxGroups)) {
-        // verification and oversized lists take the generic windowed replay
+    if ((d.draft && !UNORDERED && (PLANNED || n1 > kGroup)) || (!PLANNED && n1 > kGroup * kMaxGroups)) {
+        // verification of long lists and oversized lists take the generic windowed replay
         uint32_t n = n1;
         if (topp_active) {
             if (!have_total) {
@@ -981,7 +989,9 @@ __device__ bool sorted_tail(const mako_sample_desc& d, uint32_t row, const mako_
     }
 
     if (!PLANNED && n1 <= kGroup) {
-        // short list: one wave does everything, the chain of fp32 roundings replayed with real additions
+        // short list: one wave does everything, the chain of fp32 roundings replayed with real additions.
+        // (Verification too: 256 rows cut to 40 candidates under masks, each with a draft, take plan_kernel 10 us; sorting
+        // all of a row's candidates and replaying the sum in windows of the whole workgroup took it 80.)
         MAKO_STAMP(5);
         __syncthreads(); // the list is published; sm.flag is free
         if (wave_id() == 0) {
@@ -1029,15 +1039,55 @@ __device__ bool sorted_tail(const mako_sample_desc& d, uint32_t row, const mako_
             if (ok && need_cut && !(q_bound < qat(n - 1)))
                 ok = false;
             if (ok) {
-                const float total = exact_span_sum(kf, 0, n, 0.0f);
+                float x[4]; // (entry 64 j + lane)
+                load_span_lanes(kf, 0, n, x);
+                const float total = lanes_sum(x, n, 0.0f);
                 const float span = total - 0.0f;
                 const float prod = u_row * span;
                 float r = prod + 0.0f;
-                uint32_t pos = n - 1;
-                if (r < 0.0f)
+                uint32_t pos = n - 1, accepted = 0;
+                bool walks = true, keeps_draft = false;
+                float q_draft = 0.0f;
+                if (d.draft) { // uniform
+                    // Verification (src/gen/sampler.cpp:93-106): the draft's place in the list, one entry per lane and
+                    // ballot.  A rejected draft leaves the list for the redraw: as a weight of 0.0f it neither stops the
+                    // walk nor changes r; only where the list would begin or end with it is the place next to it meant.
+                    const int32_t draft = d.draft[row];
+                    uint32_t pd = kNone;
+#pragma unroll
+                    for (uint32_t j = 0; j < 4; ++j) {
+                        const uint32_t i = j * kWave + (uint32_t)lane_id();
+                        const unsigned long long at = __ballot(i < n && (int32_t)idat(min(i, n - 1u)) == draft);
+                        if (at)
+                            pd = j * kWave + (uint32_t)__ffsll((long long)at) - 1u;
+                    }
+                    q_draft = pd == kNone ? 0.0f : qat(pd);
+                    accepted = r < q_draft ? 1u : 0u;
+                    const uint32_t others = pd == kNone ? n : n - 1u;
+                    if (accepted || others == 0u) { // (the draft, also where it is the only candidate)
+                        keeps_draft = true;
+                        walks = false;
+                    } else {
+                        const float rest = total - q_draft;
+                        const float span2 = rest - 0.0f;
+                        const float prod2 = d.u2[row] * span2;
+                        r = prod2 + 0.0f;
+                        if (pos == pd)
+                            pos = n - 2u;
+#pragma unroll
+                        for (uint32_t j = 0; j < 4; ++j)
+                            x[j] = j * kWave + (uint32_t)lane_id() == pd ? 0.0f : x[j];
+                        if (r < 0.0f) {
+                            pos = pd == 0u ? 1u : 0u;
+                            walks = false;
+                        }
+                    }
+                } else if (r < 0.0f) {
                     pos = 0;
-                else if (r == r && r != INFINITY)
-                    exact_span_walk(kf, 0, n, r, pos);
+                    walks = false;
+                }
+                if (walks && r == r && r != INFINITY)
+                    walk_lanes(x, n, 0u, r, pos);
                 if (d.out_cand_idx && d.out_cand_q)
                     for (uint32_t j = lane_id(); j < n && j < d.cand_cap; j += kWave) {
                         d.out_cand_idx[(size_t)row * d.cand_cap + j] = (int32_t)idat(j);
@@ -1045,12 +1095,12 @@ __device__ bool sorted_tail(const mako_sample_desc& d, uint32_t row, const mako_
                     }
                 if (lane_id() == 0) {
                     RowOut o;
-                    o.token = (int32_t)idat(pos);
+                    o.token = keeps_draft ? d.draft[row] : (int32_t)idat(pos);
                     o.n_cand = n;
                     o.total = total;
-                    o.q = qat(pos);
+                    o.q = keeps_draft ? q_draft : qat(pos);
                     o.path = path;
-                    o.accepted = 0;
+                    o.accepted = accepted;
                     write_row(d, row, o);
                 }
             }
@@ -1469,7 +1519,6 @@ __device__ bool sorted_tail(const mako_sample_desc& d, uint32_t row, const mako_
     uint32_t reach_w = reach, head_n_w = head_n;
     bool head_walk_w = head_walk;
     uint32_t redraw_g = kNone, redraw_at = kNone; // the rejected draft's group and position
-    float redraw_q = 0.0f;
     if constexpr (UNORDERED && VERIFY) {
         {
             // Verification (src/gen/sampler.cpp:93-106) of a row in token order: entry i is token i, so the draft's weight is
@@ -1504,7 +1553,6 @@ __device__ bool sorted_tail(const mako_sample_desc& d, uint32_t row, const mako_
             r_begin = prod2 + 0.0f;
             if (q_draft > 0.0f) { // (the draft is a candidate, at dr < n)
                 redraw_at = dr;
-                redraw_q = q_draft;
                 redraw_g = dr / kGroup; // (a list in token order: every group but the last holds kGroup entries)
                 for (uint32_t g = redraw_g + 1u + tid; g <= groups; g += kThreads)
                     G.pg()[g] -= (double)q_draft;

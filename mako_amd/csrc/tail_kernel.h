@@ -60,7 +60,7 @@ __device__ __forceinline__ void tail_body(const mako_sample_desc& d_arg, const S
         // A top-k row is finished here, in line: there are dozens of them beside a few long tails, and through the
         // call below (whose entry and the entries of what it calls store dozens of registers per thread) each took
         // longer than the longest tail.
-        if (late_cls == kTopK && !plain && !d_arg.draft && covered) {
+        if (late_cls == kTopK && !plain && covered) {
             float m;
             uint32_t argidx, n_cands, any_overflow;
             row_summary_of(lane_stat, slices, m, argidx, n_cands, any_overflow);

@@ -316,9 +316,8 @@ __device__ __forceinline__ void topk_row(const mako_sample_desc& d, const Scratc
     uint32_t* kf = reinterpret_cast<uint32_t*>(L.sortk + kSortMax); // upper half of the dynamic block
     uint32_t* jf = kf + kSortMax;
     uint32_t n_valid = 0;
-    uint32_t n_list = kNone;
-    if (!d.draft) // the top_k-th weight's neighbourhood only
-        n_list = small_candidates(sc, row, slices, n_cands, m, inv_t, floor_q, P.top_k, 0u, kf, jf, n_valid, L, have_pre, pre);
+    // the top_k-th weight's neighbourhood only
+    uint32_t n_list = small_candidates(sc, row, slices, n_cands, m, inv_t, floor_q, P.top_k, 0u, kf, jf, n_valid, L, have_pre, pre);
     if (n_list == kNone)
         n_valid = n_cands <= 1024u ? sort_candidates<1>(sc, row, slices, n_cands, m, inv_t, floor_q, kf, jf, L)
                                    : sort_candidates<4>(sc, row, slices, n_cands, m, inv_t, floor_q, kf, jf, L);
