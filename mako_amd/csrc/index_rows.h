@@ -210,8 +210,7 @@ __global__ __launch_bounds__(kThreads) void index_groups_kernel(mako_sample_desc
     const uint32_t off = p * kSpan, cnt = min(kSpan, n_list - off);
     const uint32_t groups = (cnt + kGroup - 1u) / kGroup; // <= 16 GPW <= 64
     const GlobalKeys kf{sc_val.key[0] + (size_t)row * sc_val.vpad};
-    const GroupTable& T = sc_val.gt;
-    const size_t t_at = (size_t)row * sc_val.g_cap + p * (kSpan / kGroup);
+    GroupRec* recs = sc_val.gt + (size_t)row * sc_val.g_cap + p * (kSpan / kGroup);
     MAKO_CHECK(sc_val, kCheckGroups, p * (kSpan / kGroup) + groups <= sc_val.g_cap && (uint64_t)off + cnt <= sc_val.vpad);
     float q[GPW][4];
     uint32_t len[GPW];
@@ -235,39 +234,15 @@ __global__ __launch_bounds__(kThreads) void index_groups_kernel(mako_sample_desc
     // the sums before and behind each group: lane g holds group g's
     const double v = s_gs[lane];
     const double upto = __ockl_wfscan_add_f64(v, true);
-    const double before_l = mass + (upto - v), after_l = mass + upto;
+    const double before_l = mass + (upto - v);
     const double r0_raw = (double)u_row * total64, r0 = r0_raw == r0_raw ? r0_raw : 0.0;
 #pragma unroll
     for (uint32_t k = 0; k < GPW; ++k) {
         const uint32_t g = uniform_u32(wave + k * (uint32_t)kWaves);
         if (g >= groups) // uniform per wave
             break;
-        const double guess = readlane_f64(before_l, g), at_end = readlane_f64(after_l, g);
-        const int eg = guess > 0 ? exponent_of((float)guess) : 0;
-        const seqfp::Step32 st = span_map<true>(q[k], len[k], eg);
-        // the sum is expected to change binade inside the group (or starts at zero): records for its quarters
-        const bool split4 = uniform_u32((uint32_t)(eg == 0 || exponent_of((float)at_end) != eg)) != 0;
-        if (split4)
-            build_quarters(q[k], len[k], guess, T.quarters + (t_at + g) * 4u);
-        // the walk's map, where the walk is expected to pass the group without changing binade in it
-        const double r_here = r0 - guess, r_after = r0 - at_end;
-        const int ew = (r0 > 0.0 && r_after > 0.0) ? exponent_of((float)r_here) : 0;
-        uint4 wrec = make_uint4(0u, 0u, 0u, 0u);
-        if (ew > 0 && uniform_u32((uint32_t)(exponent_of((float)r_after) == ew)) != 0) {
-            const seqfp::Step32 sw = span_map<true>(q[k], len[k], ew);
-            const float q_top = __uint_as_float(__ockl_wfred_max_u32(max(max(__float_as_uint(q[k][0]), __float_as_uint(q[k][1])),
-                                                                         max(__float_as_uint(q[k][2]), __float_as_uint(q[k][3])))));
-            wrec = make_uint4(sw.d0, sw.d1, walk_need(q_top, ew, sw.cmax), (uint32_t)ew);
-        }
-        if (lane == 0) {
-            T.sum[t_at + g] = s_gs[g];
-            T.d0[t_at + g] = st.d0;
-            T.d1[t_at + g] = st.d1;
-            T.cmax[t_at + g] = st.cmax;
-            T.start[t_at + g] = off + g * kGroup;
-            T.pack[t_at + g] = len[k] | ((uint32_t)eg << 16) | (split4 ? kHasQuarters : 0u);
-            T.walk[t_at + g] = wrec;
-        }
+        const double sum = s_gs[g], before = readlane_f64(before_l, g);
+        group_record(q[k], off + g * kGroup, len[k], sum, before, before + sum, r0, recs + g);
     }
 }
 
@@ -320,11 +295,8 @@ __global__ __launch_bounds__(kThreads) void index_tail_kernel(mako_sample_desc d
     if (flag == kIndexReady) {
         const uint32_t* kf = sc.key[0] + (size_t)row * sc.vpad;
         // (entry i of the list is token i: no array of token ids)
-        // (verification has an instance of its own: its code costs the plain one registers)
-        const bool done = d.draft ? sorted_tail<true, false, false, false, true, true>(d, row, s_args.P, kf, nullptr, n0, true, total64, MAKO_PATH_INDEXED,
-                                                                                        L, false, 0.0f, sc.gt, (size_t)row * sc.g_cap, groups)
-                                  : sorted_tail<true, false, false, false, true, false>(d, row, s_args.P, kf, nullptr, n0, true, total64, MAKO_PATH_INDEXED,
-                                                                                         L, false, 0.0f, sc.gt, (size_t)row * sc.g_cap, groups);
+        const bool done = sorted_tail<true, false, false, false, true>(d, row, s_args.P, kf, nullptr, n0, true, total64, MAKO_PATH_INDEXED, L, false,
+                                                                       0.0f, sc.gt + (size_t)row * sc.g_cap, groups);
         if (done) {
             // (the list's length counts the gaps; the candidates are what the reference counts)
             if (tid == 0 && d.out_n_cand)

@@ -120,14 +120,7 @@ hipError_t layout_scratch(mako::Scratch& sc, uint32_t max_rows, uint32_t max_voc
     MAKO_TAKE(sc.idx[1], rv);
     sc.g_cap = (uint32_t)(sc.vpad / mako::kGroup) + mako::kWorkers;
     const size_t rg = (size_t)max_rows * sc.g_cap;
-    MAKO_TAKE(sc.gt.sum, rg);
-    MAKO_TAKE(sc.gt.d0, rg);
-    MAKO_TAKE(sc.gt.d1, rg);
-    MAKO_TAKE(sc.gt.cmax, rg);
-    MAKO_TAKE(sc.gt.start, rg);
-    MAKO_TAKE(sc.gt.pack, rg);
-    MAKO_TAKE(sc.gt.quarters, rg * 4);
-    MAKO_TAKE(sc.gt.walk, rg);
+    MAKO_TAKE(sc.gt, rg);
     MAKO_TAKE(sc.log_hist, (size_t)max_rows * sc.slices_cap * mako::kLogBins);
     MAKO_TAKE(sc.work_n, 8);
     MAKO_TAKE(sc.work_sort, (size_t)max_rows * mako::kSortItemsPerRow);
@@ -255,7 +248,7 @@ void mako_sampler_destroy(mako_sampler_ctx* ctx)
         return;
     (void)hipSetDevice(ctx->device);
     mako::Scratch& sc = ctx->sc;
-    void* ptrs[] = {sc.log_hist, sc.work_n, sc.work_sort, sc.work_tail, sc.gt.sum, sc.gt.d0, sc.gt.d1, sc.gt.cmax, sc.gt.start, sc.gt.pack, sc.gt.quarters, sc.gt.walk,
+    void* ptrs[] = {sc.log_hist, sc.work_n, sc.work_sort, sc.work_tail, sc.gt,
                     sc.cand_w, sc.cand_i, sc.part_sum, sc.plan,
                     sc.stats,      sc.wbuf,      sc.cnt,        sc.key[0],     sc.key[1],     sc.idx[0],
                     sc.idx[1],     ctx->st_logits, ctx->st_params, ctx->st_u,   ctx->st_u2,    ctx->st_mask,

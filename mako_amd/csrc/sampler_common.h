@@ -108,18 +108,20 @@ struct BigPlan {
     double mass[kWorkers];        // estimated sum of the weights above worker w's range
 };
 
-// Per-group records of a planned row's sorted list, written by the workers and read by the last of them.
-struct GroupTable {
-    double* sum;     // fp64 sum of the group's weights
-    uint32_t* d0;    // the group's map for the running fp32 sum in the epoch guessed from the mass before it
-    uint32_t* d1;
-    uint32_t* cmax;
-    uint32_t* start; // first entry of the group in the sorted list
-    uint32_t* pack;  // entries | guessed exponent << 16 | kHasQuarters if `quarters` holds records for the group
-    uint4* quarters; // [4] per group: the maps of the group's four quarters (see build_quarters)
-    uint4* walk;     // the group's map for the walk (d0, d1, the bound of group_sub_ok, exponent) in the epoch guessed
-                     // for r at the group; exponent 0: none
+// Per-group records of a planned row's list, written by sort_kernel's workers (or by the kernels of index_rows.h) and read
+// by the workgroup that adds the list up and walks it (group_chain.h).
+struct alignas(16) GroupRec {
+    double sum;         // fp64 sum of the group's weights
+    float inc[2];       // what the group adds to the running fp32 sum in the binade guessed from the mass before it, for a
+                        // sum whose last bit is even and odd (span_incs())
+    float walk[2];      // and what it takes off the walk's r in the binade guessed for that
+    uint32_t start;     // first entry of the group in the list
+    uint32_t pack;      // entries | exponent of inc's binade << kSumExpShift | of walk's << kWalkExpShift (0: none) | kOpaque
 };
+constexpr uint32_t kLenMask = 0x1ffu;
+constexpr uint32_t kSumExpShift = 9;
+constexpr uint32_t kWalkExpShift = 17;
+constexpr uint32_t kOpaque = 1u << 25; // the record stands for a whole unsorted share (unsorted_shares.h)
 
 // The large batches' work lists of sort_kernel.  Workgroups are dispatched in the order of their numbers, to the XCDs
 // in turn, and the next one waits for a CU of ITS XCD: with entries of unequal cost in row order the XCDs fall out of
@@ -151,9 +153,7 @@ struct Scratch {
     uint32_t* idx[2];  // [max_rows][vpad] candidate token ids, likewise
     uint16_t* log_hist;  // [max_rows][slices_cap][kLogBins] top_k == 0 rows: logits of the slice per bin of the slice's
                          // own frame (log_bin_in_frame(); a slice holds 16384 logits at most)
-    GroupTable gt;     // [max_rows][g_cap] each
-                       // (kept at a multiple of 16 bytes: the kernels' LDS copies of this record are read with
-                       // 128-bit operations, which stall on anything less)
+    GroupRec* gt;      // [max_rows][g_cap]
     // Work lists.  sort_kernel and tail_kernel are launched with one workgroup per POSSIBLE piece of work, but
     // workgroup i serves entry i of its kernel's list and exits if there is none: the busy workgroups are then the
     // first ones dispatched and land evenly on the XCDs, shader engines and CUs, whatever the mix of rows.
@@ -169,7 +169,7 @@ struct Scratch {
     uint32_t g_cap;    // vpad / kGroup + kWorkers
 };
 
-static_assert(offsetof(Scratch, gt) % 16 == 0 && sizeof(mako_sample_desc) % 16 == 0, "128-bit LDS reads of the staged records");
+static_assert(sizeof(mako_sample_desc) % 16 == 0, "128-bit LDS reads of the staged records");
 
 // Checked builds (-DMAKO_CHECKED, libmako_sampler_checked.so): every index a kernel computes into the context's scratch
 // arrays from counts that other kernels left is compared with the array's bound before it is used, and a failed

@@ -131,7 +131,7 @@ __device__ __forceinline__ void sort_body(const mako_sample_desc& d_arg, const S
             small_candidates(sc, row, slices, n_cands, m, inv_t, floor_q, 0u, thr_bits, kf, jf, n_valid, L, prefetched, pre);
         MAKO_STAMP(4);
         if (n_list != kNone && n_list > 0 &&
-            sorted_tail(d, row, P, kf, jf, n_list, true, total64, MAKO_PATH_NUCLEUS, L, true, q_bound))
+            sorted_tail<false, true>(d, row, P, kf, jf, n_list, true, total64, MAKO_PATH_NUCLEUS, L, true, q_bound)) // (kSmall entries at most)
             return;
         // not certifiable from the candidates: tail_kernel's launch takes a second look (narrow_second_look())
         if (tid == 0) {
@@ -179,15 +179,10 @@ __device__ __forceinline__ void sort_body(const mako_sample_desc& d_arg, const S
             bool same_tot, same_walk;
             const OpaqueGuess og = opaque_epochs(before, after_raw > before ? after_raw : before, r0, same_tot, same_walk);
             if (cnt_v == 0u) { // (nothing came: an empty group)
-                if (lane == 0u) {
-                    sc.gt.sum[t_at] = 0.0;
-                    sc.gt.d0[t_at] = sc.gt.d1[t_at] = sc.gt.cmax[t_at] = 0u;
-                    sc.gt.start[t_at] = off_v;
-                    sc.gt.pack[t_at] = 0u;
-                    sc.gt.walk[t_at] = make_uint4(0u, 0u, 0u, 0u);
-                }
+                if (lane == 0u)
+                    store_group_rec(sc.gt + t_at, 0.0, make_float2(0.0f, 0.0f), make_float2(0.0f, 0.0f), off_v, 0u);
             } else {
-                opaque_share(key1 + stage_v, cnt_v, off_v, og.e_tot, og.e_walk, t_at, sc.gt, wave_lds);
+                opaque_share(key1 + stage_v, cnt_v, off_v, og.e_tot, og.e_walk, sc.gt + t_at, wave_lds);
             }
         }
         MAKO_STAMP(12);
@@ -221,10 +216,9 @@ __device__ __forceinline__ void sort_body(const mako_sample_desc& d_arg, const S
         MAKO_STAMP(11);
         // (the guess of the running sum before the share: the plan's estimate, in the exact total's units)
         const double mass_w = readlane_f64(mass_l, w);
-        // (the walk starts from u * (the nucleus' fp32 total), which is top_p * total64 and at most one weight more;
-        // a verification row's walk is replayed by other code)
-        const double r0 = d.draft ? 0.0 : (double)u_row * ((double)s_args.P.top_p * total64);
-        worker_groups(key0, off, cnt, t_row + gbase, mass_all > 0.0 ? mass_w * (total64 / mass_all) : 0.0, sc.gt, L,
+        // (the walk starts from u * (the nucleus' fp32 total), which is top_p * total64 and at most one weight more)
+        const double r0 = (double)u_row * ((double)s_args.P.top_p * total64);
+        worker_groups(key0, off, cnt, sc.gt + t_row + gbase, mass_all > 0.0 ? mass_w * (total64 / mass_all) : 0.0, L,
                       (in_lds && sorted) ? sorted_copy : nullptr, r0 == r0 ? r0 : 0.0);
         MAKO_STAMP(12);
     }

@@ -117,7 +117,7 @@ __device__ __forceinline__ void tail_body(const mako_sample_desc& d_arg, const S
     MAKO_CHECK(sc, kCheckTailGroup, plan_n0 <= d.n_vocab && plan_groups <= min(kMaxGroups, sc.g_cap));
     bool done;
     [[clang::always_inline]] done = sorted_tail<true, false, false, UNSORTED>(d, row, s_args.P, kf, jf, n0, true, total64, MAKO_PATH_SORTED,
-                                                                              L, false, 0.0f, sc.gt, (size_t)row * sc.g_cap, groups);
+                                                                              L, false, 0.0f, sc.gt + (size_t)row * sc.g_cap, groups);
     if (done)
         return;
     // too close to call, or the list ends before the nucleus does: the whole-row path decides

@@ -23,9 +23,8 @@ namespace mako {
 // sort_kernel is bound by the number of its workgroups, one per CU at a time, and a share that needs no sorting is summed
 // by one wave of a collector workgroup that takes sixteen of them; on a small batch every worker has a CU to itself and the batch waits for the slowest anyway.
 
-// A record that stands for a whole unsorted share (in GroupTable::pack): its maps are all there is.  Never among the
-// first kHeadGroups groups of a list, and the list's entries at its positions are not written.
-constexpr uint32_t kOpaque = 1u << 30;
+// (A record with kOpaque set stands for a whole unsorted share: its increments are all there is.  Never among the first
+// kHeadGroups groups of a list, and the list's entries at its positions are not written.)
 constexpr int kOpaqueShift = 11;     // the share's largest weight lies at least this many binades below the sum and r
 constexpr uint32_t kOpaqueTies = 16; // exact ties a share may hold (expected: entries * 2^-kOpaqueShift <= 3)
 constexpr uint32_t kCollectors = 2;  // workgroups of sort_kernel that take a row's unsorted shares, one share per wave (work items kWorkers + c)

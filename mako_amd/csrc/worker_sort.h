@@ -276,22 +276,22 @@ __device__ bool lds_sort_staged_runs(const uint32_t* ks, const uint32_t* is, uin
 // of LDS of the wave's own.  The share is streamed once (sixteen loads per lane in flight): its fp64 sum, its largest
 // weight, the sums of the increments of the weights that are no exact ties, and the ties themselves (kept apart, up
 // to kOpaqueTies of either kind); only a share with ties is streamed again, for the sums between neighbouring ties.
-constexpr uint32_t kOpaqueLdsWords = 4u * kOpaqueTies + 4u * (kOpaqueTies + 1u);
-__device__ void opaque_share(const uint32_t* ks, uint32_t cnt, uint32_t off, int e_tot, int e_walk, size_t t_at,
-                             const GroupTable& T, uint32_t* lds)
+constexpr uint32_t kOpaqueLdsWords = 4u * kOpaqueTies;
+__device__ void opaque_share(const uint32_t* ks, uint32_t cnt, uint32_t off, int e_tot, int e_walk, GroupRec* rec, uint32_t* lds)
 {
     using namespace seqfp;
-    constexpr uint32_t kTrip = 16, kSegs = kOpaqueTies + 1u;
-    uint32_t* tie_key = lds;                          // [2][kOpaqueTies] as found
-    uint32_t* tie_sorted = lds + 2u * kOpaqueTies;    // [2][kOpaqueTies] heaviest first
-    unsigned long long* seg = reinterpret_cast<unsigned long long*>(lds + 4u * kOpaqueTies); // [2][kSegs]
+    constexpr uint32_t kTrip = 16;
+    uint32_t* tie_key = lds;                       // [2][kOpaqueTies] as found
+    uint32_t* tie_sorted = lds + 2u * kOpaqueTies; // [2][kOpaqueTies] heaviest first
     const GlobalKeys gk{ks};
     const uint32_t lane = (uint32_t)lane_id();
     const unsigned long long lower = (1ull << lane) - 1ull;
+    // (weights and epochs of such a share: the weights lie binades below; e_walk 0: no map for the walk)
+    const float R_t = __uint_as_float((uint32_t)e_tot << 23), half_t = half_ulp(e_tot);
+    const float R_w = __uint_as_float((uint32_t)max(e_walk, 1) << 23), half_w = half_ulp(e_walk);
     double sum = 0.0;
-    uint32_t kmax = 0u, n_t = 0u, n_w = 0u; // (the counts: uniform)
-    uint32_t acc_t = 0u, acc_w = 0u;        // a lane's increments: at most 250 of them, 2^24 at most each
-    const bool sat = cnt > (250u << 6);     // (more than that many per lane: no map)
+    uint32_t n_t = 0u, n_w = 0u; // (uniform)
+    float acc_t = 0.0f, acc_w = 0.0f; // a lane's multiples of the epochs' last places: exact up to 2^24 of them, beyond after that
     for (uint32_t base = 0; base < cnt; base += kTrip * kWave) {
         uint32_t k[kTrip];
 #pragma unroll
@@ -299,14 +299,12 @@ __device__ void opaque_share(const uint32_t* ks, uint32_t cnt, uint32_t off, int
             k[u] = gk[min(base + u * kWave + lane, cnt - 1u)];
 #pragma unroll
         for (uint32_t u = 0; u < kTrip; ++u) {
-            const bool valid = base + u * kWave + lane < cnt;
-            const uint32_t kv = valid ? k[u] : 0u;
+            const uint32_t kv = base + u * kWave + lane < cnt ? k[u] : 0u;
             const float q = __uint_as_float(kv);
             sum += (double)q;
-            kmax = max(kmax, kv);
-            const Step32 st = step32_fp(q, e_tot); // (the weights of such a share lie binades below the epochs: never the mark)
-            const bool tie_t = valid && st.d0 != st.d1;
-            acc_t += (valid && !tie_t) ? min(st.d0, 1u << 24) : 0u;
+            const float t = (R_t + q) - R_t;
+            const bool tie_t = fabsf(q - t) == half_t;
+            acc_t += tie_t ? 0.0f : t;
             const unsigned long long bal_t = __ballot(tie_t);
             if (bal_t) { // (uniform, rare)
                 const uint32_t slot = n_t + (uint32_t)__popcll(bal_t & lower);
@@ -315,9 +313,9 @@ __device__ void opaque_share(const uint32_t* ks, uint32_t cnt, uint32_t off, int
                 n_t += (uint32_t)__popcll(bal_t);
             }
             if (e_walk > 0) { // uniform
-                const Step32 sw = step32_fp(q, e_walk);
-                const bool tie_w = valid && sw.d0 != sw.d1;
-                acc_w += (valid && !tie_w) ? min(sw.d0, 1u << 24) : 0u;
+                const float w = (R_w + q) - R_w;
+                const bool tie_w = fabsf(q - w) == half_w;
+                acc_w += tie_w ? 0.0f : w;
                 const unsigned long long bal_w = __ballot(tie_w);
                 if (bal_w) {
                     const uint32_t slot = n_w + (uint32_t)__popcll(bal_w & lower);
@@ -329,107 +327,96 @@ __device__ void opaque_share(const uint32_t* ks, uint32_t cnt, uint32_t off, int
         }
     }
     const double sum64 = __ockl_wfred_add_f64(sum);
-    kmax = __ockl_wfred_max_u32(kmax);
-    // (a sum of 64 numbers below 2^31: in two halves)
-    auto wave_total = [](uint32_t v) {
-        return ((unsigned long long)__ockl_wfred_add_u32(v >> 16) << 16) + (unsigned long long)__ockl_wfred_add_u32(v & 0xffffu);
-    };
-    // One kind of map: the sums of the increments between neighbouring ties (heaviest first), with each tie's own
+    // One kind of increments: the sum of the multiples between neighbouring ties (heaviest first), with each tie's own
     // two-valued step composed in at its place.
-    auto share_map = [&](uint32_t which, uint32_t n_raw, int e, uint32_t acc) {
-        Step32 v = Step32{kSat, kSat, 0u};
-        if (e > 0 && n_raw <= kOpaqueTies && !sat) { // uniform
-            const uint32_t n = n_raw;
-            if (n == 0u) {
-                const unsigned long long S = wave_total(acc);
-                const uint32_t add = S < (1ull << 24) ? (uint32_t)S : kSat;
-                v = Step32{add, add, 0u};
-            } else {
-                // the ties by weight, heaviest first (equal ones in any order: they are the same step)
-                __builtin_amdgcn_s_waitcnt(0xc07f); // lgkmcnt(0): the wave's own writes of the ties
-                const uint32_t mine = lane < n ? tie_key[which * kOpaqueTies + lane] : 0u;
-                uint32_t rank = 0;
-                for (uint32_t j = 0; j < n; ++j) {
-                    const uint32_t other = (uint32_t)__builtin_amdgcn_readlane((int)mine, (int)j);
-                    rank += (other > mine || (other == mine && j < lane)) ? 1u : 0u;
-                }
-                if (lane < n)
-                    tie_sorted[which * kOpaqueTies + rank] = mine;
-                if (lane <= n)
-                    seg[which * kSegs + lane] = 0ull;
-                __builtin_amdgcn_s_waitcnt(0xc07f);
-                // the share again: a weight's segment is the number of ties heavier than it
-                for (uint32_t base = 0; base < cnt; base += kTrip * kWave) {
-                    uint32_t k[kTrip], sg[kTrip], dv[kTrip];
+    auto share_incs = [&](uint32_t which, uint32_t n, int e, float R, float half, float acc) {
+        if (e <= 0 || n > kOpaqueTies) // uniform
+            return make_float2(INFINITY, INFINITY);
+        const float all = readlane_f32(wave_scan_add_f32(acc), kWave - 1);
+        const uint32_t units = all < 2.0f * R ? (uint32_t)__builtin_ldexpf(all, 150 - e) : kSat; // (below 2^24, and whole)
+        if (n == 0u)
+            return make_float2(all, all);
+        // the ties by weight, heaviest first (equal ones in any order: they are the same step)
+        __builtin_amdgcn_s_waitcnt(0xc07f); // lgkmcnt(0): the wave's own writes of the ties
+        const uint32_t mine = lane < n ? tie_key[which * kOpaqueTies + lane] : 0u;
+        uint32_t rank = 0;
+        for (uint32_t j = 0; j < n; ++j) {
+            const uint32_t other = (uint32_t)__builtin_amdgcn_readlane((int)mine, (int)j);
+            rank += (other > mine || (other == mine && j < lane)) ? 1u : 0u;
+        }
+        if (lane < n)
+            tie_sorted[which * kOpaqueTies + rank] = mine;
+        __builtin_amdgcn_s_waitcnt(0xc07f);
+        // the share again, once per tie: the multiples of the weights above it (and no tie themselves)
+        Step32 v = identity32();
+        uint32_t taken = 0u;
+        for (uint32_t i = 0; i < n && units != kSat; ++i) {
+            const uint32_t tk = uniform_u32(tie_sorted[which * kOpaqueTies + i]);
+            float part = 0.0f;
+            for (uint32_t base = 0; base < cnt; base += kTrip * kWave) {
+                uint32_t k[kTrip];
 #pragma unroll
-                    for (uint32_t u = 0; u < kTrip; ++u)
-                        k[u] = gk[min(base + u * kWave + lane, cnt - 1u)];
+                for (uint32_t u = 0; u < kTrip; ++u)
+                    k[u] = gk[min(base + u * kWave + lane, cnt - 1u)];
 #pragma unroll
-                    for (uint32_t u = 0; u < kTrip; ++u) {
-                        const bool valid = base + u * kWave + lane < cnt;
-                        const Step32 st = step32_fp(__uint_as_float(k[u]), e);
-                        dv[u] = (valid && st.d0 == st.d1) ? min(st.d0, 1u << 24) : 0u;
-                        sg[u] = 0u;
-                    }
-                    for (uint32_t i = 0; i < n; ++i) {
-                        const uint32_t tk = uniform_u32(tie_sorted[which * kOpaqueTies + i]);
-#pragma unroll
-                        for (uint32_t u = 0; u < kTrip; ++u)
-                            sg[u] += tk > k[u] ? 1u : 0u;
-                    }
-                    for (uint32_t s = 0; s <= n; ++s) {
-                        uint32_t part = 0u; // (sixteen increments below 2^24 + 1 each: below 2^29)
-#pragma unroll
-                        for (uint32_t u = 0; u < kTrip; ++u)
-                            part += sg[u] == s ? dv[u] : 0u;
-                        const unsigned long long all = wave_total(part);
-                        if (lane == 0u && all)
-                            seg[which * kSegs + s] += all;
-                    }
-                }
-                __builtin_amdgcn_s_waitcnt(0xc07f);
-                v = identity32();
-                for (uint32_t s = 0; s <= n; ++s) {
-                    const unsigned long long S = seg[which * kSegs + s];
-                    const uint32_t add = S < (1ull << 24) ? (uint32_t)S : kSat;
-                    v = compose32(v, Step32{add, add, 0u});
-                    if (s < n)
-                        v = compose32(v, step32_flat(__uint_as_float(tie_sorted[which * kOpaqueTies + s]), e));
+                for (uint32_t u = 0; u < kTrip; ++u) {
+                    const float q = __uint_as_float(k[u]);
+                    const float t = (R + q) - R;
+                    part += (base + u * kWave + lane < cnt && k[u] > tk && !(fabsf(q - t) == half)) ? t : 0.0f;
                 }
             }
+            const uint32_t above = (uint32_t)__builtin_ldexpf(readlane_f32(wave_scan_add_f32(part), kWave - 1), 150 - e);
+            v = compose32(v, Step32{above - taken, above - taken, 0u});
+            v = compose32(v, step32_flat(__uint_as_float(tk), e));
+            taken = above;
         }
-        v.cmax = e > 0 ? step32_flat(__uint_as_float(kmax), e).cmax : kSat; // (a weight's step never grows as the weight falls)
-        return v;
+        const uint32_t rest = units == kSat ? kSat : units - taken;
+        v = compose32(v, Step32{rest, rest, 0u});
+        auto as_float = [e](uint32_t d) { return d < (1u << 24) ? __builtin_ldexpf((float)d, e - 150) : INFINITY; };
+        return make_float2(as_float(v.d0), as_float(v.d1));
     };
-    const Step32 m0 = share_map(0u, n_t, e_tot, acc_t);
-    const Step32 m1 = e_walk > 0 ? share_map(1u, n_w, e_walk, acc_w) : Step32{kSat, kSat, kSat};
-    if (lane == 0u) {
-        T.sum[t_at] = sum64;
-        T.d0[t_at] = m0.d0;
-        T.d1[t_at] = m0.d1;
-        T.cmax[t_at] = m0.cmax;
-        T.start[t_at] = off;
-        T.pack[t_at] = kOpaque | ((uint32_t)e_tot << 16);
-        T.walk[t_at] = e_walk > 0 ? make_uint4(m1.d0, m1.d1, walk_need(__uint_as_float(kmax), e_walk, m1.cmax), (uint32_t)e_walk)
-                                  : make_uint4(0u, 0u, 0u, 0u);
-    }
+    const float2 m0 = share_incs(0u, n_t, e_tot, R_t, half_t, acc_t);
+    const float2 m1 = share_incs(1u, n_w, e_walk, R_w, half_w, acc_w);
+    if (lane == 0u)
+        store_group_rec(rec, sum64, m0, m1, off, kOpaque | ((uint32_t)e_tot << kSumExpShift) | ((uint32_t)max(e_walk, 0) << kWalkExpShift));
 }
 
-// Group records of a worker's sorted range (cnt entries from position off of the list kf): fp64 sums, and the
-// maps of the running fp32 sum for the epoch guessed from the mass above the range plus the sums before the group.
+// The record of one group (q: its entries, four per lane; `before` / `after`: the mass in front of it and behind it; r0:
+// the estimate of where the walk starts, 0 or less: none): increments only where the binade is not expected to change
+// inside the group, which is replayed there.  One wave.
+__device__ __forceinline__ void group_record(const float (&q)[4], uint32_t start, uint32_t len, double sum, double before, double after, double r0,
+                                             GroupRec* rec)
+{
+    const uint32_t es = uniform_u32((uint32_t)exponent_of((float)before)), es_end = uniform_u32((uint32_t)exponent_of((float)after));
+    float2 inc = make_float2(INFINITY, INFINITY), walk = inc;
+    if (es == es_end)
+        inc = span_incs(q, (int)es);
+    const double r_here = r0 - before, r_after = r0 - after;
+    uint32_t ew = 0;
+    if (uniform_u32(r_here > 0.0 && r_after > 0.0 ? 1u : 0u)) {
+        ew = uniform_u32((uint32_t)exponent_of((float)r_here));
+        if (ew == es && es == es_end && ew == uniform_u32((uint32_t)exponent_of((float)r_after)))
+            walk = inc; // (one binade for both)
+        else if (ew == uniform_u32((uint32_t)exponent_of((float)r_after)))
+            walk = span_incs(q, (int)ew);
+        else
+            ew = 0;
+    }
+    if (lane_id() == 0)
+        store_group_rec(rec, sum, inc, walk, start, len | (es << kSumExpShift) | (ew << kWalkExpShift));
+}
+
+// Group records of a worker's sorted range (cnt entries from position off of the list kf).
 // kf_lds (optional): the worker's cnt sorted weights in LDS (outside L.sortk's first 16 KB), read instead of kf + off.
-// r0: the estimate of where the walk starts, u * top_p * (the row's total): the groups that r can reach also get their
-// map for the walk, for the epoch guessed from r0 less the mass before the group (0 or less: none).
-// (UNORDERED: the entries are in any order, e.g. a stretch of a row in token order: see span_map)
-template <bool UNORDERED = false>
-__device__ void worker_groups(const uint32_t* kf, uint32_t off, uint32_t cnt, size_t t_at, double mass, const GroupTable& T,
-                              const FinishLds L, const uint32_t* kf_lds = nullptr, double r0 = 0.0)
+// mass: the estimate of the sum above the range; r0: of where the walk starts, u * top_p * (the row's total).
+__device__ void worker_groups(const uint32_t* kf, uint32_t off, uint32_t cnt, GroupRec* rec, double mass, const FinishLds L,
+                              const uint32_t* kf_lds = nullptr, double r0 = 0.0)
 {
     FinishShared& sm = *L.sm;
     const uint32_t tid = threadIdx.x;
     const uint32_t* src = kf_lds ? kf_lds : kf + off; // uniform
-    double* gs = reinterpret_cast<double*>(L.sortk); // [groups] estimate of the sum before each group
-    double* ge = gs + kMaxGroups;                    // [groups] and after it
+    double* gs = reinterpret_cast<double*>(L.sortk); // [groups] their sums
+    double* gb = gs + kMaxGroups;                    // [groups] the estimate of the sum before each
     const uint32_t groups = (cnt + kGroup - 1u) / kGroup;
     if (kf_lds) // uniform: the copy is in place (its writers' barrier), nothing in device memory is waited for
         lds_barrier();
@@ -443,22 +430,17 @@ __device__ void worker_groups(const uint32_t* kf, uint32_t off, uint32_t cnt, si
             gs[g] = s;
     }
     MAKO_STAMP(16);
-    // the sums before and after each group.  Up to a wave's worth of groups, every wave scans them for itself (the
-    // values are those of the workgroup's scan, whose first wave adds them up the same way) and goes on at once.
+    // the sums before each group.  Up to a wave's worth of groups, every wave scans them for itself (the values are those
+    // of the workgroup's scan, whose first wave adds them up the same way) and goes on at once.
     const bool few = groups <= (uint32_t)kWave; // uniform
-    double before_l = 0, after_l = 0; // (few: lane g holds group g's)
+    double before_l = 0; // (few: lane g holds group g's)
     if (few) {
         if (kf_lds)
             lds_barrier();
         else
             __syncthreads();
-        const uint32_t gq = (uint32_t)lane_id();
-        const double v = gq < groups ? gs[gq] : 0.0;
-        const double incl = __ockl_wfscan_add_f64(v, true);
-        if (wave_id() == 0 && gq < groups)
-            T.sum[t_at + gq] = v;
-        before_l = mass + (incl - v);
-        after_l = mass + incl;
+        const double v = (uint32_t)lane_id() < groups ? gs[lane_id()] : 0.0;
+        before_l = mass + (__ockl_wfscan_add_f64(v, true) - v);
     } else {
         __syncthreads();
         for (uint32_t g0 = 0; g0 < groups; g0 += kThreads) {
@@ -466,11 +448,8 @@ __device__ void worker_groups(const uint32_t* kf, uint32_t off, uint32_t cnt, si
             const double v = g < groups ? gs[g] : 0.0;
             double all;
             const double incl = block_incl_scan_f64(v, all, sm.bs);
-            if (g < groups) {
-                T.sum[t_at + g] = v;
-                gs[g] = mass + (incl - v);
-                ge[g] = mass + incl;
-            }
+            if (g < groups)
+                gb[g] = mass + (incl - v);
             mass += all;
         }
         __syncthreads();
@@ -480,33 +459,8 @@ __device__ void worker_groups(const uint32_t* kf, uint32_t off, uint32_t cnt, si
         const uint32_t len = min(kGroup, cnt - g * kGroup);
         float q[4];
         load_span(src, g * kGroup, len, q);
-        const double guess = few ? readlane_f64(before_l, g) : gs[g];
-        const int eg = guess > 0 ? exponent_of((float)guess) : 0;
-        const seqfp::Step32 st = span_map<UNORDERED>(q, len, eg);
-        // the sum is expected to change binade inside the group (or starts at zero): records for its quarters
-        const double at_end = few ? readlane_f64(after_l, g) : ge[g];
-        const bool split4 = uniform_u32((uint32_t)(eg == 0 || exponent_of((float)at_end) != eg)) != 0;
-        if (split4)
-            build_quarters(q, len, guess, T.quarters + (t_at + g) * 4u);
-        // the walk's map, where the walk is expected to pass the group without changing binade in it
-        const double r_here = r0 - guess, r_after = r0 - at_end;
-        const int ew = (r0 > 0.0 && r_after > 0.0) ? exponent_of((float)r_here) : 0;
-        uint4 wrec = make_uint4(0u, 0u, 0u, 0u);
-        if (ew > 0 && uniform_u32((uint32_t)(exponent_of((float)r_after) == ew)) != 0) {
-            const seqfp::Step32 sw = span_map<UNORDERED>(q, len, ew);
-            float q_top = q[0]; // (lane 0: the group's first, largest weight)
-            if constexpr (UNORDERED)
-                q_top = __uint_as_float(__ockl_wfred_max_u32(max(max(__float_as_uint(q[0]), __float_as_uint(q[1])), max(__float_as_uint(q[2]), __float_as_uint(q[3])))));
-            wrec = make_uint4(sw.d0, sw.d1, walk_need(q_top, ew, sw.cmax), (uint32_t)ew);
-        }
-        if (lane_id() == 0) {
-            T.d0[t_at + g] = st.d0;
-            T.d1[t_at + g] = st.d1;
-            T.cmax[t_at + g] = st.cmax;
-            T.start[t_at + g] = off + g * kGroup;
-            T.pack[t_at + g] = len | ((uint32_t)eg << 16) | (split4 ? kHasQuarters : 0u);
-            T.walk[t_at + g] = wrec;
-        }
+        const double before = few ? readlane_f64(before_l, g) : gb[g], sum = gs[g];
+        group_record(q, off + g * kGroup, len, sum, before, before + sum, r0, rec + g);
     }
 }
 
