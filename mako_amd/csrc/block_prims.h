@@ -47,6 +47,14 @@ __device__ __forceinline__ global_ptr<T> as_global(T* p)
 {
     return (global_ptr<T>)p;
 }
+// The same for LDS.
+template <typename T>
+using lds_ptr = __attribute__((address_space(3))) T*;
+template <typename T>
+__device__ __forceinline__ lds_ptr<T> as_lds(T* p)
+{
+    return (lds_ptr<T>)p;
+}
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4))); // (plain vector types: they load from any address space)
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 

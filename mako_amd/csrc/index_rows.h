@@ -31,7 +31,8 @@ static_assert(kIndexMaxVocab / kSliceMax <= kWorkers && kIndexMaxVocab / kIndexB
                   kSliceMax == 4u * kIndexBlock && kIndexBlock == (uint32_t)kWaves * kGroup,
               "a piece's count and last candidate travel in the plan's per-worker words, the blocks' sums in the row's part_sum, a lane each");
 #ifdef MAKO_EMIT_INDEX_KERNELS
-// grid = (ceil(V / 16384), rows); rows of other kinds leave at once.  (VEC: V % 4 == 0 and 16-byte aligned rows, whose
+// grid = (rows rounded up to a multiple of eight, ceil(V / 16384)): workgroups go to the eight XCDs in turn, so that all of
+// these kernels work on a row on the same one; rows of other kinds leave at once.  (VEC: V % 4 == 0 and 16-byte aligned rows, whose
 // logits are loaded four at a time; the layout of a thread's sixteen logits is slice_load.h's either way.)
 template <bool VEC, int KH>
 __global__ __launch_bounds__(kThreads) void index_weights_kernel(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices)
@@ -39,7 +40,9 @@ __global__ __launch_bounds__(kThreads) void index_weights_kernel(mako_sample_des
     extern __shared__ __align__(16) unsigned long long s_dyn64[];
     __shared__ FinishShared sm;
     __shared__ ArgsLds s_args;
-    const uint32_t row = blockIdx.y, piece = blockIdx.x, tid = threadIdx.x;
+    const uint32_t row = blockIdx.x, piece = blockIdx.y, tid = threadIdx.x;
+    if (row >= d_arg.n_rows)
+        return;
     const mako_sampling_params P0 = d_arg.params[row];
     if (classify(P0) != kGeneral) // uniform
         return;
@@ -72,9 +75,8 @@ __global__ __launch_bounds__(kThreads) void index_weights_kernel(mako_sample_des
     load_penalised<VEC, KH>(d, row, lo, hi, kSliceMax, P, hl, pen, reinterpret_cast<uint32_t*>(s_dyn64), wv);
     const float inv_t = 1.0f / P.temperature;
     const float floor_q = (1.0f < P.min_p) ? 1.0f : P.min_p;
-    // (~bits(q) into the row's list, or bits(q) into the whole-row path's array)
-    uint32_t* key0 = in_order ? sc.key[0] + (size_t)row * sc.vpad : reinterpret_cast<uint32_t*>(sc.wbuf + (size_t)row * sc.vpad);
-    const uint32_t flip = in_order ? ~0u : 0u;
+    // (~bits(q), at the token's own position)
+    uint32_t* key0 = sc.key[0] + (size_t)row * sc.vpad;
     MAKO_CHECK(sc, kCheckStage, (uint64_t)hi <= sc.vpad);
     uint32_t cnt = 0, last = 0;
     double bsum[4];
@@ -96,30 +98,24 @@ __global__ __launch_bounds__(kThreads) void index_weights_kernel(mako_sample_des
                 bsum[b] += ok ? (double)q : 0.0;
             }
             if (VEC && base + 3u < hi) {
-                *reinterpret_cast<uint4*>(key0 + base) = make_uint4(k[0] ^ flip, k[1] ^ flip, k[2] ^ flip, k[3] ^ flip);
+                *reinterpret_cast<uint4*>(key0 + base) = make_uint4(~k[0], ~k[1], ~k[2], ~k[3]);
             } else {
 #pragma unroll
                 for (uint32_t c = 0; c < 4; ++c)
                     if (elem_index<VEC>(lo, tid, 4u * b + c) < hi)
-                        key0[elem_index<VEC>(lo, tid, 4u * b + c)] = k[c] ^ flip;
+                        key0[elem_index<VEC>(lo, tid, 4u * b + c)] = ~k[c];
             }
-            if (VEC && !in_order) { // uniform
-                // the whole-row path's list as well, (~bits(q), token) at the token's position: it is the row's list
-                // of candidates when every logit turns out to be one, as the pieces' counts will tell.  (Not from
-                // the instances for rows that are loaded a logit at a time: they would need more registers than
-                // two workgroups on a CU have.)
-                uint32_t* lk = sc.key[0] + (size_t)row * sc.vpad;
+            if (!in_order) { // uniform
+                // the token ids as well: with them this is the whole-row path's list of candidates when every logit turns out
+                // to be one, as the pieces' counts will tell
                 uint32_t* li = sc.idx[0] + (size_t)row * sc.vpad;
-                if (base + 3u < hi) {
-                    *reinterpret_cast<uint4*>(lk + base) = make_uint4(~k[0], ~k[1], ~k[2], ~k[3]);
+                if (VEC && base + 3u < hi) {
                     *reinterpret_cast<uint4*>(li + base) = make_uint4(base, base + 1u, base + 2u, base + 3u);
                 } else {
 #pragma unroll
                     for (uint32_t c = 0; c < 4; ++c)
-                        if (base + c < hi) {
-                            lk[base + c] = ~k[c];
-                            li[base + c] = base + c;
-                        }
+                        if (elem_index<VEC>(lo, tid, 4u * b + c) < hi)
+                            li[elem_index<VEC>(lo, tid, 4u * b + c)] = elem_index<VEC>(lo, tid, 4u * b + c);
                 }
             }
         }
@@ -166,12 +162,12 @@ __global__ __launch_bounds__(kThreads) void index_weights_kernel(mako_sample_des
             plan->flag = kIndexClaimed;
             plan->m = m;
             plan->argidx = argidx;
-            plan->n0 = VEC && !in_order ? kIndexListed : 0u;
+            plan->n0 = 0u;
         }
     }
 }
 
-// grid = (ceil(V / (4096 GPW)), rows): workgroup p leaves the records of the groups of its 4096 GPW entries.  Wave w
+// grid = (rows rounded up to a multiple of eight, ceil(V / (4096 GPW))): workgroup p leaves the records of the groups of its 4096 GPW entries.  Wave w
 // takes the groups w, w + 16, ... (GPW of them): their entries in one trip to memory, their fp64 sums to LDS, and once
 // every wave has the sums before each group, the maps from the entries it still holds.  (GPW = 4 where there are rows
 // enough to fill the chip, 1 on a small batch, which waits for one workgroup's chain of dependent steps.)
@@ -180,7 +176,9 @@ __global__ __launch_bounds__(kThreads) void index_groups_kernel(mako_sample_desc
 {
     __shared__ double s_gs[kWave];
     constexpr uint32_t kSpan = kIndexBlock * GPW; // entries per workgroup
-    const uint32_t row = blockIdx.y, p = blockIdx.x, tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+    const uint32_t row = blockIdx.x, p = blockIdx.y, tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+    if (row >= d_arg.n_rows)
+        return;
     const mako_sampling_params P0 = d_arg.params[row];
     if (!index_order_row(P0)) // uniform
         return;
@@ -283,7 +281,7 @@ __global__ __launch_bounds__(kThreads) void index_tail_kernel(mako_sample_desc d
         uint32_t counted = 0;
         for (uint32_t p = 0; p < pieces; ++p)
             counted += sc.plan[row].cursor[p];
-        general_row_from_weights<0>(d, sc, row, s_args.P, argidx, sc.plan[row].n0 == kIndexListed && uniform_u32(counted) == d.n_vocab, L);
+        general_row_from_weights<0>(d, sc, row, s_args.P, m, argidx, uniform_u32(counted) == d.n_vocab, L);
         return;
     }
     if (flag != kIndexReady && flag != kIndexWhole && flag != kIndexEmpty) // (never)

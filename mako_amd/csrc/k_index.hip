@@ -19,7 +19,7 @@ void launch_weights(int kh, dim3 grid, hipStream_t st, const mako_sample_desc& d
 
 void launch_index_weights(bool vec, int kh, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices)
 {
-    const dim3 grid((d.n_vocab + kSliceMax - 1u) / kSliceMax, d.n_rows);
+    const dim3 grid((d.n_rows + 7u) & ~7u, (d.n_vocab + kSliceMax - 1u) / kSliceMax);
     if (vec)
         launch_weights<true>(kh, grid, st, d, sc, slices);
     else
@@ -31,9 +31,9 @@ void launch_index_finish(hipStream_t st, const mako_sample_desc& d, const Scratc
     // (the group records are for rows in token order only: a workgroup per 16 384 entries where the rows fill the chip
     // anyway, per 4 096 on a small batch)
     if (in_order_rows && (uint64_t)d.n_rows * ((d.n_vocab + kSliceMax - 1u) / kSliceMax) >= 256u)
-        hipLaunchKernelGGL(index_groups_kernel<4u>, dim3((d.n_vocab + kSliceMax - 1u) / kSliceMax, d.n_rows), dim3(kThreads), 0, st, d, sc);
+        hipLaunchKernelGGL(index_groups_kernel<4u>, dim3((d.n_rows + 7u) & ~7u, (d.n_vocab + kSliceMax - 1u) / kSliceMax), dim3(kThreads), 0, st, d, sc);
     else if (in_order_rows)
-        hipLaunchKernelGGL(index_groups_kernel<1u>, dim3((d.n_vocab + kIndexBlock - 1u) / kIndexBlock, d.n_rows), dim3(kThreads), 0, st, d, sc);
+        hipLaunchKernelGGL(index_groups_kernel<1u>, dim3((d.n_rows + 7u) & ~7u, (d.n_vocab + kIndexBlock - 1u) / kIndexBlock), dim3(kThreads), 0, st, d, sc);
     hipLaunchKernelGGL(index_tail_kernel, dim3(1, d.n_rows), dim3(kThreads), kTailLds, st, d, sc);
 }
 

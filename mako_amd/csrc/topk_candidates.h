@@ -6,60 +6,12 @@
 
 namespace mako {
 
-// Bitonic sort, descending, of 1024 * ITEMS keys held ITEMS per thread: key[t] is element t * 1024 + tid.
-// Partners 1024 or more apart are other registers of the same thread, partners less than 64 apart are lanes
-// of the same wave (shuffles); only the strides in between go through LDS (two barriers each).
 // (MAKO_TOPK_PART: __attribute__((noinline)) for a translation unit whose top-k code sits inside an out-of-line
 // function: each part then has the register file to itself instead of spilling inside its loops.  No source sets it
 // today: every kernel has its top-k rows in line.)
 #ifndef MAKO_TOPK_PART
 #define MAKO_TOPK_PART
 #endif
-template <int ITEMS>
-__device__ void bitonic_sort_regs(unsigned long long (&key)[ITEMS], unsigned long long* lds)
-{
-    const uint32_t tid = threadIdx.x;
-    for (uint32_t k = 2; k <= 1024u * ITEMS; k <<= 1)
-        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
-            if (j >= 1024u) {
-                // register-to-register stage; every index below is a compile-time constant so that key[]
-                // stays in registers
-#pragma unroll
-                for (uint32_t dj = 1; dj < (uint32_t)ITEMS; dj <<= 1)
-                    if (j == dj * 1024u) {
-#pragma unroll
-                        for (uint32_t t = 0; t < (uint32_t)ITEMS; ++t)
-                            if ((t & dj) == 0) {
-                                const bool desc = ((t * 1024u + tid) & k) == 0;
-                                const unsigned long long a = key[t], b = key[t | dj];
-                                const bool swap = (a < b) == desc;
-                                key[t] = swap ? b : a;
-                                key[t | dj] = swap ? a : b;
-                            }
-                    }
-            } else if (j >= (uint32_t)kWave) {
-#pragma unroll
-                for (uint32_t t = 0; t < (uint32_t)ITEMS; ++t)
-                    lds[t * 1024u + tid] = key[t];
-                __syncthreads();
-#pragma unroll
-                for (uint32_t t = 0; t < (uint32_t)ITEMS; ++t) {
-                    const unsigned long long other = lds[t * 1024u + (tid ^ j)];
-                    const bool keep_max = ((tid & j) == 0) == (((t * 1024u + tid) & k) == 0);
-                    key[t] = keep_max ? (key[t] > other ? key[t] : other) : (key[t] < other ? key[t] : other);
-                }
-                __syncthreads();
-            } else {
-#pragma unroll
-                for (uint32_t t = 0; t < (uint32_t)ITEMS; ++t) {
-                    const unsigned long long other = __shfl_xor(key[t], (int)j);
-                    const bool keep_max = ((tid & j) == 0) == (((t * 1024u + tid) & k) == 0);
-                    key[t] = keep_max ? (key[t] > other ? key[t] : other) : (key[t] < other ? key[t] : other);
-                }
-            }
-        }
-}
-
 // Keys (bits(q) << 32 | ~token id, 0 = not a candidate) of candidates t * 1024 + tid of the row's flattened
 // candidate list (all slices; sm.soff holds the slices' offsets), t < ITEMS.  Positions first, then every load
 // from a clamped position with no branch in between (a branch around each load would make it wait for the one
@@ -152,7 +104,7 @@ __device__ MAKO_TOPK_PART uint32_t sort_candidates(const Scratch& sc, uint32_t r
     const uint32_t tid = threadIdx.x;
     unsigned long long key[ITEMS];
     candidate_keys<ITEMS>(sc, row, slices, n_cands, m, inv_t, floor_q, sm, key);
-    bitonic_sort_regs<ITEMS>(key, L.sortk);
+    bitonic_sort_regs<ITEMS>(key, as_lds(L.sortk));
     uint32_t nv = 0;
 #pragma unroll
     for (uint32_t t = 0; t < (uint32_t)ITEMS; ++t) {

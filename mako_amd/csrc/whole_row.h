@@ -100,6 +100,7 @@ __device__ bool radix_pass(const uint32_t* ksrc, const uint32_t* isrc, uint32_t*
 }
 
 __device__ void sort_segment(uint32_t* k0, uint32_t* i0, uint32_t* k1, uint32_t* i1, uint32_t n, const FinishLds& L);
+__device__ void sort_survivors(uint32_t* k0, uint32_t* i0, uint32_t* k1, uint32_t* i1, uint32_t n, const FinishLds& L);
 
 // libstdc++'s __heap_select(first, nth + 1, last) followed by iter_swap(first, nth) (bits/stl_algo.h:1956-1960,
 // stl_heap.h): where introselect ends up when its depth limit is spent.  The arrangement it leaves is the library's,
@@ -112,10 +113,9 @@ __device__ void sort_segment(uint32_t* k0, uint32_t* i0, uint32_t* k1, uint32_t*
 //    popped in (a sequential sift from the root), the lanes behind it are asked again (the root only ever moves
 //    towards the heavy end, so whoever failed before fails again).
 //  * the heap's first `cache_cap` entries (its upper levels, or all of it) live in LDS while this runs.
-// get / put: the range in device memory or LDS, as introselect_rounds() has it.  cache: room for cache_cap values in
-// LDS (0: the range is in LDS already).  All threads call.
+// get / put: the range in device memory.  cache: room for cache_cap values in LDS.  All threads call.
 template <typename Get, typename Put>
-__device__ void heap_select_rest(Get get, Put put, uint32_t first, uint32_t last, uint32_t nth, unsigned long long* cache,
+__device__ void heap_select_rest(Get get, Put put, uint32_t first, uint32_t last, uint32_t nth, lds_ptr<unsigned long long> cache,
                                  uint32_t cache_cap)
 {
     typedef unsigned long long u64;
@@ -210,191 +210,247 @@ __device__ void heap_select_rest(Get get, Put put, uint32_t first, uint32_t last
 // a cut that the rounds leave behind them is not kept up.  key/idx hold n candidates (~bits(q), token id); `desc` is
 // the order of the 64-bit values key << 32 | idx, all distinct.
 // One round = median of three to the front, then the unguarded Hoare partition of the rest around it.  That
-// partition swaps the t-th entry from the left that belongs right with the t-th entry from the right that belongs
-// left for as long as the former lies before the latter, and cuts behind the entries that belong left: the two
-// position lists come from ballots (wave w owns the w-th sixteenth of the range), the swaps are independent.
-// The depth limit's heap select is heap_select_rest() above; the last insertion sort (at most three entries) is one
-// thread's.
-//
-// introselect_rounds runs the rounds on [first, last) through get(i) / get_key(i) (the high half alone) / put(i, v)
-// until the range is no longer than `until` (3 = to the end, insertion sort included).  lsta / lstb: room for
-// last - first positions each.  cache / cache_cap: LDS for heap_select_rest().  Returns true when nothing is left to
-// do.
-template <typename Get, typename GetKey, typename Put>
-__device__ bool introselect_rounds(Get get, GetKey get_key, Put put, uint32_t& first, uint32_t& last, uint32_t nth, uint32_t& depth,
-                                   uint32_t until, uint32_t* lsta, uint32_t* lstb, FinishShared& sm,
-                                   unsigned long long* cache, uint32_t cache_cap)
+// partition swaps the t-th entry from the left that belongs right ("hole") with the t-th entry from the right that belongs
+// left ("filler") for as long as the former lies before the latter, and cuts behind the entries that belong left.
+// Three ways to make a round, as the range shrinks (nth_element_row()):
+//   in device memory   nth_rounds_memory(): one pass over the keys, sixteen bytes per lane and load, leaves a bit per
+//                      entry in LDS; what changes places goes through LDS block by block;
+//   in registers       nth_rounds_registers(): up to kNthRegs entries, sixteen per thread; what changes places goes through LDS;
+//   by one wave        nth_rounds_wave(): up to kNthWave entries, four per lane, without a barrier.
+// The depth limit's heap select is heap_select_rest() above.
+// (A batch of 32 rows of 12 000 candidates, 40 kept: 81 us with every round in device memory or LDS, two passes over the keys
+// each and through pointers that the compiler could not tell from each other; 60 us now.  64 rows of 129 280, bound by the
+// rounds in device memory of the row with the unluckiest pivots: 240 and 230 us.)
+constexpr uint32_t kNthChunks = 4;                                     // of four entries in a row per thread:
+constexpr uint32_t kNthRegs = kNthChunks * 4u * (uint32_t)kThreads; // what a workgroup takes into registers
+constexpr uint32_t kNthWave = 256;                                     // and one wave
+
+__device__ __forceinline__ uint32_t mask_rank(unsigned long long m)
+{
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+// The median of three and its position (__move_median_to_first(first, first + 1, mid, last - 1)).
+template <typename T>
+__device__ __forceinline__ void median_of_three(T vx, T vy, T vz, uint32_t ix, uint32_t iy, uint32_t iz, T& med, uint32_t& im)
+{
+    const bool xy = vx < vy, yz = vy < vz, xz = vx < vz;
+    im = xy == yz ? iy : (xy == xz ? iz : ix);
+    med = xy == yz ? vy : (xy == xz ? vz : vx);
+}
+
+// Rounds on entries [first, last) in device memory until no more than `until` are left or the depth limit is reached.
+// far: room for n / 32 words of device memory behind which nobody looks (the bits of ranges that LDS has no room for).
+// lds: kTailLds bytes.  All threads call.
+// (A workgroup's four SIMDs look at 256 entries a cycle, one instruction each, and a CU fetches 40 GB/s from the memory
+// behind its L2: a row of 129 280 keys takes it 13 us to read, 0.2 us to give one instruction to.  So the keys are read
+// once a round, a bit per entry is kept in LDS, and the entries that change places are read and written where they lie, block
+// by block, through LDS.  The first round of such a row takes 49 us: the keys 14, what moves 33.)
+__device__ __forceinline__ void nth_rounds_memory(global_ptr<uint32_t> key, global_ptr<uint32_t> idx, uint32_t& first, uint32_t& last, uint32_t nth,
+                                                  uint32_t& depth, uint32_t until, global_ptr<uint32_t> far, lds_ptr<unsigned long long> lds,
+                                                  FinishShared& sm)
 {
     typedef unsigned long long u64;
     const uint32_t tid = threadIdx.x, lane = lane_id(), wave = wave_id();
-    while (last - first > until) {
-        if (depth == 0) {
-            heap_select_rest(get, put, first, last, nth, cache, cache_cap);
-            return true;
-        }
+    static_assert(kGroup == 4u * (uint32_t)kWave, "a block of entries: entry 64 j + l is lane l's j-th");
+    constexpr uint32_t kBlocksMax = (kMaxSlices * kSliceMax) / kGroup + 1u, kBlocksInLds = 2048;
+    static_assert(kBlocksMax <= 4u * (uint32_t)kThreads + 1u && kTailLds >= kBlocksInLds * 36u + 8192u && kTailLds >= (kBlocksMax + 1u) * 4u + 8192u, "");
+    while (last - first > until && depth > 0u) {
         --depth;
-        if (tid == 0) { // __move_median_to_first(first, first + 1, mid, last - 1)
-            const uint32_t ix = first + 1u, iy = first + (last - first) / 2u, iz = last - 1u;
-            const u64 x = get(ix), y = get(iy), z = get(iz), r = get(first); // (one trip to memory)
-            uint32_t im;
+        const uint32_t lo = uniform_u32(first + 1u), end = uniform_u32(last);
+        if (wave == 0) { // (one trip to memory)
+            const uint32_t ix = lo, iy = first + (end - first) / 2u, iz = end - 1u;
+            const uint32_t p = lane == 0 ? ix : (lane == 1 ? iy : (lane == 2 ? iz : first));
+            const uint32_t k = key[p], i = idx[p];
+            auto at = [&](int l) { return ((u64)(uint32_t)__builtin_amdgcn_readlane((int)k, l) << 32) | (u64)(uint32_t)__builtin_amdgcn_readlane((int)i, l); };
             u64 med;
-            if (x < y) {
-                im = y < z ? iy : (x < z ? iz : ix);
-                med = y < z ? y : (x < z ? z : x);
-            } else {
-                im = x < z ? ix : (y < z ? iz : iy);
-                med = x < z ? x : (y < z ? z : y);
+            uint32_t im;
+            median_of_three(at(0), at(1), at(2), ix, iy, iz, med, im);
+            if (lane == 3) {
+                key[im] = k;
+                idx[im] = i;
+                key[first] = (uint32_t)(med >> 32);
+                idx[first] = (uint32_t)med;
+                sm.bs.f64[0] = __longlong_as_double((long long)med); // (the pivot, for everyone)
             }
-            put(first, med);
-            put(im, r);
-            sm.bs.f64[0] = __longlong_as_double((long long)med); // (the pivot, for everyone)
-            sm.bs.bcast = 0;                                     // the pairs that change places, counted below
         }
         __syncthreads();
         const u64 pivot = (u64)__double_as_longlong(sm.bs.f64[0]);
-        // (scalars, like all of a wave's bounds and counts below)
-        const uint32_t lo0 = uniform_u32(first + 1u), last_s = uniform_u32(last), len = last_s - lo0;
-        const uint32_t chunk = ((len + kThreads - 1u) / kThreads) * kWave; // per wave, a multiple of 64
-        const uint32_t beg = uniform_u32(min(last_s, lo0 + wave * chunk)), end = min(last_s, beg + chunk);
-        // entries of the wave's chunk that belong left of the cut
-        // (kTrip loads in flight per lane: a trip costs one round trip to memory, not kTrip; the high halves decide
-        // but for an entry whose weight is the pivot's; one workgroup's instruction issue bounds these passes, so they
-        // keep what they can in wave masks: per entry one compare, the masks' scalar arithmetic, and for an entry
-        // that is listed its rank among the mask's lanes)
-        constexpr uint32_t kTrip = 8;
-        const uint32_t pivot_key = uniform_u32((uint32_t)(pivot >> 32));
-        // left[u] / in[u]: the lanes whose entry base + 64 u + lane belongs left / lies in the chunk
-        auto trip_masks = [&](uint32_t base, u64 (&left)[kTrip], u64 (&in)[kTrip]) {
-            uint32_t k[kTrip];
-            u64 ties = 0;
-            if (base + kWave * kTrip <= end) { // (uniform)
-                const size_t at = (size_t)base + lane;
-#pragma unroll
-                for (uint32_t u = 0; u < kTrip; ++u)
-                    k[u] = get_key(at + u * kWave);
-#pragma unroll
-                for (uint32_t u = 0; u < kTrip; ++u) {
-                    in[u] = ~0ull;
-                    left[u] = __builtin_amdgcn_ballot_w64(k[u] < pivot_key);
-                    ties |= __builtin_amdgcn_ballot_w64(k[u] == pivot_key);
-                }
-            } else {
-                // (the chunk's last trip: only its loads that reach into the chunk, which on the short ranges of the
-                // rounds in LDS is one in eight; scalar branches)
-#pragma unroll
-                for (uint32_t u = 0; u < kTrip; ++u) {
-                    k[u] = 0u;
-                    if (base + u * kWave < end)
-                        k[u] = get_key((size_t)min(base + u * kWave + lane, last_s - 1u));
-                }
-#pragma unroll
-                for (uint32_t u = 0; u < kTrip; ++u) {
-                    in[u] = left[u] = 0ull;
-                    if (base + u * kWave < end) {
-                        in[u] = __builtin_amdgcn_ballot_w64(base + u * kWave + lane < end);
-                        left[u] = __builtin_amdgcn_ballot_w64(k[u] < pivot_key) & in[u];
-                        ties |= __builtin_amdgcn_ballot_w64(k[u] == pivot_key) & in[u];
-                    }
-                }
-            }
-            if (ties) { // (rare)
-#pragma unroll
-                for (uint32_t u = 0; u < kTrip; ++u) {
-                    if (!in[u])
-                        continue;
-                    const uint32_t pos = base + u * kWave + lane;
-                    bool l = false;
-                    if (pos < end && k[u] == pivot_key)
-                        l = get(pos) < pivot;
-                    left[u] |= __builtin_amdgcn_ballot_w64(l);
-                }
-            }
-        };
-        auto rank_in = [](u64 m) { return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u)); };
-        uint32_t mine = 0;
-        for (uint32_t base = beg; base < end; base += kWave * kTrip) {
-            u64 left[kTrip], in[kTrip];
-            trip_masks(base, left, in);
+        const uint32_t pivot_key = uniform_u32((uint32_t)(pivot >> 32)), pivot_id = uniform_u32((uint32_t)pivot);
+        // blocks of 256 positions, to the waves in turn
+        const uint32_t b0 = lo / kGroup, n_blocks = (end - 1u) / kGroup + 1u - b0;
+        const bool bits_in_lds = n_blocks <= kBlocksInLds; // uniform
+        // LDS: smalls before each block, the blocks' bits (four words, word j: the entries at 64 j + l), entries on the move
+        const lds_ptr<uint32_t> pre = (lds_ptr<uint32_t>)lds;
+        const lds_ptr<u64> bits = lds + (n_blocks + 2u) / 2u;
+        const global_ptr<u64> bits_far = (global_ptr<u64>)far;
+        const lds_ptr<u64> moving = bits + (bits_in_lds ? n_blocks * 4u : 0u);
+        const uint32_t room = kTailLds / 8u - (n_blocks + 2u) / 2u - (bits_in_lds ? n_blocks * 4u : 0u);
+        constexpr uint32_t kTrip = 8, kFills = 4;
+        for (uint32_t b = wave; b < n_blocks; b += kTrip * (uint32_t)kWaves) {
+            uint32_t k[kTrip][4];
 #pragma unroll
             for (uint32_t u = 0; u < kTrip; ++u)
-                mine += (uint32_t)__popcll(left[u]);
-        }
-        if (lane == 0)
-            sm.bs.u64[wave] = mine;
-        __syncthreads();
-        uint32_t small_before = 0, smalls = 0;
-        for (int w = 0; w < kWaves; ++w) {
-            const uint32_t x = (uint32_t)sm.bs.u64[w];
-            if (w < (int)wave)
-                small_before += x;
-            smalls += x;
-        }
-        small_before = uniform_u32(small_before);
-        smalls = uniform_u32(smalls);
-        const uint32_t cut = lo0 + smalls;
-        // Only the big entries before the cut and the small ones behind it change places, the t-th of the former
-        // with the t-th of the latter counted from the right: as many of one kind as of the other.  When the rounds go
-        // on in the left part (cut > nth), what lies behind the cut is never read again (nth_element's caller keeps the
-        // first nth entries only): the big entries need not be moved there.
-        const bool right_kept = cut <= nth;
-        uint32_t big_before = (beg - lo0) - small_before;
-        // position lists: lsta[t] = the t-th big entry from the left (those before the cut), lstb[t] = the t-th small
-        // entry from the left (those behind it)
-        uint32_t moving = 0; // big entries of the wave's chunk before the cut
-        for (uint32_t base = beg; base < end; base += kWave * kTrip) {
-            u64 left[kTrip], in[kTrip];
-            trip_masks(base, left, in);
-            if (base + kWave * kTrip <= cut) { // (uniform; all but one of the chunks' trips lie on one side of the cut)
 #pragma unroll
-                for (uint32_t u = 0; u < kTrip; ++u) {
-                    if (!in[u]) // (scalar: a trip's part beyond the chunk)
-                        continue;
-                    const u64 big = in[u] & ~left[u];
-                    if ((big >> lane) & 1ull)
-                        lsta[big_before + rank_in(big)] = base + u * kWave + lane;
-                    const uint32_t nb = (uint32_t)__popcll(big);
-                    big_before += nb;
-                    moving += nb;
-                    small_before += (uint32_t)__popcll(left[u]);
-                }
-            } else if (base >= cut) {
+                for (uint32_t j = 0; j < 4; ++j)
+                    k[u][j] = key[(size_t)(b0 + min(b + u * (uint32_t)kWaves, n_blocks - 1u)) * kGroup + (uint32_t)kWave * j + lane];
 #pragma unroll
-                for (uint32_t u = 0; u < kTrip; ++u) {
-                    if (!left[u])
-                        continue;
-                    if ((left[u] >> lane) & 1ull)
-                        lstb[small_before + rank_in(left[u])] = base + u * kWave + lane;
-                    small_before += (uint32_t)__popcll(left[u]);
-                }
-            } else {
+            for (uint32_t u = 0; u < kTrip; ++u) {
+                const uint32_t bb = b + u * (uint32_t)kWaves;
+                if (bb >= n_blocks) // uniform
+                    break;
+                const uint32_t p0 = (b0 + bb) * kGroup;
+                u64 m[4], ties = 0;
 #pragma unroll
-                for (uint32_t u = 0; u < kTrip; ++u) {
-                    if (!in[u])
-                        continue;
-                    const uint32_t pos = base + u * kWave + lane;
-                    const u64 big = in[u] & ~left[u];
-                    const u64 before = __builtin_amdgcn_ballot_w64(pos < cut);
-                    if ((left[u] >> lane) & 1ull) {
-                        if (pos >= cut)
-                            lstb[small_before + rank_in(left[u])] = pos;
-                    } else if (((big >> lane) & 1ull) && pos < cut)
-                        lsta[big_before + rank_in(big)] = pos;
-                    big_before += (uint32_t)__popcll(big);
-                    moving += (uint32_t)__popcll(big & before);
-                    small_before += (uint32_t)__popcll(left[u]);
+                for (uint32_t j = 0; j < 4; ++j) {
+                    m[j] = __builtin_amdgcn_ballot_w64(k[u][j] < pivot_key);
+                    ties |= __builtin_amdgcn_ballot_w64(k[u][j] == pivot_key);
                 }
+                if (p0 < lo || p0 + kGroup > end) { // uniform: the range's first and last block
+#pragma unroll
+                    for (uint32_t j = 0; j < 4; ++j)
+                        m[j] &= __builtin_amdgcn_ballot_w64(p0 + (uint32_t)kWave * j + lane >= lo && p0 + (uint32_t)kWave * j + lane < end);
+                }
+                if (ties) { // (rare: entries of the pivot's weight)
+#pragma unroll
+                    for (uint32_t j = 0; j < 4; ++j) {
+                        const uint32_t p = p0 + (uint32_t)kWave * j + lane;
+                        bool l = false;
+                        if (k[u][j] == pivot_key && p >= lo && p < end)
+                            l = idx[p] < pivot_id;
+                        m[j] |= __builtin_amdgcn_ballot_w64(l);
+                    }
+                }
+                const u64 w = lane == 0 ? m[0] : (lane == 1 ? m[1] : (lane == 2 ? m[2] : m[3]));
+                if (lane < 4) {
+                    if (bits_in_lds) // uniform
+                        bits[bb * 4u + lane] = w;
+                    else
+                        bits_far[bb * 4u + lane] = w;
+                }
+                if (lane == 0)
+                    pre[bb] = (uint32_t)(__popcll(m[0]) + __popcll(m[1]) + __popcll(m[2]) + __popcll(m[3]));
             }
         }
-        if (lane == 0 && moving)
-            atomicAdd(&sm.bs.bcast, (u64)moving);
         __syncthreads();
-        const uint32_t pairs = (uint32_t)sm.bs.bcast;
-        for (uint32_t t = tid; t < pairs; t += kThreads) {
-            const uint32_t a = lsta[t], b = lstb[smalls - 1u - t];
-            const u64 vb = get(b);
-            if (right_kept)
-                put(b, get(a));
-            put(a, vb);
+        // the counts' prefix sums, up to four blocks a thread
+        uint32_t smalls;
+        {
+            uint32_t c[4], mine = 0;
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                c[j] = 4u * tid + j < n_blocks ? pre[4u * tid + j] : 0u;
+                mine += c[j];
+            }
+            uint32_t at = block_excl_scan_u32(mine, smalls, sm.bs);
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j)
+                if (4u * tid + j < n_blocks) {
+                    pre[4u * tid + j] = at;
+                    at += c[j];
+                }
+            if (tid == 0)
+                pre[n_blocks] = smalls;
+        }
+        __syncthreads();
+        smalls = uniform_u32(smalls);
+        const uint32_t cut = lo + smalls, cut_block = cut / kGroup - b0;
+        // When the rounds go on in the left part (cut > nth), what lies behind the cut is never read again (nth_element's
+        // caller keeps the first nth entries only): the holes' entries need not be moved there.
+        const bool right_kept = cut <= nth;
+        auto block_bits = [&](uint32_t b, u64 (&m)[4]) {
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j)
+                m[j] = bits_in_lds ? bits[b * 4u + j] : bits_far[b * 4u + j];
+        };
+        // smalls in front of the cut, of all; so many pairs change places
+        uint32_t before_cut = smalls;
+        if (cut_block < n_blocks) {
+            u64 m[4];
+            block_bits(cut_block, m);
+            before_cut = pre[cut_block];
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j)
+                before_cut += (uint32_t)__popcll(m[j] & __builtin_amdgcn_ballot_w64((b0 + cut_block) * kGroup + (uint32_t)kWave * j + lane < cut));
+        }
+        const uint32_t pairs = uniform_u32(smalls - before_cut);
+        // The fillers (small s of all is the filler of pair smalls - 1 - s) go to LDS, from there to the holes (the entry at p
+        // is the hole of pair (p - lo) - smalls before it): from the range's end on as many blocks at a time as there is
+        // room for the smalls of, up to four a wave, whose loads are in flight together.
+        for (uint32_t t0 = 0, b_hi = n_blocks; t0 < pairs;) {
+            uint32_t b_lo = b_hi - min(b_hi - cut_block, kFills * (uint32_t)kWaves);
+            const uint32_t s_hi = uniform_u32(pre[b_hi]);
+            while (s_hi - uniform_u32(pre[b_lo]) > room)
+                b_lo = b_hi - (b_hi - b_lo) / 2u;
+            const uint32_t s_lo = max(uniform_u32(pre[b_lo]), before_cut), t1 = t0 + (s_hi - s_lo);
+            uint32_t k[kFills][4], i[kFills][4];
+#pragma unroll
+            for (uint32_t u = 0; u < kFills; ++u) {
+                const size_t at = (size_t)(b0 + min(b_lo + wave + u * (uint32_t)kWaves, b_hi - 1u)) * kGroup + lane;
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j) {
+                    k[u][j] = key[at + (uint32_t)kWave * j];
+                    i[u][j] = idx[at + (uint32_t)kWave * j];
+                }
+            }
+            // (turn 1, where the right part is kept: the holes' entries, left in LDS in the fillers' stead, to the fillers)
+            auto fills = [&](bool to_fillers) {
+#pragma unroll
+                for (uint32_t u = 0; u < kFills; ++u) {
+                    const uint32_t b = b_lo + wave + u * (uint32_t)kWaves;
+                    if (b >= b_hi) // uniform
+                        break;
+                    u64 m[4];
+                    block_bits(b, m);
+                    uint32_t s0 = uniform_u32(pre[b]);
+#pragma unroll
+                    for (uint32_t j = 0; j < 4; ++j) {
+                        const uint32_t s = s0 + mask_rank(m[j]);
+                        if (((m[j] >> lane) & 1ull) && s >= s_lo) { // (all but those in front of the cut in its block)
+                            if (!to_fillers) {
+                                moving[s_hi - 1u - s] = ((u64)k[u][j] << 32) | (u64)i[u][j];
+                            } else {
+                                const u64 v = moving[s_hi - 1u - s];
+                                const uint32_t p = (b0 + b) * kGroup + (uint32_t)kWave * j + lane;
+                                key[p] = (uint32_t)(v >> 32);
+                                idx[p] = (uint32_t)v;
+                            }
+                        }
+                        s0 += (uint32_t)__popcll(m[j]);
+                    }
+                }
+            };
+            fills(false);
+            lds_barrier();
+            for (uint32_t b = wave; b <= min(cut_block, n_blocks - 1u); b += (uint32_t)kWaves) {
+                const uint32_t p0 = (b0 + b) * kGroup, s0 = uniform_u32(pre[b]);
+                // holes before the block, and before the next
+                const uint32_t h0 = max(p0, lo) - lo - s0, h1 = p0 + kGroup - lo - uniform_u32(pre[b + 1u]);
+                if (h1 <= t0 || h0 >= t1) // uniform
+                    continue;
+                u64 m[4];
+                block_bits(b, m);
+                uint32_t s = s0;
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j) {
+                    const uint32_t p = p0 + (uint32_t)kWave * j + lane, t = p - lo - (s + mask_rank(m[j]));
+                    if (!((m[j] >> lane) & 1ull) && p >= lo && p < cut && t >= t0 && t < t1) {
+                        const u64 v = moving[t - t0];
+                        if (right_kept)
+                            moving[t - t0] = ((u64)key[p] << 32) | (u64)idx[p];
+                        key[p] = (uint32_t)(v >> 32);
+                        idx[p] = (uint32_t)v;
+                    }
+                    s += (uint32_t)__popcll(m[j]);
+                }
+            }
+            lds_barrier();
+            if (right_kept) { // uniform
+                fills(true);
+                lds_barrier();
+            }
+            t0 = t1;
+            b_hi = b_lo;
         }
         __syncthreads();
         if (right_kept)
@@ -402,62 +458,299 @@ __device__ bool introselect_rounds(Get get, GetKey get_key, Put put, uint32_t& f
         else
             last = cut;
     }
-    if (last - first > 3u)
-        return false;
-    if (tid == 0) // __insertion_sort(first, last)
-        for (uint32_t i = first + 1u; i < last; ++i) {
-            const u64 v = get(i);
-            uint32_t j = i;
-            if (v < get(first)) {
-                for (; j > first; --j)
-                    put(j, get(j - 1u));
-            } else {
-                for (; v < get(j - 1u); --j)
-                    put(j, get(j - 1u));
-            }
-            put(j, v);
-        }
-    __syncthreads();
-    return true;
 }
 
-// The row's candidates in device memory (key[i], idx[i]; lsta / lstb: room for n positions each).  The rounds run on
-// device memory, ten or so dependent trips to memory each, until the range fits the dynamic LDS block (kSortMax
-// entries and two position lists); the remaining dozen rounds run on a copy there.
-__device__ void nth_element_row(uint32_t* key, uint32_t* idx, uint32_t n, uint32_t nth, uint32_t* lsta, uint32_t* lstb,
-                                const FinishLds& L)
+// Rounds on at most kNthRegs entries in registers: position origin + 4096 c + 4 tid + j is x[c][j] (first, last, nth and the
+// positions here: less origin).  buf: kNthRegs / 2 values in LDS.  All threads call.
+__device__ __forceinline__ void nth_rounds_registers(unsigned long long (&x)[kNthChunks][4], uint32_t& first, uint32_t& last, uint32_t nth, uint32_t& depth,
+                                                     uint32_t until, lds_ptr<unsigned long long> buf, FinishShared& sm)
+{
+    typedef unsigned long long u64;
+    const uint32_t tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+    constexpr uint32_t kChunk = 4u * (uint32_t)kThreads;
+    const lds_ptr<u64> piv = as_lds(sm.bs.u64);   // [4]
+    const lds_ptr<uint32_t> cnt = as_lds(sm.hist); // [kNthChunks][kWaves]
+    while (last - first > until && depth > 0u) {
+        --depth;
+        first = uniform_u32(first);
+        last = uniform_u32(last);
+        const uint32_t ps[4] = {first + 1u, first + (last - first) / 2u, last - 1u, first};
+        // (the owners of the three, and of the first entry, say what they are)
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i)
+            if (((ps[i] >> 8) & ((uint32_t)kWaves - 1u)) == wave && ((ps[i] >> 2) & 63u) == lane) {
+                const uint32_t j = ps[i] & 3u;
+#pragma unroll
+                for (uint32_t c = 0; c < kNthChunks; ++c)
+                    if (ps[i] / kChunk == c) // uniform
+                        piv[i] = j == 0u ? x[c][0] : (j == 1u ? x[c][1] : (j == 2u ? x[c][2] : x[c][3]));
+            }
+        lds_barrier();
+        const u64 vr = piv[3];
+        u64 med;
+        uint32_t im;
+        median_of_three((u64)piv[0], (u64)piv[1], (u64)piv[2], ps[0], ps[1], ps[2], med, im);
+        const uint32_t lo = first + 1u;
+        uint32_t own = 0; // bit 4 c + j: the entry belongs left
+#pragma unroll
+        for (uint32_t c = 0; c < kNthChunks; ++c) {
+            uint32_t mine = 0;
+            if (c * kChunk < last && (c + 1u) * kChunk > first) { // uniform
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j) {
+                    const uint32_t p = c * kChunk + 4u * tid + j;
+                    x[c][j] = p == im ? vr : (p == first ? med : x[c][j]);
+                    const bool left = p >= lo && p < last && x[c][j] < med;
+                    own |= (left ? 1u : 0u) << (4u * c + j);
+                    mine += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(left));
+                }
+            }
+            if (lane == 0)
+                cnt[c * (uint32_t)kWaves + wave] = mine;
+        }
+        lds_barrier();
+        static_assert(kNthChunks * (uint32_t)kWaves == (uint32_t)kWave, "a count per lane");
+        const uint32_t c_l = cnt[lane], upto = __ockl_wfscan_add_u32(c_l, true);
+        const uint32_t smalls = (uint32_t)__builtin_amdgcn_readlane((int)upto, kWave - 1), cut = lo + smalls;
+        const bool right_kept = cut <= nth;
+        uint32_t place[kNthChunks][4]; // in buf, of what changes places
+#pragma unroll
+        for (uint32_t c = 0; c < kNthChunks; ++c) {
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j)
+                place[c][j] = kNone;
+            if (!(c * kChunk < last && (c + 1u) * kChunk > first)) // uniform
+                continue;
+            uint32_t rank = (uint32_t)__builtin_amdgcn_readlane((int)(upto - c_l), (int)(c * (uint32_t)kWaves + wave));
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                rank += mask_rank(__builtin_amdgcn_ballot_w64((own >> (4u * c + j)) & 1u));
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) { // (rank: entries before the position that belong left)
+                const uint32_t p = c * kChunk + 4u * tid + j;
+                const bool left = (own >> (4u * c + j)) & 1u;
+                if (left && p >= cut) { // the t-th from the right
+                    place[c][j] = smalls - 1u - rank;
+                    buf[place[c][j]] = x[c][j];
+                } else if (!left && p >= lo && p < cut) { // the t-th from the left
+                    place[c][j] = p - lo - rank;
+                }
+                rank += left ? 1u : 0u;
+            }
+        }
+        lds_barrier();
+#pragma unroll
+        for (uint32_t c = 0; c < kNthChunks; ++c)
+            if (c * kChunk < cut && (c + 1u) * kChunk > first) { // uniform
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j)
+                    if (place[c][j] != kNone && c * kChunk + 4u * tid + j < cut) {
+                        const u64 v = buf[place[c][j]];
+                        if (right_kept)
+                            buf[place[c][j]] = x[c][j];
+                        x[c][j] = v;
+                    }
+            }
+        if (right_kept) { // uniform
+            lds_barrier();
+#pragma unroll
+            for (uint32_t c = 0; c < kNthChunks; ++c)
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j)
+                    if (place[c][j] != kNone && c * kChunk + 4u * tid + j >= cut)
+                        x[c][j] = buf[place[c][j]];
+            first = cut;
+        } else {
+            last = cut;
+        }
+    }
+    first = uniform_u32(first);
+    last = uniform_u32(last);
+}
+
+// The last rounds by one wave: entries [f, l) of the len <= kNthWave at `range`, four in a lane's registers (entry
+// 64 j + lane), of which only those of the range are looked at.  tmp: kNthWave values.  Leaves `range` as introselect arranges
+// it; returns false when the depth limit is reached first.  One wave calls.
+// (A round of the whole workgroup takes 2 us on a range this short, most of it barriers and trips through LDS; one of a
+// wave 0.6 us.  From 512 or 1 024 entries on the wave is the slower one, with 50 instructions per 64 entries.)
+__device__ __forceinline__ bool nth_rounds_wave(lds_ptr<unsigned long long> range, uint32_t len, uint32_t& f, uint32_t& l, uint32_t nth,
+                                                uint32_t& depth, lds_ptr<unsigned long long> tmp)
+{
+    typedef unsigned long long u64;
+    constexpr uint32_t kItems = kNthWave / (uint32_t)kWave;
+    const uint32_t lane = lane_id();
+    const lds_ptr<u64> tmp_a = tmp;
+    const lds_ptr<u64> tmp_b = tmp + kNthWave / 2u; // (at most half of the entries change places with the other half)
+    auto lds_turn = []() { // (a wave's LDS operations complete in order: only the compiler has to be told)
+        __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+        __builtin_amdgcn_wave_barrier();
+    };
+    u64 x[kItems];
+#pragma unroll
+    for (uint32_t j = 0; j < kItems; ++j)
+        x[j] = range[min(j * kWave + lane, len - 1u)];
+    f = uniform_u32(f);
+    l = uniform_u32(l);
+    while (l - f > 3u && depth > 0u) {
+        --depth;
+        const uint32_t ix = f + 1u, iy = f + (l - f) / 2u, iz = l - 1u;
+        // (the three and the first entry through LDS: picked out of the registers they would take a chain of moves)
+        const u64 vx = range[ix], vy = range[iy], vz = range[iz], vr = range[f];
+        u64 med;
+        uint32_t im;
+        median_of_three(vx, vy, vz, ix, iy, iz, med, im);
+        im = uniform_u32(im);
+        const uint32_t lo = f + 1u;
+        u64 left[kItems];
+        uint32_t smalls = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < kItems; ++j) {
+            left[j] = 0ull;
+            if (j * kWave < l && (j + 1u) * kWave > f) { // uniform
+                const uint32_t p = j * kWave + lane;
+                x[j] = p == f ? med : (p == im ? vr : x[j]);
+                left[j] = __builtin_amdgcn_ballot_w64(p >= lo && p < l && x[j] < med);
+                smalls += (uint32_t)__popcll(left[j]);
+            }
+        }
+        const uint32_t cut = lo + smalls;
+        uint32_t before = 0; // smalls in front of the register's entries
+#pragma unroll
+        for (uint32_t j = 0; j < kItems; ++j)
+            if (j * kWave < l && (j + 1u) * kWave > f) { // uniform
+                const uint32_t p = j * kWave + lane, s = before + mask_rank(left[j]);
+                const bool is_left = (left[j] >> lane) & 1ull;
+                if (is_left && p >= cut)
+                    tmp_b[smalls - 1u - s] = x[j];
+                if (!is_left && p >= lo && p < cut)
+                    tmp_a[p - lo - s] = x[j];
+                before += (uint32_t)__popcll(left[j]);
+            }
+        lds_turn();
+        before = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < kItems; ++j)
+            if (j * kWave < l && (j + 1u) * kWave > f) { // uniform
+                const uint32_t p = j * kWave + lane, s = before + mask_rank(left[j]);
+                const bool is_left = (left[j] >> lane) & 1ull;
+                if (is_left && p >= cut)
+                    x[j] = tmp_a[smalls - 1u - s];
+                if (!is_left && p >= lo && p < cut)
+                    x[j] = tmp_b[p - lo - s];
+                if (p < l)
+                    range[p] = x[j];
+                before += (uint32_t)__popcll(left[j]);
+            }
+        lds_turn();
+        if (cut <= nth)
+            f = cut;
+        else
+            l = cut;
+    }
+    const bool done = l - f <= 3u;
+    if (done && l > f) { // __insertion_sort: the entries are distinct
+        u64 a = range[f], b = f + 1u < l ? range[f + 1u] : ~0ull, c = f + 2u < l ? range[f + 2u] : ~0ull;
+        auto order = [](u64& lo, u64& hi) {
+            const u64 t = lo < hi ? lo : hi;
+            hi = lo < hi ? hi : lo;
+            lo = t;
+        };
+        order(a, b);
+        order(b, c);
+        order(a, b);
+        lds_turn();
+        range[f] = a; // (every lane the same)
+        if (f + 1u < l)
+            range[f + 1u] = b;
+        if (f + 2u < l)
+            range[f + 2u] = c;
+    }
+    return done;
+}
+
+// The row's candidates in device memory (key[i], idx[i]; far: n / 32 words of it that are free).  All threads call.
+__device__ MAKO_RARE_CALL void nth_element_row(uint32_t* key_p, uint32_t* idx_p, uint32_t n, uint32_t nth, uint32_t* far, const FinishLds& L)
 {
     assume_lds(L);
     typedef unsigned long long u64;
+    FinishShared& sm = *L.sm;
     const uint32_t tid = threadIdx.x;
     if (n == 0 || nth >= n)
         return;
     uint32_t first = 0, last = n;
     uint32_t depth = 2u * (31u - (uint32_t)__clz((int)n));
-    __syncthreads();
+    const global_ptr<uint32_t> key = as_global(key_p), idx = as_global(idx_p);
+    const lds_ptr<u64> lds = as_lds(L.sortk);
     auto get = [=](uint32_t i) { return ((u64)key[i] << 32) | (u64)idx[i]; };
     auto put = [=](uint32_t i, u64 v) {
         key[i] = (uint32_t)(v >> 32);
         idx[i] = (uint32_t)v;
     };
-    // (the rounds in device memory use no LDS of their own: the whole block holds the heap's upper levels if the
-    // depth limit is reached here)
-    if (introselect_rounds(get, [=](size_t i) { return key[i]; }, put, first, last, nth, depth, kSortMax, lsta, lstb, *L.sm, L.sortk,
-                           kDynLds / 8u))
-        return;
-    u64* lds = L.sortk;
-    uint32_t* la = reinterpret_cast<uint32_t*>(L.sortk + kSortMax);
-    uint32_t* lb = la + kSortMax;
-    static_assert(kSortMax * 16u <= kDynLds, "the range and its two position lists fit the dynamic LDS block");
-    const uint32_t base = first, len = last - first;
-    for (uint32_t i = tid; i < len; i += kThreads)
-        lds[i] = get(base + i);
     __syncthreads();
-    introselect_rounds([=](uint32_t i) { return lds[i - base]; }, [=](size_t i) { return (uint32_t)(lds[i - base] >> 32); },
-                       [=](uint32_t i, u64 v) { lds[i - base] = v; }, first, last, nth, depth, 3u, la, lb, *L.sm, nullptr, 0u);
-    for (uint32_t i = tid; i < len; i += kThreads)
-        put(base + i, lds[i]);
-    __syncthreads();
+    MAKO_STAMP(20);
+    nth_rounds_memory(key, idx, first, last, nth, depth, kNthRegs - 4u, as_global(far), lds, sm);
+    MAKO_STAMP(21);
+    first = uniform_u32(first);
+    last = uniform_u32(last);
+    if (last - first <= kNthRegs - 4u) { // uniform
+        const uint32_t origin = first & ~3u, from = first;
+        u64 x[kNthChunks][4];
+#pragma unroll
+        for (uint32_t c = 0; c < kNthChunks; ++c) {
+            // (rows' arrays are a multiple of 1 024 long)
+            const uint32_t p = min(origin + c * 4u * (uint32_t)kThreads + 4u * tid, (last - 1u) & ~3u);
+            const u32x4 k = *(global_ptr<const u32x4>)(key + p), i = *(global_ptr<const u32x4>)(idx + p);
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j)
+                x[c][j] = ((u64)k[j] << 32) | (u64)i[j];
+        }
+        first -= origin;
+        last -= origin;
+        nth_rounds_registers(x, first, last, nth - origin, depth, kNthWave, lds, sm);
+        MAKO_STAMP(22);
+        // what is settled goes back, the rest to one wave's list in LDS, or back too if the depth limit has been reached
+        const uint32_t len = last - first;
+        const bool by_wave = len <= kNthWave; // uniform
+        const lds_ptr<u64> range = lds;       // [kNthWave], and twice as much for the wave's own use
+        lds_barrier(); // (the exchange buffer has been read)
+#pragma unroll
+        for (uint32_t c = 0; c < kNthChunks; ++c)
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                const uint32_t p = c * 4u * (uint32_t)kThreads + 4u * tid + j;
+                if (p + origin >= from && p < (by_wave ? first : last))
+                    put(origin + p, x[c][j]);
+                else if (by_wave && p >= first && p < last)
+                    range[p - first] = x[c][j];
+            }
+        lds_barrier();
+        bool done = false;
+        if (by_wave) { // uniform
+            if (wave_id() == 0) {
+                uint32_t f = 0, l = len, dep = depth;
+                const bool ok = nth_rounds_wave(range, len, f, l, nth - origin - first, dep, range + kNthWave);
+                if (lane_id() == 0) {
+                    sm.bs.u64[0] = ok ? 1u : 0u;
+                    sm.bs.u64[1] = ((u64)f << 32) | (u64)l;
+                }
+            }
+            lds_barrier();
+            done = sm.bs.u64[0] != 0u;
+            if (tid < len)
+                put(origin + first + tid, range[tid]);
+            last = first + (uint32_t)sm.bs.u64[1];
+            first += (uint32_t)(sm.bs.u64[1] >> 32);
+        }
+        first += origin;
+        last += origin;
+        __syncthreads();
+        MAKO_STAMP(23);
+        if (done)
+            return;
+    }
+    // the depth limit
+    heap_select_rest(get, put, first, last, nth, lds, kDynLds / 8u);
 }
 
 // key0 / idx0 <- the row's candidates in index order (~bits(q), token id), from its bits(q) array qb[0 .. V) (bits(q)
@@ -496,21 +789,19 @@ __device__ MAKO_RARE_CALL void compact_candidates(const uint32_t* qb, uint32_t V
 // Common tail of the whole-row paths.  key[0]/idx[0] of the row hold n0 candidates (~bits(q), token id) in index
 // order.  Sorts them by (q desc, idx asc) when top-k or top-p is active, truncates (src/gen/sampler.cpp:39-61)
 // and draws.  `total64` (when have_total) is the fp64 sum of q over all candidates of the row, of which the list
-// may be only the heaviest part; otherwise it is summed from the list.  The row's bits(q) array (sc.wbuf: bits(q) of
-// every candidate at its index, 0 elsewhere) must be in place.
+// may be only the heaviest part; otherwise it is summed from the list.  key0 / idx0: the list, key1 / idx1: a second buffer.
+// qk: the row's bits(q) array (bits(q) of every candidate at its index, 0 elsewhere), wanted for a second look at a cut too
+// close to call; without one (nullptr) such a row is left undone and false is returned.
 // (TOPK_ALONE = false leaves the top-k-without-top-p branch out of the instance inside plan_kernel: that kernel is
 // only launched for batches whose host copy of the parameters shows a top-p on every sampled row, and the branch's
 // registers would be spilled around the top-k rows' fast path, +3.5 us on a 256-row batch.)
 template <bool TOPK_ALONE>
-__device__ void sort_truncate_draw(const mako_sample_desc& d, const Scratch& sc, uint32_t row, const mako_sampling_params& P,
-                                   uint32_t n0, bool have_total, double total64, uint32_t path, const FinishLds& L)
+__device__ bool sort_truncate_draw(const mako_sample_desc& d, uint32_t row, const mako_sampling_params& P, uint32_t* key0, uint32_t* idx0,
+                                   uint32_t* key1, uint32_t* idx1, const uint32_t* qk, uint32_t n0, bool have_total, double total64,
+                                   uint32_t path, const FinishLds& L)
 {
     assume_lds(L);
     FinishShared& sm = *L.sm;
-    uint32_t* key0 = sc.key[0] + (size_t)row * sc.vpad;
-    uint32_t* key1 = sc.key[1] + (size_t)row * sc.vpad;
-    uint32_t* idx0 = sc.idx[0] + (size_t)row * sc.vpad;
-    uint32_t* idx1 = sc.idx[1] + (size_t)row * sc.vpad;
 
     // order by (q desc, idx asc): stable LSD radix sort of ~bits(q), ascending
     const bool topk_active = P.top_k > 0 && P.top_k < n0;
@@ -518,14 +809,13 @@ __device__ void sort_truncate_draw(const mako_sample_desc& d, const Scratch& sc,
     // top-k alone: the survivors stay in the order nth_element leaves them (sampler.cpp:39-43, then :79-83)
     const bool nth_order = TOPK_ALONE && topk_active && !topp_active;
     if (nth_order)
-        nth_element_row(key0, idx0, n0, P.top_k, key1, idx1, L);
+        nth_element_row(key0, idx0, n0, P.top_k, key1, L);
     else if (topk_active) {
         // a top-p follows: the survivors are sorted, so only which candidates they are matters, and `desc` is a total
         // order: nth_element's first top_k entries are the top_k first of the sorted list, in some order.  The
         // partitions and a sort of top_k entries cost a quarter of the sort of all candidates.
-        nth_element_row(key0, idx0, n0, P.top_k, key1, idx1, L);
-        sort_segment(idx0, key0, idx1, key1, P.top_k, L); // (stable sorts: token ids first, then the weights)
-        sort_segment(key0, idx0, key1, idx1, P.top_k, L);
+        nth_element_row(key0, idx0, n0, P.top_k, key1, L);
+        sort_survivors(key0, idx0, key1, idx1, P.top_k, L);
     } else if (topp_active)
         sort_segment(key0, idx0, key1, idx1, n0, L);
     const uint32_t *ks = key0, *is = idx0;
@@ -533,31 +823,32 @@ __device__ void sort_truncate_draw(const mako_sample_desc& d, const Scratch& sc,
     const uint32_t n1 = topk_active ? P.top_k : n0; // sampler.cpp:40-43
     // (sorted_tail's one-wave path for lists of up to kGroup entries adds and walks them in the order given, whatever
     // it is, and without a top-p it cuts nothing: nth_element's survivors take it too)
-    if (nth_order ? (!d.draft && n1 <= kGroup) : (topk_active || topp_active)) {
+    if (nth_order ? n1 <= kGroup : (topk_active || topp_active)) {
         if (sorted_tail(d, row, P, ks, is, n1, have_total, total64, path, L))
-            return;
+            return true;
         // Too close to call (top-p rows only): the reference's total decides, summed in the order its candidates have
         // at that point (sampler.cpp:40-48).
+        if (!qk)
+            return false;
         if (topk_active) {
             // the order nth_element leaves the survivors in: from the candidates in index order again
-            compact_candidates(reinterpret_cast<const uint32_t*>(sc.wbuf + (size_t)row * sc.vpad), d.n_vocab, key0, idx0, sm);
-            nth_element_row(key0, idx0, n0, P.top_k, key1, idx1, L);
+            compact_candidates(qk, d.n_vocab, key0, idx0, sm);
+            nth_element_row(key0, idx0, n0, P.top_k, key1, L);
             total64 = reference_total([=](uint32_t i) { return __uint_as_float(~key0[i]); }, n1, sm);
-            sort_segment(idx0, key0, idx1, key1, n1, L); // (equal weights by token id, as in the list of all candidates)
-            sort_segment(key0, idx0, key1, idx1, n1, L);
+            sort_survivors(key0, idx0, key1, idx1, n1, L); // (equal weights by token id, as in the list of all candidates)
         } else {
             // index order: the row's bits(q) array (the zeros of the logits that are no candidates add nothing)
-            const uint32_t* qk = reinterpret_cast<const uint32_t*>(sc.wbuf + (size_t)row * sc.vpad);
             total64 = reference_total([=](uint32_t i) { return __uint_as_float(qk[i]); }, d.n_vocab, sm);
         }
         sorted_tail_exact(d, row, P, ks, is, n1, total64, path, L);
-        return;
+        return true;
     }
-    // nth_element's order (long lists, verification), or neither top-k nor top-p: the candidates stay in index order
+    // nth_element's order (long lists), or neither top-k nor top-p: the candidates stay in index order
     const uint32_t* kf = ks;
     const uint32_t* jf = is;
     draw_from_list(
         d, row, [=](uint32_t i) { return __uint_as_float(~kf[i]); }, [=](uint32_t i) { return jf[i]; }, n1, path, sm);
+    return true;
 }
 
 // Sorts n (key, id) pairs at (k0, i0) by key ascending, stably, with (k1, i1) as the second buffer; the result
@@ -586,6 +877,92 @@ __device__ void sort_segment(uint32_t* k0, uint32_t* i0, uint32_t* k1, uint32_t*
         }
         __syncthreads();
     }
+}
+
+// Bitonic sort, descending, of 1024 * ITEMS keys held ITEMS per thread: key[t] is element t * 1024 + tid.
+// Partners 1024 or more apart are other registers of the same thread, partners less than 64 apart are lanes
+// of the same wave (shuffles); only the strides in between go through LDS (two barriers each).
+template <int ITEMS>
+__device__ void bitonic_sort_regs(unsigned long long (&key)[ITEMS], lds_ptr<unsigned long long> lds)
+{
+    const uint32_t tid = threadIdx.x;
+    for (uint32_t k = 2; k <= 1024u * ITEMS; k <<= 1)
+        for (uint32_t j = k >> 1; j > 0; j >>= 1) {
+            if (j >= 1024u) {
+                // register-to-register stage; every index below is a compile-time constant so that key[]
+                // stays in registers
+#pragma unroll
+                for (uint32_t dj = 1; dj < (uint32_t)ITEMS; dj <<= 1)
+                    if (j == dj * 1024u) {
+#pragma unroll
+                        for (uint32_t t = 0; t < (uint32_t)ITEMS; ++t)
+                            if ((t & dj) == 0) {
+                                const bool desc = ((t * 1024u + tid) & k) == 0;
+                                const unsigned long long a = key[t], b = key[t | dj];
+                                const bool swap = (a < b) == desc;
+                                key[t] = swap ? b : a;
+                                key[t | dj] = swap ? a : b;
+                            }
+                    }
+            } else if (j >= (uint32_t)kWave) {
+#pragma unroll
+                for (uint32_t t = 0; t < (uint32_t)ITEMS; ++t)
+                    lds[t * 1024u + tid] = key[t];
+                __syncthreads();
+#pragma unroll
+                for (uint32_t t = 0; t < (uint32_t)ITEMS; ++t) {
+                    const unsigned long long other = lds[t * 1024u + (tid ^ j)];
+                    const bool keep_max = ((tid & j) == 0) == (((t * 1024u + tid) & k) == 0);
+                    key[t] = keep_max ? (key[t] > other ? key[t] : other) : (key[t] < other ? key[t] : other);
+                }
+                __syncthreads();
+            } else {
+#pragma unroll
+                for (uint32_t t = 0; t < (uint32_t)ITEMS; ++t) {
+                    const unsigned long long other = __shfl_xor(key[t], (int)j);
+                    const bool keep_max = ((tid & j) == 0) == (((t * 1024u + tid) & k) == 0);
+                    key[t] = keep_max ? (key[t] > other ? key[t] : other) : (key[t] < other ? key[t] : other);
+                }
+            }
+        }
+}
+
+// Sorts n (key, id) pairs in any order at (k0, i0) by key, then id, both ascending; (k1, i1): a second buffer.
+// (Up to 4096 of them in registers, by one bitonic sort of both: 1000 pairs took the radix sorts' eight passes through
+// device memory 60 us.)
+__device__ void sort_survivors(uint32_t* k0, uint32_t* i0, uint32_t* k1, uint32_t* i1, uint32_t n, const FinishLds& L)
+{
+    assume_lds(L);
+    typedef unsigned long long u64;
+    const uint32_t tid = threadIdx.x;
+    if (n > 4096u) { // (stable sorts: ids first, then the keys)
+        sort_segment(i0, k0, i1, k1, n, L);
+        sort_segment(k0, i0, k1, i1, n, L);
+        return;
+    }
+    const global_ptr<uint32_t> k = as_global(k0), i = as_global(i0);
+    __syncthreads();
+    auto sort = [&](auto items) {
+        constexpr int kItems = decltype(items)::value;
+        u64 key[kItems]; // (complements: the sort is a descending one)
+#pragma unroll
+        for (uint32_t t = 0; t < (uint32_t)kItems; ++t) {
+            const uint32_t e = t * kThreads + tid, at = min(e, n - 1u);
+            key[t] = e < n ? ~(((u64)k[at] << 32) | (u64)i[at]) : 0ull;
+        }
+        bitonic_sort_regs<kItems>(key, as_lds(L.sortk));
+#pragma unroll
+        for (uint32_t t = 0; t < (uint32_t)kItems; ++t)
+            if (t * kThreads + tid < n) {
+                k[t * kThreads + tid] = ~(uint32_t)(key[t] >> 32);
+                i[t * kThreads + tid] = ~(uint32_t)key[t];
+            }
+    };
+    if (n <= 1024u)
+        sort(std::integral_constant<int, 1>());
+    else
+        sort(std::integral_constant<int, 4>());
+    __syncthreads();
 }
 
 // Whole-row path: exact for every parameter combination.  One workgroup rebuilds the penalised
@@ -719,123 +1096,103 @@ __device__ MAKO_RARE_CALL void general_row(const mako_sample_desc& d, const Scra
         fallback_row(d, row, argidx);
         return;
     }
-    sort_truncate_draw<SITE == 0>(d, sc, row, P, n0, false, 0.0, MAKO_PATH_GENERAL, L);
+    sort_truncate_draw<SITE == 0>(d, row, P, key0, idx0, sc.key[1] + (size_t)row * sc.vpad, sc.idx[1] + (size_t)row * sc.vpad, qb, n0, false,
+                                  0.0, MAKO_PATH_GENERAL, L);
 }
 
-// The whole-row path for a row whose weights are already in place: sc.wbuf of the row holds bits(q) of every candidate at
-// its index and 0 elsewhere, as general_row()'s first sweep leaves it (index_weights_kernel writes the same array with a
-// workgroup per 16 384 logits instead of one for the row).  Counts and compacts the candidates in index order and goes
-// on like general_row().  All threads call; `argidx`: the row's first maximum, for a row without candidates.
+// The whole-row path for a row whose weights are already in place: key[0] of the row holds ~bits(q) of every candidate at
+// its index and ~0 elsewhere (index_weights_kernel, with a workgroup per 16 384 logits instead of one for the row).  Counts
+// and compacts the candidates in index order into the row's second buffers and goes on like general_row().  All threads
+// call; m, argidx: the row's maximum and where it is first.
 // `listed`: true when that kernel found every logit a candidate (no mask, no floor, no underflow: the usual row) and
-// has left the list itself as well, (~bits(q), i) at i in key[0] / idx[0] of the row: nothing to count or to compact.
+// has left the token ids as well, i at i in idx[0] of the row: the list is there, nothing to count or to compact.
 template <int SITE>
 __device__ MAKO_RARE_CALL void general_row_from_weights(const mako_sample_desc& d, const Scratch& sc, uint32_t row,
-                                                        const mako_sampling_params& P, uint32_t argidx, bool listed,
+                                                        const mako_sampling_params& P, float m, uint32_t argidx, bool listed,
                                                         const FinishLds& L)
 {
     assume_lds(L);
     FinishShared& sm = *L.sm;
     const uint32_t V = d.n_vocab;
-    if (listed) { // uniform
-        sort_truncate_draw<SITE == 0>(d, sc, row, P, V, false, 0.0, MAKO_PATH_GENERAL, L);
-        return;
-    }
-    const uint32_t* qb = reinterpret_cast<const uint32_t*>(sc.wbuf + (size_t)row * sc.vpad);
-    uint32_t* key0 = sc.key[0] + (size_t)row * sc.vpad;
-    uint32_t* idx0 = sc.idx[0] + (size_t)row * sc.vpad;
-    const uint32_t lane = lane_id(), wave = wave_id();
-    // (wave w owns the w-th sixteenth of the row, a multiple of 256 logits, lane l entries 4l..4l+3 of each 256; eight
-    // such blocks' loads are in flight per trip, from clamped addresses and masked afterwards: one round trip to memory
-    // per 2 048 entries of the wave instead of one per 256)
-    const uint32_t chunk = ((V + kThreads * 4u - 1u) / (kThreads * 4u)) * kGroup;
-    const uint32_t beg = min(V, wave * chunk), end = min(V, beg + chunk);
-    const uint32_t last_vec = (uint32_t)sc.vpad - 4u; // (vpad is a multiple of 1024)
-    constexpr uint32_t kTrip = 8;
-    auto load_trip = [&](uint32_t base, uint32_t (&k)[kTrip][4]) {
-        uint4 x[kTrip];
+    uint32_t* k_from = sc.key[0] + (size_t)row * sc.vpad;
+    uint32_t* i_from = sc.idx[0] + (size_t)row * sc.vpad;
+    uint32_t* k_to = sc.key[1] + (size_t)row * sc.vpad;
+    uint32_t* i_to = sc.idx[1] + (size_t)row * sc.vpad;
+    uint32_t n0 = V;
+    if (!listed) { // uniform
+        const global_ptr<const uint32_t> from = as_global(k_from);
+        const global_ptr<uint32_t> kd = as_global(k_to), id = as_global(i_to);
+        const uint32_t lane = lane_id(), wave = wave_id();
+        // (wave w owns the w-th sixteenth of the row, a multiple of 256 logits; of each 256, lane l takes l, l + 64, ...;
+        // eight such blocks' loads are in flight per trip, from clamped addresses and masked afterwards: one round trip to
+        // memory per 2 048 entries of the wave instead of one per 256)
+        const uint32_t chunk = ((V + kThreads * 4u - 1u) / (kThreads * 4u)) * kGroup;
+        const uint32_t beg = uniform_u32(min(V, wave * chunk)), end = uniform_u32(min(V, beg + chunk));
+        constexpr uint32_t kTrip = 8;
+        auto load_trip = [&](uint32_t base, uint32_t (&k)[kTrip][4]) {
 #pragma unroll
-        for (uint32_t u = 0; u < kTrip; ++u)
-            x[u] = *reinterpret_cast<const uint4*>(qb + min(base + u * kGroup + lane * 4u, last_vec));
-#pragma unroll
-        for (uint32_t u = 0; u < kTrip; ++u) {
-            const uint32_t i = base + u * kGroup + lane * 4u;
-            k[u][0] = i < end ? x[u].x : 0u;
-            k[u][1] = i + 1u < end ? x[u].y : 0u;
-            k[u][2] = i + 2u < end ? x[u].z : 0u;
-            k[u][3] = i + 3u < end ? x[u].w : 0u;
-        }
-    };
-    uint32_t mine = 0;
-    for (uint32_t base = beg; base < end; base += kGroup * kTrip) {
-        uint32_t k[kTrip][4];
-        load_trip(base, k);
-#pragma unroll
-        for (uint32_t u = 0; u < kTrip; ++u)
-            mine += (k[u][0] ? 1u : 0u) + (k[u][1] ? 1u : 0u) + (k[u][2] ? 1u : 0u) + (k[u][3] ? 1u : 0u);
-    }
-    mine = __ockl_wfred_add_u32(mine);
-    __syncthreads();
-    if (lane == 0)
-        sm.bs.u64[wave] = mine;
-    __syncthreads();
-    uint32_t n0 = 0, at = 0;
-    for (int w = 0; w < kWaves; ++w) {
-        const uint32_t x = (uint32_t)sm.bs.u64[w];
-        if (w < (int)wave)
-            at += x;
-        n0 += x;
-    }
-    if (n0 == V) {
-        // every logit is a candidate (no mask, no floor, no underflow: the usual row): the list is the array itself,
-        // written four entries per lane and store
-        for (uint32_t base = beg; base < end; base += kGroup * kTrip) {
-            uint32_t k[kTrip][4];
-            load_trip(base, k);
-#pragma unroll
-            for (uint32_t u = 0; u < kTrip; ++u) {
-                const uint32_t i = base + u * kGroup + lane * 4u;
-                if (i + 3u < end) {
-                    *reinterpret_cast<uint4*>(key0 + i) = make_uint4(~k[u][0], ~k[u][1], ~k[u][2], ~k[u][3]);
-                    *reinterpret_cast<uint4*>(idx0 + i) = make_uint4(i, i + 1u, i + 2u, i + 3u);
-                } else {
-#pragma unroll
-                    for (uint32_t j = 0; j < 4; ++j)
-                        if (i + j < end) {
-                            key0[i + j] = ~k[u][j];
-                            idx0[i + j] = i + j;
-                        }
-                }
-            }
-        }
-    } else {
-        for (uint32_t base = beg; base < end; base += kGroup * kTrip) {
-            uint32_t k[kTrip][4];
-            load_trip(base, k);
-#pragma unroll
-            for (uint32_t u = 0; u < kTrip; ++u) {
-                const uint32_t i = base + u * kGroup + lane * 4u;
-                const uint32_t c = (k[u][0] ? 1u : 0u) + (k[u][1] ? 1u : 0u) + (k[u][2] ? 1u : 0u) + (k[u][3] ? 1u : 0u);
-                const uint32_t incl = __ockl_wfscan_add_u32(c, true);
-                uint32_t pos = at + incl - c;
+            for (uint32_t u = 0; u < kTrip; ++u)
 #pragma unroll
                 for (uint32_t j = 0; j < 4; ++j)
-                    if (k[u][j]) {
-                        MAKO_CHECK(sc, kCheckCompact, pos < n0 && (uint64_t)pos < sc.vpad);
-                        key0[pos] = ~k[u][j];
-                        idx0[pos] = i + j;
-                        ++pos;
-                    }
-                at += (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
-            }
+                    k[u][j] = from[min(base + u * kGroup + j * (uint32_t)kWave + lane, V - 1u)];
+#pragma unroll
+            for (uint32_t u = 0; u < kTrip; ++u)
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j)
+                    k[u][j] = base + u * kGroup + j * (uint32_t)kWave + lane < end ? k[u][j] : ~0u;
+        };
+        uint32_t mine = 0;
+        for (uint32_t base = beg; base < end; base += kGroup * kTrip) {
+            uint32_t k[kTrip][4];
+            load_trip(base, k);
+#pragma unroll
+            for (uint32_t u = 0; u < kTrip; ++u)
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j)
+                    mine += (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(k[u][j] != ~0u));
         }
+        __syncthreads();
+        if (lane == 0)
+            sm.bs.u64[wave] = mine;
+        __syncthreads();
+        uint32_t at = 0;
+        n0 = 0;
+        for (int w = 0; w < kWaves; ++w) {
+            const uint32_t x = (uint32_t)sm.bs.u64[w];
+            if (w < (int)wave)
+                at += x;
+            n0 += x;
+        }
+        at = uniform_u32(at);
+        n0 = uniform_u32(n0);
+        for (uint32_t base = beg; base < end; base += kGroup * kTrip) {
+            uint32_t k[kTrip][4];
+            load_trip(base, k);
+#pragma unroll
+            for (uint32_t u = 0; u < kTrip; ++u)
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j) {
+                    const unsigned long long is = __builtin_amdgcn_ballot_w64(k[u][j] != ~0u);
+                    if (k[u][j] != ~0u) {
+                        const uint32_t pos = at + mask_rank(is);
+                        MAKO_CHECK(sc, kCheckCompact, pos < n0 && (uint64_t)pos < sc.vpad);
+                        kd[pos] = k[u][j];
+                        id[pos] = base + u * kGroup + j * (uint32_t)kWave + lane;
+                    }
+                    at += (uint32_t)__popcll(is);
+                }
+        }
+        __syncthreads();
     }
-    __syncthreads();
     if (n0 == 0) {
         fallback_row(d, row, argidx);
         return;
     }
-    sort_truncate_draw<SITE == 0>(d, sc, row, P, n0, false, 0.0, MAKO_PATH_GENERAL, L);
+    if (!sort_truncate_draw<SITE == 0>(d, row, P, listed ? k_from : k_to, listed ? i_from : i_to, listed ? k_to : k_from, listed ? i_to : i_from,
+                                       nullptr, n0, false, 0.0, MAKO_PATH_GENERAL, L)) {
+        __syncthreads();
+        general_row<SITE>(d, sc, row, P, m, argidx, L); // (a cut too close to call: from the logits again)
+    }
 }
-
 
 } // namespace mako
