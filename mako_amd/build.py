@@ -7,7 +7,8 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 # the C ABI, and one translation unit per kernel family (a kernel's register allocation then does not depend on
 # which other kernels exist; they also compile side by side)
-SOURCES = ["mako_sampler.hip", "k_scan.hip", "k_finish.hip", "k_plan_alone.hip", "k_sort.hip", "k_sort_unsorted.hip", "k_tail.hip", "k_tail_unsorted.hip", "k_index.hip"]
+SOURCES = ["mako_sampler.hip", "k_scan.hip", "k_finish.hip", "k_plan_alone.hip", "k_sort.hip", "k_sort_unsorted.hip", "k_tail.hip", "k_tail_unsorted.hip", "k_index.hip",
+           "k_beside_finish.hip", "k_beside_sort.hip", "k_beside_tail.hip"]
 OBJ_DIR = os.path.join(HERE, "csrc", "_obj")
 OUT = os.path.join(HERE, "libmako_sampler.so")
 # the same library with the kernels' index checks compiled in (-DMAKO_CHECKED): for the test that runs the workloads
@@ -41,13 +42,14 @@ SOURCE_FLAGS = {
     "k_tail.hip": ["-DMAKO_TOPK_GENERAL_SITE=0", *RARE_CALLS],
     "k_tail_unsorted.hip": ["-DMAKO_TOPK_GENERAL_SITE=0", *RARE_CALLS],
     "k_index.hip": ["-DMAKO_TOPK_GENERAL_SITE=0", *RARE_CALLS],
+    "k_beside_tail.hip": ["-DMAKO_TOPK_GENERAL_SITE=0", *RARE_CALLS],
     # the whole-row path and the second look at a cut that is too close to call, out of line beside the top-k rows
     "k_plan_alone.hip": RARE_CALLS,
 }
 
 
 # and the checked library with plans that leave shares unsorted which they should not (-DMAKO_RASH_PLANS, only
-# finish_kernel differs): for the test that expects the oracle's results all the same, through rows given up to the
+# the second pass differs): for the test that expects the oracle's results all the same, through rows given up to the
 # whole-row path
 OUT_RASH = os.path.join(HERE, "libmako_sampler_rash.so")
 
@@ -60,7 +62,7 @@ def build(verbose=False, extra=(), jobs=8, checked=False, rash=False):
         extra = (*extra, "-DMAKO_CHECKED=1")
 
     def compile_one(name):
-        mine = rash and name == "k_finish.hip"
+        mine = rash and name in ("k_finish.hip", "k_beside_finish.hip")
         suffix = "_rash.o" if mine else ("_checked.o" if checked or rash else ".o")
         obj = os.path.join(OBJ_DIR, os.path.splitext(name)[0] + suffix)
         if rash and not mine:

@@ -1,7 +1,7 @@
 // Rows that are cut neither to a top-k nor to a nucleus (top_k == 0, top_p >= 1, temperature > 0): the reference adds
-// up and walks the candidates in token order (src/gen/sampler.cpp:29-36, :79-83, :64-72), so nothing is sorted.  With
-// the caller's host copy of the parameters the library knows that a batch has such rows and gives them three launches
-// of their own instead of one workgroup per row on the whole-row path:
+// up and walks the candidates in token order (src/gen/sampler.cpp:29-36, :79-83, :64-72), so nothing is sorted.  A batch that
+// the caller's host copy of the parameters shows to have none but rows of the whole-row class gets three launches for them
+// instead of one workgroup per row on the whole-row path:
 //   index_weights_kernel  a workgroup per 16 384 logits: masks and penalties as everywhere, q = expf((w - m) / T), and
 //                         ~bits(q) (0.0f for a logit that is no candidate) stored at the token's own position (entry i
 //                         of the list is token i: no array of token ids);
@@ -10,13 +10,15 @@
 //                         as sort_kernel's workers leave them for a sorted list;
 //   index_tail_kernel     a workgroup per row: the exact fp32 total and the walk over the group records
 //                         (sorted_tail's planned instance for lists in any order).
+// Where there are, or may be, rows of other kinds beside them, the same work is done in the launches of those (beside_*.h):
+// the weights with finish_kernel's, the groups with sort_kernel's, the rest with tail_kernel's.
 // A logit that is no candidate stays in the list as a weight of 0.0f: adding it changes no sum, and the walk's
 // `r < q` is never true for it.  The list ends behind the row's last candidate, which is where the reference's walk
 // ends when it runs off its list.  Verification works on the same list: the draft's weight is entry `draft`, and a
 // rejected draft is redrawn with that entry taken as 0.0f (sorted_tail's UNORDERED instance).
 // The other rows of the whole-row class (top-k without top-p, top-k beyond the candidate lists) only get their weights
-// here (index_weights_kernel, into the array general_row_from_weights() starts from) and one workgroup each in
-// index_tail_kernel's launch for the rest of the whole-row path.
+// here (into the array general_row_from_weights() starts from) and one workgroup each in the last launch for the rest of the
+// whole-row path.
 #pragma once
 
 #include "sorted_tail.h"
@@ -30,19 +32,13 @@ constexpr uint32_t kIndexMaxVocab = kMaxGroups * kGroup; // the group records of
 static_assert(kIndexMaxVocab / kSliceMax <= kWorkers && kIndexMaxVocab / kIndexBlock <= kMaxSlices && kIndexMaxVocab / kIndexBlock <= (uint32_t)kWave &&
                   kSliceMax == 4u * kIndexBlock && kIndexBlock == (uint32_t)kWaves * kGroup,
               "a piece's count and last candidate travel in the plan's per-worker words, the blocks' sums in the row's part_sum, a lane each");
-#ifdef MAKO_EMIT_INDEX_KERNELS
-// grid = (rows rounded up to a multiple of eight, ceil(V / 16384)): workgroups go to the eight XCDs in turn, so that all of
-// these kernels work on a row on the same one; rows of other kinds leave at once.  (VEC: V % 4 == 0 and 16-byte aligned rows, whose
+// Piece `piece` of row `row`; of a row of another kind nothing.  (VEC: V % 4 == 0 and 16-byte aligned rows, whose
 // logits are loaded four at a time; the layout of a thread's sixteen logits is slice_load.h's either way.)
 template <bool VEC, int KH>
-__global__ __launch_bounds__(kThreads) void index_weights_kernel(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices)
+__device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_arg, const Scratch& sc_val, uint32_t slices, uint32_t row, uint32_t piece,
+                                                    unsigned long long* s_dyn64, FinishShared& sm, ArgsLds& s_args)
 {
-    extern __shared__ __align__(16) unsigned long long s_dyn64[];
-    __shared__ FinishShared sm;
-    __shared__ ArgsLds s_args;
-    const uint32_t row = blockIdx.x, piece = blockIdx.y, tid = threadIdx.x;
-    if (row >= d_arg.n_rows)
-        return;
+    const uint32_t tid = threadIdx.x;
     const mako_sampling_params P0 = d_arg.params[row];
     if (classify(P0) != kGeneral) // uniform
         return;
@@ -167,18 +163,15 @@ __global__ __launch_bounds__(kThreads) void index_weights_kernel(mako_sample_des
     }
 }
 
-// grid = (rows rounded up to a multiple of eight, ceil(V / (4096 GPW))): workgroup p leaves the records of the groups of its 4096 GPW entries.  Wave w
+// Workgroup p of a row leaves the records of the groups of its 4096 GPW entries.  Wave w
 // takes the groups w, w + 16, ... (GPW of them): their entries in one trip to memory, their fp64 sums to LDS, and once
 // every wave has the sums before each group, the maps from the entries it still holds.  (GPW = 4 where there are rows
 // enough to fill the chip, 1 on a small batch, which waits for one workgroup's chain of dependent steps.)
 template <uint32_t GPW>
-__global__ __launch_bounds__(kThreads) void index_groups_kernel(mako_sample_desc d_arg, Scratch sc_val)
+__device__ __forceinline__ void index_groups_block(const mako_sample_desc& d_arg, const Scratch& sc_val, uint32_t row, uint32_t p, double* s_gs)
 {
-    __shared__ double s_gs[kWave];
     constexpr uint32_t kSpan = kIndexBlock * GPW; // entries per workgroup
-    const uint32_t row = blockIdx.x, p = blockIdx.y, tid = threadIdx.x, lane = lane_id(), wave = wave_id();
-    if (row >= d_arg.n_rows)
-        return;
+    const uint32_t tid = threadIdx.x, lane = lane_id(), wave = wave_id();
     const mako_sampling_params P0 = d_arg.params[row];
     if (!index_order_row(P0)) // uniform
         return;
@@ -244,48 +237,31 @@ __global__ __launch_bounds__(kThreads) void index_groups_kernel(mako_sample_desc
     }
 }
 
-// grid = (1, rows).
-__global__ __launch_bounds__(kThreads) void index_tail_kernel(mako_sample_desc d_arg, Scratch sc_val)
+// What these kernels have left of a row of theirs (flag: of its plan, which is zero again behind this), by one workgroup: the
+// rest of the whole-row path, or the total and the draw.  path: MAKO_PATH_* of a row in token order.  All threads call; sm.tab
+// must hold the exp2 table.
+__device__ __forceinline__ void finish_index_row_here(const mako_sample_desc& d, const Scratch& sc, const mako_sampling_params& P, uint32_t row,
+                                                      uint32_t path, const FinishLds& L)
 {
-    extern __shared__ __align__(16) unsigned long long s_dyn64[];
-    __shared__ FinishShared sm;
-    __shared__ ArgsLds s_args;
-    const uint32_t row = blockIdx.y, tid = threadIdx.x;
-    const mako_sampling_params P0 = d_arg.params[row];
-    if (classify(P0) != kGeneral) // uniform
-        return;
-    const bool in_order = index_order_row(P0);
-    const BigPlan* planned = sc_val.plan + row;
-    const uint32_t flag = planned->flag, n0 = min(planned->n0, d_arg.n_vocab), n_cand = planned->thr;
-    const uint32_t groups = min(planned->groups, min(kMaxGroups, sc_val.g_cap));
-    const double total64 = planned->total64;
-    const float m = planned->m;
-    const uint32_t argidx = planned->argidx;
-    MAKO_ROW(row);
-    stage_args(d_arg, sc_val, row, s_args); // (with a barrier: the plan has been read)
-    const mako_sample_desc& d = s_args.d;
-    const Scratch& sc = s_args.sc;
+    const uint32_t tid = threadIdx.x;
+    BigPlan* plan = sc.plan + row;
+    const uint32_t flag = plan->flag, n0 = min(plan->n0, d.n_vocab), n_cand = plan->thr;
+    const uint32_t groups = min(plan->groups, min(kMaxGroups, sc.g_cap));
+    const double total64 = plan->total64;
+    const float m = plan->m;
+    const uint32_t argidx = plan->argidx;
+    // (the pieces' counts of candidates: when every logit is one, index_weights_kernel's list is the row's list)
+    const uint32_t pieces = (d.n_vocab + kSliceMax - 1u) / kSliceMax;
+    const uint32_t counted = __ockl_wfred_add_u32((uint32_t)lane_id() < pieces ? plan->cursor[min((uint32_t)lane_id(), kWorkers - 1u)] : 0u);
+    __syncthreads(); // (the plan has been read)
     if (tid == 0)
-        sc.plan[row].flag = 0;
-    const FinishLds L = finish_lds_views(sm, s_dyn64);
-    if (!in_order) {
+        plan->flag = 0;
+    if (!index_order_row(P)) {
         // the whole-row path from the weights index_weights_kernel left (the group records' kernel has not touched the row)
-        if (flag != kIndexClaimed) // (never)
-            return;
-        __syncthreads();
-        if (tid < 32)
-            sm.tab[tid] = k_exp2_tab[tid];
-        __syncthreads();
-        // (the pieces' counts of candidates: when every logit is one, index_weights_kernel's list is the row's list)
-        const uint32_t pieces = (d.n_vocab + kSliceMax - 1u) / kSliceMax;
-        uint32_t counted = 0;
-        for (uint32_t p = 0; p < pieces; ++p)
-            counted += sc.plan[row].cursor[p];
-        general_row_from_weights<0>(d, sc, row, s_args.P, m, argidx, uniform_u32(counted) == d.n_vocab, L);
+        if (flag == kIndexClaimed)
+            general_row_from_weights<0>(d, sc, row, P, m, argidx, uniform_u32(counted) == d.n_vocab, L);
         return;
     }
-    if (flag != kIndexReady && flag != kIndexWhole && flag != kIndexEmpty) // (never)
-        return;
     if (flag == kIndexEmpty) {
         fallback_row(d, row, argidx);
         return;
@@ -293,8 +269,8 @@ __global__ __launch_bounds__(kThreads) void index_tail_kernel(mako_sample_desc d
     if (flag == kIndexReady) {
         const uint32_t* kf = sc.key[0] + (size_t)row * sc.vpad;
         // (entry i of the list is token i: no array of token ids)
-        const bool done = sorted_tail<true, false, false, false, true>(d, row, s_args.P, kf, nullptr, n0, true, total64, MAKO_PATH_INDEXED, L, false,
-                                                                       0.0f, sc.gt + (size_t)row * sc.g_cap, groups);
+        const bool done = sorted_tail<true, false, false, false, true>(d, row, P, kf, nullptr, n0, true, total64, path, L, false, 0.0f,
+                                                                       sc.gt + (size_t)row * sc.g_cap, groups);
         if (done) {
             // (the list's length counts the gaps; the candidates are what the reference counts)
             if (tid == 0 && d.out_n_cand)
@@ -302,11 +278,73 @@ __global__ __launch_bounds__(kThreads) void index_tail_kernel(mako_sample_desc d
             return;
         }
     }
-    __syncthreads();
-    if (tid < 32)
-        sm.tab[tid] = k_exp2_tab[tid];
-    __syncthreads();
-    general_row<0>(d, sc, row, s_args.P, m, argidx, L);
+    if (flag == kIndexReady || flag == kIndexWhole)
+        general_row<0>(d, sc, row, P, m, argidx, L);
+}
+__device__ MAKO_RARE_CALL void finish_index_row(const mako_sample_desc& d, const Scratch& sc, const mako_sampling_params& P, uint32_t row,
+                                                uint32_t path, const FinishLds& L)
+{
+    assume_lds(L);
+    finish_index_row_here(d, sc, P, row, path, L);
+}
+
+// The row of `rank` among those that want says (kGeneral, or those of them that are in token order).  The same for the whole
+// workgroup.
+template <typename Want>
+__device__ __forceinline__ bool ranked_row(const mako_sample_desc& d, uint32_t rank, Want want, uint32_t& row)
+{
+    for (uint32_t base = 0; base < d.n_rows; base += (uint32_t)kWave) {
+        const uint32_t r = base + (uint32_t)lane_id();
+        const bool is = r < d.n_rows && want(d.params[min(r, d.n_rows - 1u)]);
+        const unsigned long long all = __builtin_amdgcn_ballot_w64(is);
+        const uint32_t n = (uint32_t)__popcll(all);
+        if (rank < n) {
+            const unsigned long long hit = __builtin_amdgcn_ballot_w64(is && mask_rank(all) == rank);
+            row = base + (uint32_t)__ffsll((long long)hit) - 1u;
+            return true;
+        }
+        rank -= n;
+    }
+    return false;
+}
+
+#ifdef MAKO_EMIT_INDEX_KERNELS
+// grid = (rows rounded up to a multiple of eight, ceil(V / 16384)): workgroups go to the eight XCDs in turn, so that all of
+// these kernels work on a row on the same one.
+template <bool VEC, int KH>
+__global__ __launch_bounds__(kThreads) void index_weights_kernel(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices)
+{
+    extern __shared__ __align__(16) unsigned long long s_dyn64[];
+    __shared__ FinishShared sm;
+    __shared__ ArgsLds s_args;
+    if (blockIdx.x < d_arg.n_rows)
+        index_weights_piece<VEC, KH>(d_arg, sc_val, slices, blockIdx.x, blockIdx.y, s_dyn64, sm, s_args);
+}
+
+// grid = (rows rounded up to a multiple of eight, ceil(V / (4096 GPW))).
+template <uint32_t GPW>
+__global__ __launch_bounds__(kThreads) void index_groups_kernel(mako_sample_desc d_arg, Scratch sc_val)
+{
+    __shared__ double s_gs[kWave];
+    if (blockIdx.x < d_arg.n_rows)
+        index_groups_block<GPW>(d_arg, sc_val, blockIdx.x, blockIdx.y, s_gs);
+}
+
+// grid = (1, rows).
+__global__ __launch_bounds__(kThreads) void index_tail_kernel(mako_sample_desc d_arg, Scratch sc_val)
+{
+    extern __shared__ __align__(16) unsigned long long s_dyn64[];
+    __shared__ FinishShared sm;
+    __shared__ ArgsLds s_args;
+    const uint32_t row = blockIdx.y;
+    if (classify(d_arg.params[row]) != kGeneral || sc_val.plan[row].flag == 0u) // uniform (none: its token is forced)
+        return;
+    MAKO_ROW(row);
+    if (threadIdx.x < 32)
+        sm.tab[threadIdx.x] = k_exp2_tab[threadIdx.x];
+    stage_args(d_arg, sc_val, row, s_args);
+    const FinishLds views = finish_lds_views(sm, s_dyn64);
+    finish_index_row_here(s_args.d, s_args.sc, s_args.P, row, MAKO_PATH_INDEXED, views);
 }
 #endif // MAKO_EMIT_INDEX_KERNELS
 

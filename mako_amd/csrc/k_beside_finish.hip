@@ -1,0 +1,53 @@
+// finish_beside_kernel's variants: the second pass over the top_k == 0 rows and the weights of the whole-row class in one launch.
+#define MAKO_EMIT_BESIDE_FINISH
+#include "launch.h"
+#include "sampler_kernels.h"
+
+namespace mako {
+namespace {
+template <bool VEC, int KH, bool UNSORTED>
+void launch_one(uint32_t wgs, uint32_t more, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices)
+{
+    hipLaunchKernelGGL((finish_beside_kernel<VEC, KH, UNSORTED>), dim3(1, wgs + more), dim3(kThreads), kDynLds, st, d, sc, slices, wgs);
+}
+template <bool VEC, bool UNSORTED>
+void launch_vec(int kh, uint32_t wgs, uint32_t more, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices)
+{
+    if (kh == 2)
+        launch_one<VEC, 2, UNSORTED>(wgs, more, st, d, sc, slices);
+    else if (kh == 8)
+        launch_one<VEC, 8, UNSORTED>(wgs, more, st, d, sc, slices);
+    else
+        launch_one<VEC, 0, UNSORTED>(wgs, more, st, d, sc, slices);
+}
+} // namespace
+
+void launch_finish_beside(bool vec, int kh, bool unsorted, uint32_t wgs, uint32_t more, hipStream_t st, const mako_sample_desc& d,
+                          const Scratch& sc, uint32_t slices)
+{
+    if (vec && unsorted)
+        launch_vec<true, true>(kh, wgs, more, st, d, sc, slices);
+    else if (vec)
+        launch_vec<true, false>(kh, wgs, more, st, d, sc, slices);
+    else if (unsorted)
+        launch_vec<false, true>(kh, wgs, more, st, d, sc, slices);
+    else
+        launch_vec<false, false>(kh, wgs, more, st, d, sc, slices);
+}
+
+hipError_t init_beside_finish()
+{
+    const void* kernels[] = {(const void*)finish_beside_kernel<true, 0, false>, (const void*)finish_beside_kernel<false, 0, false>,
+                             (const void*)finish_beside_kernel<true, 2, false>, (const void*)finish_beside_kernel<false, 2, false>,
+                             (const void*)finish_beside_kernel<true, 8, false>, (const void*)finish_beside_kernel<false, 8, false>,
+                             (const void*)finish_beside_kernel<true, 0, true>,  (const void*)finish_beside_kernel<false, 0, true>,
+                             (const void*)finish_beside_kernel<true, 2, true>,  (const void*)finish_beside_kernel<false, 2, true>,
+                             (const void*)finish_beside_kernel<true, 8, true>,  (const void*)finish_beside_kernel<false, 8, true>};
+    for (const void* k : kernels) {
+        const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDynLds);
+        if (e != hipSuccess)
+            return e;
+    }
+    return hipSuccess;
+}
+} // namespace mako

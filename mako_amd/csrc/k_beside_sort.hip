@@ -1,0 +1,24 @@
+// sort_beside_kernel: the wide rows' sort and the group records of the rows in token order in one launch.
+#define MAKO_EMIT_BESIDE_SORT
+#include "launch.h"
+#include "sampler_kernels.h"
+
+namespace mako {
+void launch_sort_beside(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices, uint32_t grid_rows, bool unsorted,
+                        uint32_t more)
+{
+    // (a large batch's lists are sized by the batch's rows: large_batch_lists())
+    const uint32_t x = unsorted ? kSortItemsPerRow : kWorkers, rows = unsorted && grid_rows ? d.n_rows : grid_rows;
+    const dim3 grid(x, rows + (more + x - 1u) / x);
+    if (unsorted)
+        hipLaunchKernelGGL(sort_beside_kernel<true>, grid, dim3(kThreads), kSortLds, st, d, sc, slices, rows);
+    else
+        hipLaunchKernelGGL(sort_beside_kernel<false>, grid, dim3(kThreads), kSortLds, st, d, sc, slices, rows);
+}
+
+hipError_t init_beside_sort()
+{
+    const hipError_t e = hipFuncSetAttribute((const void*)sort_beside_kernel<true>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSortLds);
+    return e != hipSuccess ? e : hipFuncSetAttribute((const void*)sort_beside_kernel<false>, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSortLds);
+}
+} // namespace mako

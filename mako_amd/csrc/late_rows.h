@@ -7,6 +7,7 @@
 #include "sorted_tail.h"
 #include "topk_candidates.h"
 #include "whole_row.h"
+#include "index_rows.h"
 
 namespace mako {
 
@@ -95,15 +96,21 @@ __device__ MAKO_RARE_CALL bool late_plain_row(const mako_sample_desc& d, const S
 
 // What the earlier kernels leave of row `row`, by one workgroup (all threads call; sm.tab must hold the exp2 table):
 // rows whose token is forced, greedy rows, top-k rows, rows for the whole-row path, second looks.
+// BESIDE: the rows that the launches before have begun for index_rows.h are finished here too; index_path: MAKO_PATH_* of
+// those in token order.
+template <bool BESIDE>
 __device__ MAKO_RARE_CALL void finish_late_row(const mako_sample_desc& d, const Scratch& sc, const mako_sampling_params& P,
-                                               uint32_t row, uint32_t slices, const FinishLds& L)
+                                               uint32_t row, uint32_t slices, uint32_t index_path, const FinishLds& L)
 {
     assume_lds(L);
     const RowClass cls = classify(P);
     if ((d.force_token || d.close_token || cls == kGreedy) && late_plain_row(d, sc, cls, row, slices))
         return;
-    if (cls == kGeneral && sc.plan[row].flag == kIndexClaimed) // (a row in token order that the kernels of index_rows.h finish)
-        return;
+    if constexpr (BESIDE)
+        if (cls == kGeneral && sc.plan[row].flag != 0u) { // uniform
+            finish_index_row(d, sc, P, row, index_path, L);
+            return;
+        }
     if (cls == kNucleus) {
         // (the flag is never set for a row whose token is forced: the second pass leaves such a row alone)
         const uint32_t flag = sc.plan[row].flag;

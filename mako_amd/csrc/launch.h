@@ -34,9 +34,20 @@ void launch_plan_alone(hipStream_t st, const mako_sample_desc& d, const Scratch&
 void launch_sort(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices, uint32_t grid_rows, bool unsorted); // (host copy)
 // (tail_kernel: `tail_cap` workgroups for the possible wide rows, then one per row for what is left of every row)
 void launch_tail(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices, uint32_t tail_cap, bool unsorted); // (host copy, by value)
-// the three kernels of the rows whose candidates stay in token order (index_rows.h): the weights (before tail_kernel's
-// launch, which then leaves such rows alone), the group records, the total and the draw (behind it)
+// the three kernels of a batch with none but rows of the whole-row class (index_rows.h): the weights, the group records, the
+// total and the draw
 hipError_t init_index_kernels();
 void launch_index_weights(bool vec, int kh, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices);
 void launch_index_finish(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, bool in_order_rows);
+// finish, sort and tail of a batch where such rows are, or may be, beside others (beside_rows.h): the same launches with
+// `more` workgroups behind their own for those rows; index_path: MAKO_PATH_* of the rows in token order
+hipError_t init_beside_finish();
+hipError_t init_beside_sort();
+hipError_t init_beside_tail();
+void launch_finish_beside(bool vec, int kh, bool unsorted, uint32_t wgs, uint32_t more, hipStream_t st, const mako_sample_desc& d,
+                          const Scratch& sc, uint32_t slices);
+void launch_sort_beside(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices, uint32_t grid_rows, bool unsorted,
+                        uint32_t more);
+void launch_tail_beside(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices, uint32_t tail_cap, bool unsorted,
+                        uint32_t index_path);
 } // namespace mako

@@ -239,6 +239,9 @@ int mako_sampler_create(mako_sampler_ctx** out, int device, uint32_t max_rows, u
     MAKO_HIP(ctx, mako::init_sort_kernels());
     MAKO_HIP(ctx, mako::init_tail_kernels());
     MAKO_HIP(ctx, mako::init_index_kernels());
+    MAKO_HIP(ctx, mako::init_beside_finish());
+    MAKO_HIP(ctx, mako::init_beside_sort());
+    MAKO_HIP(ctx, mako::init_beside_tail());
     return MAKO_OK;
 }
 
@@ -396,18 +399,16 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
     } while (0)
     // which kernels have work: all of them unless the caller's host copy of the parameters says otherwise
     // (any_late: rows that are finished in tail_kernel's launch, after the plan)
-    // (any_index: rows cut neither to a top-k nor to a nucleus, whose candidates stay in token order; known only from
-    // the caller's copy of the parameters, they get the kernels of index_rows.h instead of a workgroup each on the
-    // whole-row path, unless the vocabulary is beyond 262 144)
-    bool any_nucleus = true, any_late = true, any_index = false, only_index = false, any_in_order = false;
-    uint32_t nucleus_rows = d.n_rows;
+    // (index_rows.h: the rows of the whole-row class, unless the vocabulary is beyond 262 144; only_index: the batch has no
+    // others, and they get launches of their own; beside: it has, or may have, and they take part in the others' launches)
+    const bool index_served = d.n_vocab <= mako::kIndexMaxVocab;
+    bool any_nucleus = true, any_late = true, only_index = false, any_in_order = false, beside = index_served;
+    uint32_t nucleus_rows = d.n_rows, index_rows = d.n_rows;
     if (params_host) {
         any_nucleus = any_late = false;
         uint32_t n_nucleus = 0, n_index = 0;
-        const bool index_served = d.n_vocab <= mako::kIndexMaxVocab;
         for (uint32_t r = 0; r < d.n_rows; ++r) {
             const mako::RowClass c = mako::classify(params_host[r]);
-            // (with them every other row of the whole-row class, whose weights the first of those kernels leaves too)
             const bool index_row = index_served && c == mako::kGeneral;
             any_nucleus |= c == mako::kNucleus;
             any_late |= c == mako::kGeneral && !index_row;
@@ -416,13 +417,11 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
             n_nucleus += c == mako::kNucleus;
         }
         nucleus_rows = std::max(n_nucleus, 1u);
-        any_index = n_index != 0;
         only_index = n_index == d.n_rows && !d.force_token && !d.close_token; // (a forced row is written by the late rows' launch)
-        // (rows of other kinds beside them are finished in tail_kernel's launch, which leaves alone what the index
-        // kernels have claimed; plan_kernel would not)
-        any_late |= any_index && !only_index;
+        beside = n_index != 0 && !only_index;
+        index_rows = n_index;
     }
-    const bool launch_sort = any_nucleus || any_late;
+    const bool launch_sort = any_nucleus || any_late || beside;
     // (finish_kernel's grid: scan_kernel, which cuts the second pass up, is told of it)
     const uint32_t finish_wgs = mako::second_pass_grid(d.n_rows, nucleus_rows, ctx->cus);
     // Batches with many top_k == 0 rows leave the shares of their sorted lists that need no order unsorted
@@ -447,20 +446,33 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
     // top_k == 0 rows: planned and handed out by the second pass, sorted, cut and drawn from; the stages talk through
     // kernel boundaries (device-wide fences inside a kernel cost far more on this chip).  A batch without such rows
     // (and without rows for the whole-row path) ends with plan_kernel instead.
-    if (any_index) // (before the launch that finishes late rows: it leaves alone what this one has claimed)
-        MAKO_LAUNCH(mako::launch_index_weights(vec, kh, st, d, sc, slices));
-    if (any_nucleus)
-        MAKO_LAUNCH(mako::launch_finish(vec, kh, unsorted, finish_wgs, st, d, sc, slices));
-    if (!launch_sort && !only_index)
-        MAKO_LAUNCH(mako::launch_plan_alone(st, d, sc, slices));
-    MAKO_MARK(2);
-    if (any_nucleus)
-        MAKO_LAUNCH(mako::launch_sort(st, d, sc, slices, nucleus_rows, unsorted));
-    MAKO_MARK(3);
-    if (launch_sort) // (also finishes every row the kernels before it leave: finish_late_row())
-        MAKO_LAUNCH(mako::launch_tail(st, d, sc, slices, nucleus_rows, unsorted));
-    if (any_index)
-        MAKO_LAUNCH(mako::launch_index_finish(st, d, sc, any_in_order));
+    if (beside) {
+        // (workgroups for the rows of index_rows.h: a round of them at most, each takes several pieces in turn)
+        const uint32_t pieces = (d.n_vocab + mako::kSliceMax - 1u) / mako::kSliceMax, blocks = (d.n_vocab + mako::kIndexBlock - 1u) / mako::kIndexBlock;
+        const uint32_t for_weights = (uint32_t)std::min<uint64_t>((uint64_t)index_rows * pieces, ctx->cus);
+        const uint32_t for_groups = (uint32_t)std::min<uint64_t>((uint64_t)index_rows * blocks, ctx->cus);
+        MAKO_LAUNCH(mako::launch_finish_beside(vec, kh, unsorted, any_nucleus ? finish_wgs : 0u, for_weights, st, d, sc, slices));
+        MAKO_MARK(2);
+        if (any_nucleus || any_in_order || !params_host)
+            MAKO_LAUNCH(mako::launch_sort_beside(st, d, sc, slices, any_nucleus ? nucleus_rows : 0u, unsorted, for_groups));
+        MAKO_MARK(3);
+        MAKO_LAUNCH(mako::launch_tail_beside(st, d, sc, slices, nucleus_rows, unsorted, params_host ? MAKO_PATH_INDEXED : MAKO_PATH_GENERAL));
+    } else {
+        if (only_index)
+            MAKO_LAUNCH(mako::launch_index_weights(vec, kh, st, d, sc, slices));
+        if (any_nucleus)
+            MAKO_LAUNCH(mako::launch_finish(vec, kh, unsorted, finish_wgs, st, d, sc, slices));
+        if (!launch_sort && !only_index)
+            MAKO_LAUNCH(mako::launch_plan_alone(st, d, sc, slices));
+        MAKO_MARK(2);
+        if (any_nucleus)
+            MAKO_LAUNCH(mako::launch_sort(st, d, sc, slices, nucleus_rows, unsorted));
+        MAKO_MARK(3);
+        if (launch_sort) // (also finishes every row the kernels before it leave: finish_late_row())
+            MAKO_LAUNCH(mako::launch_tail(st, d, sc, slices, nucleus_rows, unsorted));
+        if (only_index)
+            MAKO_LAUNCH(mako::launch_index_finish(st, d, sc, any_in_order));
+    }
     MAKO_MARK(4);
 #undef MAKO_MARK
 #undef MAKO_LAUNCH

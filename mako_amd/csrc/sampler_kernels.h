@@ -35,3 +35,4 @@
 #include "late_rows.h"
 #include "tail_kernel.h"
 #include "index_rows.h"
+#include "beside_rows.h"

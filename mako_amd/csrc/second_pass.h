@@ -250,14 +250,11 @@ __device__ void row_pieces(const mako_sample_desc& d, const Scratch& sc, uint32_
 // workgroups are then the first ones dispatched and land evenly on the XCDs, shader engines and CUs, whatever the
 // mix of rows.
 // (UNSORTED: the instance for batches of many such rows, whose plans leave shares unsorted: unsorted_shares.h)
+// (n_wgs: workgroups of the launch that are finish_kernel's)
 template <bool VEC, int KH, bool UNSORTED>
-__global__ __launch_bounds__(kThreads) void finish_kernel(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices)
+__device__ __forceinline__ void finish_body(const mako_sample_desc& d_arg, const Scratch& sc_arg, uint32_t slices, uint32_t n_wgs,
+                                            unsigned long long* s_dyn64, FinishShared& sm, ArgsLds& s_args, CoarsePlan& s_plan)
 {
-    const Scratch& sc_arg = sc_val; // (by value: the cut is one trip to memory away, not two)
-    extern __shared__ __align__(16) unsigned long long s_dyn64[]; // (128-bit LDS operations need the alignment)
-    __shared__ FinishShared sm;
-    __shared__ ArgsLds s_args;
-    __shared__ CoarsePlan s_plan;
 #ifdef MAKO_TIMING_FINISH
     MAKO_WG_TIMER;
 #endif
@@ -265,7 +262,7 @@ __global__ __launch_bounds__(kThreads) void finish_kernel(mako_sample_desc d_arg
     // (each costs most of a microsecond here, and the pass starts with nothing else to do): the rows' parameters
     // for find_piece() and the arguments' copy go out together with the cut, and the row's own parameters are then
     // taken from the lane that loaded them.
-    uint32_t wg = blockIdx.y * gridDim.x + blockIdx.x;
+    uint32_t wg = blockIdx.y;
     const uint32_t tid = threadIdx.x;
     const bool by_lane = d_arg.n_rows <= (uint32_t)kWave; // uniform
     mako_sampling_params P_lane = mako_sampling_params{};
@@ -288,7 +285,7 @@ __global__ __launch_bounds__(kThreads) void finish_kernel(mako_sample_desc d_arg
             return;
     } else {
         const uint32_t per_xcd = (cut.z + 7u) / 8u;
-        if (per_xcd * 8u <= gridDim.x * gridDim.y) {
+        if (per_xcd * 8u <= n_wgs) {
             if ((wg >> 3) >= per_xcd)
                 return;
             wg = (wg & 7u) * per_xcd + (wg >> 3);
@@ -351,6 +348,17 @@ __global__ __launch_bounds__(kThreads) void finish_kernel(mako_sample_desc d_arg
         row_pieces<VEC, KH, true, UNSORTED>(d, sc, row, piece, pieces, n_pieces, piece_len, P, hl, slices, L, s_plan, opaque_first);
     else
         row_pieces<VEC, KH, false, UNSORTED>(d, sc, row, piece, pieces, n_pieces, piece_len, P, hl, slices, L, s_plan, opaque_first);
+}
+
+// (its arguments by value: the cut is one trip to memory away, not two)
+template <bool VEC, int KH, bool UNSORTED>
+__global__ __launch_bounds__(kThreads) void finish_kernel(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices)
+{
+    extern __shared__ __align__(16) unsigned long long s_dyn64[]; // (128-bit LDS operations need the alignment)
+    __shared__ FinishShared sm;
+    __shared__ ArgsLds s_args;
+    __shared__ CoarsePlan s_plan;
+    finish_body<VEC, KH, UNSORTED>(d_arg, sc_val, slices, gridDim.y, s_dyn64, sm, s_args, s_plan);
 }
 
 } // namespace mako

@@ -6,7 +6,6 @@
 
 namespace mako {
 
-#ifdef MAKO_EMIT_SORT_KERNELS // (not templates: defined by the one translation unit that launches them)
 // grid = (kWorkers, rows) workgroups, of which workgroup i serves entry i of the work list.  Worker w sorts the share
 // of the row's weights that the second pass handed it and stores it at its place in the row's sorted list, with
 // the group records tail_kernel works from; worker 0 of a narrow row finishes the row from the candidate lists.
@@ -15,14 +14,12 @@ namespace mako {
 // UNSORTED: the instance for batches whose plans leave shares unsorted (unsorted_shares.h; a translation unit of its own,
 // k_sort_unsorted.hip): it knows the rows' collectors and that an unsorted share is one record.
 template <bool UNSORTED>
-__device__ __forceinline__ void sort_body(const mako_sample_desc& d_arg, const Scratch& sc_val, uint32_t slices)
+__device__ __forceinline__ void sort_body(const mako_sample_desc& d_arg, const Scratch& sc_val, uint32_t slices, unsigned long long* s_dyn64,
+                                          FinishShared& sm, ArgsLds& s_args)
 {
     // (the context's record by value: its first loads, the list's length and this workgroup's entry, go out together
     // and at once; the list has room for every workgroup of the grid)
     const Scratch& sc_arg = sc_val;
-    extern __shared__ __align__(16) unsigned long long s_dyn64[]; // (128-bit LDS operations need the alignment)
-    __shared__ FinishShared sm;
-    __shared__ ArgsLds s_args;
     const uint32_t piece = blockIdx.y * gridDim.x + blockIdx.x, tid = threadIdx.x;
     // A workgroup's time here is a chain of round trips to device memory, and each one left out shortens it by half
     // a microsecond.  Three remain: the work list's entry (with the arguments' copy for LDS), everything of the row's
@@ -223,15 +220,22 @@ __device__ __forceinline__ void sort_body(const mako_sample_desc& d_arg, const S
         MAKO_STAMP(12);
     }
 }
+#ifdef MAKO_EMIT_SORT_KERNELS // (not templates: defined by the one translation unit that launches them)
 #ifdef MAKO_SORT_UNSORTED
 __global__ __launch_bounds__(kThreads) void sort_kernel_unsorted(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices)
 {
-    sort_body<true>(d_arg, sc_val, slices);
+    extern __shared__ __align__(16) unsigned long long s_dyn64[]; // (128-bit LDS operations need the alignment)
+    __shared__ FinishShared sm;
+    __shared__ ArgsLds s_args;
+    sort_body<true>(d_arg, sc_val, slices, s_dyn64, sm, s_args);
 }
 #else
 __global__ __launch_bounds__(kThreads) void sort_kernel(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices)
 {
-    sort_body<false>(d_arg, sc_val, slices);
+    extern __shared__ __align__(16) unsigned long long s_dyn64[]; // (128-bit LDS operations need the alignment)
+    __shared__ FinishShared sm;
+    __shared__ ArgsLds s_args;
+    sort_body<false>(d_arg, sc_val, slices, s_dyn64, sm, s_args);
 }
 #endif
 #endif // MAKO_EMIT_SORT_KERNELS
