@@ -1,0 +1,51 @@
+"""mako_sampler_sample_host() against the call on device pointers: inputs of every size on their way through the staging
+memory (copies of 1 MiB, 16 MiB of pinned memory that is used again), rows apart from each other, histories as pairs."""
+import ctypes
+
+import numpy as np
+import pytest
+
+from mako_amd import api, workloads
+from parity import gpu_rows
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("rows,vocab,apart", [(1, 1, 0), (1, 3, 5), (3, 4099, 0), (2, 131072, 0), (5, 65536, 64), (1, 262145, 0), (33, 140001, 3)])
+@pytest.mark.parametrize("verify", [False, True])
+def test_same_as_the_device_call(rows, vocab, apart, verify):
+    rng = np.random.Generator(np.random.PCG64([rows, vocab]))
+    whole = (rng.standard_normal((rows, vocab + apart)) * 3.0).astype(np.float32)
+    p = api.make_params(rows, 0.8, 40, 0.95)
+    p["repetition_penalty"], p["frequency_penalty"], p["presence_penalty"] = 1.1, 0.2, 0.3
+    p["temperature"][::5] = 0.0
+    n = min(vocab, 300)
+    hist = np.stack([rng.permutation(vocab)[:n] for _ in range(rows)]).astype(np.int32)
+    counts = rng.integers(1, 4, (rows, n)).astype(np.uint32)
+    length = rng.integers(0, n + 1, rows).astype(np.uint32)
+    words = (vocab + 31) // 32
+    mask = rng.integers(0, 1 << 32, (rows, words + 1), dtype=np.uint64).astype(np.uint32)
+    mask[:, 0] |= 1
+    u, u2 = workloads._uniforms(rng, rows), workloads._uniforms(rng, rows)
+    draft = rng.integers(0, vocab, rows).astype(np.int32)
+    tokens, accepted = np.full(rows, -1, np.int32), np.zeros(rows, np.uint8)
+    ctx = api.SamplerContext(max_rows=rows, max_vocab=vocab, max_hist=512)
+
+    def at(a):
+        return ctypes.c_void_p(a.ctypes.data)
+
+    try:
+        for _ in range(2):
+            rc = ctx.lib.mako_sampler_sample_host(
+                ctypes.c_void_p(ctx.ptr), at(whole), vocab + apart, rows, vocab, at(p), at(u), at(mask), words + 1, at(hist), at(counts), n,
+                at(length), at(draft) if verify else None, at(u2) if verify else None, at(accepted) if verify else None, at(tokens))
+            assert rc == api.MAKO_OK, ctx.last_error()
+            w = dict(logits=np.ascontiguousarray(whole[:, :vocab]), params=p, u=u, mask=np.ascontiguousarray(mask[:, :words]), hist=hist,
+                     hist_len=length)
+            g = gpu_rows(ctx, w, hist_counts=counts, draft=draft if verify else None, u2=u2 if verify else None)
+            assert np.array_equal(tokens, g["tokens"])
+            if verify:
+                assert np.array_equal(accepted, g["accepted"])
+            whole[:] = np.roll(whole, 1, axis=1)
+    finally:
+        ctx.close()
