@@ -25,8 +25,8 @@ struct alignas(16) CoarsePlan {
     double mass_all;
     uint32_t count[kWorkers]; // hand-over: this workgroup's entries for each worker
     uint32_t lbase[kWorkers + 1]; // where its run starts in the workgroup's own ordering of what it keeps
-    uint32_t goff[kWorkers];      // entry e of that ordering, if worker w's, goes to goff[w] + e of the row's staging arrays
-    uint32_t lim[kWorkers];       // if e < lim[w] (the share's room allows it)
+    uint2 run[kWorkers]; // entry e of that ordering, if worker w's, goes to run[w].x + e of the row's staging arrays if
+                         // e < run[w].y (the share's room allows it)
     uint32_t flag, thr, n0_est;
     uint32_t opq_mask; // workers whose shares are left unsorted (opaque_guess())
 };

@@ -8,7 +8,7 @@ namespace {
 template <bool VEC, int KH, bool UNSORTED>
 void launch_one(uint32_t wgs, uint32_t more, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices)
 {
-    hipLaunchKernelGGL((finish_beside_kernel<VEC, KH, UNSORTED>), dim3(1, wgs + more), dim3(kThreads), kDynLds, st, d, sc, slices, wgs);
+    hipLaunchKernelGGL((finish_beside_kernel<VEC, KH, UNSORTED>), dim3(1, wgs + more), dim3(kThreads), kFinishLds, st, d, sc, slices, wgs);
 }
 template <bool VEC, bool UNSORTED>
 void launch_vec(int kh, uint32_t wgs, uint32_t more, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices)
@@ -44,7 +44,7 @@ hipError_t init_beside_finish()
                              (const void*)finish_beside_kernel<true, 2, true>,  (const void*)finish_beside_kernel<false, 2, true>,
                              (const void*)finish_beside_kernel<true, 8, true>,  (const void*)finish_beside_kernel<false, 8, true>};
     for (const void* k : kernels) {
-        const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDynLds);
+        const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFinishLds);
         if (e != hipSuccess)
             return e;
     }

@@ -7,7 +7,7 @@ namespace {
 template <bool VEC, int KH, bool UNSORTED>
 void launch_one(uint32_t wgs, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices)
 {
-    hipLaunchKernelGGL((finish_kernel<VEC, KH, UNSORTED>), dim3(1, wgs), dim3(kThreads), kDynLds, st, d, sc, slices);
+    hipLaunchKernelGGL((finish_kernel<VEC, KH, UNSORTED>), dim3(1, wgs), dim3(kThreads), kFinishLds, st, d, sc, slices);
 }
 template <bool VEC, bool UNSORTED>
 void launch_vec(int kh, uint32_t wgs, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices)
@@ -43,7 +43,7 @@ hipError_t init_finish_kernels()
                              (const void*)finish_kernel<true, 2, true>,  (const void*)finish_kernel<false, 2, true>,
                              (const void*)finish_kernel<true, 8, true>,  (const void*)finish_kernel<false, 8, true>};
     for (const void* k : kernels) {
-        const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDynLds);
+        const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kFinishLds);
         if (e != hipSuccess)
             return e;
     }

@@ -103,29 +103,51 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
     // (a piece may be shorter than the sixteen logits per thread: whole blocks past its end are skipped; the test is
     // the same for every thread)
 #pragma unroll
-    for (uint32_t j = 0; j < 16; ++j) {
-        qb[j] = 0u;
-        slot[j] = kNone;
-        if (lo + (VEC ? (j / 4u) * 4096u : j * (uint32_t)kThreads) < hi) {
-            // (the large batches' instance: a wave whose weights all underflow to zero, as those of a peaked row far
-            // below its maximum do, skips the arithmetic that would tell it so; expf_glibc() returns 0 below that bound)
-            float q = 0.0f;
-            if (!UNSORTED || __ballot(!((wv[j] - m) * inv_t < -0x1.9fe368p6f)) != 0ull)
-                q = weight_of(wv[j], m, inv_t, sm.tab);
-            qb[j] = (q >= floor_q && q > 0.0f) ? __float_as_uint(q) : 0u;
-            if (qb[j])
-                sum += (double)q;
-            if (qb[j] >= thr && qb[j]) {
-                // the worker whose range of bits(q) holds the weight (equal weights always meet in one share): the
-                // number of workers whose lower edge lies above it, by bisection over the edges
-                // (the first two steps against edges held in scalar registers, the other three from LDS)
+    for (uint32_t g = 0; g < 16u; g += 4u) {
+#pragma unroll
+        for (uint32_t j = g; j < g + 4u; ++j) {
+            qb[j] = 0u;
+            slot[j] = kNone;
+        }
+        if (lo + (VEC ? (g / 4u) * 4096u : g * (uint32_t)kThreads) < hi) {
+            bool keeps[4];
+#pragma unroll
+            for (uint32_t j = g; j < g + 4u; ++j) {
+                // (the large batches' instance: a wave whose weights all underflow to zero, as those of a peaked row far
+                // below its maximum do, skips the arithmetic that would tell it so; expf_glibc() returns 0 below that bound)
+                float q = 0.0f;
+                if (!UNSORTED || __ballot(!((wv[j] - m) * inv_t < -0x1.9fe368p6f)) != 0ull)
+                    q = weight_of(wv[j], m, inv_t, sm.tab);
+                qb[j] = (q >= floor_q && q > 0.0f) ? __float_as_uint(q) : 0u;
+                sum += qb[j] ? (double)q : 0.0;
+                keeps[j - g] = qb[j] >= thr && qb[j];
+            }
+            // the worker whose range of bits(q) holds the weight (equal weights always meet in one share): the number of
+            // workers whose lower edge lies above it, by bisection over the edges (the first two steps against edges held in
+            // scalar registers, the other three from LDS), and a place among the workgroup's entries for it.
+            // (Four logits side by side: one after the other, each with its own branch, they wait for three reads and an
+            // atomic's answer every time.  A flat row's piece of 16 384: FIN_BEFORE -> FIN_AFTER us.)
+            if (__ballot(keeps[0] || keeps[1] || keeps[2] || keeps[3]) != 0ull) { // uniform
                 static_assert(kWorkers == 32, "five steps");
-                uint32_t w = qb[j] < edge15 ? 16u : 0u;
-                w += qb[j] < (w ? edge23 : edge7) ? 8u : 0u;
+                uint32_t w[4], place[4];
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j) {
+                    w[j] = qb[g + j] < edge15 ? 16u : 0u;
+                    w[j] += qb[g + j] < (w[j] ? edge23 : edge7) ? 8u : 0u;
+                    place[j] = 0u;
+                }
 #pragma unroll
                 for (uint32_t step = 4u; step; step >>= 1)
-                    w += qb[j] < pl.key_lo[w + step - 1u] ? step : 0u;
-                slot[j] = (w << 16) | atomicAdd(&pl.count[w], 1u);
+#pragma unroll
+                    for (uint32_t j = 0; j < 4; ++j)
+                        w[j] += qb[g + j] < pl.key_lo[w[j] + step - 1u] ? step : 0u;
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j)
+                    if (keeps[j])
+                        place[j] = atomicAdd(&pl.count[w[j]], 1u);
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j)
+                    slot[g + j] = keeps[j] ? (w[j] << 16) | place[j] : kNone;
             }
         }
     }
@@ -161,14 +183,15 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
         pl.count[tid] = 0; // (for the workgroup's next piece)
     const global_ptr<uint32_t> kstage = as_global(sc.key[1]) + (size_t)row * sc.vpad;
     const global_ptr<uint32_t> istage = as_global(sc.idx[1]) + (size_t)row * sc.vpad;
-    uint2* buf = reinterpret_cast<uint2*>(L.cnt); // [kSliceMax / 2] (weight, token id)
-    constexpr uint32_t kHalf = kSliceMax / 2u;
+    // (room for all a piece can hold: with half as much, a flat row's pieces, which keep nearly everything, went through
+    // it twice, 2 us more each, and the workgroup has its CU to itself anyway)
+    uint2* buf = reinterpret_cast<uint2*>(L.cnt); // [kSliceMax] (weight, token id)
+    static_assert(kFinishLds >= kSliceMax * sizeof(uint2), "");
     const uint32_t kept = pl.lbase[kWorkers];
-    // (the entries' workers travel beside them, a byte each, in the plan's count arrays, which are done with)
-    static_assert(offsetof(CoarsePlan, incl) == offsetof(CoarsePlan, cnt) + sizeof(uint32_t) * kLogBins && 2u * sizeof(uint32_t) * kLogBins >= kHalf &&
-                      kSliceMax <= 0x10000u && kWorkers <= 256u,
-                  "a byte per buffered entry; an entry's place fits sixteen bits beside its worker");
-    uint8_t* wbuf = reinterpret_cast<uint8_t*>(pl.cnt);
+    // (an entry's worker travels in the upper bits of its token id)
+    constexpr uint32_t kIdBits = 27;
+    static_assert(kMaxSlices * kSliceMax <= 1u << kIdBits && kWorkers <= 1u << (32u - kIdBits) && kSliceMax <= 0x10000u,
+                  "a token id and a worker in a word; an entry's place fits sixteen bits beside its worker");
     // (from here on: worker << 16 | the entry's place in the workgroup's order.  The runs' starts are read for all
     // sixteen at once, kept or not: behind sixteen branches each read would be a wait of its own.)
     {
@@ -183,35 +206,29 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
     }
     bool dropped = false;
     const uint32_t unsorted_mask = UNSORTED ? uniform_u32(pl.opq_mask) : 0u;
-    for (uint32_t from = 0; from < kept; from += kHalf) { // (what fits the buffer at a time: usually everything)
+    if (kept) { // uniform
 #pragma unroll
         for (uint32_t j = 0; j < 16; ++j)
-            if (slot[j] != kNone && (slot[j] & 0xffffu) - from < kHalf) {
-                buf[(slot[j] & 0xffffu) - from] = make_uint2(qb[j], elem_index<VEC>(lo, tid, j));
-                wbuf[(slot[j] & 0xffffu) - from] = (uint8_t)(slot[j] >> 16);
-            }
-        if (from == 0 && tid < kWorkers) { // (wave 0: where each worker's run goes and where its room ends, in the
-                                           // workgroup's order)
+            if (slot[j] != kNone)
+                buf[slot[j] & 0xffffu] = make_uint2(qb[j], elem_index<VEC>(lo, tid, j) | ((slot[j] >> 16) << kIdBits));
+        if (tid < kWorkers) { // (wave 0: where each worker's run goes and where its room ends, in the workgroup's order)
             const uint32_t room = pl.cap[tid];
-            pl.goff[tid] = pl.stage_off[tid] + base_mine - lbase_mine;
-            pl.lim[tid] = lbase_mine + (room > base_mine ? room - base_mine : 0u);
+            pl.run[tid] = make_uint2(pl.stage_off[tid] + base_mine - lbase_mine, lbase_mine + (room > base_mine ? room - base_mine : 0u));
         }
         lds_barrier();
 #pragma unroll 4 // (fully unrolled, the unaligned variants spill dozens of registers for no gain)
-        for (uint32_t t = 0; t < kHalf / kThreads; ++t) {
-            const uint32_t e = from + t * kThreads + tid;
-            if (e < kept) { // (uniform per wave but for the last one)
-                const uint32_t w = wbuf[e - from];
-                if (e < pl.lim[w]) {
-                    const uint2 x = buf[e - from];
-                    MAKO_CHECK(sc, kCheckStage, (uint64_t)(pl.goff[w] + e) < sc.vpad && pl.goff[w] + e >= pl.stage_off[w] &&
-                                                    pl.goff[w] + e < pl.stage_off[w] + pl.cap[w]);
-                    kstage[pl.goff[w] + e] = x.x;
-                    if (!UNSORTED || !((unsorted_mask >> w) & 1u)) // (a share that is only summed has no use for the token ids)
-                        istage[pl.goff[w] + e] = x.y;
-                } else {
-                    dropped = true;
-                }
+        for (uint32_t e = tid; e < kept; e += kThreads) { // (uniform per wave but for the last trip)
+            const uint2 x = buf[e];
+            const uint32_t w = x.y >> kIdBits;
+            const uint2 run = pl.run[w];
+            if (e < run.y) {
+                MAKO_CHECK(sc, kCheckStage, (uint64_t)(run.x + e) < sc.vpad && run.x + e >= pl.stage_off[w] &&
+                                                run.x + e < pl.stage_off[w] + pl.cap[w]);
+                kstage[run.x + e] = x.x;
+                if (!UNSORTED || !((unsorted_mask >> w) & 1u)) // (a share that is only summed has no use for the token ids)
+                    istage[run.x + e] = x.y & ((1u << kIdBits) - 1u);
+            } else {
+                dropped = true;
             }
         }
         lds_barrier();
