@@ -192,21 +192,12 @@ __device__ __forceinline__ bool walk_lanes(const float (&x)[4], uint32_t n, uint
 
 // ---- increments ----------------------------------------------------------------------------------------------------
 //
-// Inside one binade of the running value (seqfp.h) an addend q is rounded to a multiple of the binade's last place U,
-// whatever the value it is added to, unless it is an exact tie.  With R0 the binade's first float, (R0 + q) - R0 is that
-// multiple, as a float; sums of such multiples are exact in fp32 up to 2^24 U, in any order, and anything beyond stays
+// Inside one binade of the running value an addend that is no exact tie adds a multiple of the binade's last place U
+// (seqfp.h's increment()); sums of such multiples are exact in fp32 up to 2^24 U, in any order, and anything beyond stays
 // beyond.  So a span without ties is ONE float, its sum of multiples, the value behind it is S + that sum, and it is the
 // sequential loop's value if (and only if) it still lies in the binade: additions never fall, so that nothing inside the
 // span can have left a binade that its end lies in; and going down, a value that ends above R0 never was at or below R0
 // on the way, nor was it below the next weight (it would have turned negative), so the walk cannot have stopped there.
-
-// Half of the last place of the binade with exponent e, which an exact tie is off its multiple by.  (The lowest binade
-// has no such thing: there every float is a multiple.)
-__device__ __forceinline__ float half_ulp(int e)
-{
-    const uint32_t normal = (uint32_t)(e - 24) << 23, tiny = e >= 2 ? 1u << ((e - 2) & 31) : 0x7fc00000u;
-    return __uint_as_float(e >= 25 ? normal : tiny);
-}
 
 // Inclusive sum over the lanes, for values whose sums are exact.
 __device__ __forceinline__ float wave_scan_add_f32(float v)
@@ -229,19 +220,19 @@ __device__ __forceinline__ float2 span_incs(const float (&q)[4], int e)
     using namespace seqfp;
     if (e <= 0 || e > 200) // uniform (weights are at most 1: no sum of them gets near the upper bound)
         return make_float2(INFINITY, INFINITY);
-    const float R0 = __uint_as_float((uint32_t)e << 23), half = half_ulp(e);
+    const float base = binade_base(e), half = half_ulp(e);
     float t[4];
     bool tie = false;
 #pragma unroll
     for (uint32_t j = 0; j < 4; ++j) {
-        t[j] = (R0 + q[j]) - R0;
-        tie |= fabsf(q[j] - t[j]) == half;
+        t[j] = increment(q[j], base);
+        tie |= is_tie(q[j], t[j], half);
     }
     if (__ballot(tie) == 0ull) {
         const float all = readlane_f32(wave_scan_add_f32(((t[0] + t[1]) + t[2]) + t[3]), kWave - 1);
         return make_float2(all, all);
     }
-    Step32 st = identity32();
+    Step32 st = identity32(); // (ties: not the lowest binade)
 #pragma unroll
     for (uint32_t j = 0; j < 4; ++j)
         st = compose32(st, step32_fp(q[j], e));
@@ -285,8 +276,8 @@ __device__ __forceinline__ SpanEnd span_steps(float (&q_io)[4], float& S_io, uin
     for (uint32_t round = 0;; ++round) {
         const uint32_t ex = uniform_u32((__float_as_uint(S) >> 23) & 0xffu);
         const int e = ex ? (int)ex : 1;
-        const float R0 = __uint_as_float((uint32_t)e << 23), top = R0 + R0, half = half_ulp(e);
-        const float t0 = (R0 + q0) - R0, t1 = (R0 + q1) - R0, t2 = (R0 + q2) - R0, t3 = (R0 + q3) - R0;
+        const float base = seqfp::binade_base(e), top = seqfp::binade_top(e), low = seqfp::binade_low(e), half = seqfp::half_ulp(e);
+        const float t0 = seqfp::increment(q0, base), t1 = seqfp::increment(q1, base), t2 = seqfp::increment(q2, base), t3 = seqfp::increment(q3, base);
         const float p1 = t0 + t1, p2 = p1 + t2, p3 = p2 + t3;
         const float incl = wave_scan_add_f32(p3);
         const float excl = __uint_as_float((uint32_t)__builtin_amdgcn_update_dpp(0, (int)__float_as_uint(incl), 0x138 /* wave_shr:1 */, 0xf, 0xf, false));
@@ -294,8 +285,7 @@ __device__ __forceinline__ SpanEnd span_steps(float (&q_io)[4], float& S_io, uin
         const float before = SUB ? S - excl : S + excl;
         const float a0 = SUB ? before - t0 : before + t0, a1 = SUB ? before - p1 : before + p1;
         const float a2 = SUB ? before - p2 : before + p2, a3 = SUB ? before - p3 : before + p3;
-        const float low = e > 1 ? R0 : -0x1p-149f; // (in the lowest binade the walk may go down to zero)
-        auto event = [&](float a, float q, float t) { return !(SUB ? a > low : a < top) || fabsf(q - t) == half; };
+        auto event = [&](float a, float q, float t) { return !(SUB ? a > low : a < top) || seqfp::is_tie(q, t, half); };
         const bool v0 = event(a0, q0, t0), v1 = event(a1, q1, t1), v2 = event(a2, q2, t2), v3 = event(a3, q3, t3);
         const unsigned long long bal = __ballot(v0 || v1 || v2 || v3);
         if (bal == 0ull) {
@@ -643,7 +633,7 @@ __device__ __forceinline__ bool chain_sum(Keys kf, const GroupLds G, uint32_t gr
         uint32_t done = base == 0u ? lead : 0u;
         while (done < cnt) {
             const uint32_t ex = uniform_u32((__float_as_uint(S) >> 23) & 0xffu), e = ex ? ex : 1u;
-            const float top = __uint_as_float((e + 1u) << 23);
+            const float top = seqfp::binade_top((int)e);
             const bool plain = ((pk_l >> kSumExpShift) & 0xffu) == e && inc_l.x == inc_l.y;
             const float after = S + wave_scan_add_f32(lane < done ? 0.0f : (plain ? inc_l.x : INFINITY));
             const unsigned long long bad = __ballot(lane >= done && lane < cnt && !(after < top));
@@ -693,11 +683,10 @@ __device__ __forceinline__ WalkEnd chain_walk(Keys kf, const GroupLds G, uint32_
         uint32_t done = 0;
         while (done < cnt) {
             const uint32_t ex = uniform_u32((__float_as_uint(r) >> 23) & 0xffu), e = ex ? ex : 1u;
-            const float low = e > 1u ? __uint_as_float(e << 23) : -1.0f; // (in the lowest binade r may go down to zero)
-            auto stays = [&](float x) { return e > 1u ? x > low : x >= 0.0f; };
+            const float low = seqfp::binade_low((int)e);
             const bool plain = ((pk_l >> kWalkExpShift) & 0xffu) == e && inc_l.x == inc_l.y;
             const float after = r - wave_scan_add_f32(lane < done ? 0.0f : (plain ? inc_l.x : INFINITY));
-            const unsigned long long bad = __ballot(lane >= done && lane < cnt && !stays(after));
+            const unsigned long long bad = __ballot(lane >= done && lane < cnt && !(after > low));
             const uint32_t f = bad ? (uint32_t)__ffsll((long long)bad) - 1u : cnt;
             if (f > done)
                 r = readlane_f32(after, f - 1u);
@@ -708,7 +697,7 @@ __device__ __forceinline__ WalkEnd chain_walk(Keys kf, const GroupLds G, uint32_
             const bool for_here = ((pk >> kWalkExpShift) & 0xffu) == e;
             if (for_here) {
                 const float behind = r - ((__float_as_uint(r) & 1u) ? readlane_f32(inc_l.y, f) : readlane_f32(inc_l.x, f));
-                if (__ballot(stays(behind)) != 0ull) {
+                if (__ballot(behind > low) != 0ull) {
                     r = behind;
                     continue;
                 }

@@ -198,6 +198,47 @@ SEQFP_HD long long sub_apply(long long m, float q, int e)
     return m - ((m & 1) ? s.d1 : s.d0);
 }
 
+// ---- increments ------------------------------------------------------------
+//
+// Inside one binade of the running value an addend q is rounded to a multiple of the binade's last place, whatever the value
+// it is added to, unless it is an exact tie.  With R0 the binade's first float, (R0 + q) - R0 is that multiple, as a float.
+// (Right for q < R0, for which R0 + q stays in the binade.  A larger q gives something of at least R0, which no state of the
+// binade can take without leaving it: additions end at or above its top, subtractions below its first float.)
+// The lowest binade holds the subnormals too, and its states start at zero: a q of R0 or more may well stay inside it, where
+// R0 + q would not.  But there every float IS a multiple, nothing is rounded and nothing is a tie: with 0.0f in R0's place
+// the same expression gives q itself.
+
+// What stands in R0's place for the binade with exponent e >= 1.
+SEQFP_HD float binade_base(int e)
+{
+    return e > 1 ? u2f(uint32_t(e) << 23) : 0.0f;
+}
+// The first float above the binade.
+SEQFP_HD float binade_top(int e)
+{
+    return u2f(uint32_t(e + 1) << 23);
+}
+// What a value going down has to stay strictly above: at the binade's first float the last place halves.  (In the lowest
+// binade it does not: a value may go down to zero.)
+SEQFP_HD float binade_low(int e)
+{
+    return e > 1 ? u2f(uint32_t(e) << 23) : -0x1p-149f;
+}
+SEQFP_HD float increment(float q, float base)
+{
+    return (base + q) - base;
+}
+// Half of the last place, which an exact tie is off its multiple by.  (A NaN, off which nothing is, in the lowest binade.)
+SEQFP_HD float half_ulp(int e)
+{
+    const uint32_t normal = uint32_t(e - 24) << 23, tiny = e >= 2 ? 1u << ((e - 2) & 31) : 0x7fc00000u;
+    return u2f(e >= 25 ? normal : tiny);
+}
+SEQFP_HD bool is_tie(float q, float inc, float half)
+{
+    return fabsf(q - inc) == half;
+}
+
 // ---- groups ----------------------------------------------------------------
 //
 // A long sorted list is cut into groups.  The map of a whole group under a GUESSED epoch (taken from an

@@ -287,8 +287,8 @@ __device__ void opaque_share(const uint32_t* ks, uint32_t cnt, uint32_t off, int
     const uint32_t lane = (uint32_t)lane_id();
     const unsigned long long lower = (1ull << lane) - 1ull;
     // (weights and epochs of such a share: the weights lie binades below; e_walk 0: no map for the walk)
-    const float R_t = __uint_as_float((uint32_t)e_tot << 23), half_t = half_ulp(e_tot);
-    const float R_w = __uint_as_float((uint32_t)max(e_walk, 1) << 23), half_w = half_ulp(e_walk);
+    const float base_t = binade_base(e_tot), half_t = half_ulp(e_tot);
+    const float base_w = binade_base(e_walk), half_w = half_ulp(e_walk);
     double sum = 0.0;
     uint32_t n_t = 0u, n_w = 0u; // (uniform)
     float acc_t = 0.0f, acc_w = 0.0f; // a lane's multiples of the epochs' last places: exact up to 2^24 of them, beyond after that
@@ -302,8 +302,8 @@ __device__ void opaque_share(const uint32_t* ks, uint32_t cnt, uint32_t off, int
             const uint32_t kv = base + u * kWave + lane < cnt ? k[u] : 0u;
             const float q = __uint_as_float(kv);
             sum += (double)q;
-            const float t = (R_t + q) - R_t;
-            const bool tie_t = fabsf(q - t) == half_t;
+            const float t = increment(q, base_t);
+            const bool tie_t = is_tie(q, t, half_t);
             acc_t += tie_t ? 0.0f : t;
             const unsigned long long bal_t = __ballot(tie_t);
             if (bal_t) { // (uniform, rare)
@@ -313,8 +313,8 @@ __device__ void opaque_share(const uint32_t* ks, uint32_t cnt, uint32_t off, int
                 n_t += (uint32_t)__popcll(bal_t);
             }
             if (e_walk > 0) { // uniform
-                const float w = (R_w + q) - R_w;
-                const bool tie_w = fabsf(q - w) == half_w;
+                const float w = increment(q, base_w);
+                const bool tie_w = is_tie(q, w, half_w);
                 acc_w += tie_w ? 0.0f : w;
                 const unsigned long long bal_w = __ballot(tie_w);
                 if (bal_w) {
@@ -329,11 +329,11 @@ __device__ void opaque_share(const uint32_t* ks, uint32_t cnt, uint32_t off, int
     const double sum64 = __ockl_wfred_add_f64(sum);
     // One kind of increments: the sum of the multiples between neighbouring ties (heaviest first), with each tie's own
     // two-valued step composed in at its place.
-    auto share_incs = [&](uint32_t which, uint32_t n, int e, float R, float half, float acc) {
+    auto share_incs = [&](uint32_t which, uint32_t n, int e, float from, float half, float acc) {
         if (e <= 0 || n > kOpaqueTies) // uniform
             return make_float2(INFINITY, INFINITY);
         const float all = readlane_f32(wave_scan_add_f32(acc), kWave - 1);
-        const uint32_t units = all < 2.0f * R ? (uint32_t)__builtin_ldexpf(all, 150 - e) : kSat; // (below 2^24, and whole)
+        const uint32_t units = all < binade_top(e) ? (uint32_t)__builtin_ldexpf(all, 150 - e) : kSat; // (below 2^24, and whole)
         if (n == 0u)
             return make_float2(all, all);
         // the ties by weight, heaviest first (equal ones in any order: they are the same step)
@@ -361,8 +361,8 @@ __device__ void opaque_share(const uint32_t* ks, uint32_t cnt, uint32_t off, int
 #pragma unroll
                 for (uint32_t u = 0; u < kTrip; ++u) {
                     const float q = __uint_as_float(k[u]);
-                    const float t = (R + q) - R;
-                    part += (base + u * kWave + lane < cnt && k[u] > tk && !(fabsf(q - t) == half)) ? t : 0.0f;
+                    const float t = increment(q, from);
+                    part += (base + u * kWave + lane < cnt && k[u] > tk && !is_tie(q, t, half)) ? t : 0.0f;
                 }
             }
             const uint32_t above = (uint32_t)__builtin_ldexpf(readlane_f32(wave_scan_add_f32(part), kWave - 1), 150 - e);
@@ -375,8 +375,8 @@ __device__ void opaque_share(const uint32_t* ks, uint32_t cnt, uint32_t off, int
         auto as_float = [e](uint32_t d) { return d < (1u << 24) ? __builtin_ldexpf((float)d, e - 150) : INFINITY; };
         return make_float2(as_float(v.d0), as_float(v.d1));
     };
-    const float2 m0 = share_incs(0u, n_t, e_tot, R_t, half_t, acc_t);
-    const float2 m1 = share_incs(1u, n_w, e_walk, R_w, half_w, acc_w);
+    const float2 m0 = share_incs(0u, n_t, e_tot, base_t, half_t, acc_t);
+    const float2 m1 = share_incs(1u, n_w, e_walk, base_w, half_w, acc_w);
     if (lane == 0u)
         store_group_rec(rec, sum64, m0, m1, off, kOpaque | ((uint32_t)e_tot << kSumExpShift) | ((uint32_t)max(e_walk, 0) << kWalkExpShift));
 }

@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from mako_amd import api
-from parity import assert_parity
+from parity import assert_parity, oracle_rows
 
 pytestmark = pytest.mark.gpu
 
@@ -34,3 +34,24 @@ def test_totals_and_walks(gpu_ctx, vocab, kind, top_p):
     w = dict(name="%s %d" % (kind, vocab), logits=_logits(kind, rows, vocab, rng), u=us,
              params=api.make_params(rows, np.linspace(0.6, 1.4, rows), 0, top_p))
     assert_parity(gpu_ctx, w, cap=64, hinted=True)
+
+
+@pytest.mark.parametrize("vocab", [9000, 129280])
+@pytest.mark.parametrize("hinted", [False, True])
+def test_walks_in_the_lowest_binade(gpu_ctx, vocab, hinted):
+    """A weight in [2^-126, 2^-125) far in front of the only other one, 1.0, and a walk that starts one last place below
+    it, at it, above it, and at the ends of the binade: sums with such a weight lie in the next binade, whose last place is
+    twice as large."""
+    at = 5000
+    r = [float.fromhex(x + "p-126") for x in ("0x1.01b1b8", "0x1.01b1ba", "0x1.01b1bc", "0x1.fffffe")]
+    r += [2.0**-126, 2.0**-127, 2.0**-149, 0.0, 0.5]
+    u = np.array(r, np.float32)
+    logits = np.full((len(r), vocab), -np.inf, np.float32)
+    logits[:, at] = np.float32(-87.3299484)
+    logits[:, -1] = 0.0
+    w = dict(name="lowest binade", logits=logits, u=u, params=api.make_params(len(r), 1.0, 0, 1.0))
+    ref = oracle_rows(w, cap=4)
+    assert ref[0][1]["cand_q"][0] == np.float32(float.fromhex("0x1.01b1bap-126"))
+    assert [t for t, _ in ref] == [at, vocab - 1, vocab - 1, vocab - 1, at, at, at, at, vocab - 1]
+    g = assert_parity(gpu_ctx, w, cap=0, hinted=hinted)
+    assert (g["n_cand"] == 2).all()

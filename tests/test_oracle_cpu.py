@@ -224,6 +224,16 @@ def test_seqfp_host():
     assert " 0 failures" in out, out
 
 
+def test_group_chain_host():
+    """The kernels' chains over groups of 256 weights (mako_amd/csrc/group_chain.h) restated on the host, on the
+    arithmetic they share (seqfp.h): sums, walks and their stops against real fp32 loops, over every binade."""
+    exe = os.path.join(HERE, "cpu", "group_chain_test")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-I", os.path.join(HERE, "..", "mako_amd", "csrc"),
+                    os.path.join(HERE, "cpu", "group_chain_test.cpp"), "-o", exe], check=True)
+    out = subprocess.run([exe], capture_output=True, text=True)
+    assert out.returncode == 0 and ": 0 failures" in out.stdout, out.stdout
+
+
 def test_unsorted_share_host():
     """The record that stands for an unsorted share of a sorted list (opaque_share, mako_amd/csrc/worker_sort.h)
     restated on the host: sums of the increments between neighbouring exact ties, the ties' own steps composed in
@@ -357,7 +367,7 @@ def test_oracle_under_sanitizers():
     assert out.returncode == 0 and out.stdout.strip().endswith(" 0 failures"), out.stdout + out.stderr
 
 
-@pytest.mark.parametrize("name", ["seqfp_test", "gen_helpers_test", "log_bins_test", "unsorted_share_test"])
+@pytest.mark.parametrize("name", ["seqfp_test", "gen_helpers_test", "log_bins_test", "unsorted_share_test", "group_chain_test"])
 def test_host_code_under_sanitizers(name):
     """The host-side C++ the library shares with its kernels (seqfp.h) and ships (include/gen/), likewise."""
     exe = os.path.join(HERE, "cpu", name + "_san")
