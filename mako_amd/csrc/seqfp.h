@@ -211,7 +211,7 @@ SEQFP_HD long long sub_apply(long long m, float q, int e)
 // What stands in R0's place for the binade with exponent e >= 1.
 SEQFP_HD float binade_base(int e)
 {
-    return e > 1 ? u2f(uint32_t(e) << 23) : 0.0f;
+    return u2f(e > 1 ? uint32_t(e) << 23 : 0u); // (chosen as bits: a scalar select where e is one)
 }
 // The first float above the binade.
 SEQFP_HD float binade_top(int e)
@@ -222,7 +222,7 @@ SEQFP_HD float binade_top(int e)
 // binade it does not: a value may go down to zero.)
 SEQFP_HD float binade_low(int e)
 {
-    return e > 1 ? u2f(uint32_t(e) << 23) : -0x1p-149f;
+    return u2f(e > 1 ? uint32_t(e) << 23 : 0x80000001u); // (-2^-149)
 }
 SEQFP_HD float increment(float q, float base)
 {
