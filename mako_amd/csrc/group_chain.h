@@ -485,14 +485,14 @@ struct GroupLds { // carved from the dynamic LDS block once sorting is over
     __device__ __forceinline__ uint32_t* pack() const { return start() + kMaxGroups; } // as GroupRec::pack, and the slot + 1
     __device__ __forceinline__ uint32_t* misc() const { return pack() + kMaxGroups; }  // [16]
     __device__ __forceinline__ uint32_t* staged() const { return misc() + 16; }        // [64] the groups in the slots
-    __device__ __forceinline__ uint16_t* todo() const { return reinterpret_cast<uint16_t*>(staged() + 64); } // [2 * kMaxGroups] increments to be made
+    // [kMaxGroups] groups whose increment for the running sum is to be made, then [kMaxGroups] those for the walk
+    __device__ __forceinline__ uint16_t* todo() const { return reinterpret_cast<uint16_t*>(staged() + 64); }
     // [kHeadLen + kWave] the first entries of the list
     __device__ __forceinline__ float* head() const { return reinterpret_cast<float*>(todo() + 2u * kMaxGroups); }
     // [kSlots][kGroup] entries of the groups that are expected to be replayed; the last slot is for any other
     __device__ __forceinline__ float* slot(uint32_t s) const { return head() + kHeadLen + kWave + s * kGroup; }
 };
 constexpr uint32_t kSlots = 39;
-constexpr uint32_t kTodoSum = 0x8000u; // (of a todo entry: the running sum's increment, not the walk's)
 constexpr uint32_t kSlotShift = 26; // (of GroupLds::pack())
 constexpr uint32_t kGroupLdsHead = (kMaxGroups + 2u) * 8u + kMaxGroups * (8u + 8u + 4u + 4u + 4u) + (16u + 64u) * 4u;
 static_assert(kGroupLdsHead % 16u == 0 && kGroupLdsHead + (kHeadLen + kWave + kSlots * kGroup + kWave) * 4u <= kTailLds && kSlots < 64u,
@@ -535,17 +535,24 @@ __device__ __forceinline__ bool walk_changes_binade(const GroupLds G, uint32_t g
 
 // Which groups are expected to be replayed (their entries go to the slots), and which others lack an increment for the
 // binade expected now: thread g decides for group g, of those from `from` on; `sum`, `walk`: for which of the two, the
-// latter from r0 (the sum's first `lead` groups need neither).  (All threads call, the caller's barriers around it.)  A group that is expected to be replayed anyway, and
-// one the walk is not expected to reach, gets no increment.  G.misc()[3] counts the slots, G.misc()[7] the increments to
-// be made.
-template <bool UNSORTED>
+// latter from r0 (the sum's first `lead` groups need neither).  (All threads call, the caller's barriers around it.)  A group
+// that is expected to be replayed anyway, and one the walk is not expected to reach, gets no increment.  G.misc()[3] counts the
+// slots, G.misc()[7] and [8] the increments to be made, the sum's and the walk's.
+// PLANNED: a worker has left the sum's increments, and a group of which it took another binade than is expected now (four at
+// most in a row where it happened at all) is replayed too.  Its increment is not made again, as only the chain could wait for
+// that: an increment and the binade it is for (in pack()) are two words, and a chain beside the writer could find the old binade
+// with the new increment.  That binade may be the running value's own, where the fp64 sums that the guesses come from lie on the
+// other side of a power of two.  (Made in front of the chain by all the waves, with a trip to memory of their own: no faster.)
+template <bool UNSORTED, bool PLANNED>
 __device__ __forceinline__ void plan_groups(const GroupLds G, uint32_t lead, uint32_t from, uint32_t groups, bool sum, bool walk, double r0, const LeftOut out)
 {
     const uint32_t g = threadIdx.x;
     const uint32_t pk = G.pack()[min(g, groups - 1u)];
     if (g < from || g >= groups || (UNSORTED && (pk & kOpaque)))
         return;
-    const bool replay_s = sum && g >= lead && sum_changes_binade(G, g), replay_w = walk && walk_changes_binade(G, g, r0);
+    const double b = G.pg()[g];
+    const bool made = ((pk >> kSumExpShift) & 0xffu) == (uint32_t)exponent_of((float)b);
+    const bool replay_s = sum && g >= lead && (sum_changes_binade(G, g) || (PLANNED && !made)), replay_w = walk && walk_changes_binade(G, g, r0);
     if (replay_s || replay_w) {
         const uint32_t s = atomicAdd(&G.misc()[3], 1u);
         if (s < kSlots - 1u) {
@@ -553,11 +560,10 @@ __device__ __forceinline__ void plan_groups(const GroupLds G, uint32_t lead, uin
             G.pack()[g] = pk | ((s + 1u) << kSlotShift);
         }
     }
-    const double b = G.pg()[g];
-    if (sum && g >= lead && !replay_s && ((pk >> kSumExpShift) & 0xffu) != (uint32_t)exponent_of((float)b))
-        G.todo()[atomicAdd(&G.misc()[7], 1u)] = (uint16_t)(g | kTodoSum);
-    if (walk && !replay_w && r0 - b > 0.0 && g != out.group && ((pk >> kWalkExpShift) & 0xffu) != (uint32_t)exponent_of((float)(r0 - b)))
+    if (!PLANNED && sum && g >= lead && !replay_s && !made)
         G.todo()[atomicAdd(&G.misc()[7], 1u)] = (uint16_t)g;
+    if (walk && !replay_w && r0 - b > 0.0 && g != out.group && ((pk >> kWalkExpShift) & 0xffu) != (uint32_t)exponent_of((float)(r0 - b)))
+        G.todo()[kMaxGroups + atomicAdd(&G.misc()[8], 1u)] = (uint16_t)g;
 }
 template <typename Keys>
 __device__ __forceinline__ void fill_staged(Keys kf, const GroupLds G, const LeftOut out = LeftOut{})
@@ -568,32 +574,32 @@ __device__ __forceinline__ void fill_staged(Keys kf, const GroupLds G, const Lef
 }
 
 // The increments to be made.  The calling wave is number `part` of `parts` that share the work; up to four groups per trip
-// to memory.
+// to memory.  (Never beside the chain that uses them: plan_groups().)
 template <typename Keys>
 __device__ __forceinline__ void build_incs(Keys kf, double r0, const GroupLds G, uint32_t part, uint32_t parts)
 {
-    const uint32_t n = uniform_u32(G.misc()[7]);
+    const uint32_t n_sum = uniform_u32(G.misc()[7]), n = n_sum + uniform_u32(G.misc()[8]);
     for (uint32_t i0 = part; i0 < n; i0 += parts * 4u) {
         float q[4][4];
         uint32_t item[4];
 #pragma unroll
         for (uint32_t u = 0; u < 4; ++u) {
-            item[u] = uniform_u32(G.todo()[min(i0 + u * parts, n - 1u)]);
-            const uint32_t g = item[u] & ~kTodoSum;
-            load_span(kf, uniform_u32(G.start()[g]), i0 + u * parts < n ? uniform_u32(G.pack()[g]) & kLenMask : 0u, q[u]);
+            const uint32_t i = min(i0 + u * parts, n - 1u);
+            item[u] = uniform_u32(G.todo()[i < n_sum ? i : kMaxGroups + (i - n_sum)]);
+            load_span(kf, uniform_u32(G.start()[item[u]]), i0 + u * parts < n ? uniform_u32(G.pack()[item[u]]) & kLenMask : 0u, q[u]);
         }
 #pragma unroll
         for (uint32_t u = 0; u < 4; ++u) {
             if (i0 + u * parts >= n) // uniform
                 break;
-            const uint32_t g = item[u] & ~kTodoSum;
-            const bool sum = (item[u] & kTodoSum) != 0u;
+            const uint32_t g = item[u];
+            const bool for_sum = i0 + u * parts < n_sum;
             const double b = G.pg()[g];
-            const uint32_t e = uniform_u32((uint32_t)exponent_of((float)(sum ? b : r0 - b)));
+            const uint32_t e = uniform_u32((uint32_t)exponent_of((float)(for_sum ? b : r0 - b)));
             const float2 inc = span_incs(q[u], (int)e);
             if (lane_id() == 0) {
-                const uint32_t shift = sum ? kSumExpShift : kWalkExpShift;
-                (sum ? G.inc() : G.winc())[g] = inc;
+                const uint32_t shift = for_sum ? kSumExpShift : kWalkExpShift;
+                (for_sum ? G.inc() : G.winc())[g] = inc;
                 atomicAnd(&G.pack()[g], ~(0xffu << shift)); // (another wave may be at work on the other one)
                 atomicOr(&G.pack()[g], e << shift);
             }

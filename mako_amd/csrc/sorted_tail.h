@@ -306,7 +306,8 @@ __device__ bool sorted_tail(const mako_sample_desc& d, uint32_t row, const mako_
     const uint32_t groups1 = PLANNED ? t_groups : (n1 + kGroup - 1) / kGroup;
     if (tid == 0) {
         G.misc()[3] = 0; // slots in use
-        G.misc()[7] = 0; // increments to be made
+        G.misc()[7] = 0; // increments to be made for the running sum
+        G.misc()[8] = 0; // and for the walk
         if (UNSORTED) {
             sm.ticket = 0; // set: a record of an unsorted share where the code below needs the list itself
             sm.flag = 0;   // set: the list has such records
@@ -585,7 +586,8 @@ __device__ bool sorted_tail(const mako_sample_desc& d, uint32_t row, const mako_
 
     // The exact fp32 total, then the walk from u times it (group_chain.h).  Where the binades change, and where the walk
     // ends, is known beforehand but for what the fp64 sums leave open: those groups' entries are fetched now, by all the
-    // waves, and while one wave chains the running sum the others see to the increments for the walk that are missing.
+    // waves, and while one wave chains the running sum the others see to the increments for the walk that are missing (the
+    // sum's, where nobody has left any, are made first).
     const double r0_raw = (double)u_row * G.pg()[groups], r0_guess = r0_raw == r0_raw ? r0_raw : 0.0;
     // (the sum's leading groups: up to the last of the first two in which it changes binade; the second costs half a
     // microsecond one by one, a replay nearly one)
@@ -594,7 +596,7 @@ __device__ bool sorted_tail(const mako_sample_desc& d, uint32_t row, const mako_
     // through costs a microsecond, twelve groups at two nanoseconds an entry six.
     const double head_mass = G.pg()[min(kHeadStaged, groups)];
     bool head_walk = r0_guess * 1.001 <= head_mass || groups <= kHeadStaged;
-    plan_groups<UNSORTED>(G, lead, 0u, groups, true, !head_walk, r0_guess, LeftOut{});
+    plan_groups<UNSORTED, PLANNED>(G, lead, 0u, groups, true, !head_walk, r0_guess, LeftOut{});
     __syncthreads();
     MAKO_STAMP(13);
     fill_staged(kf, G);
@@ -602,8 +604,6 @@ __device__ bool sorted_tail(const mako_sample_desc& d, uint32_t row, const mako_
         build_incs(kf, r0_guess, G, (uint32_t)wave_id(), (uint32_t)kWaves);
         __syncthreads();
     } else {
-        // (what a worker left for another binade than is expected now, little if anything: whoever is not yet done with it
-        // when the chain gets there has the group replayed)
         lds_barrier();
     }
     if (wave_id() == 0) {
@@ -630,12 +630,12 @@ __device__ bool sorted_tail(const mako_sample_desc& d, uint32_t row, const mako_
     auto prepare_walk = [&](uint32_t from, double r_here) __attribute__((always_inline)) {
         __syncthreads();
         if (tid == 0)
-            G.misc()[3] = G.misc()[7] = 0;
+            G.misc()[3] = G.misc()[7] = G.misc()[8] = 0;
         if (tid < groups)
             G.pack()[tid] &= (1u << kSlotShift) - 1u;
         const double r0_here = r_here + G.pg()[from];
         __syncthreads();
-        plan_groups<UNSORTED>(G, 0u, from, groups, false, true, r0_here, out);
+        plan_groups<UNSORTED, PLANNED>(G, 0u, from, groups, false, true, r0_here, out);
         __syncthreads();
         fill_staged(kf, G, out);
         build_incs(kf, r0_here, G, (uint32_t)wave_id(), (uint32_t)kWaves);

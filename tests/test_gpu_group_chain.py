@@ -55,3 +55,33 @@ def test_walks_in_the_lowest_binade(gpu_ctx, vocab, hinted):
     assert [t for t, _ in ref] == [at, vocab - 1, vocab - 1, vocab - 1, at, at, at, at, vocab - 1]
     g = assert_parity(gpu_ctx, w, cap=0, hinted=hinted)
     assert (g["n_cand"] == 2).all()
+
+
+@pytest.mark.parametrize("rows", [24, 64])
+@pytest.mark.parametrize("hinted", [False, True])
+def test_running_sum_ahead_of_its_estimates(rows, hinted):
+    """Two weights near 1 and a tail of weights of about 2^-24, in a sum just below 2: each is rounded up or down to a whole
+    last place, so that the running sum passes 2 dozens of groups before or behind the fp64 sums, which in some of the larger
+    batch's rows pass it a few groups away from where the plan's estimates do.  The increments of those groups are for neither
+    the binade that is expected in the end nor, maybe, for the one that the running sum is in."""
+    vocab = 65540
+    rng = np.random.default_rng([rows, 11])
+    ctx = api.SamplerContext(max_rows=rows, max_vocab=vocab)
+    logits = np.empty((rows, vocab), np.float32)
+    for r in range(rows):
+        c = [0.55, 0.8, 1.1, 1.4, 1.6, 1.9][r % 6] * (1.0 + 0.02 * rng.random())
+        mass = vocab * c * 2.0**-24
+        heads = rng.uniform(0.01, 0.02, r % 5)
+        second = 1.0 - heads.sum() - mass * rng.uniform(0.1, 0.9)
+        logits[r] = np.log(c * 2.0**-24) + 1e-3 * rng.standard_normal(vocab)
+        at = rng.permutation(vocab)[:2 + len(heads)]
+        logits[r, at] = np.log(np.concatenate([[1.0, second], heads]))
+    u = rng.random(rows).astype(np.float32)
+    u[::2] = np.float32(1.0) - rng.uniform(0.0, 2e-3, len(u[::2])).astype(np.float32)
+    w = dict(name="ahead of its estimates", logits=logits, u=u, params=api.make_params(rows, 1.0, 0, 1.0))
+    try:
+        for top_p in (1.0, 1.0 - 2.0**-20):
+            w["params"]["top_p"] = np.float32(top_p)
+            assert_parity(ctx, w, cap=0, hinted=hinted)
+    finally:
+        ctx.close()
