@@ -562,7 +562,8 @@ __device__ __forceinline__ void plan_groups(const GroupLds G, uint32_t lead, uin
     }
     if (!PLANNED && sum && g >= lead && !replay_s && !made)
         G.todo()[atomicAdd(&G.misc()[7], 1u)] = (uint16_t)g;
-    if (walk && !replay_w && r0 - b > 0.0 && g != out.group && ((pk >> kWalkExpShift) & 0xffu) != (uint32_t)exponent_of((float)(r0 - b)))
+    // (at r = 0 too: the walk passes what weighs nothing there, in a row whose first candidates are behind a masked stretch)
+    if (walk && !replay_w && r0 - b >= 0.0 && g != out.group && ((pk >> kWalkExpShift) & 0xffu) != (uint32_t)exponent_of((float)(r0 - b)))
         G.todo()[kMaxGroups + atomicAdd(&G.misc()[8], 1u)] = (uint16_t)g;
 }
 template <typename Keys>

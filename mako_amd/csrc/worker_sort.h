@@ -382,8 +382,9 @@ __device__ void opaque_share(const uint32_t* ks, uint32_t cnt, uint32_t off, int
 }
 
 // The record of one group (q: its entries, four per lane; `before` / `after`: the mass in front of it and behind it; r0:
-// the estimate of where the walk starts, 0 or less: none): increments only where the binade is not expected to change
-// inside the group, which is replayed there.  One wave.
+// the estimate of where the walk starts): increments only where the binade is not expected to change inside the group,
+// which is replayed there.  (A walk that starts at 0 passes the groups in front of the first weight.  Left without increments
+// for that, 64 rows drawn at u = 0 behind a masked half of 129 280 logits took 372 us, with them 84.)  One wave.
 __device__ __forceinline__ void group_record(const float (&q)[4], uint32_t start, uint32_t len, double sum, double before, double after, double r0,
                                              GroupRec* rec)
 {
@@ -393,7 +394,7 @@ __device__ __forceinline__ void group_record(const float (&q)[4], uint32_t start
         inc = span_incs(q, (int)es);
     const double r_here = r0 - before, r_after = r0 - after;
     uint32_t ew = 0;
-    if (uniform_u32(r_here > 0.0 && r_after > 0.0 ? 1u : 0u)) {
+    if (uniform_u32(r_here >= 0.0 && r_after >= 0.0 ? 1u : 0u)) {
         ew = uniform_u32((uint32_t)exponent_of((float)r_here));
         if (ew == es && es == es_end && ew == uniform_u32((uint32_t)exponent_of((float)r_after)))
             walk = inc; // (one binade for both)

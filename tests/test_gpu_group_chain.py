@@ -4,7 +4,7 @@ import numpy as np
 import pytest
 
 from mako_amd import api
-from parity import assert_parity, oracle_rows
+from parity import assert_parity, gpu_rows, oracle_rows
 
 pytestmark = pytest.mark.gpu
 
@@ -85,3 +85,22 @@ def test_running_sum_ahead_of_its_estimates(rows, hinted):
             assert_parity(ctx, w, cap=0, hinted=hinted)
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("masked", [3072, 3073, 20000, 65536, 129278])
+def test_walks_from_zero_behind_a_masked_stretch(gpu_ctx, masked):
+    """u = 0 and the first tokens masked: the walk passes every group in front of the first candidate at r = 0."""
+    rng = np.random.default_rng(masked)
+    rows, vocab = 6, 129280
+    logits = (rng.standard_normal((rows, vocab)) * 2.0).astype(np.float32)
+    logits[:, :masked] = -np.inf
+    logits[3, 5] = 3.0  # (one row with a candidate in front of the stretch, drawn behind it)
+    u = np.array([0.0, 0.0, 2.0**-24, 0.9, 0.5, 2.0**-149], np.float32)
+    w = dict(name="from zero", logits=logits, u=u, params=api.make_params(rows, 1.0, 0, 1.0))
+    draft = np.array([masked, vocab - 1, masked + 1, 5, 0, masked], np.int32)
+    assert_parity(gpu_ctx, w, cap=0, hinted=True)
+    assert_parity(gpu_ctx, w, cap=0)
+    for u2 in (np.zeros(rows, np.float32), u):
+        g = gpu_rows(gpu_ctx, w, draft=draft, u2=u2, hinted=True)
+        for r, (t, tr) in enumerate(oracle_rows(w, draft=draft, u2=u2)):
+            assert g["tokens"][r] == t and bool(g["accepted"][r]) == bool(tr["accepted"]), (r, g["tokens"][r], t)
