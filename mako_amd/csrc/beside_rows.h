@@ -27,9 +27,10 @@ __global__ __launch_bounds__(kThreads) void finish_beside_kernel(mako_sample_des
         return;
     }
     const uint32_t pieces = (d_arg.n_vocab + kSliceMax - 1u) / kSliceMax;
+    RankedRows rows;
     for (uint32_t p = blockIdx.y - finish_wgs;; p += gridDim.y - finish_wgs) {
         uint32_t row;
-        if (!ranked_row(d_arg, p / pieces, [](const mako_sampling_params& P) { return classify(P) == kGeneral; }, row))
+        if (!rows.find(d_arg, p / pieces, [](const mako_sampling_params& P) { return classify(P) == kGeneral; }, row))
             return;
         index_weights_piece<VEC, KH>(d_arg, sc_val, slices, row, p % pieces, s_dyn64, sm, s_args);
         __syncthreads(); // (the next piece's table of counts and arguments)
@@ -50,9 +51,10 @@ __global__ __launch_bounds__(kThreads) void sort_beside_kernel(mako_sample_desc 
         return;
     }
     const uint32_t blocks = (d_arg.n_vocab + kIndexBlock - 1u) / kIndexBlock;
+    RankedRows rows;
     for (uint32_t p = (blockIdx.y - sort_rows) * gridDim.x + blockIdx.x;; p += (gridDim.y - sort_rows) * gridDim.x) {
         uint32_t row;
-        if (!ranked_row(d_arg, p / blocks, [](const mako_sampling_params& P) { return index_order_row(P); }, row))
+        if (!rows.find(d_arg, p / blocks, [](const mako_sampling_params& P) { return index_order_row(P); }, row))
             return;
         index_groups_block<1u>(d_arg, sc_val, row, p % blocks, reinterpret_cast<double*>(s_dyn64));
         __syncthreads();

@@ -47,3 +47,17 @@ def test_every_kind_beside_every_other(rows, vocab, kinds):
         assert not (b["path"] == api.PATH_INDEXED).any()
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("kinds", [ALL, ["top_k"], ["nucleus", "temperature"]])
+def test_more_pieces_than_workgroups(kinds):
+    """Thousands of rows: a workgroup beside the others' takes dozens of pieces in turn and looks for each one's row."""
+    rows, vocab = 5003, 300
+    ctx = api.SamplerContext(max_rows=rows, max_vocab=vocab)
+    try:
+        w = _batch(rows, vocab, kinds, 9)
+        a = assert_parity(ctx, w, cap=8)
+        b = gpu_rows(ctx, w, hinted=True)
+        assert np.array_equal(a["tokens"], b["tokens"])
+    finally:
+        ctx.close()
