@@ -2,8 +2,9 @@
 // parameters shows them, or there is none): the kernels of index_rows.h as workgroups of the others' launches, so that a
 // batch has four launches whatever its rows are.  (Launches of their own would cost a batch without such rows three times
 // 2 us; one workgroup for all of a row's work, as a batch without the host copy had it, took 500 to 700 us a row.)
-// Workgroups behind those of the launch's own kernel take the rows' pieces in turn; without such rows they leave after
-// a look at the parameters.
+// Workgroups behind those of the launch's own kernel take the rows' pieces in turn; scan_kernel has counted the rows, and
+// without any of them they leave at once.  (Looked for in the parameters instead, 64 rows a trip to memory, their absence kept
+// finish's launch of 4 000 top-k rows 50 us, 10 without these workgroups, 12 now.)
 #pragma once
 
 #include "index_rows.h"
@@ -27,8 +28,9 @@ __global__ __launch_bounds__(kThreads) void finish_beside_kernel(mako_sample_des
         return;
     }
     const uint32_t pieces = (d_arg.n_vocab + kSliceMax - 1u) / kSliceMax;
+    const uint32_t all = sc_val.work_n[8] * pieces;
     RankedRows rows;
-    for (uint32_t p = blockIdx.y - finish_wgs;; p += gridDim.y - finish_wgs) {
+    for (uint32_t p = blockIdx.y - finish_wgs; p < all; p += gridDim.y - finish_wgs) {
         uint32_t row;
         if (!rows.find(d_arg, p / pieces, [](const mako_sampling_params& P) { return classify(P) == kGeneral; }, row))
             return;
@@ -46,13 +48,21 @@ __global__ __launch_bounds__(kThreads) void sort_beside_kernel(mako_sample_desc 
     extern __shared__ __align__(16) unsigned long long s_dyn64[]; // (128-bit LDS operations need the alignment)
     __shared__ FinishShared sm;
     __shared__ ArgsLds s_args;
+    // (what either way needs first in one trip, and ahead of the branch: behind it, where stores of the other way might have
+    // been, the compiler takes no scalar loads, and thousands of workgroups without work wait for nothing but this trip.
+    // 8 704 of them: 31 us with vector loads, a trip of their own for the arguments and, short of registers, scratch memory; 23 now, 20.6 in
+    // sort_kernel)
+    const uint32_t in_order = sc_val.work_n[9];
+    SortFirstTrip first;
+    fetch_sort_entry<UNSORTED>(d_arg, sc_val, min(blockIdx.y, max(sort_rows, 1u) - 1u) * gridDim.x + blockIdx.x, first);
     if (blockIdx.y < sort_rows) {
-        sort_body<UNSORTED>(d_arg, sc_val, slices, s_dyn64, sm, s_args);
+        sort_body<UNSORTED>(d_arg, sc_val, slices, first, s_dyn64, sm, s_args);
         return;
     }
     const uint32_t blocks = (d_arg.n_vocab + kIndexBlock - 1u) / kIndexBlock;
+    const uint32_t all = in_order * blocks;
     RankedRows rows;
-    for (uint32_t p = (blockIdx.y - sort_rows) * gridDim.x + blockIdx.x;; p += (gridDim.y - sort_rows) * gridDim.x) {
+    for (uint32_t p = (blockIdx.y - sort_rows) * gridDim.x + blockIdx.x; p < all; p += (gridDim.y - sort_rows) * gridDim.x) {
         uint32_t row;
         if (!rows.find(d_arg, p / blocks, [](const mako_sampling_params& P) { return index_order_row(P); }, row))
             return;

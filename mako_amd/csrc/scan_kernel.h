@@ -94,8 +94,10 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(VEC ? 
     }
     if (row == 0 && slice == 0 && wave_id() == 1) { // how the second pass will be cut up
         const SecondPassCut cut = second_pass_cut(d, n_slices, slice_len, cus_and_grid & 0xffffu, (cus_and_grid >> 16) * 8u);
-        if (lane_id() == 0)
+        if (lane_id() == 0) {
             *reinterpret_cast<uint4*>(sc.work_n + 4) = make_uint4(cut.per_row, cut.piece_len, cut.busy, cut.pieces);
+            *reinterpret_cast<uint2*>(sc.work_n + 8) = make_uint2(cut.general, cut.in_order);
+        }
     }
     // ReasoningBudget::forced's question (src/server/openai.cpp:598-602), answered in the same pass over the logits
     bool want_above = false;

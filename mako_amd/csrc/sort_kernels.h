@@ -11,36 +11,49 @@ namespace mako {
 // the group records tail_kernel works from; worker 0 of a narrow row finishes the row from the candidate lists.
 // What the row's list looks like as a whole (the workers' counts, the exact total) every worker adds up for itself
 // from what the second pass left; worker 0 stores it for tail_kernel.
+//
+// A workgroup's time here is a chain of round trips to device memory, and each one left out shortens it by half
+// a microsecond.  Three remain: the work list's entry (with the arguments' copy for LDS), everything of the row's
+// record (a worker per lane), the worker's share.  (The empty asm statements keep each trip's loads together:
+// the compiler would let those that only a later branch needs wait for that branch.)
+// The first trip: asked for by the kernel, ahead of any branch.  (The context's record by value: the loads go out at once; the
+// list has room for every workgroup of the grid that it is for.)
+struct SortFirstTrip {
+    ArgWords arg_words;
+    uint32_t n_work, pieces_raw, item, n_collectors;
+    uint64_t tab_word;
+};
+template <bool UNSORTED>
+__device__ __forceinline__ void fetch_sort_entry(const mako_sample_desc& d_arg, const Scratch& sc_arg, uint32_t entry, SortFirstTrip& f)
+{
+    fetch_arg_words(d_arg, sc_arg, f.arg_words);
+    f.n_work = sc_arg.work_n[0];
+    f.pieces_raw = sc_arg.work_n[7];
+    f.item = sc_arg.work_sort[entry];
+    f.tab_word = k_exp2_tab[threadIdx.x & 31u];
+    f.n_collectors = UNSORTED ? sc_arg.work_n[3] : 0u;
+    asm volatile("" ::"s"(f.item), "s"(f.n_work), "s"(f.n_collectors), "s"(f.pieces_raw), "v"(f.arg_words.d), "v"(f.arg_words.sc), "v"(f.tab_word));
+}
+
 // UNSORTED: the instance for batches whose plans leave shares unsorted (unsorted_shares.h; a translation unit of its own,
 // k_sort_unsorted.hip): it knows the rows' collectors and that an unsorted share is one record.
 template <bool UNSORTED>
-__device__ __forceinline__ void sort_body(const mako_sample_desc& d_arg, const Scratch& sc_val, uint32_t slices, unsigned long long* s_dyn64,
-                                          FinishShared& sm, ArgsLds& s_args)
+__device__ __forceinline__ void sort_body(const mako_sample_desc& d_arg, const Scratch& sc_val, uint32_t slices, const SortFirstTrip& first,
+                                          unsigned long long* s_dyn64, FinishShared& sm, ArgsLds& s_args)
 {
-    // (the context's record by value: its first loads, the list's length and this workgroup's entry, go out together
-    // and at once; the list has room for every workgroup of the grid)
     const Scratch& sc_arg = sc_val;
     const uint32_t piece = blockIdx.y * gridDim.x + blockIdx.x, tid = threadIdx.x;
-    // A workgroup's time here is a chain of round trips to device memory, and each one left out shortens it by half
-    // a microsecond.  Three remain: the work list's entry (with the arguments' copy for LDS), everything of the row's
-    // record (a worker per lane), the worker's share.  (The empty asm statements keep each trip's loads together:
-    // the compiler would let those that only a later branch needs wait for that branch.)
-    ArgWords arg_words;
-    fetch_arg_words(d_arg, sc_arg, arg_words);
-    const uint32_t n_work = sc_arg.work_n[0];
-    const uint32_t pieces_raw = sc_arg.work_n[7];
-    const uint32_t item = sc_arg.work_sort[piece];
-    const uint64_t tab_word = k_exp2_tab[tid & 31u];
+    ArgWords arg_words = first.arg_words;
+    const uint32_t n_work = first.n_work, pieces_raw = first.pieces_raw, item = first.item;
+    const uint64_t tab_word = first.tab_word;
     if constexpr (UNSORTED) {
         // (two lists that meet at workgroup number sorted_at: large_batch_lists())
-        const uint32_t n_collectors = sc_arg.work_n[3];
-        asm volatile("" ::"s"(item), "s"(n_work), "s"(n_collectors), "s"(pieces_raw), "v"(arg_words.d), "v"(arg_words.sc), "v"(tab_word));
+        const uint32_t n_collectors = first.n_collectors;
         const SortLists lists = large_batch_lists(d_arg.n_rows);
         const bool with_work = piece < lists.sorted_at ? lists.sorted_at - piece <= n_collectors : piece - lists.sorted_at < n_work;
         if (!with_work)
             return;
     } else {
-        asm volatile("" ::"s"(item), "s"(n_work), "s"(pieces_raw), "v"(arg_words.d), "v"(arg_words.sc), "v"(tab_word));
         if (piece >= n_work)
             return;
     }
@@ -227,7 +240,9 @@ __global__ __launch_bounds__(kThreads) void sort_kernel_unsorted(mako_sample_des
     extern __shared__ __align__(16) unsigned long long s_dyn64[]; // (128-bit LDS operations need the alignment)
     __shared__ FinishShared sm;
     __shared__ ArgsLds s_args;
-    sort_body<true>(d_arg, sc_val, slices, s_dyn64, sm, s_args);
+    SortFirstTrip first;
+    fetch_sort_entry<true>(d_arg, sc_val, blockIdx.y * gridDim.x + blockIdx.x, first);
+    sort_body<true>(d_arg, sc_val, slices, first, s_dyn64, sm, s_args);
 }
 #else
 __global__ __launch_bounds__(kThreads) void sort_kernel(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices)
@@ -235,7 +250,9 @@ __global__ __launch_bounds__(kThreads) void sort_kernel(mako_sample_desc d_arg, 
     extern __shared__ __align__(16) unsigned long long s_dyn64[]; // (128-bit LDS operations need the alignment)
     __shared__ FinishShared sm;
     __shared__ ArgsLds s_args;
-    sort_body<false>(d_arg, sc_val, slices, s_dyn64, sm, s_args);
+    SortFirstTrip first;
+    fetch_sort_entry<false>(d_arg, sc_val, blockIdx.y * gridDim.x + blockIdx.x, first);
+    sort_body<false>(d_arg, sc_val, slices, first, s_dyn64, sm, s_args);
 }
 #endif
 #endif // MAKO_EMIT_SORT_KERNELS

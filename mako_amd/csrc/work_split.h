@@ -17,17 +17,24 @@ struct SecondPassCut {
     uint32_t piece_len;
     uint32_t busy;      // workgroups with work
     uint32_t pieces;    // pieces per row: workgroup g of a row takes the pieces g, g + per_row, ...
+    // and of the rows of the whole-row class (index_rows.h): all of them, those in token order
+    uint32_t general, in_order;
 };
 // finish_grid: the workgroups finish_kernel is launched with (second_pass_grid()).
 __device__ __forceinline__ SecondPassCut second_pass_cut(const mako_sample_desc& d, uint32_t slices, uint32_t slice_len,
                                                          uint32_t cus, uint32_t finish_grid)
 {
     uint32_t rows = 0; // top_k == 0 rows of the batch (every lane ends up with the count)
+    SecondPassCut cut;
+    cut.general = cut.in_order = 0;
     for (uint32_t base = 0; base < d.n_rows; base += (uint32_t)kWave) {
         const uint32_t r = base + (uint32_t)lane_id();
-        rows += (uint32_t)__popcll(__ballot(r < d.n_rows && classify(d.params[r]) == kNucleus));
+        const mako_sampling_params P = d.params[min(r, d.n_rows - 1u)];
+        const RowClass cls = classify(P);
+        rows += (uint32_t)__popcll(__ballot(r < d.n_rows && cls == kNucleus));
+        cut.general += (uint32_t)__popcll(__ballot(r < d.n_rows && cls == kGeneral));
+        cut.in_order += (uint32_t)__popcll(__ballot(r < d.n_rows && index_order_row(P)));
     }
-    SecondPassCut cut;
     cut.piece_len = slice_len;
     cut.pieces = slices;
     for (uint32_t blocks = 1; blocks < 4u; ++blocks) {
