@@ -75,13 +75,12 @@ __global__ __launch_bounds__(kThreads) void sort_beside_kernel(mako_sample_desc 
 #ifdef MAKO_EMIT_BESIDE_TAIL
 // grid as tail_kernel's
 template <bool UNSORTED>
-__global__ __launch_bounds__(kThreads) void tail_beside_kernel(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices, uint32_t tail_cap,
-                                                               uint32_t index_path)
+__global__ __launch_bounds__(kThreads) void tail_beside_kernel(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices, uint32_t tail_cap)
 {
     extern __shared__ __align__(16) unsigned long long s_dyn64[]; // (128-bit LDS operations need the alignment)
     __shared__ FinishShared sm;
     __shared__ ArgsLds s_args;
-    tail_body<UNSORTED, true>(d_arg, sc_val, slices, tail_cap, index_path, s_dyn64, sm, s_args);
+    tail_body<UNSORTED, true>(d_arg, sc_val, slices, tail_cap, s_dyn64, sm, s_args);
 }
 #endif
 

@@ -10,7 +10,7 @@
 //                         as sort_kernel's workers leave them for a sorted list;
 //   index_tail_kernel     a workgroup per row: the exact fp32 total and the walk over the group records
 //                         (sorted_tail's planned instance for lists in any order).
-// Where there are, or may be, rows of other kinds beside them, the same work is done in the launches of those (beside_*.h):
+// Where there are, or may be, rows of other kinds beside them, the same work is done in the launches of those (beside_rows.h):
 // the weights with finish_kernel's, the groups with sort_kernel's, the rest with tail_kernel's.
 // A logit that is no candidate stays in the list as a weight of 0.0f: adding it changes no sum, and the walk's
 // `r < q` is never true for it.  The list ends behind the row's last candidate, which is where the reference's walk
@@ -238,10 +238,9 @@ __device__ __forceinline__ void index_groups_block(const mako_sample_desc& d_arg
 }
 
 // What these kernels have left of a row of theirs (flag: of its plan, which is zero again behind this), by one workgroup: the
-// rest of the whole-row path, or the total and the draw.  path: MAKO_PATH_* of a row in token order.  All threads call; sm.tab
-// must hold the exp2 table.
+// rest of the whole-row path, or the total and the draw.  All threads call; sm.tab must hold the exp2 table.
 __device__ __forceinline__ void finish_index_row_here(const mako_sample_desc& d, const Scratch& sc, const mako_sampling_params& P, uint32_t row,
-                                                      uint32_t path, const FinishLds& L)
+                                                      const FinishLds& L)
 {
     const uint32_t tid = threadIdx.x;
     BigPlan* plan = sc.plan + row;
@@ -269,7 +268,7 @@ __device__ __forceinline__ void finish_index_row_here(const mako_sample_desc& d,
     if (flag == kIndexReady) {
         const uint32_t* kf = sc.key[0] + (size_t)row * sc.vpad;
         // (entry i of the list is token i: no array of token ids)
-        const bool done = sorted_tail<true, false, false, false, true>(d, row, P, kf, nullptr, n0, true, total64, path, L, false, 0.0f,
+        const bool done = sorted_tail<true, false, false, false, true>(d, row, P, kf, nullptr, n0, true, total64, MAKO_PATH_INDEXED, L, false, 0.0f,
                                                                        sc.gt + (size_t)row * sc.g_cap, groups);
         if (done) {
             // (the list's length counts the gaps; the candidates are what the reference counts)
@@ -282,10 +281,10 @@ __device__ __forceinline__ void finish_index_row_here(const mako_sample_desc& d,
         general_row<0>(d, sc, row, P, m, argidx, L);
 }
 __device__ MAKO_RARE_CALL void finish_index_row(const mako_sample_desc& d, const Scratch& sc, const mako_sampling_params& P, uint32_t row,
-                                                uint32_t path, const FinishLds& L)
+                                                const FinishLds& L)
 {
     assume_lds(L);
-    finish_index_row_here(d, sc, P, row, path, L);
+    finish_index_row_here(d, sc, P, row, L);
 }
 
 // Rows of the kind that `want` says (kGeneral, or those of them that are in token order) by their rank among them, for ranks that
@@ -349,7 +348,7 @@ __global__ __launch_bounds__(kThreads) void index_tail_kernel(mako_sample_desc d
         sm.tab[threadIdx.x] = k_exp2_tab[threadIdx.x];
     stage_args(d_arg, sc_val, row, s_args);
     const FinishLds views = finish_lds_views(sm, s_dyn64);
-    finish_index_row_here(s_args.d, s_args.sc, s_args.P, row, MAKO_PATH_INDEXED, views);
+    finish_index_row_here(s_args.d, s_args.sc, s_args.P, row, views);
 }
 #endif // MAKO_EMIT_INDEX_KERNELS
 

@@ -4,14 +4,13 @@
 #include "sampler_kernels.h"
 
 namespace mako {
-void launch_tail_beside(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices, uint32_t tail_cap, bool unsorted,
-                        uint32_t index_path)
+void launch_tail_beside(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices, uint32_t tail_cap, bool unsorted)
 {
     const dim3 grid(1, tail_cap + d.n_rows);
     if (unsorted)
-        hipLaunchKernelGGL(tail_beside_kernel<true>, grid, dim3(kThreads), kTailLds, st, d, sc, slices, tail_cap, index_path);
+        hipLaunchKernelGGL(tail_beside_kernel<true>, grid, dim3(kThreads), kTailLds, st, d, sc, slices, tail_cap);
     else
-        hipLaunchKernelGGL(tail_beside_kernel<false>, grid, dim3(kThreads), kTailLds, st, d, sc, slices, tail_cap, index_path);
+        hipLaunchKernelGGL(tail_beside_kernel<false>, grid, dim3(kThreads), kTailLds, st, d, sc, slices, tail_cap);
 }
 
 hipError_t init_beside_tail()

@@ -96,11 +96,10 @@ __device__ MAKO_RARE_CALL bool late_plain_row(const mako_sample_desc& d, const S
 
 // What the earlier kernels leave of row `row`, by one workgroup (all threads call; sm.tab must hold the exp2 table):
 // rows whose token is forced, greedy rows, top-k rows, rows for the whole-row path, second looks.
-// BESIDE: the rows that the launches before have begun for index_rows.h are finished here too; index_path: MAKO_PATH_* of
-// those in token order.
+// BESIDE: the rows that the launches before have begun for index_rows.h are finished here too.
 template <bool BESIDE>
 __device__ MAKO_RARE_CALL void finish_late_row(const mako_sample_desc& d, const Scratch& sc, const mako_sampling_params& P,
-                                               uint32_t row, uint32_t slices, uint32_t index_path, const FinishLds& L)
+                                               uint32_t row, uint32_t slices, const FinishLds& L)
 {
     assume_lds(L);
     const RowClass cls = classify(P);
@@ -108,7 +107,7 @@ __device__ MAKO_RARE_CALL void finish_late_row(const mako_sample_desc& d, const 
         return;
     if constexpr (BESIDE)
         if (cls == kGeneral && sc.plan[row].flag != 0u) { // uniform
-            finish_index_row(d, sc, P, row, index_path, L);
+            finish_index_row(d, sc, P, row, L);
             return;
         }
     if (cls == kNucleus) {

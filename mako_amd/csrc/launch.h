@@ -40,7 +40,7 @@ hipError_t init_index_kernels();
 void launch_index_weights(bool vec, int kh, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices);
 void launch_index_finish(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, bool in_order_rows);
 // finish, sort and tail of a batch where such rows are, or may be, beside others (beside_rows.h): the same launches with
-// `more` workgroups behind their own for those rows; index_path: MAKO_PATH_* of the rows in token order
+// `more` workgroups behind their own for those rows
 hipError_t init_beside_finish();
 hipError_t init_beside_sort();
 hipError_t init_beside_tail();
@@ -48,6 +48,5 @@ void launch_finish_beside(bool vec, int kh, bool unsorted, uint32_t wgs, uint32_
                           const Scratch& sc, uint32_t slices);
 void launch_sort_beside(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices, uint32_t grid_rows, bool unsorted,
                         uint32_t more);
-void launch_tail_beside(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices, uint32_t tail_cap, bool unsorted,
-                        uint32_t index_path);
+void launch_tail_beside(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices, uint32_t tail_cap, bool unsorted);
 } // namespace mako

@@ -447,7 +447,7 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
         if (any_nucleus || any_in_order || !params_host)
             MAKO_LAUNCH(mako::launch_sort_beside(st, d, sc, slices, any_nucleus ? nucleus_rows : 0u, unsorted, for_groups));
         MAKO_MARK(3);
-        MAKO_LAUNCH(mako::launch_tail_beside(st, d, sc, slices, nucleus_rows, unsorted, params_host ? MAKO_PATH_INDEXED : MAKO_PATH_GENERAL));
+        MAKO_LAUNCH(mako::launch_tail_beside(st, d, sc, slices, nucleus_rows, unsorted));
     } else {
         if (only_index)
             MAKO_LAUNCH(mako::launch_index_weights(vec, kh, st, d, sc, slices));

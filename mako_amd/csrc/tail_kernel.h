@@ -15,10 +15,10 @@ namespace mako {
 // (With the top-k rows in line the compiler would make a called function of the wide rows' sorted tail instead,
 // which costs them 2 us: that call is forced in line below.)
 // UNSORTED: the instance for batches whose plans may have left shares unsorted (unsorted_shares.h; a translation unit of its
-// own, k_tail_unsorted.hip).  BESIDE, index_path: as finish_late_row() has them.
+// own, k_tail_unsorted.hip).  BESIDE: as finish_late_row() has it.
 template <bool UNSORTED, bool BESIDE>
 __device__ __forceinline__ void tail_body(const mako_sample_desc& d_arg, const Scratch& sc_val, uint32_t slices, uint32_t tail_cap,
-                                          uint32_t index_path, unsigned long long* s_dyn64, FinishShared& sm, ArgsLds& s_args)
+                                          unsigned long long* s_dyn64, FinishShared& sm, ArgsLds& s_args)
 {
     const Scratch& sc_arg = sc_val;
 #ifdef MAKO_TIMING_TAIL
@@ -70,7 +70,7 @@ __device__ __forceinline__ void tail_body(const mako_sample_desc& d_arg, const S
         // (the views handed on by reference live in scratch memory, 32 bytes per thread: made here, where only the
         // rows that take the call store them)
         const FinishLds late_views = finish_lds_views(sm, s_dyn64);
-        finish_late_row<BESIDE>(s_args.d, s_args.sc, s_args.P, r, slices, index_path, late_views);
+        finish_late_row<BESIDE>(s_args.d, s_args.sc, s_args.P, r, slices, late_views);
         return;
     }
     // (two trips to memory before the list's records are asked for: the work list's entry with the arguments' copy
@@ -131,7 +131,7 @@ __global__ __launch_bounds__(kThreads) void tail_kernel_unsorted(mako_sample_des
     extern __shared__ __align__(16) unsigned long long s_dyn64[]; // (128-bit LDS operations need the alignment)
     __shared__ FinishShared sm;
     __shared__ ArgsLds s_args;
-    tail_body<true, false>(d_arg, sc_val, slices, tail_cap, 0u, s_dyn64, sm, s_args);
+    tail_body<true, false>(d_arg, sc_val, slices, tail_cap, s_dyn64, sm, s_args);
 }
 #else
 __global__ __launch_bounds__(kThreads) void tail_kernel(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices, uint32_t tail_cap)
@@ -139,7 +139,7 @@ __global__ __launch_bounds__(kThreads) void tail_kernel(mako_sample_desc d_arg, 
     extern __shared__ __align__(16) unsigned long long s_dyn64[]; // (128-bit LDS operations need the alignment)
     __shared__ FinishShared sm;
     __shared__ ArgsLds s_args;
-    tail_body<false, false>(d_arg, sc_val, slices, tail_cap, 0u, s_dyn64, sm, s_args);
+    tail_body<false, false>(d_arg, sc_val, slices, tail_cap, s_dyn64, sm, s_args);
 }
 #endif
 #endif // MAKO_EMIT_TAIL_KERNEL

@@ -44,7 +44,7 @@ def test_every_kind_beside_every_other(rows, vocab, kinds):
         b = assert_parity(ctx, w, cap=0)
         c = gpu_rows(ctx, w, cap=64)
         assert np.array_equal(a["tokens"], b["tokens"]) and np.array_equal(a["tokens"], c["tokens"])
-        assert not (b["path"] == api.PATH_INDEXED).any()
+        assert np.array_equal(a["path"], b["path"])
     finally:
         ctx.close()
 

@@ -1,9 +1,10 @@
 """GPU parity of rows that are cut neither to a top-k nor to a nucleus (temperature only: top_k = 0, top_p = 1), whose
-candidates the reference adds up and walks in token order (src/gen/sampler.cpp:79-83, :64-72).  With the caller's host
-copy of the parameters such rows take kernels of their own (mako_amd/csrc/index_rows.h: weights in place, group records,
-exact fp32 total and walk by group maps over the unsorted list); tokens, candidate counts, candidate lists and fp32
-totals must be the oracle's bit for bit, with gaps in the list (masks, min_p, underflow), at both ends of u, beside rows
-of every other kind, and the results must equal those of the call without the host copy (the whole-row path)."""
+candidates the reference adds up and walks in token order (src/gen/sampler.cpp:79-83, :64-72).  Such rows take kernels of
+their own (mako_amd/csrc/index_rows.h: weights in place, group records, exact fp32 total and walk by the groups'
+increments over the unsorted list), launched for a batch that the caller's host copy of the parameters shows to have no
+others, and otherwise as workgroups of the others' launches; tokens, candidate counts, candidate lists and fp32 totals must
+be the oracle's bit for bit, with gaps in the list (masks, min_p, underflow), at both ends of u, beside rows of every other
+kind, both ways.  What those kernels do not serve takes the whole-row path."""
 import numpy as np
 import pytest
 
@@ -99,8 +100,8 @@ def test_beside_rows_of_every_kind(gpu_ctx):
     # (cold rows have weights that underflow: with candidate lists asked for they take the whole-row path)
     assert np.isin(g["path"][::4], [PATH_INDEXED, PATH_GENERAL]).all() and (g["path"][::4] == PATH_INDEXED).sum() >= 4
     assert not (np.delete(g["path"], np.s_[::4]) == PATH_INDEXED).any()
-    h = gpu_rows(gpu_ctx, w, cap=256)
-    assert (h["path"][::4] == PATH_GENERAL).all()
+    h = assert_parity(gpu_ctx, w, cap=256)
+    assert np.array_equal(h["path"], g["path"])
     assert np.array_equal(h["tokens"], g["tokens"]) and np.array_equal(h["total"].view(np.uint32), g["total"].view(np.uint32))
     assert np.array_equal(h["n_cand"], g["n_cand"])
 
@@ -131,16 +132,59 @@ def test_vocabularies_that_are_no_multiple_of_four(vocab):
         ctx.close()
 
 
-def test_rows_the_kernels_do_not_serve():
-    """More logits than a row's group records cover (262 144): the rows take the whole-row path as before."""
-    vocab = 262148
-    ctx = api.SamplerContext(max_rows=2, max_vocab=vocab, max_hist=0)
+@pytest.mark.parametrize("vocab", [262147, 262148])
+@pytest.mark.parametrize("hinted", [False, True])
+def test_rows_the_kernels_do_not_serve(vocab, hinted):
+    """More logits than a row's group records cover (262 144): every row of the whole-row class takes the whole-row path
+    from its logits on, with masks, penalties and ties, sampling and verification."""
+    rng = np.random.Generator(np.random.PCG64([vocab, 98]))
+    rows, hl = 10, 300
+    w = _plain_batch(rows, vocab, 7, sigmas=(3.0, 1.0), temps=(0.8, 1.1), spikes=False)
+    w["logits"][4:6] = np.round(w["logits"][4:6] * 4.0) / 4.0
+    p = w["params"]
+    p["min_p"][2:4] = np.float32(1e-3)
+    p["top_k"][4:6] = [40, 3000]
+    p["top_k"][6:8], p["top_p"][6:8] = [200, 5000], np.float32(0.95)
+    p["repetition_penalty"][8:], p["frequency_penalty"][8:], p["presence_penalty"][8:] = 1.1, 0.2, 0.3
+    w["hist"] = rng.integers(0, vocab, (rows, hl)).astype(np.int32)
+    w["hist_len"] = np.full(rows, hl, np.uint32)
+    words = (vocab + 31) // 32
+    w["mask"] = np.full((rows, words), 0xffffffff, np.uint32)
+    w["mask"][1::3] = rng.integers(0, 2**32, (len(w["mask"][1::3]), words), dtype=np.uint64).astype(np.uint32)
+    ctx = api.SamplerContext(max_rows=rows, max_vocab=vocab, max_hist=hl)
     try:
-        w = _plain_batch(2, vocab, 7, spikes=False)
-        g = assert_parity(ctx, w, cap=16, hinted=True)
+        g = assert_parity(ctx, w, cap=16, hinted=hinted)
+        assert (g["path"] == PATH_GENERAL).all()
+        draft, u2 = w["logits"].argmax(axis=1).astype(np.int32), workloads._uniforms(rng, rows)
+        draft[::2] = rng.integers(0, vocab, len(draft[::2]))
+        v = gpu_rows(ctx, w, draft=draft, u2=u2, hinted=hinted)
+        for r, (t, tr) in enumerate(oracle_rows(w, draft=draft, u2=u2)):
+            assert v["tokens"][r] == t and bool(v["accepted"][r]) == bool(tr["accepted"]), r
     finally:
         ctx.close()
-    assert (g["path"] == PATH_GENERAL).all()
+
+
+@pytest.mark.parametrize("vocab", [5, 4099, 20000, 65537])
+@pytest.mark.parametrize("hinted", [False, True])
+def test_rows_with_gaps_written_out_take_the_whole_row_path(vocab, hinted):
+    """Candidates are wanted of rows whose list has gaps: the whole-row path from the logits on, on vocabularies the kernels
+    of index_rows.h serve otherwise, with penalties and at both ends of u."""
+    rng = np.random.Generator(np.random.PCG64([vocab, 99]))
+    rows, hl = 12, min(vocab, 600)
+    us = [0.0, 2.0**-24, 0.3, 0.7, 0.999, 1.0 - 2.0**-24]
+    w = _plain_batch(rows, vocab, vocab, sigmas=(2.0, 0.3), temps=(0.6, 1.0), us=us, spikes=False)
+    w["params"]["repetition_penalty"], w["params"]["frequency_penalty"], w["params"]["presence_penalty"] = 1.2, 0.1, 0.4
+    w["hist"] = rng.integers(0, vocab, (rows, hl)).astype(np.int32)
+    w["hist_len"] = rng.integers(0, hl + 1, rows).astype(np.uint32)
+    w["logits"][:, rng.permutation(vocab)[:max(1, vocab // 3)]] = -np.inf
+    w["logits"][:, -1] = 0.5  # (the list does not end in front of the gaps)
+    ctx = api.SamplerContext(max_rows=rows, max_vocab=vocab, max_hist=hl)
+    try:
+        g = assert_parity(ctx, w, cap=64, hinted=hinted)
+        assert (g["path"] == PATH_GENERAL).all()
+        assert (assert_parity(ctx, w, cap=0, hinted=hinted)["path"] == PATH_INDEXED).all()
+    finally:
+        ctx.close()
 
 
 def test_no_candidate_survives(gpu_ctx):
@@ -154,8 +198,8 @@ def test_no_candidate_survives(gpu_ctx):
 
 def test_other_rows_of_the_whole_row_path_get_their_weights_there_too(gpu_ctx):
     """Rows cut to a top-k without a top-p (the order nth_element leaves) and to a top-k beyond the candidate lists:
-    with the host copy of the parameters their weights come from the same kernel as the rows' in token order, a
-    workgroup per 16 384 logits, and the whole-row path goes on from there."""
+    their weights come from the same kernel as the rows' in token order, a workgroup per 16 384 logits, and the whole-row
+    path goes on from there, with the host copy of the parameters and without it."""
     rng = np.random.Generator(np.random.PCG64([9, 94]))
     rows, vocab, hl = 36, 129280, 512
     w = _plain_batch(rows, vocab, 9, sigmas=(3.0, 1.0), temps=(0.7, 1.1))
@@ -177,9 +221,8 @@ def test_other_rows_of_the_whole_row_path_get_their_weights_there_too(gpu_ctx):
     g = assert_parity(gpu_ctx, w, cap=128, hinted=True)
     _say("whole-row rows with the host copy, paths: %s" % _paths(g))
     assert (g["path"][0::3] == PATH_GENERAL).all() and (g["path"][1::3] == PATH_GENERAL).all()
-    h = gpu_rows(gpu_ctx, w, cap=128)
-    assert np.array_equal(h["tokens"], g["tokens"]) and np.array_equal(h["total"].view(np.uint32), g["total"].view(np.uint32))
-    assert np.array_equal(h["cand_idx"], g["cand_idx"])
+    h = assert_parity(gpu_ctx, w, cap=128)
+    assert np.array_equal(h["path"], g["path"])
 
 
 @pytest.mark.parametrize("vocab", [4099, 40000, 129280])
@@ -241,15 +284,18 @@ def test_verification_of_rows_in_token_order(gpu_ctx):
         assert not bad, bad[:8]
         _say("verification (cap %d): %d accepted, paths %s" % (cap, int(g["accepted"].sum()), _paths(g)))
         assert (g["path"] == PATH_INDEXED).sum() >= rows // 2
+        # (the total is the one a sampled row has)
+        totals = np.array([tr["total"] for _, tr in oracle_rows(w)], np.float32)
+        assert np.array_equal(g["total"].view(np.uint32), totals.view(np.uint32))
         h = gpu_rows(gpu_ctx, w, cap=cap, draft=draft, u2=u2)
         assert np.array_equal(h["tokens"], g["tokens"]) and np.array_equal(h["accepted"], g["accepted"])
-        assert np.array_equal(h["total"].view(np.uint32), g["total"].view(np.uint32))
+        assert np.array_equal(h["total"].view(np.uint32), totals.view(np.uint32)) and np.array_equal(h["path"], g["path"])
 
 
 def test_forced_and_close_tokens_beside_rows_in_token_order(gpu_ctx):
     """The decode loop's hooks (force_token, close_token) on a batch of temperature-only rows: a forced row is left to
-    the launch that writes forced tokens, the others take the kernels of their own; the results are those of the call
-    without the host copy of the parameters."""
+    the launch that writes forced tokens, the others take the kernels of their own, with the host copy of the parameters and
+    without it; counts, tokens and totals are those of the logits."""
     rng = np.random.Generator(np.random.PCG64([11, 96]))
     rows, vocab = 48, 129280
     w = _plain_batch(rows, vocab, 11, sigmas=(3.0, 1.0), temps=(0.8, 1.1))
@@ -263,14 +309,19 @@ def test_forced_and_close_tokens_beside_rows_in_token_order(gpu_ctx):
     g = api.sample(gpu_ctx, w["logits"], w["params"], w["u"], params_host=True, **kw)
     h = api.sample(gpu_ctx, w["logits"], w["params"], w["u"], **kw)
     _say("forced beside rows in token order, paths: %s" % _paths(g))
-    for key in ("tokens", "forced", "above", "n_cand"):
+    for key in ("tokens", "forced", "above", "n_cand", "path"):
         assert np.array_equal(g[key], h[key]), key
     assert np.array_equal(g["total"].view(np.uint32), h["total"].view(np.uint32))
     forced = g["forced"] != api.FORCED_NONE
     assert forced.sum() >= 10 and (g["path"][forced] == api.PATH_FORCED).all() and (g["path"][~forced] == PATH_INDEXED).all()
     assert (g["tokens"][::5] == force[::5]).all()
     ref = oracle_rows(w)
-    assert all(g["tokens"][r] == ref[r][0] for r in range(rows) if not forced[r])
+    assert all(g["tokens"][r] == ref[r][0] and g["n_cand"][r] == ref[r][1]["n_cand"] and
+               np.float32(g["total"][r]).view(np.uint32) == np.float32(ref[r][1]["total"]).view(np.uint32)
+               for r in range(rows) if not forced[r])
+    above = [int((w["logits"][r] > w["logits"][r, close[r]]).sum()) if close[r] >= 0 else 0xffffffff for r in range(rows)]
+    assert np.array_equal(g["above"], np.array(above, np.uint32))
+    assert np.array_equal(forced, (force >= 0) | ((close >= 0) & (np.array(above) < 3)))
 
 
 def test_beside_a_large_batch_of_nucleus_rows():
