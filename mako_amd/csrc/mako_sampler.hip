@@ -12,6 +12,7 @@
 #include <string>
 
 #include "../../include/mako_sampler.h"
+#include "host_stage.h"
 #include "launch.h"
 #include "sampler_kernels.h"
 
@@ -473,71 +474,14 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
 } // namespace
 
 namespace {
-constexpr size_t kStageAlign = 256;
-constexpr size_t kStagePinned = (size_t)16 << 20; // pinned memory kept per context, at most
-constexpr size_t kStageCopy = (size_t)1 << 20;    // bytes per copy: a copy costs 8 us and a MiB's transfer 20, putting it together 12
-
-// The inputs of a host-pointer call on their way to device memory: put one after the other, each at a multiple of
-// kStageAlign, into pinned memory, from where every kStageCopy bytes are copied to the same places of the context's block.
-struct HostStage {
+// HostStage's copies, on the default stream.
+struct DeviceLink {
     mako_sampler_ctx* ctx;
-    size_t at = 0, sent = 0; // bytes put and bytes copied, of the block
-    size_t base = 0;         // byte of the block that is at the pinned memory's start
-    hipError_t status = hipSuccess;
-
-    void flush()
+    int copy(size_t to, const void* from, size_t bytes)
     {
-        if (at > sent && status == hipSuccess)
-            status = hipMemcpyAsync(ctx->st_dev + sent, ctx->st_pin + (sent - base), at - sent, hipMemcpyHostToDevice, nullptr);
-        sent = at;
+        return hipMemcpyAsync(ctx->st_dev + to, from, bytes, hipMemcpyHostToDevice, nullptr);
     }
-    void append(const void* src, size_t bytes)
-    {
-        const unsigned char* from = static_cast<const unsigned char*>(src);
-        while (bytes && status == hipSuccess) {
-            if (at - base == ctx->st_pin_bytes) { // (the pinned memory is full: again from its start, when it has been read)
-                flush();
-                if (status == hipSuccess)
-                    status = hipStreamSynchronize(nullptr);
-                base = at;
-            }
-            const size_t n = std::min({bytes, ctx->st_pin_bytes - (at - base), kStageCopy - (at - sent)});
-            memcpy(ctx->st_pin + (at - base), from, n);
-            at += n;
-            from += n;
-            bytes -= n;
-            if (at - sent == kStageCopy)
-                flush();
-        }
-    }
-    void skip(size_t bytes) // (nobody reads what these hold)
-    {
-        while (bytes) {
-            const size_t n = std::min(bytes, kStageAlign);
-            static const unsigned char zeros[kStageAlign] = {};
-            append(zeros, n);
-            if (status != hipSuccess)
-                return;
-            bytes -= n;
-        }
-    }
-    void* put_rows(const void* src, size_t src_stride, size_t bytes, size_t stride, uint32_t rows)
-    {
-        skip((kStageAlign - at % kStageAlign) % kStageAlign);
-        unsigned char* dst = ctx->st_dev + at;
-        if (at + rows * stride > ctx->st_dev_bytes) // (never: the block holds the context's largest call)
-            status = hipErrorInvalidValue;
-        if (src_stride == bytes && stride == bytes) {
-            append(src, bytes * rows);
-            return dst;
-        }
-        for (uint32_t r = 0; r < rows; ++r) {
-            append(static_cast<const unsigned char*>(src) + r * src_stride, bytes);
-            skip(stride - bytes);
-        }
-        return dst;
-    }
-    void* put(const void* src, size_t bytes) { return put_rows(src, bytes, bytes, bytes, 1u); }
+    int wait() { return hipStreamSynchronize(nullptr); }
 };
 } // namespace
 
@@ -573,8 +517,8 @@ int mako_sampler_sample_host(mako_sampler_ctx* ctx, const float* logits, int64_t
     // staging buffers are created on first use and kept
     if (!ctx->st_dev) {
         const size_t R = ctx->max_rows, mwords = ((size_t)ctx->max_vocab + 31) / 32, hist = ctx->max_hist;
-        const size_t bytes = R * (((size_t)ctx->max_vocab + 3) / 4 * 16 + sizeof(mako_sampling_params) + mwords * 4 + hist * 8 + 16) + 16 * kStageAlign;
-        const size_t pinned = std::min(bytes, kStagePinned);
+        const size_t bytes = R * (((size_t)ctx->max_vocab + 3) / 4 * 16 + sizeof(mako_sampling_params) + mwords * 4 + hist * 8 + 16) + 16 * mako::kStageAlign;
+        const size_t pinned = std::min(bytes, mako::kStagePinned);
         void* p = nullptr;
         if (!ctx->st_pin) {
             MAKO_HIP(ctx, hipHostMalloc(&p, pinned, hipHostMallocDefault));
@@ -592,36 +536,35 @@ int mako_sampler_sample_host(mako_sampler_ctx* ctx, const float* logits, int64_t
     // All inputs one after the other in one block of device memory, through pinned memory, in copies that run while the
     // next part is put together: one copy for a row of 129 280 logits, 17 us, where a copy from the caller's own memory for
     // each of seven arrays took 100.
-    HostStage stage{ctx};
+    mako::HostStage<DeviceLink> stage(DeviceLink{ctx}, ctx->st_pin, ctx->st_pin_bytes, ctx->st_dev_bytes);
     mako_sample_desc d;
     memset(&d, 0, sizeof d);
     const int64_t stride = ((int64_t)n_vocab + 3) & ~3ll;
-    d.params = static_cast<const mako_sampling_params*>(stage.put(params, n_rows * sizeof(*params)));
-    d.u = static_cast<const float*>(stage.put(u, n_rows * sizeof(float)));
+    d.params = reinterpret_cast<const mako_sampling_params*>(ctx->st_dev + stage.put(params, n_rows * sizeof(*params)));
+    d.u = reinterpret_cast<const float*>(ctx->st_dev + stage.put(u, n_rows * sizeof(float)));
     d.n_rows = n_rows;
     d.n_vocab = n_vocab;
     if (mask) {
         const size_t w = ((size_t)n_vocab + 31) / 32;
-        d.mask = static_cast<const uint32_t*>(stage.put_rows(mask, (size_t)mask_stride * 4, w * 4, w * 4, n_rows));
+        d.mask = reinterpret_cast<const uint32_t*>(ctx->st_dev + stage.put_rows(mask, (size_t)mask_stride * 4, w * 4, w * 4, n_rows));
         d.mask_stride = (int64_t)w;
     }
     if (hist_tokens && hist_stride > 0) {
-        d.hist_tokens = static_cast<int32_t*>(stage.put(hist_tokens, n_rows * (size_t)hist_stride * 4));
+        d.hist_tokens = reinterpret_cast<int32_t*>(ctx->st_dev + stage.put(hist_tokens, n_rows * (size_t)hist_stride * 4));
         if (hist_counts)
-            d.hist_counts = static_cast<const uint32_t*>(stage.put(hist_counts, n_rows * (size_t)hist_stride * 4));
-        d.hist_len = static_cast<uint32_t*>(stage.put(hist_len, n_rows * 4u));
+            d.hist_counts = reinterpret_cast<const uint32_t*>(ctx->st_dev + stage.put(hist_counts, n_rows * (size_t)hist_stride * 4));
+        d.hist_len = reinterpret_cast<uint32_t*>(ctx->st_dev + stage.put(hist_len, n_rows * 4u));
         d.hist_stride = hist_stride;
     }
     if (draft) {
-        d.draft = static_cast<const int32_t*>(stage.put(draft, n_rows * 4u));
-        d.u2 = static_cast<const float*>(stage.put(u2, n_rows * 4u));
+        d.draft = reinterpret_cast<const int32_t*>(ctx->st_dev + stage.put(draft, n_rows * 4u));
+        d.u2 = reinterpret_cast<const float*>(ctx->st_dev + stage.put(u2, n_rows * 4u));
         d.out_accepted = ctx->st_out + n_rows * sizeof(int32_t);
     }
-    d.logits = static_cast<const float*>(stage.put_rows(logits, (size_t)logits_stride * 4, (size_t)n_vocab * 4, (size_t)stride * 4, n_rows));
+    d.logits = reinterpret_cast<const float*>(ctx->st_dev + stage.put_rows(logits, (size_t)logits_stride * 4, (size_t)n_vocab * 4, (size_t)stride * 4, n_rows));
     d.logits_stride = stride;
-    stage.flush();
-    if (stage.status != hipSuccess)
-        return fail(ctx, MAKO_ERR_HIP, std::string("sampler: copying a call's inputs: ") + hipGetErrorString(stage.status));
+    if (const int e = stage.send())
+        return fail(ctx, MAKO_ERR_HIP, std::string("sampler: copying a call's inputs: ") + (e > 0 ? hipGetErrorString((hipError_t)e) : "they do not fit"));
     d.out_tokens = reinterpret_cast<int32_t*>(ctx->st_out);
     // (the caller's parameters are in host memory: the call looks at them and leaves out what no row needs)
     const int rc = mako_sampler_sample_batch_hinted(ctx, &d, params, nullptr);

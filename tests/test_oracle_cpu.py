@@ -255,6 +255,16 @@ def test_log_bins_host():
     assert out.returncode == 0 and " 0 failures" in out.stdout, out.stdout
 
 
+def test_host_stage_host():
+    """The host-pointer call's way to device memory (mako_amd/csrc/host_stage.h) over copies that read their source as late
+    as they may, some of which fail."""
+    exe = os.path.join(HERE, "cpu", "host_stage_test")
+    subprocess.run(["g++", "-O2", "-std=c++17", "-I", os.path.join(HERE, "..", "mako_amd", "csrc"),
+                    os.path.join(HERE, "cpu", "host_stage_test.cpp"), "-o", exe], check=True)
+    out = subprocess.run([exe], capture_output=True, text=True)
+    assert out.returncode == 0 and ": 0 failures" in out.stdout, out.stdout
+
+
 def test_heap_select_host():
     """The depth-limit branch of the kernels' nth_element (heap_select_rest, mako_amd/csrc/whole_row.h) restated on
     the host: libstdc++'s __make_heap level by level and its sweep 64 entries per ballot leave exactly what
@@ -367,7 +377,8 @@ def test_oracle_under_sanitizers():
     assert out.returncode == 0 and out.stdout.strip().endswith(" 0 failures"), out.stdout + out.stderr
 
 
-@pytest.mark.parametrize("name", ["seqfp_test", "gen_helpers_test", "log_bins_test", "unsorted_share_test", "group_chain_test"])
+@pytest.mark.parametrize("name", ["seqfp_test", "gen_helpers_test", "log_bins_test", "unsorted_share_test", "group_chain_test",
+                                  "host_stage_test"])
 def test_host_code_under_sanitizers(name):
     """The host-side C++ the library shares with its kernels (seqfp.h) and ships (include/gen/), likewise."""
     exe = os.path.join(HERE, "cpu", name + "_san")
