@@ -161,8 +161,13 @@ int mako_sampler_sample_batch_static(mako_sampler_ctx* ctx, const mako_sample_de
 
 /* Host-pointer convenience call with the reference's calling convention
  * (host logits, src/gen/session.cpp:443): copies the rows to the device,
- * samples, waits and copies the ids back.  Arrays are host arrays here; mask,
- * hist_*, draft/u2/accepted may be null.  PCIe-bound, not the measured path. */
+ * samples, waits and hands the ids back.  Arrays are host arrays here; mask,
+ * hist_*, draft/u2/accepted may be null.  PCIe-bound, not the measured path.
+ * A context's first such call allocates what its largest could need: device
+ * memory for all its inputs, and pinned host memory (16 MiB at most, and 5
+ * bytes a row for the results) that the inputs pass through and the kernels
+ * write the results to.  Both are the context's until it is destroyed.  Where
+ * the system has no pinned memory to give, ordinary memory takes its place. */
 int mako_sampler_sample_host(mako_sampler_ctx* ctx, const float* logits, int64_t logits_stride, uint32_t n_rows,
                              uint32_t n_vocab, const mako_sampling_params* params, const float* u,
                              const uint32_t* mask, int64_t mask_stride, const int32_t* hist_tokens,

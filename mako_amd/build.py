@@ -48,10 +48,12 @@ SOURCE_FLAGS = {
 }
 
 
-# and the checked library with plans that leave shares unsorted which they should not (-DMAKO_RASH_PLANS, only
-# the second pass differs): for the test that expects the oracle's results all the same, through rows given up to the
-# whole-row path
+# and the checked library with plans that leave shares unsorted which they should not (-DMAKO_RASH_PLANS, the second
+# pass), for the test that expects the oracle's results all the same, through rows given up to the whole-row path; and
+# without pinned memory (-DMAKO_NO_PINNED, the C ABI), for the host-pointer call's way round it
 OUT_RASH = os.path.join(HERE, "libmako_sampler_rash.so")
+RASH_FLAGS = {"k_finish.hip": ["-DMAKO_RASH_PLANS=1"], "k_beside_finish.hip": ["-DMAKO_RASH_PLANS=1"],
+              "mako_sampler.hip": ["-DMAKO_NO_PINNED=1"]}
 
 
 def build(verbose=False, extra=(), jobs=8, checked=False, rash=False):
@@ -62,12 +64,12 @@ def build(verbose=False, extra=(), jobs=8, checked=False, rash=False):
         extra = (*extra, "-DMAKO_CHECKED=1")
 
     def compile_one(name):
-        mine = rash and name in ("k_finish.hip", "k_beside_finish.hip")
+        mine = rash and name in RASH_FLAGS
         suffix = "_rash.o" if mine else ("_checked.o" if checked or rash else ".o")
         obj = os.path.join(OBJ_DIR, os.path.splitext(name)[0] + suffix)
         if rash and not mine:
             return obj # (the checked build's)
-        cmd = ["hipcc", *FLAGS, *SOURCE_FLAGS.get(name, INLINE_ALL), *extra, *(["-DMAKO_RASH_PLANS=1"] if mine else []), "-c",
+        cmd = ["hipcc", *FLAGS, *SOURCE_FLAGS.get(name, INLINE_ALL), *extra, *(RASH_FLAGS[name] if mine else []), "-c",
                os.path.join(CSRC, name), "-o", obj]
         if verbose:
             print(" ".join(cmd), flush=True)

@@ -4,6 +4,7 @@
 
 #include <stdint.h>
 #include <stdio.h>
+#include <stdlib.h>
 #include <string.h>
 
 #include <algorithm>
@@ -40,12 +41,14 @@ struct mako_sampler_ctx {
     int device = 0;
     uint32_t max_rows = 0, max_vocab = 0, max_hist = 0;
     mako::Scratch sc{};
-    // staging for the host-pointer call: device memory for all of a call's inputs, pinned memory they pass through on the
-    // way, and pinned memory the kernels write the results to
+    // staging for the host-pointer call: device memory for all of a call's inputs (and, behind them, its results), the host
+    // memory they pass through on the way, and pinned memory the kernels write the results to.  Where the system has no
+    // pinned memory to give (st_pinned false) the host memory is ordinary memory, and the results are copied back.
     unsigned char* st_dev = nullptr;
-    unsigned char* st_pin = nullptr;
+    unsigned char* st_host = nullptr;
     unsigned char* st_out = nullptr;
-    size_t st_dev_bytes = 0, st_pin_bytes = 0;
+    size_t st_dev_bytes = 0, st_host_bytes = 0;
+    bool st_pinned = false;
     std::string err = "";
     bool profile = false, profiled = false;
     bool dirty = false; // a launch of the last batch failed: the scratch memory is cleared again before the next one
@@ -248,9 +251,12 @@ void mako_sampler_destroy(mako_sampler_ctx* ctx)
     for (void* p : ptrs)
         if (p)
             (void)hipFree(p);
-    for (void* p : {ctx->st_pin, ctx->st_out})
-        if (p)
-            (void)hipHostFree(p);
+    if (ctx->st_pinned) {
+        (void)hipHostFree(ctx->st_host);
+        (void)hipHostFree(ctx->st_out);
+    } else {
+        free(ctx->st_host);
+    }
     for (hipEvent_t e : ctx->ev)
         if (e)
             (void)hipEventDestroy(e);
@@ -474,12 +480,26 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
 } // namespace
 
 namespace {
-// HostStage's copies, on the default stream.
+// Pinned memory, or null (a build for tests has none).
+unsigned char* pinned_memory(size_t bytes)
+{
+    void* p = nullptr;
+#ifndef MAKO_NO_PINNED
+    if (hipHostMalloc(&p, bytes, hipHostMallocDefault) != hipSuccess) {
+        (void)hipGetLastError(); // (not the next launch's)
+        p = nullptr;
+    }
+#endif
+    return static_cast<unsigned char*>(p);
+}
+
+// HostStage's copies on the default stream, from ordinary memory those of a program that has no other.
 struct DeviceLink {
     mako_sampler_ctx* ctx;
     int copy(size_t to, const void* from, size_t bytes)
     {
-        return hipMemcpyAsync(ctx->st_dev + to, from, bytes, hipMemcpyHostToDevice, nullptr);
+        return ctx->st_pinned ? hipMemcpyAsync(ctx->st_dev + to, from, bytes, hipMemcpyHostToDevice, nullptr)
+                              : hipMemcpy(ctx->st_dev + to, from, bytes, hipMemcpyHostToDevice);
     }
     int wait() { return hipStreamSynchronize(nullptr); }
 };
@@ -515,28 +535,35 @@ int mako_sampler_sample_host(mako_sampler_ctx* ctx, const float* logits, int64_t
                 return fail(ctx, MAKO_ERR_INVALID_ARG, "sampler: hist_len[r] > hist_stride");
     MAKO_HIP(ctx, hipSetDevice(ctx->device));
     // staging buffers are created on first use and kept
+    const size_t R = ctx->max_rows, out_bytes = R * (sizeof(int32_t) + 1);
     if (!ctx->st_dev) {
-        const size_t R = ctx->max_rows, mwords = ((size_t)ctx->max_vocab + 31) / 32, hist = ctx->max_hist;
-        const size_t bytes = R * (((size_t)ctx->max_vocab + 3) / 4 * 16 + sizeof(mako_sampling_params) + mwords * 4 + hist * 8 + 16) + 16 * mako::kStageAlign;
-        const size_t pinned = std::min(bytes, mako::kStagePinned);
+        const size_t mwords = ((size_t)ctx->max_vocab + 31) / 32, hist = ctx->max_hist;
+        const size_t need = R * (((size_t)ctx->max_vocab + 3) / 4 * 16 + sizeof(mako_sampling_params) + mwords * 4 + hist * 8 + 16) + 16 * mako::kStageAlign;
+        const size_t bytes = (need + mako::kStageAlign - 1) / mako::kStageAlign * mako::kStageAlign;
+        if (!ctx->st_host) {
+            ctx->st_host_bytes = std::min(bytes, mako::kStagePinned);
+            ctx->st_host = pinned_memory(ctx->st_host_bytes);
+            ctx->st_out = ctx->st_host ? pinned_memory(out_bytes) : nullptr;
+            ctx->st_pinned = ctx->st_out != nullptr;
+            if (!ctx->st_pinned) {
+                if (ctx->st_host)
+                    (void)hipHostFree(ctx->st_host);
+                ctx->st_host_bytes = std::min(bytes, mako::kStageCopy);
+                ctx->st_host = static_cast<unsigned char*>(malloc(ctx->st_host_bytes));
+            }
+            if (!ctx->st_host)
+                return fail(ctx, MAKO_ERR_NO_MEMORY, "sampler: no host memory for a call's inputs");
+        }
         void* p = nullptr;
-        if (!ctx->st_pin) {
-            MAKO_HIP(ctx, hipHostMalloc(&p, pinned, hipHostMallocDefault));
-            ctx->st_pin = static_cast<unsigned char*>(p);
-            ctx->st_pin_bytes = pinned;
-        }
-        if (!ctx->st_out) {
-            MAKO_HIP(ctx, hipHostMalloc(&p, R * (sizeof(int32_t) + 1), hipHostMallocDefault));
-            ctx->st_out = static_cast<unsigned char*>(p);
-        }
-        MAKO_HIP(ctx, hipMalloc(&p, bytes));
+        MAKO_HIP(ctx, hipMalloc(&p, bytes + out_bytes));
         ctx->st_dev = static_cast<unsigned char*>(p);
         ctx->st_dev_bytes = bytes;
     }
     // All inputs one after the other in one block of device memory, through pinned memory, in copies that run while the
     // next part is put together: one copy for a row of 129 280 logits, 17 us, where a copy from the caller's own memory for
     // each of seven arrays took 100.
-    mako::HostStage<DeviceLink> stage(DeviceLink{ctx}, ctx->st_pin, ctx->st_pin_bytes, ctx->st_dev_bytes);
+    mako::HostStage<DeviceLink> stage(DeviceLink{ctx}, ctx->st_host, ctx->st_host_bytes, ctx->st_dev_bytes);
+    unsigned char* const out = ctx->st_pinned ? ctx->st_out : ctx->st_dev + ctx->st_dev_bytes;
     mako_sample_desc d;
     memset(&d, 0, sizeof d);
     const int64_t stride = ((int64_t)n_vocab + 3) & ~3ll;
@@ -559,21 +586,27 @@ int mako_sampler_sample_host(mako_sampler_ctx* ctx, const float* logits, int64_t
     if (draft) {
         d.draft = reinterpret_cast<const int32_t*>(ctx->st_dev + stage.put(draft, n_rows * 4u));
         d.u2 = reinterpret_cast<const float*>(ctx->st_dev + stage.put(u2, n_rows * 4u));
-        d.out_accepted = ctx->st_out + n_rows * sizeof(int32_t);
+        d.out_accepted = out + n_rows * sizeof(int32_t);
     }
     d.logits = reinterpret_cast<const float*>(ctx->st_dev + stage.put_rows(logits, (size_t)logits_stride * 4, (size_t)n_vocab * 4, (size_t)stride * 4, n_rows));
     d.logits_stride = stride;
     if (const int e = stage.send())
         return fail(ctx, MAKO_ERR_HIP, std::string("sampler: copying a call's inputs: ") + (e > 0 ? hipGetErrorString((hipError_t)e) : "they do not fit"));
-    d.out_tokens = reinterpret_cast<int32_t*>(ctx->st_out);
+    d.out_tokens = reinterpret_cast<int32_t*>(out);
     // (the caller's parameters are in host memory: the call looks at them and leaves out what no row needs)
     const int rc = mako_sampler_sample_batch_hinted(ctx, &d, params, nullptr);
     MAKO_HIP(ctx, hipStreamSynchronize(nullptr)); // (also behind a failed launch: the copies read the pinned memory)
     if (rc != MAKO_OK)
         return rc;
-    memcpy(out_tokens, ctx->st_out, n_rows * sizeof(int32_t));
-    if (draft)
-        memcpy(out_accepted, ctx->st_out + n_rows * sizeof(int32_t), n_rows);
+    if (ctx->st_pinned) {
+        memcpy(out_tokens, out, n_rows * sizeof(int32_t));
+        if (draft)
+            memcpy(out_accepted, out + n_rows * sizeof(int32_t), n_rows);
+    } else {
+        MAKO_HIP(ctx, hipMemcpy(out_tokens, out, n_rows * sizeof(int32_t), hipMemcpyDeviceToHost));
+        if (draft)
+            MAKO_HIP(ctx, hipMemcpy(out_accepted, out + n_rows * sizeof(int32_t), n_rows, hipMemcpyDeviceToHost));
+    }
     return MAKO_OK;
 }
 

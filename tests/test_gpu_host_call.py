@@ -1,5 +1,6 @@
 """mako_sampler_sample_host() against the call on device pointers: inputs of every size on their way through the staging
-memory (copies of 1 MiB, 16 MiB of pinned memory that is used again), rows apart from each other, histories as pairs."""
+memory (copies of 1 MiB, 16 MiB of pinned memory that is used again), rows apart from each other, histories as pairs; and on a
+system that has no pinned memory to give."""
 import ctypes
 
 import numpy as np
@@ -13,7 +14,8 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("rows,vocab,apart", [(1, 1, 0), (1, 3, 5), (3, 4099, 0), (2, 131072, 0), (5, 65536, 64), (1, 262145, 0), (33, 140001, 3)])
 @pytest.mark.parametrize("verify", [False, True])
-def test_same_as_the_device_call(rows, vocab, apart, verify):
+@pytest.mark.parametrize("lib", [api.LIB_PATH, api.RASH_LIB_PATH], ids=["pinned", "no pinned memory"])
+def test_same_as_the_device_call(rows, vocab, apart, verify, lib):
     rng = np.random.Generator(np.random.PCG64([rows, vocab]))
     whole = (rng.standard_normal((rows, vocab + apart)) * 3.0).astype(np.float32)
     p = api.make_params(rows, 0.8, 40, 0.95)
@@ -29,7 +31,7 @@ def test_same_as_the_device_call(rows, vocab, apart, verify):
     u, u2 = workloads._uniforms(rng, rows), workloads._uniforms(rng, rows)
     draft = rng.integers(0, vocab, rows).astype(np.int32)
     tokens, accepted = np.full(rows, -1, np.int32), np.zeros(rows, np.uint8)
-    ctx = api.SamplerContext(max_rows=rows, max_vocab=vocab, max_hist=512)
+    ctx = api.SamplerContext(max_rows=rows, max_vocab=vocab, max_hist=512, lib_path=lib)
 
     def at(a):
         return ctypes.c_void_p(a.ctypes.data)
