@@ -38,14 +38,14 @@ __device__ __forceinline__ uint32_t dpp_or_zero(uint32_t v)
     return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, CTRL, ROW_MASK, 0xf, false);
 }
 
-// Inclusive scan, in lane order, of the 64 lanes' maps under composition (cmax is not touched).
+// Inclusive scan, in lane order, of the 64 lanes' maps under composition.
 __device__ __forceinline__ void wave_scan_maps(uint32_t& d0, uint32_t& d1)
 {
     using seqfp::Step32;
 #define MAKO_SCAN_STEP(CTRL, ROW_MASK)                                                                               \
     {                                                                                                                \
-        const Step32 t = Step32{dpp_or_zero<CTRL, ROW_MASK>(d0), dpp_or_zero<CTRL, ROW_MASK>(d1), 0u};               \
-        const Step32 r = seqfp::compose32(t, Step32{d0, d1, 0u}); /* earlier lanes first; {0, 0} is the identity */  \
+        const Step32 t = Step32{dpp_or_zero<CTRL, ROW_MASK>(d0), dpp_or_zero<CTRL, ROW_MASK>(d1)};                   \
+        const Step32 r = seqfp::compose32(t, Step32{d0, d1}); /* earlier lanes first; {0, 0} is the identity */      \
         d0 = r.d0;                                                                                                   \
         d1 = r.d1;                                                                                                   \
     }

@@ -366,12 +366,12 @@ __device__ void opaque_share(const uint32_t* ks, uint32_t cnt, uint32_t off, int
                 }
             }
             const uint32_t above = (uint32_t)__builtin_ldexpf(readlane_f32(wave_scan_add_f32(part), kWave - 1), 150 - e);
-            v = compose32(v, Step32{above - taken, above - taken, 0u});
+            v = compose32(v, Step32{above - taken, above - taken});
             v = compose32(v, step32_flat(__uint_as_float(tk), e));
             taken = above;
         }
         const uint32_t rest = units == kSat ? kSat : units - taken;
-        v = compose32(v, Step32{rest, rest, 0u});
+        v = compose32(v, Step32{rest, rest});
         auto as_float = [e](uint32_t d) { return d < (1u << 24) ? __builtin_ldexpf((float)d, e - 150) : INFINITY; };
         return make_float2(as_float(v.d0), as_float(v.d1));
     };

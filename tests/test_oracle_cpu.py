@@ -236,9 +236,9 @@ def test_group_chain_host():
 
 def test_unsorted_share_host():
     """The record that stands for an unsorted share of a sorted list (opaque_share, mako_amd/csrc/worker_sort.h)
-    restated on the host: sums of the increments between neighbouring exact ties, the ties' own steps composed in
-    between.  Wherever it passes the tests under which tail_kernel applies it, it gives the state that adding
-    (subtracting) the sorted weights one by one with real fp32 operations gives: 60000 shares."""
+    restated on the host: sums of the weights' multiples between neighbouring exact ties, the ties' own steps composed in
+    between.  Wherever it passes the test under which the chains apply it, it gives the value that adding (subtracting) the
+    sorted weights one by one with real fp32 operations gives: 60000 shares."""
     exe = os.path.join(HERE, "cpu", "unsorted_share_test")
     subprocess.run(["g++", "-O2", "-std=c++17", "-ffp-contract=off", "-I", os.path.join(HERE, "..", "mako_amd", "csrc"),
                     os.path.join(HERE, "cpu", "unsorted_share_test.cpp"), "-o", exe], check=True)
