@@ -135,12 +135,12 @@ int mako_sampler_sample_batch(mako_sampler_ctx* ctx, const mako_sample_desc* des
 
 /* The same call for a caller that still has the batch's parameters in HOST memory (the SamplingParams originate
  * there, src/gen/session.hpp:19-21): params_host[n_rows] must hold the same values as desc->params.  The call
- * looks at them on the calling thread and leaves out the kernels that no row of the batch needs (a batch without
- * top_k == 0 rows takes two launches instead of four).  Rows that are cut neither to a top-k nor to a nucleus
- * (temperature only: top_k == 0, top_p >= 1), whose candidates stay in token order, get three launches of their own
- * instead of one workgroup each for the whole row (up to 262 144 logits per row), verification and the decode loop's
- * hooks included; the other rows of the whole-row path (a top-k without a top-p, a top-k beyond 128) then get their
- * weights from many workgroups instead of one.  The results never depend on it; null = the call above. */
+ * looks at them on the calling thread and leaves out the kernels and the workgroups that no row of the batch needs: a
+ * batch of top-k rows takes two launches instead of four, and a batch with none but rows that are cut neither to a top-k
+ * nor to a nucleus (temperature only: top_k == 0, top_p >= 1), to a top-k without a top-p or to a top-k beyond 128 takes
+ * four of its own.  Without the copy such rows are served by more workgroups of the four launches that every batch
+ * then has (up to 262 144 logits per row, both ways; rows of more take one workgroup each).  The results never depend on
+ * it; null = the call above. */
 int mako_sampler_sample_batch_hinted(mako_sampler_ctx* ctx, const mako_sample_desc* desc,
                                      const mako_sampling_params* params_host, void* stream);
 

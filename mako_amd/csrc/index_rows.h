@@ -5,8 +5,8 @@
 //   index_weights_kernel  a workgroup per 16 384 logits: masks and penalties as everywhere, q = expf((w - m) / T), and
 //                         ~bits(q) (0.0f for a logit that is no candidate) stored at the token's own position (entry i
 //                         of the list is token i: no array of token ids);
-//   index_groups_kernel   a workgroup per 16 384 entries: the group records of its 64 groups of 256 (fp64 sums, the maps
-//                         of the running fp32 sum and of the walk for the binades guessed from the sums before them),
+//   index_groups_kernel   a workgroup per 16 384 entries: the group records of its 64 groups of 256 (fp64 sums, the
+//                         increments of the running fp32 sum and of the walk in the binades guessed from the sums before them),
 //                         as sort_kernel's workers leave them for a sorted list;
 //   index_tail_kernel     a workgroup per row: the exact fp32 total and the walk over the group records
 //                         (sorted_tail's planned instance for lists in any order).
@@ -165,7 +165,7 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
 
 // Workgroup p of a row leaves the records of the groups of its 4096 GPW entries.  Wave w
 // takes the groups w, w + 16, ... (GPW of them): their entries in one trip to memory, their fp64 sums to LDS, and once
-// every wave has the sums before each group, the maps from the entries it still holds.  (GPW = 4 where there are rows
+// every wave has the sums before each group, the increments from the entries it still holds.  (GPW = 4 where there are rows
 // enough to fill the chip, 1 on a small batch, which waits for one workgroup's chain of dependent steps.)
 template <uint32_t GPW>
 __device__ __forceinline__ void index_groups_block(const mako_sample_desc& d_arg, const Scratch& sc_val, uint32_t row, uint32_t p, double* s_gs)

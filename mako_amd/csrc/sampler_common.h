@@ -241,8 +241,8 @@ __host__ __device__ __forceinline__ RowClass classify(const mako_sampling_params
     return p.top_k <= kTopKFast ? kTopK : kGeneral;
 }
 
-// Rows that are cut neither to a top-k nor to a nucleus: their candidates stay in token order.  With the caller's host
-// copy of the parameters such rows get kernels of their own (index_rows.h), which hand a row on through BigPlan::flag:
+// Rows that are cut neither to a top-k nor to a nucleus: their candidates stay in token order.  Their kernels (index_rows.h,
+// beside_rows.h) hand a row on through BigPlan::flag:
 __host__ __device__ __forceinline__ bool index_order_row(const mako_sampling_params& p)
 {
     return p.temperature > 0.0f && !(p.top_p < 1.0f) && p.top_k == 0u;

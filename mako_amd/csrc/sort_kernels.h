@@ -169,7 +169,7 @@ __device__ __forceinline__ void sort_body(const mako_sample_desc& d_arg, const S
     const size_t t_row = (size_t)row * sc.g_cap;
     if (UNSORTED && w >= kWorkers) {
         // One of the row's collectors: each of its waves takes one of the shares that are left unsorted (collector c the
-        // shares 16 c .. 16 c + 15 of them) and leaves its record.  (The binades of the maps from the plan's estimates in
+        // shares 16 c .. 16 c + 15 of them) and leaves its record.  (The binades of the increments from the plan's estimates in
         // the exact total's units; any guess is safe, the tail tests what it applies.  A verification row has no such
         // shares.)
         MAKO_WG_TAG(0xc0000000u);

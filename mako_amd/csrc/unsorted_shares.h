@@ -13,11 +13,11 @@ namespace mako {
 // value is an exact tie with probability 2^-(difference of the exponents).  A share that the plan's estimates place
 // (a) behind the head of the list that the tail keeps in LDS, (b) inside one binade of the running sum, (c) above the
 // top-p cut and (d) where r stays inside one binade and cannot stop (or where the walk never gets) is not sorted: it
-// is left as ONE record, its fp64 sum, the sum of its increments as the map of the running sum, the same for the walk
+// is left as ONE record, its fp64 sum, the sum of its increments for the running sum, the same for the walk
 // (opaque_share()).  The few exact ties are kept apart: between two neighbouring ties (in value) the increments are
 // summed, and the tie's own two-valued step is composed in at its place.  The estimates only decide who tries:
-// tail_kernel applies such a record under the same exact tests as a group's map, and gives the row to the whole-row
-// path if one fails (the share's order would be needed then and does not exist).
+// tail_kernel applies such a record under the same exact test as a group's increment, and gives the row to the whole-row
+// path if it fails (the share's order would be needed then and does not exist).
 //
 // Only batches with many top_k == 0 rows do this (the host decides and launches the kernels' instances for it): there
 // sort_kernel is bound by the number of its workgroups, one per CU at a time, and a share that needs no sorting is summed
@@ -46,7 +46,7 @@ struct OpaqueGuess {
     int e_walk; // of r's; 0: the walk is not expected to reach the share
 };
 
-// The binades for a share's maps.  `before` / `after`: the mass above the share and above the next one; r0: where the
+// The binades for a share's increments.  `before` / `after`: the mass above the share and above the next one; r0: where the
 // walk starts (0: none), all in the same units.  same_tot / same_walk: the margins leave no doubt about them.
 __device__ __forceinline__ OpaqueGuess opaque_epochs(double before, double after, double r0, bool& same_tot, bool& same_walk)
 {

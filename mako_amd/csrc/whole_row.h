@@ -219,8 +219,8 @@ __device__ void heap_select_rest(Get get, Put put, uint32_t first, uint32_t last
 //   by one wave        nth_rounds_wave(): up to kNthWave entries, four per lane, without a barrier.
 // The depth limit's heap select is heap_select_rest() above.
 // (A batch of 32 rows of 12 000 candidates, 40 kept: 81 us with every round in device memory or LDS, two passes over the keys
-// each and through pointers that the compiler could not tell from each other; 60 us now.  64 rows of 129 280, bound by the
-// rounds in device memory of the row with the unluckiest pivots: 240 and 230 us.)
+// each and through pointers that the compiler could not tell from each other; 60 us now.  64 rows of 129 280 are bound by
+// the rounds in device memory of the row with the unluckiest pivots, and no faster: 235 to 270 us, as the box will have it.)
 constexpr uint32_t kNthChunks = 4;                                     // of four entries in a row per thread:
 constexpr uint32_t kNthRegs = kNthChunks * 4u * (uint32_t)kThreads; // what a workgroup takes into registers
 constexpr uint32_t kNthWave = 256;                                     // and one wave

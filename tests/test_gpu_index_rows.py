@@ -253,7 +253,7 @@ def test_wide_top_k_before_a_top_p_with_many_equal_weights(gpu_ctx, vocab):
 
 def test_verification_of_rows_in_token_order(gpu_ctx):
     """Sampler::verify (src/gen/sampler.cpp:86-107) on temperature-only rows: the draft's weight read off the list,
-    the total by the chain of group maps, and for a rejected draft the walk over the list without it.  Drafts that
+    the total by the chain over the groups, and for a rejected draft the walk over the list without it.  Drafts that
     are likely and unlikely tokens, no candidates (masked), the row's last candidate, and beyond the vocabulary's
     candidates; both uniforms from 0 to 1 - 2^-24."""
     rng = np.random.Generator(np.random.PCG64([10, 95]))
