@@ -538,21 +538,14 @@ __device__ __forceinline__ bool walk_changes_binade(const GroupLds G, uint32_t g
 // latter from r0 (the sum's first `lead` groups need neither).  (All threads call, the caller's barriers around it.)  A group
 // that is expected to be replayed anyway, and one the walk is not expected to reach, gets no increment.  G.misc()[3] counts the
 // slots, G.misc()[7] and [8] the increments to be made, the sum's and the walk's.
-// PLANNED: a worker has left the sum's increments, and a group of which it took another binade than is expected now (four at
-// most in a row where it happened at all) is replayed too.  Its increment is not made again, as only the chain could wait for
-// that: an increment and the binade it is for (in pack()) are two words, and a chain beside the writer could find the old binade
-// with the new increment.  That binade may be the running value's own, where the fp64 sums that the guesses come from lie on the
-// other side of a power of two.  (Made in front of the chain by all the waves, with a trip to memory of their own: no faster.)
-template <bool UNSORTED, bool PLANNED>
+template <bool UNSORTED>
 __device__ __forceinline__ void plan_groups(const GroupLds G, uint32_t lead, uint32_t from, uint32_t groups, bool sum, bool walk, double r0, const LeftOut out)
 {
     const uint32_t g = threadIdx.x;
     const uint32_t pk = G.pack()[min(g, groups - 1u)];
     if (g < from || g >= groups || (UNSORTED && (pk & kOpaque)))
         return;
-    const double b = G.pg()[g];
-    const bool made = ((pk >> kSumExpShift) & 0xffu) == (uint32_t)exponent_of((float)b);
-    const bool replay_s = sum && g >= lead && (sum_changes_binade(G, g) || (PLANNED && !made)), replay_w = walk && walk_changes_binade(G, g, r0);
+    const bool replay_s = sum && g >= lead && sum_changes_binade(G, g), replay_w = walk && walk_changes_binade(G, g, r0);
     if (replay_s || replay_w) {
         const uint32_t s = atomicAdd(&G.misc()[3], 1u);
         if (s < kSlots - 1u) {
@@ -560,7 +553,8 @@ __device__ __forceinline__ void plan_groups(const GroupLds G, uint32_t lead, uin
             G.pack()[g] = pk | ((s + 1u) << kSlotShift);
         }
     }
-    if (!PLANNED && sum && g >= lead && !replay_s && !made)
+    const double b = G.pg()[g];
+    if (sum && g >= lead && !replay_s && ((pk >> kSumExpShift) & 0xffu) != (uint32_t)exponent_of((float)b))
         G.todo()[atomicAdd(&G.misc()[7], 1u)] = (uint16_t)g;
     // (at r = 0 too: the walk passes what weighs nothing there, in a row whose first candidates are behind a masked stretch)
     if (walk && !replay_w && r0 - b >= 0.0 && g != out.group && ((pk >> kWalkExpShift) & 0xffu) != (uint32_t)exponent_of((float)(r0 - b)))
@@ -574,12 +568,15 @@ __device__ __forceinline__ void fill_staged(Keys kf, const GroupLds G, const Lef
         stage_group(kf, G, uniform_u32(G.staged()[s]), s, out);
 }
 
-// The increments to be made.  The calling wave is number `part` of `parts` that share the work; up to four groups per trip
-// to memory.  (Never beside the chain that uses them: plan_groups().)
+// The increments to be made: the running sum's, the walk's.  The calling wave is number `part` of `parts` that share the work; up
+// to four groups per trip to memory.
+// Never beside the chain that uses them: an increment and the binade it is for (in pack()) are two words, and a chain beside the
+// writer could find the old binade with the new increment.  That binade may be the running value's own, where the fp64 sums
+// that the guesses come from lie on the other side of a power of two.
 template <typename Keys>
-__device__ __forceinline__ void build_incs(Keys kf, double r0, const GroupLds G, uint32_t part, uint32_t parts)
+__device__ __forceinline__ void build_incs(Keys kf, double r0, const GroupLds G, bool sum, bool walk, uint32_t part, uint32_t parts)
 {
-    const uint32_t n_sum = uniform_u32(G.misc()[7]), n = n_sum + uniform_u32(G.misc()[8]);
+    const uint32_t n_sum = sum ? uniform_u32(G.misc()[7]) : 0u, n = n_sum + (walk ? uniform_u32(G.misc()[8]) : 0u);
     for (uint32_t i0 = part; i0 < n; i0 += parts * 4u) {
         float q[4][4];
         uint32_t item[4];

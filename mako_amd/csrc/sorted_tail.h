@@ -586,8 +586,8 @@ __device__ bool sorted_tail(const mako_sample_desc& d, uint32_t row, const mako_
 
     // The exact fp32 total, then the walk from u times it (group_chain.h).  Where the binades change, and where the walk
     // ends, is known beforehand but for what the fp64 sums leave open: those groups' entries are fetched now, by all the
-    // waves, and while one wave chains the running sum the others see to the increments for the walk that are missing (the
-    // sum's, where nobody has left any, are made first).
+    // waves, the sum's increments that are missing are made, and while one wave then chains the running sum the others see to
+    // those for the walk.
     const double r0_raw = (double)u_row * G.pg()[groups], r0_guess = r0_raw == r0_raw ? r0_raw : 0.0;
     // (the sum's leading groups: up to the last of the first two in which it changes binade; the second costs half a
     // microsecond one by one, a replay nearly one)
@@ -596,16 +596,17 @@ __device__ bool sorted_tail(const mako_sample_desc& d, uint32_t row, const mako_
     // through costs a microsecond, twelve groups at two nanoseconds an entry six.
     const double head_mass = G.pg()[min(kHeadStaged, groups)];
     bool head_walk = r0_guess * 1.001 <= head_mass || groups <= kHeadStaged;
-    plan_groups<UNSORTED, PLANNED>(G, lead, 0u, groups, true, !head_walk, r0_guess, LeftOut{});
+    plan_groups<UNSORTED>(G, lead, 0u, groups, true, !head_walk, r0_guess, LeftOut{});
     __syncthreads();
     MAKO_STAMP(13);
     fill_staged(kf, G);
-    if (!PLANNED) {
-        build_incs(kf, r0_guess, G, (uint32_t)wave_id(), (uint32_t)kWaves);
+    // (what a worker left for another binade than is expected now: none in most rows, four in some, and the trip is only taken
+    // for some.  Left to the chain to replay instead, tail_kernel took 22.9 us on the 64-row decode batch, 22.4 so)
+    build_incs(kf, r0_guess, G, true, !PLANNED, (uint32_t)wave_id(), (uint32_t)kWaves);
+    if (!PLANNED)
         __syncthreads();
-    } else {
+    else
         lds_barrier();
-    }
     if (wave_id() == 0) {
         float S = 0.0f;
         const bool ok = chain_sum<UNSORTED>(kf, G, groups, lead, lead == groups ? n : uniform_u32(G.start()[lead]), S);
@@ -613,7 +614,7 @@ __device__ bool sorted_tail(const mako_sample_desc& d, uint32_t row, const mako_
         if (lane_id() == 0)
             G.misc()[1] = ok ? __float_as_uint(S) : 0xffffffffu; // (a sum of weights is never a NaN)
     } else if (PLANNED) {
-        build_incs(kf, r0_guess, G, (uint32_t)wave_id() - 1u, (uint32_t)kWaves - 1u);
+        build_incs(kf, r0_guess, G, false, true, (uint32_t)wave_id() - 1u, (uint32_t)kWaves - 1u);
     }
     __syncthreads();
     MAKO_STAMP(8);
@@ -635,10 +636,10 @@ __device__ bool sorted_tail(const mako_sample_desc& d, uint32_t row, const mako_
             G.pack()[tid] &= (1u << kSlotShift) - 1u;
         const double r0_here = r_here + G.pg()[from];
         __syncthreads();
-        plan_groups<UNSORTED, PLANNED>(G, 0u, from, groups, false, true, r0_here, out);
+        plan_groups<UNSORTED>(G, 0u, from, groups, false, true, r0_here, out);
         __syncthreads();
         fill_staged(kf, G, out);
-        build_incs(kf, r0_here, G, (uint32_t)wave_id(), (uint32_t)kWaves);
+        build_incs(kf, r0_here, G, false, true, (uint32_t)wave_id(), (uint32_t)kWaves);
         __syncthreads();
     };
     uint32_t dp = kNone;
