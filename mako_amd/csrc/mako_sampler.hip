@@ -439,7 +439,7 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
         }                                                                                                          \
     } while (0)
     MAKO_MARK(0);
-    MAKO_LAUNCH(mako::launch_scan(vec, kh, d.close_token != nullptr, grid, lds, st, d, sc, slice_len, (ctx->cus & 0xffffu) | ((finish_wgs / 8u) << 16)));
+    MAKO_LAUNCH(mako::launch_scan(vec, kh, d.close_token != nullptr, grid, lds, st, d, sc, slice_len, std::min(ctx->cus, mako::kCountGeneral - 1u) | (beside ? mako::kCountGeneral : 0u) | ((finish_wgs / 8u) << 16)));
     MAKO_MARK(1);
     // top_k == 0 rows: planned and handed out by the second pass, sorted, cut and drawn from; the stages talk through
     // kernel boundaries (device-wide fences inside a kernel cost far more on this chip).  A batch without such rows

@@ -140,7 +140,8 @@ __host__ __device__ inline SortLists large_batch_lists(uint32_t n_rows)
     return SortLists{2u * n_rows};
 }
 
-constexpr uint32_t kWorkWords = 12; // of Scratch::work_n
+constexpr uint32_t kWorkWords = 12;        // of Scratch::work_n
+constexpr uint32_t kCountGeneral = 0x8000u; // scan_kernel: leave the number of rows of the whole-row class (beside_rows.h)
 struct Scratch {
     SliceStat* stats;  // [max_rows][kMaxSlices]
     float* cand_w;     // [max_rows][slices_cap][kCap] penalised logits of the slice's candidates
@@ -162,8 +163,8 @@ struct Scratch {
     // (finish_kernel and plan_kernel get the same effect from find_piece().)
     uint32_t* work_n;      // [kWorkWords] entries in work_sort, work_tail (zeroed by scan_kernel); [3]: the large batches' collectors; [2]: failed checks of a checked
                            // build (MAKO_CHECK); then, 16-byte aligned at [4], how the second pass is cut up
-                           // (SecondPassCut; scan_kernel's first workgroup decides), and at [8] the rows of the
-                           // whole-row class and those of them in token order
+                           // (SecondPassCut; scan_kernel's first workgroup decides), and at [8], for launches that serve
+                           // them beside others, the rows of the whole-row class and those of them in token order
     uint32_t* work_sort;   // [max_rows * kSortItemsPerRow] row << 8 | worker; appended by finish_kernel.  The large batches'
                            // instances keep two lists in it that meet, the costliest entries in front (large_batch_lists())
     uint32_t* work_tail;   // [max_rows] row; appended by finish_kernel

@@ -20,9 +20,10 @@ struct SecondPassCut {
     // and of the rows of the whole-row class (index_rows.h): all of them, those in token order
     uint32_t general, in_order;
 };
-// finish_grid: the workgroups finish_kernel is launched with (second_pass_grid()).
+// finish_grid: the workgroups finish_kernel is launched with (second_pass_grid()).  count_general: the rows of the whole-row
+// class are wanted too (counted for every batch, they cost a 64-row decode batch without any 0.3 of its 66 us).
 __device__ __forceinline__ SecondPassCut second_pass_cut(const mako_sample_desc& d, uint32_t slices, uint32_t slice_len,
-                                                         uint32_t cus, uint32_t finish_grid)
+                                                         uint32_t cus, uint32_t finish_grid, bool count_general)
 {
     uint32_t rows = 0; // top_k == 0 rows of the batch (every lane ends up with the count)
     SecondPassCut cut;
@@ -32,8 +33,10 @@ __device__ __forceinline__ SecondPassCut second_pass_cut(const mako_sample_desc&
         const mako_sampling_params P = d.params[min(r, d.n_rows - 1u)];
         const RowClass cls = classify(P);
         rows += (uint32_t)__popcll(__ballot(r < d.n_rows && cls == kNucleus));
-        cut.general += (uint32_t)__popcll(__ballot(r < d.n_rows && cls == kGeneral));
-        cut.in_order += (uint32_t)__popcll(__ballot(r < d.n_rows && index_order_row(P)));
+        if (count_general) { // uniform
+            cut.general += (uint32_t)__popcll(__ballot(r < d.n_rows && cls == kGeneral));
+            cut.in_order += (uint32_t)__popcll(__ballot(r < d.n_rows && index_order_row(P)));
+        }
     }
     cut.piece_len = slice_len;
     cut.pieces = slices;

@@ -1,5 +1,5 @@
 """Kernels that many workgroups run must not use scratch memory: it slows down the start of every workgroup, those without
-work included (sort_beside_kernel with 20 bytes of it: 8 704 workgroups without work 31 us instead of 20)."""
+work included (20 bytes of it: 3 us for a launch of 8 704 workgroups without work)."""
 import os
 import re
 import struct
