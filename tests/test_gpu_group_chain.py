@@ -104,3 +104,25 @@ def test_walks_from_zero_behind_a_masked_stretch(gpu_ctx, masked):
         g = gpu_rows(gpu_ctx, w, draft=draft, u2=u2, hinted=True)
         for r, (t, tr) in enumerate(oracle_rows(w, draft=draft, u2=u2)):
             assert g["tokens"][r] == t and bool(g["accepted"][r]) == bool(tr["accepted"]), (r, g["tokens"][r], t)
+
+
+@pytest.mark.parametrize("first", [3070, 3071, 3072, 3200, 3385, 65536, 129000])
+@pytest.mark.parametrize("hinted", [False, True])
+def test_redraws_from_zero_behind_the_staged_head(gpu_ctx, first, hinted):
+    """A rejected draft that is the row's first candidate, behind the part of the list that is kept in LDS, and a redraw from
+    u2 = 0: the walk passes the head at r = 0 and must not find the draft in its group's entries, which were fetched for
+    the sum."""
+    rng = np.random.default_rng(first)
+    rows, vocab = 8, 129280
+    logits = np.full((rows, vocab), -np.inf, np.float32)
+    logits[:, first] = rng.uniform(-1.0, 1.0, rows)
+    for r in range(rows):
+        others = rng.integers(first + 1, vocab, 2 + 40 * r)
+        logits[r, others] = rng.uniform(-2.0, 2.0, len(others))
+    u = np.linspace(0.6, 0.99, rows).astype(np.float32)
+    w = dict(name="redraw from zero", logits=logits, u=u, params=api.make_params(rows, 1.0, 0, 1.0))
+    draft = np.full(rows, first, np.int32)
+    for u2 in (np.zeros(rows, np.float32), np.full(rows, 2.0**-149, np.float32), np.full(rows, 2.0**-24, np.float32)):
+        g = gpu_rows(gpu_ctx, w, draft=draft, u2=u2, hinted=hinted)
+        for r, (t, tr) in enumerate(oracle_rows(w, draft=draft, u2=u2)):
+            assert g["tokens"][r] == t and bool(g["accepted"][r]) == bool(tr["accepted"]), (r, g["tokens"][r], t)
