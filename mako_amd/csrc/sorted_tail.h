@@ -664,23 +664,18 @@ __device__ bool sorted_tail(const mako_sample_desc& d, uint32_t row, const mako_
                 __syncthreads();
                 if (tid == 0) {
                     G.winc()[out.group] = make_float2(INFINITY, INFINITY);
-                    G.pack()[out.group] &= ~(0xffu << kWalkExpShift);
+                    // (nor a slot: what was fetched for the sum holds the draft, and a walk that was expected to end in the head
+                    // passes it at r = 0 where nothing in it weighs anything)
+                    G.pack()[out.group] &= ~(0xffu << kWalkExpShift) & ((1u << kSlotShift) - 1u);
                 }
             }
         }
         const double rg = r == r ? (double)r : 0.0;
         head_walk = rg * 1.001 <= G.pg()[min(kHeadStaged, groups)] || groups <= kHeadStaged;
-        if (!head_walk) {
+        if (!head_walk)
             prepare_walk(0u, rg);
-        } else if (q_draft > 0.0f && tid == 0) { // (read by wave 0 alone)
-            // (in the staged head, and in the slot of its group: a walk expected to end in the head passes it where nothing in
-            // it weighs anything, and goes on with the slots as they were filled for the sum)
-            if (dp < kHeadLen)
-                head[dp] = 0.0f;
-            const uint32_t slot = out.group != kNone ? G.pack()[out.group] >> kSlotShift : 0u;
-            if (slot)
-                G.slot(slot - 1u)[out.entry] = 0.0f;
-        }
+        else if (q_draft > 0.0f && dp < kHeadLen && tid == 0) // (read by wave 0 alone)
+            head[dp] = 0.0f;
     }
 
     uint32_t pos = n - 1;
