@@ -34,7 +34,7 @@ __global__ __launch_bounds__(kThreads) void finish_beside_kernel(mako_sample_des
         uint32_t row;
         if (!rows.find(d_arg, p / pieces, [](const mako_sampling_params& P) { return classify(P) == kGeneral; }, row))
             return;
-        index_weights_piece<VEC, KH>(d_arg, sc_val, slices, row, p % pieces, s_dyn64, sm, s_args);
+        index_weights_piece<VEC, KH, true>(d_arg, sc_val, slices, row, p % pieces, s_dyn64, sm, s_args);
         __syncthreads(); // (the next piece's table of counts and arguments)
     }
 }
@@ -52,7 +52,7 @@ __global__ __launch_bounds__(kThreads) void sort_beside_kernel(mako_sample_desc 
     // been, the compiler takes no scalar loads, and thousands of workgroups without work wait for nothing but this trip.
     // 8 704 of them: 31 us with vector loads, a trip of their own for the arguments and, short of registers, scratch memory; 23 now, 20.6 in
     // sort_kernel)
-    const uint32_t in_order = sc_val.work_n[9];
+    const uint32_t general = sc_val.work_n[8], in_order = sc_val.work_n[9];
     SortFirstTrip first;
     fetch_sort_entry<UNSORTED>(d_arg, sc_val, min(blockIdx.y, max(sort_rows, 1u) - 1u) * gridDim.x + blockIdx.x, first);
     if (blockIdx.y < sort_rows) {
@@ -61,8 +61,22 @@ __global__ __launch_bounds__(kThreads) void sort_beside_kernel(mako_sample_desc 
     }
     const uint32_t blocks = (d_arg.n_vocab + kIndexBlock - 1u) / kIndexBlock;
     const uint32_t all = in_order * blocks;
+    const uint32_t me = (blockIdx.y - sort_rows) * gridDim.x + blockIdx.x, wgs = (gridDim.y - sort_rows) * gridDim.x;
+    // (nth_steps.h's first step, as many workgroups a row as there are; the groups' workgroups are counted from the other end)
+    const uint32_t nth_rows = nth_steps_for(d_arg.n_vocab) ? general - in_order : 0u;
+    if (nth_rows) { // uniform
+        const uint32_t per_row = min(max(wgs / nth_rows, 1u), (d_arg.n_vocab + kNthChunk - 1u) / kNthChunk);
+        RankedRows rows;
+        for (uint32_t p = me; p < nth_rows * per_row; p += wgs) {
+            uint32_t row;
+            if (!rows.find(d_arg, p / per_row, [](const mako_sampling_params& P) { return nth_row(P); }, row))
+                break;
+            nth_step(d_arg, sc_val, row, p % per_row, per_row, 1u, s_dyn64, sm.bs);
+            __syncthreads();
+        }
+    }
     RankedRows rows;
-    for (uint32_t p = (blockIdx.y - sort_rows) * gridDim.x + blockIdx.x; p < all; p += (gridDim.y - sort_rows) * gridDim.x) {
+    for (uint32_t p = wgs - 1u - me; p < all; p += wgs) {
         uint32_t row;
         if (!rows.find(d_arg, p / blocks, [](const mako_sampling_params& P) { return index_order_row(P); }, row))
             return;

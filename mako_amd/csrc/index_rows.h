@@ -17,12 +17,13 @@
 // ends when it runs off its list.  Verification works on the same list: the draft's weight is entry `draft`, and a
 // rejected draft is redrawn with that entry taken as 0.0f (sorted_tail's UNORDERED instance).
 // The other rows of the whole-row class (top-k without top-p, top-k beyond the candidate lists) only get their weights
-// here (into the array general_row_from_weights() starts from) and one workgroup each in the last launch for the rest of the
-// whole-row path.
+// here (into the array general_row_from_weights() starts from), the first rounds of their nth_element (nth_steps.h), and one
+// workgroup each in the last launch for the rest of the whole-row path.
 #pragma once
 
 #include "sorted_tail.h"
 #include "worker_sort.h"
+#include "nth_steps.h"
 #include "whole_row.h"
 
 namespace mako {
@@ -32,9 +33,71 @@ constexpr uint32_t kIndexMaxVocab = kMaxGroups * kGroup; // the group records of
 static_assert(kIndexMaxVocab / kSliceMax <= kWorkers && kIndexMaxVocab / kIndexBlock <= kMaxSlices && kIndexMaxVocab / kIndexBlock <= (uint32_t)kWave &&
                   kSliceMax == 4u * kIndexBlock && kIndexBlock == (uint32_t)kWaves * kGroup,
               "a piece's count and last candidate travel in the plan's per-worker words, the blocks' sums in the row's part_sum, a lane each");
+// The pivot of the first round of nth_element on a row that is its own list (no gaps): the median of the weights of its second
+// logit, its middle and its last one.  A barrier later sm.bs.u64[0] is the pivot, [1] the first entry, sm.aux where the pivot
+// is.  hl: the history's length, 0 where there is nothing to penalise.  All threads call.
+__device__ __forceinline__ void first_pivot(const mako_sample_desc& d, uint32_t row, const mako_sampling_params& P, uint32_t hl, float m, FinishShared& sm)
+{
+    typedef unsigned long long u64;
+    const uint32_t places[4] = {1u, d.n_vocab / 2u, d.n_vocab - 1u, 0u}, mine = min((uint32_t)lane_id(), 3u);
+    const uint32_t at = mine == 0u ? places[0] : (mine == 1u ? places[1] : (mine == 2u ? places[2] : places[3]));
+    if (hl) { // uniform
+        if (threadIdx.x < 4u)
+            sm.run[threadIdx.x] = 0u;
+        lds_barrier();
+        const global_ptr<const int32_t> ht = as_global(d.hist_tokens) + (int64_t)row * d.hist_stride;
+        const global_ptr<const uint32_t> hc = d.hist_counts ? as_global(d.hist_counts) + (int64_t)row * d.hist_stride : nullptr;
+        for (uint32_t h = threadIdx.x; h < hl; h += kThreads) {
+            const uint32_t t = (uint32_t)ht[h];
+#pragma unroll
+            for (uint32_t i = 0; i < 4; ++i)
+                if (t == places[i])
+                    atomicAdd(&sm.run[i], hc ? hc[h] : 1u);
+        }
+        lds_barrier();
+    }
+    if (wave_id() == 0) {
+        float w = as_global(d.logits)[(int64_t)row * d.logits_stride + at];
+        const uint32_t word = d.mask ? as_global(d.mask)[(int64_t)row * d.mask_stride + (at >> 5)] : ~0u;
+        w = (word >> (at & 31u)) & 1u ? w : -INFINITY;
+        const uint32_t c = hl ? sm.run[mine] : 0u;
+        if (c)
+            w = penalize(w, c, P.repetition_penalty, P.presence_penalty, P.frequency_penalty);
+        const uint32_t key = ~__float_as_uint(weight_of(w, m, 1.0f / P.temperature, sm.tab));
+        auto entry = [&](int i) { return ((u64)(uint32_t)__builtin_amdgcn_readlane((int)key, i) << 32) | (u64)places[i]; };
+        u64 med;
+        uint32_t from;
+        median_of_three<u64>(entry(0), entry(1), entry(2), places[0], places[1], places[2], med, from);
+        if (lane_id() == 0) {
+            sm.bs.u64[0] = med;
+            sm.bs.u64[1] = entry(3);
+            sm.aux = from;
+        }
+    }
+}
+
+// A thread's four bits (entries as elem_index() has them, the first at `base`), whole blocks of 256 entries at a time.
+template <bool VEC>
+__device__ __forceinline__ void store_nth_bits(global_ptr<uint32_t> words, uint32_t base, uint32_t four)
+{
+    if (VEC) {
+        const uint32_t word = eight_nibbles(four);
+        if ((lane_id() & 7) == 0)
+            words[base >> 5] = word;
+    } else {
+#pragma unroll
+        for (uint32_t c = 0; c < 4; ++c) {
+            const unsigned long long m = __builtin_amdgcn_ballot_w64((four >> c) & 1u);
+            if (lane_id() == 0)
+                *(global_ptr<unsigned long long>)(words + ((base + c * (uint32_t)kThreads) >> 5)) = m;
+        }
+    }
+}
+
 // Piece `piece` of row `row`; of a row of another kind nothing.  (VEC: V % 4 == 0 and 16-byte aligned rows, whose
-// logits are loaded four at a time; the layout of a thread's sixteen logits is slice_load.h's either way.)
-template <bool VEC, int KH>
+// logits are loaded four at a time; the layout of a thread's sixteen logits is slice_load.h's either way.  STEPS: there may be
+// rows for nth_steps.h, whose bits take the registers that let two workgroups share a CU.)
+template <bool VEC, int KH, bool STEPS>
 __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_arg, const Scratch& sc_val, uint32_t slices, uint32_t row, uint32_t piece,
                                                     unsigned long long* s_dyn64, FinishShared& sm, ArgsLds& s_args)
 {
@@ -68,9 +131,20 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
     const bool pen = d.hist_tokens && !penalties_neutral(P);
     const uint32_t lo = piece * kSliceMax, hi = min(d.n_vocab, lo + kSliceMax);
     float wv[16];
-    load_penalised<VEC, KH>(d, row, lo, hi, kSliceMax, P, hl, pen, reinterpret_cast<uint32_t*>(s_dyn64), wv);
+    // (a row for nth_steps.h: the first round's pivot if every logit should turn out to be a candidate)
+    const bool steps = STEPS && !in_order && nth_steps_for(d.n_vocab); // uniform
+    load_penalised<VEC, KH>(d, row, lo, hi, kSliceMax, P, hl, pen, reinterpret_cast<uint32_t*>(s_dyn64), wv, [&]() {
+        if (steps)
+            first_pivot(d, row, P, pen ? hl : 0u, m, sm);
+    });
     const float inv_t = 1.0f / P.temperature;
     const float floor_q = (1.0f < P.min_p) ? 1.0f : P.min_p;
+    NthFirst first = {0u, 0u, 0u, 0u}; // (in scalar registers)
+    if (steps) {
+        lds_barrier();
+        first = NthFirst{uniform_u32((uint32_t)(sm.bs.u64[0] >> 32)), uniform_u32((uint32_t)sm.bs.u64[0]), uniform_u32(sm.aux),
+                         uniform_u32((uint32_t)(sm.bs.u64[1] >> 32))};
+    }
     // (~bits(q), at the token's own position)
     uint32_t* key0 = sc.key[0] + (size_t)row * sc.vpad;
     MAKO_CHECK(sc, kCheckStage, (uint64_t)hi <= sc.vpad);
@@ -101,7 +175,22 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
                     if (elem_index<VEC>(lo, tid, 4u * b + c) < hi)
                         key0[elem_index<VEC>(lo, tid, 4u * b + c)] = ~k[c];
             }
-            if (!in_order) { // uniform
+            if (steps) { // uniform
+                // who is a candidate, and who belongs left of the pivot: bits for nth_steps.h's first step
+                uint32_t is = 0, left = 0;
+#pragma unroll
+                for (uint32_t c = 0; c < 4; ++c) {
+                    const uint32_t at = elem_index<VEC>(lo, tid, 4u * b + c);
+                    // (where the pivot was, the first entry is now, token 0)
+                    const bool moved = at == first.from;
+                    const uint32_t key = moved ? first.first_key : ~k[c];
+                    const bool lighter = key < first.pivot_key || (key == first.pivot_key && (moved || at < first.pivot_id));
+                    is |= (k[c] ? 1u : 0u) << c;
+                    left |= (at != 0u && at < hi && lighter ? 1u : 0u) << c;
+                }
+                store_nth_bits<VEC>(as_global(nth_bits(sc, row, 2u)), base, is);
+                store_nth_bits<VEC>(as_global(nth_bits(sc, row, 0u)), base, left);
+            } else if (!in_order) { // uniform
                 // the token ids as well: with them this is the whole-row path's list of candidates when every logit turns out
                 // to be one, as the pieces' counts will tell
                 uint32_t* li = sc.idx[0] + (size_t)row * sc.vpad;
@@ -155,6 +244,10 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
         plan->cursor[piece] = cnt; // (the pieces' counts and last candidates travel in the plan's per-worker words)
         plan->key_lo[piece] = last;
         if (piece == 0) {
+            if (STEPS) {
+                nth_state(plan, 0u)->seq = nth_state(plan, 1u)->seq = 0u;
+                *nth_first(plan) = first;
+            }
             plan->flag = kIndexClaimed;
             plan->m = m;
             plan->argidx = argidx;
@@ -238,7 +331,9 @@ __device__ __forceinline__ void index_groups_block(const mako_sample_desc& d_arg
 }
 
 // What these kernels have left of a row of theirs (flag: of its plan, which is zero again behind this), by one workgroup: the
-// rest of the whole-row path, or the total and the draw.  All threads call; sm.tab must hold the exp2 table.
+// rest of the whole-row path, or the total and the draw.  All threads call; sm.tab must hold the exp2 table.  ALL_KINDS: rows
+// that are not in token order are among them (their code costs the others' kernel scratch memory, 0.7 of 78 us on 64 rows).
+template <bool ALL_KINDS = true>
 __device__ __forceinline__ void finish_index_row_here(const mako_sample_desc& d, const Scratch& sc, const mako_sampling_params& P, uint32_t row,
                                                       const FinishLds& L)
 {
@@ -257,8 +352,9 @@ __device__ __forceinline__ void finish_index_row_here(const mako_sample_desc& d,
         plan->flag = 0;
     if (!index_order_row(P)) {
         // the whole-row path from the weights index_weights_kernel left (the group records' kernel has not touched the row)
-        if (flag == kIndexClaimed)
-            general_row_from_weights<0>(d, sc, row, P, m, argidx, uniform_u32(counted) == d.n_vocab, L);
+        if constexpr (ALL_KINDS)
+            if (flag == kIndexClaimed)
+                general_row_from_weights<0>(d, sc, row, P, m, argidx, uniform_u32(counted), L);
         return;
     }
     if (flag == kIndexEmpty) {
@@ -315,14 +411,14 @@ struct RankedRows {
 #ifdef MAKO_EMIT_INDEX_KERNELS
 // grid = (rows rounded up to a multiple of eight, ceil(V / 16384)): workgroups go to the eight XCDs in turn, so that all of
 // these kernels work on a row on the same one.
-template <bool VEC, int KH>
+template <bool VEC, int KH, bool STEPS>
 __global__ __launch_bounds__(kThreads) void index_weights_kernel(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices)
 {
     extern __shared__ __align__(16) unsigned long long s_dyn64[];
     __shared__ FinishShared sm;
     __shared__ ArgsLds s_args;
     if (blockIdx.x < d_arg.n_rows)
-        index_weights_piece<VEC, KH>(d_arg, sc_val, slices, blockIdx.x, blockIdx.y, s_dyn64, sm, s_args);
+        index_weights_piece<VEC, KH, STEPS>(d_arg, sc_val, slices, blockIdx.x, blockIdx.y, s_dyn64, sm, s_args);
 }
 
 // grid = (rows rounded up to a multiple of eight, ceil(V / (4096 GPW))).
@@ -334,7 +430,19 @@ __global__ __launch_bounds__(kThreads) void index_groups_kernel(mako_sample_desc
         index_groups_block<GPW>(d_arg, sc_val, blockIdx.x, blockIdx.y, s_gs);
 }
 
+// grid = (rows rounded up to a multiple of eight, workgroups per row): a step of nth_steps.h.
+// (Two workgroups share a CU only with 80 scalar registers each, all in all: with 82 the second half of the first step's 512
+// started 16 us after the first.)
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_num_sgpr(80))) void nth_step_kernel(mako_sample_desc d_arg, Scratch sc_val, uint32_t step)
+{
+    extern __shared__ __align__(16) unsigned long long s_dyn64[];
+    __shared__ BlockScratch s_bs;
+    if (blockIdx.x < d_arg.n_rows)
+        nth_step(d_arg, sc_val, blockIdx.x, blockIdx.y, gridDim.y, step, s_dyn64, s_bs);
+}
+
 // grid = (1, rows).
+template <bool ALL_KINDS>
 __global__ __launch_bounds__(kThreads) void index_tail_kernel(mako_sample_desc d_arg, Scratch sc_val)
 {
     extern __shared__ __align__(16) unsigned long long s_dyn64[];
@@ -348,7 +456,7 @@ __global__ __launch_bounds__(kThreads) void index_tail_kernel(mako_sample_desc d
         sm.tab[threadIdx.x] = k_exp2_tab[threadIdx.x];
     stage_args(d_arg, sc_val, row, s_args);
     const FinishLds views = finish_lds_views(sm, s_dyn64);
-    finish_index_row_here(s_args.d, s_args.sc, s_args.P, row, views);
+    finish_index_row_here<ALL_KINDS>(s_args.d, s_args.sc, s_args.P, row, views);
 }
 #endif // MAKO_EMIT_INDEX_KERNELS
 

@@ -37,8 +37,11 @@ void launch_tail(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, u
 // the three kernels of a batch with none but rows of the whole-row class (index_rows.h): the weights, the group records, the
 // total and the draw
 hipError_t init_index_kernels();
-void launch_index_weights(bool vec, int kh, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices);
-void launch_index_finish(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, bool in_order_rows);
+// (steps: there are rows for nth_steps.h)
+void launch_index_weights(bool vec, int kh, bool steps, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices);
+// a step of nth_steps.h, `wgs` workgroups per row
+void launch_nth_step(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t step, uint32_t wgs);
+void launch_index_finish(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, bool in_order_rows, bool other_rows);
 // finish, sort and tail of a batch where such rows are, or may be, beside others (beside_rows.h): the same launches with
 // `more` workgroups behind their own for those rows
 hipError_t init_beside_finish();

@@ -400,10 +400,11 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
     // (index_rows.h: the rows of the whole-row class, unless the vocabulary is beyond 262 144; only_index: the batch has no
     // others, and they get launches of their own; beside: it has, or may have, and they take part in the others' launches)
     const bool index_served = d.n_vocab <= mako::kIndexMaxVocab;
-    bool any_nucleus = true, any_late = true, only_index = false, any_in_order = false, beside = index_served;
+    // (any_unordered: those of the class that are not in token order)
+    bool any_nucleus = true, any_late = true, only_index = false, any_in_order = false, beside = index_served, any_unordered = index_served;
     uint32_t nucleus_rows = d.n_rows, index_rows = d.n_rows;
     if (params_host) {
-        any_nucleus = any_late = false;
+        any_nucleus = any_late = any_unordered = false;
         uint32_t n_nucleus = 0, n_index = 0;
         for (uint32_t r = 0; r < d.n_rows; ++r) {
             const mako::RowClass c = mako::classify(params_host[r]);
@@ -412,6 +413,7 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
             any_late |= c == mako::kGeneral && !index_row;
             n_index += index_row;
             any_in_order |= index_row && mako::index_order_row(params_host[r]);
+            any_unordered |= index_row && !mako::index_order_row(params_host[r]);
             n_nucleus += c == mako::kNucleus;
         }
         nucleus_rows = std::max(n_nucleus, 1u);
@@ -419,6 +421,12 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
         beside = n_index != 0 && !only_index;
         index_rows = n_index;
     }
+    const bool any_nth = any_unordered && mako::nth_steps_for(d.n_vocab);
+    // (their steps: a launch each, of about two workgroups per CU.  Beside other rows the sort's launch has the first.  A launch
+    // costs 8 to 10 us and leaves 0.44 of a row: as many as bring the 64 rows' unluckiest near what a workgroup takes into its
+    // registers.  64 rows of 129 280: 185 us with two, 172, 164, 162, 168 with six; of 40 000: 104 with two, 105, 110)
+    const uint32_t nth_wgs = std::min(std::max(2u * ctx->cus / ((d.n_rows + 7u) & ~7u), 1u), (d.n_vocab + mako::kNthChunk - 1u) / mako::kNthChunk);
+    const uint32_t nth_steps = !any_nth ? 0u : (d.n_vocab <= 65536u ? 2u : 4u);
     const bool launch_sort = any_nucleus || any_late || beside;
     // (finish_kernel's grid: scan_kernel, which cuts the second pass up, is told of it)
     const uint32_t finish_wgs = mako::second_pass_grid(d.n_rows, nucleus_rows, ctx->cus);
@@ -451,13 +459,15 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
         const uint32_t for_groups = (uint32_t)std::min<uint64_t>((uint64_t)index_rows * blocks, ctx->cus);
         MAKO_LAUNCH(mako::launch_finish_beside(vec, kh, unsorted, any_nucleus ? finish_wgs : 0u, for_weights, st, d, sc, slices));
         MAKO_MARK(2);
-        if (any_nucleus || any_in_order || !params_host)
+        if (any_nucleus || any_in_order || any_nth || !params_host)
             MAKO_LAUNCH(mako::launch_sort_beside(st, d, sc, slices, any_nucleus ? nucleus_rows : 0u, unsorted, for_groups));
         MAKO_MARK(3);
+        for (uint32_t step = 2u; params_host && step <= nth_steps; ++step)
+            MAKO_LAUNCH(mako::launch_nth_step(st, d, sc, step, nth_wgs));
         MAKO_LAUNCH(mako::launch_tail_beside(st, d, sc, slices, nucleus_rows, unsorted));
     } else {
         if (only_index)
-            MAKO_LAUNCH(mako::launch_index_weights(vec, kh, st, d, sc, slices));
+            MAKO_LAUNCH(mako::launch_index_weights(vec, kh, any_nth, st, d, sc, slices));
         if (any_nucleus)
             MAKO_LAUNCH(mako::launch_finish(vec, kh, unsorted, finish_wgs, st, d, sc, slices));
         if (!launch_sort && !only_index)
@@ -468,8 +478,10 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
         MAKO_MARK(3);
         if (launch_sort) // (also finishes every row the kernels before it leave: finish_late_row())
             MAKO_LAUNCH(mako::launch_tail(st, d, sc, slices, nucleus_rows, unsorted));
+        for (uint32_t step = 1u; only_index && step <= nth_steps; ++step)
+            MAKO_LAUNCH(mako::launch_nth_step(st, d, sc, step, nth_wgs));
         if (only_index)
-            MAKO_LAUNCH(mako::launch_index_finish(st, d, sc, any_in_order));
+            MAKO_LAUNCH(mako::launch_index_finish(st, d, sc, any_in_order, any_unordered));
     }
     MAKO_MARK(4);
 #undef MAKO_MARK

@@ -1,0 +1,331 @@
+// The first rounds of the whole-row class's nth_element (whole_row.h), with several workgroups per row.
+//
+// libstdc++'s introselect halves its range round by round, and one workgroup is bound by what its CU can read and move: a row
+// of 129 280 candidates kept it 88 us before what is left fits its registers (186 for the row with the unluckiest pivots of
+// 64), while three quarters of the chip had nothing to do.  A round needs its pivot, the number of entries that belong left of
+// it, and for every entry that moves its place, all of which follow from one bit per entry ("belongs left").  So a launch in
+// which several workgroups share a row (a "step") makes a round out of the bits that the launch before left, and leaves the
+// next round's:
+//   index_weights_kernel   weights a workgroup per 16 384 logits; a row whose every logit is a candidate is its own list, so
+//                          the first pivot is the median of three logits known beforehand: leaves the first round's bits
+//                          (and the bits of who is a candidate);
+//   step 1                 such a row: the first round.  Any other: the candidates moved together.
+//   step 2, 3, ...         a round each, until what is left fits a workgroup's registers (kNthUntil), where the row's one
+//                          workgroup goes on in the last launch.
+// A step writes the list it makes beside the old one, with the next round's pivot already swapped to the front; its workgroups
+// take 4 096 entries of the new list at a time.  An entry that belongs left and lies in front of the cut stays where it is; a
+// hole's filler comes through LDS: the holes of 4 096 places in a row are filled from one stretch of the old list, from its
+// end backwards.
+#pragma once
+
+#include "sampler_common.h"
+#include "workgroup_state.h"
+
+namespace mako {
+
+constexpr uint32_t kNthUntil = 16380;       // entries that a workgroup takes into registers wherever they begin
+constexpr uint32_t kNthChunk = 4096;        // of the new list, per workgroup and turn: four per thread
+constexpr uint32_t kNthMaxVocab = kMaxGroups * kGroup;
+constexpr uint32_t kNthWords = kNthMaxVocab / 64u; // of a row's bits
+constexpr uint32_t kNthLds = kNthChunk * 8u + kNthWords * 12u + 64u;
+
+// Where a row stands: two records in turn in the row's plan (a step reads one and writes the other), in the words its workers
+// would use.  seq: steps made, 0: none yet.  len entries of key[buf] / idx[buf] are what is left of the list, `used` rounds
+// behind them.  pre: the next round's pivot is at the front and its bits are in place.
+struct alignas(4) NthState {
+    uint32_t seq, len, pre, used, buf;
+};
+static_assert(2u * sizeof(NthState) <= sizeof(BigPlan::cap), "");
+// The first pivot of a row that is its own list, where it came from, and the key of its first entry.
+struct NthFirst {
+    uint32_t pivot_key, pivot_id, from, first_key;
+};
+__device__ __forceinline__ NthState* nth_state(BigPlan* plan, uint32_t slot)
+{
+    return reinterpret_cast<NthState*>(plan->cap) + slot;
+}
+__device__ __forceinline__ NthFirst* nth_first(BigPlan* plan)
+{
+    return reinterpret_cast<NthFirst*>(plan->stage_off);
+}
+// A row's bits, entry i at bit i & 31 of word i >> 5, in the memory of its penalised logits: of the list in key[buf], and of
+// the row's candidates (buf = 2).  (Written in blocks of 256 entries.)
+__device__ __forceinline__ uint32_t* nth_bits(const Scratch& sc, uint32_t row, uint32_t buf)
+{
+    return reinterpret_cast<uint32_t*>(sc.wbuf + (size_t)row * sc.vpad) + buf * (uint32_t)(sc.vpad / 32u + 256u);
+}
+// Is the row one of these?  (The others of its class stay in token order: index_rows.h.)
+__device__ __forceinline__ bool nth_row(const mako_sampling_params& P)
+{
+    return classify(P) == kGeneral && P.top_k != 0u;
+}
+// Are there steps for rows of this many logits?
+__host__ __device__ __forceinline__ bool nth_steps_for(uint32_t n_vocab)
+{
+    return n_vocab > kNthUntil && n_vocab <= kNthMaxVocab;
+}
+
+__device__ __forceinline__ uint32_t mask_rank(unsigned long long m)
+{
+    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
+}
+
+// The median of three and its position (__move_median_to_first(first, first + 1, mid, last - 1)).
+template <typename T>
+__device__ __forceinline__ void median_of_three(T vx, T vy, T vz, uint32_t ix, uint32_t iy, uint32_t iz, T& med, uint32_t& im)
+{
+    const bool xy = vx < vy, yz = vy < vz, xz = vx < vz;
+    im = xy == yz ? iy : (xy == xz ? iz : ix);
+    med = xy == yz ? vy : (xy == xz ? vz : vx);
+}
+
+// Four bits per lane (of entries 4 l .. 4 l + 3) as words of 32: the first lane of every eight holds theirs.
+__device__ __forceinline__ uint32_t eight_nibbles(uint32_t nibble)
+{
+    uint32_t v = nibble << (4u * ((uint32_t)lane_id() & 7u));
+    v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0xb1, 0xf, 0xf, false);  // quad_perm: lane ^ 1
+    v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x4e, 0xf, 0xf, false);  // quad_perm: lane ^ 2
+    v |= (uint32_t)__builtin_amdgcn_mov_dpp((int)v, 0x141, 0xf, 0xf, false); // row_half_mirror: the other four
+    return v;
+}
+
+// One step of row `row`, by workgroup w of W.  lds: kNthLds bytes (what the row's bits take of it).  All threads call.
+__device__ __forceinline__ void nth_step(const mako_sample_desc& d, const Scratch& sc, uint32_t row, uint32_t w, uint32_t W, uint32_t step,
+                                         unsigned long long* lds_dyn, BlockScratch& bs)
+{
+    typedef unsigned long long u64;
+    const uint32_t tid = threadIdx.x, lane = lane_id(), wave = wave_id();
+    BigPlan* plan = sc.plan + row;
+    const uint32_t pieces = (d.n_vocab + kSliceMax - 1u) / kSliceMax;
+    // (one trip to memory)
+    const uint32_t flag = plan->flag, counted = plan->cursor[min(lane, kWorkers - 1u)];
+    const mako_sampling_params P = d.params[row];
+    NthState now = *nth_state(plan, (step - 1u) & 1u);
+    const NthFirst first = *nth_first(plan);
+    static_assert(kNthWords <= 4u * (uint32_t)kThreads, "four words of bits a thread");
+    const uint32_t usual = (step - 1u) & 1u, words_max = (d.n_vocab + 63u) / 64u; // (where the bits of a row that goes on are)
+    u64 x[4];
+    auto load_bits = [&](uint32_t buf, uint32_t words) {
+        const global_ptr<const u64> from = (global_ptr<const u64>)as_global(nth_bits(sc, row, buf));
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i)
+            x[i] = from[min(4u * tid + i, words - 1u)];
+    };
+    load_bits(usual, words_max);
+    const uint32_t nth = P.top_k;
+    if (!nth_row(P) || flag != kIndexClaimed) // uniform (a row of another kind; one whose token is forced)
+        return;
+    bool compact = false;
+    if (step == 1u) {
+        const uint32_t n0 = uniform_u32(__ockl_wfred_add_u32(lane < pieces ? counted : 0u));
+        compact = n0 != d.n_vocab;
+        // (a whole list that nothing is cut off stays as it is)
+        now = NthState{0u, d.n_vocab, compact || nth < n0 ? 1u : 0u, 0u, 0u};
+    }
+    const uint32_t len = uniform_u32(now.len), from_buf = uniform_u32(now.buf), used = now.used;
+    auto leave = [&](uint32_t n, uint32_t pre, uint32_t rounds, uint32_t in) {
+        if (w == 0u && tid == 0u) {
+            NthState* s = nth_state(plan, step & 1u);
+            s->seq = step;
+            s->len = n;
+            s->pre = pre;
+            s->used = rounds;
+            s->buf = in;
+        }
+    };
+    const lds_ptr<u64> buf = as_lds(lds_dyn);                // [kNthChunk] fillers
+    const lds_ptr<u64> bits = buf + kNthChunk;               // [words]
+    const uint32_t words = (len + 63u) / 64u;
+    const lds_ptr<uint32_t> pre = (lds_ptr<uint32_t>)(bits + words); // [words + 1] set bits in front of each
+    const uint32_t to_buf = from_buf ^ 1u;
+    const global_ptr<const uint32_t> kin = as_global(sc.key[from_buf]) + (size_t)row * sc.vpad, iin = as_global(sc.idx[from_buf]) + (size_t)row * sc.vpad;
+    const global_ptr<uint32_t> kout = as_global(sc.key[to_buf]) + (size_t)row * sc.vpad, iout = as_global(sc.idx[to_buf]) + (size_t)row * sc.vpad;
+    bool go = uniform_u32(now.pre) != 0u;
+    uint32_t smalls = 0;
+    if (go) { // uniform
+        if (compact || from_buf != usual) // uniform
+            load_bits(compact ? 2u : from_buf, words);
+        uint32_t mine = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i)
+            mine += 4u * tid + i < words ? (uint32_t)__popcll(x[i]) : 0u;
+        uint32_t at = block_excl_scan_u32(mine, smalls, bs);
+#pragma unroll
+        for (uint32_t i = 0; i < 4; ++i)
+            if (4u * tid + i < words) {
+                bits[4u * tid + i] = x[i];
+                pre[4u * tid + i] = at;
+                at += (uint32_t)__popcll(x[i]);
+            }
+        smalls = uniform_u32(smalls);
+        if (tid == 0)
+            pre[words] = smalls;
+        __syncthreads();
+    }
+    const uint32_t out_len = compact ? smalls : smalls + 1u; // (the cut: behind the pivot and what belongs left)
+    if (go && !compact && out_len <= nth)                    // uniform: the rounds go on in the right part, by one workgroup
+        go = false;
+    if (!go) { // uniform
+        if (step == 1u) {
+            // (a list that stays where it is has no token ids yet)
+            const global_ptr<uint32_t> ids = as_global(sc.idx[0]) + (size_t)row * sc.vpad;
+            for (uint32_t i = w * (uint32_t)kThreads + tid; i < len; i += W * (uint32_t)kThreads)
+                ids[i] = i;
+        }
+        leave(len, step == 1u ? 0u : now.pre, used, from_buf);
+        return;
+    }
+    const bool goes_on = out_len > kNthUntil && nth < out_len; // uniform
+    // the entry at i of the old list; a row that is its own list has no token ids, and its first entry has yet to change places
+    // with the pivot
+    NthFirst own = {0u, 0u, kNone, 0u};
+    if (step == 1u && !compact)
+        own = first;
+    const bool ids_implied = step == 1u;
+    auto entry = [&](uint32_t i) {
+        i = min(i, len - 1u);
+        const uint32_t k = kin[i], id = ids_implied ? i : iin[i];
+        return i == own.from ? ((u64)own.first_key << 32) : (((u64)k << 32) | (u64)id);
+    };
+    auto ones_before = [&](uint32_t p) { return pre[p >> 6] + (uint32_t)__popcll(bits[p >> 6] & ((1ull << (p & 63u)) - 1ull)); };
+    // the place of the s-th set bit, by one wave
+    auto word_of = [&](uint32_t s) {
+        const uint32_t c = (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(lane * 64u <= words && pre[min(lane * 64u, words)] <= s)) - 1u;
+        const uint32_t i = c * 64u + lane;
+        return c * 64u + (uint32_t)__popcll(__builtin_amdgcn_ballot_w64(i < words && pre[min(i, words)] <= s)) - 1u;
+    };
+    auto place_of = [&](uint32_t s) {
+        const uint32_t j = word_of(s);
+        const u64 x = bits[j];
+        const u64 hit = __builtin_amdgcn_ballot_w64(((x >> lane) & 1ull) && mask_rank(x) == s - pre[j]);
+        return j * 64u + (uint32_t)__ffsll((long long)hit) - 1u;
+    };
+    // what the new list has at p (> 0 unless the list is only moved together)
+    auto source = [&](uint32_t p) {
+        if (compact)
+            return place_of(p);
+        if ((bits[p >> 6] >> (p & 63u)) & 1ull) // uniform
+            return p;
+        return place_of(smalls - 1u - (p - 1u - ones_before(p)));
+    };
+    // Which entries the next pivot is chosen from, and what is at the front until then (the waves ask for one each, and go on)
+    u64 mine = 0, pivot = 0, front = 0;
+    uint32_t pivot_at = kNone;
+    if (wave < 4u && out_len != 0u && (goes_on || wave == 3u)) {
+        const uint32_t p = wave == 0u ? 1u : (wave == 1u ? out_len / 2u : (wave == 2u ? out_len - 1u : 0u));
+        if (wave == 3u && !compact)
+            mine = step == 1u ? ((u64)own.pivot_key << 32) | (u64)own.pivot_id : entry(0u);
+        else
+            mine = entry(uniform_u32(source(p)));
+    }
+    uint32_t* bits_out = nth_bits(sc, row, to_buf);
+    // (equal shares for the workgroups, in as few turns as hold them.  Where few entries are left their fillers come from far
+    // apart, and in pieces of 4 096 one workgroup of eight went through half of the old list for them, 22 us)
+    const uint32_t shares = W * ((out_len + W * kNthChunk - 1u) / (W * kNthChunk));
+    const uint32_t chunk = out_len ? (((out_len + shares - 1u) / shares) + kGroup - 1u) & ~(kGroup - 1u) : kNthChunk;
+    for (uint32_t c = w; c * chunk < out_len; c += W) { // uniform
+        const uint32_t p0 = c * chunk, p1 = min(p0 + chunk, out_len);
+        const uint32_t p = p0 + 4u * tid, pc = min(p, (out_len - 1u) & ~3u); // (rows' arrays are a multiple of 1 024 long)
+        u32x4 k = {0u, 0u, 0u, 0u}, id = {0u, 0u, 0u, 0u};
+        // set bits [s_lo, s_hi) are wanted here: those of the holes' fillers, of which the hole in front takes the last, or
+        // the entries themselves
+        uint32_t s_lo = p0, s_hi = p1, holes_before = 0;
+        if (!compact) { // uniform
+            k = *(global_ptr<const u32x4>)(kin + pc);
+            if (ids_implied)
+                id = u32x4{pc, pc + 1u, pc + 2u, pc + 3u};
+            else
+                id = *(global_ptr<const u32x4>)(iin + pc);
+            holes_before = p0 ? p0 - 1u - uniform_u32(ones_before(p0)) : 0u;
+            const uint32_t holes_to = p1 - 1u - uniform_u32(p1 < len ? ones_before(p1) : smalls);
+            s_lo = smalls - holes_to;
+            s_hi = smalls - holes_before;
+        }
+        if (s_lo < s_hi) { // uniform
+            const uint32_t b_lo = uniform_u32(word_of(s_lo)) / 4u, b_hi = uniform_u32(word_of(s_hi - 1u)) / 4u;
+            constexpr uint32_t kTrip = 2;
+            for (uint32_t b = b_lo + wave; b <= b_hi; b += kTrip * (uint32_t)kWaves) { // uniform per wave
+                u32x4 fk[kTrip], fi[kTrip];
+#pragma unroll
+                for (uint32_t u = 0; u < kTrip; ++u) {
+                    const uint32_t at = min((b + u * (uint32_t)kWaves) * kGroup + 4u * lane, (len - 1u) & ~3u);
+                    fk[u] = *(global_ptr<const u32x4>)(kin + at);
+                    if (ids_implied)
+                        fi[u] = u32x4{at, at + 1u, at + 2u, at + 3u};
+                    else
+                        fi[u] = *(global_ptr<const u32x4>)(iin + at);
+                }
+#pragma unroll
+                for (uint32_t u = 0; u < kTrip; ++u) {
+                    const uint32_t at = (b + u * (uint32_t)kWaves) * kGroup + 4u * lane;
+                    if (b + u * (uint32_t)kWaves > b_hi || at >= len)
+                        continue;
+                    const u64 x = bits[at >> 6];
+                    uint32_t s = pre[at >> 6] + (uint32_t)__popcll(x & ((1ull << (at & 63u)) - 1ull));
+                    const uint32_t nibble = (uint32_t)(x >> (at & 63u)) & 15u;
+#pragma unroll
+                    for (uint32_t j = 0; j < 4; ++j)
+                        if ((nibble >> j) & 1u) {
+                            const u64 v = at + j == own.from ? ((u64)own.first_key << 32) : (((u64)fk[u][j] << 32) | (u64)fi[u][j]);
+                            if (s >= s_lo && s < s_hi)
+                                buf[compact ? s - s_lo : s_hi - 1u - s] = v;
+                            ++s;
+                        }
+                }
+            }
+        }
+        if (c == w && wave < 4u && lane == 0u)
+            bs.u64[wave] = mine;
+        __syncthreads();
+        if (c == w) { // uniform
+            front = bs.u64[3];
+            if (goes_on)
+                median_of_three<u64>(bs.u64[0], bs.u64[1], bs.u64[2], 1u, out_len / 2u, out_len - 1u, pivot, pivot_at);
+        }
+        u64 v[4];
+        uint32_t hole = 0, nibble = 0;
+        if (!compact) { // uniform
+            const u64 x = bits[pc >> 6];
+            nibble = (uint32_t)(x >> (pc & 63u)) & 15u;
+            hole = (pc ? pc - 1u : 0u) - (pre[pc >> 6] + (uint32_t)__popcll(x & ((1ull << (pc & 63u)) - 1ull))) - holes_before;
+        }
+#pragma unroll
+        for (uint32_t j = 0; j < 4; ++j) {
+            const uint32_t pj = p + j;
+            if (compact) {
+                v[j] = buf[min(pj - p0, kNthChunk - 1u)];
+            } else if (pj == 0u) {
+                v[j] = front;
+            } else if ((nibble >> j) & 1u) {
+                v[j] = pj == own.from ? ((u64)own.first_key << 32) : (((u64)k[j] << 32) | (u64)id[j]);
+            } else {
+                v[j] = buf[min(hole, kNthChunk - 1u)];
+                ++hole;
+            }
+        }
+        uint32_t left = 0;
+        if (goes_on) { // uniform: the next pivot to the front, and who belongs left of it
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                const uint32_t pj = p + j;
+                v[j] = pj == pivot_at ? front : v[j];
+                left |= (pj != 0u && pj < out_len && v[j] < pivot ? 1u : 0u) << j;
+                v[j] = pj == 0u ? pivot : v[j];
+            }
+        }
+        if (p < p1) {
+            MAKO_CHECK(sc, kCheckCompact, (uint64_t)p + 3u < sc.vpad);
+            *(global_ptr<u32x4>)(kout + p) = u32x4{(uint32_t)(v[0] >> 32), (uint32_t)(v[1] >> 32), (uint32_t)(v[2] >> 32), (uint32_t)(v[3] >> 32)};
+            *(global_ptr<u32x4>)(iout + p) = u32x4{(uint32_t)v[0], (uint32_t)v[1], (uint32_t)v[2], (uint32_t)v[3]};
+        }
+        if (goes_on) { // uniform
+            const uint32_t word = eight_nibbles(left);
+            if ((lane & 7u) == 0u && (p & ~(kGroup - 1u)) < p1)
+                as_global(bits_out)[p >> 5] = word;
+        }
+        __syncthreads(); // (the fillers' buffer)
+    }
+    leave(out_len, goes_on ? 1u : 0u, used + (compact ? 0u : 1u), to_buf);
+}
+
+} // namespace mako

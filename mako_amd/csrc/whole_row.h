@@ -1,6 +1,7 @@
 // The whole-row path: exact for every parameter combination, one workgroup per row.
 #pragma once
 
+#include "nth_steps.h"
 #include "sorted_tail.h"
 
 namespace mako {
@@ -212,43 +213,33 @@ __device__ void heap_select_rest(Get get, Put put, uint32_t first, uint32_t last
 // One round = median of three to the front, then the unguarded Hoare partition of the rest around it.  That
 // partition swaps the t-th entry from the left that belongs right ("hole") with the t-th entry from the right that belongs
 // left ("filler") for as long as the former lies before the latter, and cuts behind the entries that belong left.
-// Three ways to make a round, as the range shrinks (nth_element_row()):
+// Three ways to make a round, as the range shrinks (nth_element_row()), behind those that several workgroups have made of a long
+// row (nth_steps.h):
 //   in device memory   nth_rounds_memory(): one pass over the keys, sixteen bytes per lane and load, leaves a bit per
 //                      entry in LDS; what changes places goes through LDS block by block;
 //   in registers       nth_rounds_registers(): up to kNthRegs entries, sixteen per thread; what changes places goes through LDS;
 //   by one wave        nth_rounds_wave(): up to kNthWave entries, four per lane, without a barrier.
 // The depth limit's heap select is heap_select_rest() above.
 // (A batch of 32 rows of 12 000 candidates, 40 kept: 81 us with every round in device memory or LDS, two passes over the keys
-// each and through pointers that the compiler could not tell from each other; 60 us now.  64 rows of 129 280 are bound by
-// the rounds in device memory of the row with the unluckiest pivots, and no faster: 235 to 270 us, as the box will have it.)
+// each and through pointers that the compiler could not tell from each other; 60 us now.  64 rows of 129 280, bound by the
+// rounds in device memory of the row with the unluckiest pivots: 225 to 235 us, 150 to 162 with the first rounds made by several
+// workgroups; one such row 144, 72 so.)
 constexpr uint32_t kNthChunks = 4;                                     // of four entries in a row per thread:
 constexpr uint32_t kNthRegs = kNthChunks * 4u * (uint32_t)kThreads; // what a workgroup takes into registers
 constexpr uint32_t kNthWave = 256;                                     // and one wave
-
-__device__ __forceinline__ uint32_t mask_rank(unsigned long long m)
-{
-    return __builtin_amdgcn_mbcnt_hi((uint32_t)(m >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)m, 0u));
-}
-
-// The median of three and its position (__move_median_to_first(first, first + 1, mid, last - 1)).
-template <typename T>
-__device__ __forceinline__ void median_of_three(T vx, T vy, T vz, uint32_t ix, uint32_t iy, uint32_t iz, T& med, uint32_t& im)
-{
-    const bool xy = vx < vy, yz = vy < vz, xz = vx < vz;
-    im = xy == yz ? iy : (xy == xz ? iz : ix);
-    med = xy == yz ? vy : (xy == xz ? vz : vx);
-}
+static_assert(kNthUntil == kNthRegs - 4u, "wherever the range begins, from a multiple of four on");
 
 // Rounds on entries [first, last) in device memory until no more than `until` are left or the depth limit is reached.
 // far: room for n / 32 words of device memory behind which nobody looks (the bits of ranges that LDS has no room for).
+// ready: the first round's pivot is at `first` already, and these are its bits (nth_steps.h); nullptr: they are not.
 // lds: kTailLds bytes.  All threads call.
 // (A workgroup's four SIMDs look at 256 entries a cycle, one instruction each, and a CU fetches 40 GB/s from the memory
 // behind its L2: a row of 129 280 keys takes it 13 us to read, 0.2 us to give one instruction to.  So the keys are read
 // once a round, a bit per entry is kept in LDS, and the entries that change places are read and written where they lie, block
 // by block, through LDS.  The first round of such a row takes 49 us: the keys 14, what moves 33.)
 __device__ __forceinline__ void nth_rounds_memory(global_ptr<uint32_t> key, global_ptr<uint32_t> idx, uint32_t& first, uint32_t& last, uint32_t nth,
-                                                  uint32_t& depth, uint32_t until, global_ptr<uint32_t> far, lds_ptr<unsigned long long> lds,
-                                                  FinishShared& sm)
+                                                  uint32_t& depth, uint32_t until, global_ptr<uint32_t> far, const uint32_t* ready,
+                                                  lds_ptr<unsigned long long> lds, FinishShared& sm)
 {
     typedef unsigned long long u64;
     const uint32_t tid = threadIdx.x, lane = lane_id(), wave = wave_id();
@@ -258,7 +249,7 @@ __device__ __forceinline__ void nth_rounds_memory(global_ptr<uint32_t> key, glob
     while (last - first > until && depth > 0u) {
         --depth;
         const uint32_t lo = uniform_u32(first + 1u), end = uniform_u32(last);
-        if (wave == 0) { // (one trip to memory)
+        if (wave == 0 && !ready) { // (one trip to memory)
             const uint32_t ix = lo, iy = first + (end - first) / 2u, iz = end - 1u;
             const uint32_t p = lane == 0 ? ix : (lane == 1 ? iy : (lane == 2 ? iz : first));
             const uint32_t k = key[p], i = idx[p];
@@ -275,7 +266,7 @@ __device__ __forceinline__ void nth_rounds_memory(global_ptr<uint32_t> key, glob
             }
         }
         __syncthreads();
-        const u64 pivot = (u64)__double_as_longlong(sm.bs.f64[0]);
+        const u64 pivot = (u64)__double_as_longlong(sm.bs.f64[0]); // (of no use where the bits are there)
         const uint32_t pivot_key = uniform_u32((uint32_t)(pivot >> 32)), pivot_id = uniform_u32((uint32_t)pivot);
         // blocks of 256 positions, to the waves in turn
         const uint32_t b0 = lo / kGroup, n_blocks = (end - 1u) / kGroup + 1u - b0;
@@ -287,7 +278,23 @@ __device__ __forceinline__ void nth_rounds_memory(global_ptr<uint32_t> key, glob
         const lds_ptr<u64> moving = bits + (bits_in_lds ? n_blocks * 4u : 0u);
         const uint32_t room = kTailLds / 8u - (n_blocks + 2u) / 2u - (bits_in_lds ? n_blocks * 4u : 0u);
         constexpr uint32_t kTrip = 8, kFills = 4;
-        for (uint32_t b = wave; b < n_blocks; b += kTrip * (uint32_t)kWaves) {
+        if (ready) { // uniform
+            const global_ptr<const u64> done = (global_ptr<const u64>)as_global(ready);
+            for (uint32_t b = tid; b < n_blocks; b += (uint32_t)kThreads) {
+                uint32_t n = 0;
+#pragma unroll
+                for (uint32_t j = 0; j < 4; ++j) {
+                    const u64 m = done[(b0 + b) * 4u + j];
+                    n += (uint32_t)__popcll(m);
+                    if (bits_in_lds) // uniform
+                        bits[b * 4u + j] = m;
+                    else
+                        bits_far[b * 4u + j] = m;
+                }
+                pre[b] = n;
+            }
+        }
+        for (uint32_t b = wave; !ready && b < n_blocks; b += kTrip * (uint32_t)kWaves) {
             uint32_t k[kTrip][4];
 #pragma unroll
             for (uint32_t u = 0; u < kTrip; ++u)
@@ -333,6 +340,7 @@ __device__ __forceinline__ void nth_rounds_memory(global_ptr<uint32_t> key, glob
             }
         }
         __syncthreads();
+        ready = nullptr;
         // the counts' prefix sums, up to four blocks a thread
         uint32_t smalls;
         {
@@ -669,8 +677,15 @@ __device__ __forceinline__ bool nth_rounds_wave(lds_ptr<unsigned long long> rang
     return done;
 }
 
-// The row's candidates in device memory (key[i], idx[i]; far: n / 32 words of it that are free).  All threads call.
-__device__ MAKO_RARE_CALL void nth_element_row(uint32_t* key_p, uint32_t* idx_p, uint32_t n, uint32_t nth, uint32_t* far, const FinishLds& L)
+// What other workgroups have done of it (nth_steps.h): `used` rounds, which left `len` entries; `ready` as for
+// nth_rounds_memory().
+struct NthDone {
+    uint32_t used, len;
+    const uint32_t* ready;
+};
+// The row's candidates in device memory (key[i], idx[i]; far: n / 32 words of it that are free), n of them to begin with.  All threads call.
+__device__ MAKO_RARE_CALL void nth_element_row(uint32_t* key_p, uint32_t* idx_p, uint32_t n, uint32_t nth, uint32_t* far, const FinishLds& L,
+                                               NthDone done = NthDone{0u, kNone, nullptr})
 {
     assume_lds(L);
     typedef unsigned long long u64;
@@ -678,8 +693,8 @@ __device__ MAKO_RARE_CALL void nth_element_row(uint32_t* key_p, uint32_t* idx_p,
     const uint32_t tid = threadIdx.x;
     if (n == 0 || nth >= n)
         return;
-    uint32_t first = 0, last = n;
-    uint32_t depth = 2u * (31u - (uint32_t)__clz((int)n));
+    uint32_t first = 0, last = min(n, done.len);
+    uint32_t depth = 2u * (31u - (uint32_t)__clz((int)n)) - done.used;
     const global_ptr<uint32_t> key = as_global(key_p), idx = as_global(idx_p);
     const lds_ptr<u64> lds = as_lds(L.sortk);
     auto get = [=](uint32_t i) { return ((u64)key[i] << 32) | (u64)idx[i]; };
@@ -689,11 +704,11 @@ __device__ MAKO_RARE_CALL void nth_element_row(uint32_t* key_p, uint32_t* idx_p,
     };
     __syncthreads();
     MAKO_STAMP(20);
-    nth_rounds_memory(key, idx, first, last, nth, depth, kNthRegs - 4u, as_global(far), lds, sm);
+    nth_rounds_memory(key, idx, first, last, nth, depth, kNthUntil, as_global(far), done.ready, lds, sm);
     MAKO_STAMP(21);
     first = uniform_u32(first);
     last = uniform_u32(last);
-    if (last - first <= kNthRegs - 4u) { // uniform
+    if (last - first <= kNthUntil) { // uniform
         const uint32_t origin = first & ~3u, from = first;
         u64 x[kNthChunks][4];
 #pragma unroll
@@ -725,7 +740,7 @@ __device__ MAKO_RARE_CALL void nth_element_row(uint32_t* key_p, uint32_t* idx_p,
                     range[p - first] = x[c][j];
             }
         lds_barrier();
-        bool done = false;
+        bool arranged = false;
         if (by_wave) { // uniform
             if (wave_id() == 0) {
                 uint32_t f = 0, l = len, dep = depth;
@@ -736,7 +751,7 @@ __device__ MAKO_RARE_CALL void nth_element_row(uint32_t* key_p, uint32_t* idx_p,
                 }
             }
             lds_barrier();
-            done = sm.bs.u64[0] != 0u;
+            arranged = sm.bs.u64[0] != 0u;
             if (tid < len)
                 put(origin + first + tid, range[tid]);
             last = first + (uint32_t)sm.bs.u64[1];
@@ -746,7 +761,7 @@ __device__ MAKO_RARE_CALL void nth_element_row(uint32_t* key_p, uint32_t* idx_p,
         last += origin;
         __syncthreads();
         MAKO_STAMP(23);
-        if (done)
+        if (arranged)
             return;
     }
     // the depth limit
@@ -790,6 +805,7 @@ __device__ MAKO_RARE_CALL void compact_candidates(const uint32_t* qb, uint32_t V
 // order.  Sorts them by (q desc, idx asc) when top-k or top-p is active, truncates (src/gen/sampler.cpp:39-61)
 // and draws.  `total64` (when have_total) is the fp64 sum of q over all candidates of the row, of which the list
 // may be only the heaviest part; otherwise it is summed from the list.  key0 / idx0: the list, key1 / idx1: a second buffer.
+// done: what is behind a row's nth_element already (then the list is what the rounds left of it; n0 as it was).
 // qk: the row's bits(q) array (bits(q) of every candidate at its index, 0 elsewhere), wanted for a second look at a cut too
 // close to call; without one (nullptr) such a row is left undone and false is returned.
 // (TOPK_ALONE = false leaves the top-k-without-top-p branch out of the instance inside plan_kernel: that kernel is
@@ -798,7 +814,7 @@ __device__ MAKO_RARE_CALL void compact_candidates(const uint32_t* qb, uint32_t V
 template <bool TOPK_ALONE>
 __device__ bool sort_truncate_draw(const mako_sample_desc& d, uint32_t row, const mako_sampling_params& P, uint32_t* key0, uint32_t* idx0,
                                    uint32_t* key1, uint32_t* idx1, const uint32_t* qk, uint32_t n0, bool have_total, double total64,
-                                   uint32_t path, const FinishLds& L)
+                                   uint32_t path, const FinishLds& L, NthDone done = NthDone{0u, kNone, nullptr})
 {
     assume_lds(L);
     FinishShared& sm = *L.sm;
@@ -809,12 +825,12 @@ __device__ bool sort_truncate_draw(const mako_sample_desc& d, uint32_t row, cons
     // top-k alone: the survivors stay in the order nth_element leaves them (sampler.cpp:39-43, then :79-83)
     const bool nth_order = TOPK_ALONE && topk_active && !topp_active;
     if (nth_order)
-        nth_element_row(key0, idx0, n0, P.top_k, key1, L);
+        nth_element_row(key0, idx0, n0, P.top_k, key1, L, done);
     else if (topk_active) {
         // a top-p follows: the survivors are sorted, so only which candidates they are matters, and `desc` is a total
         // order: nth_element's first top_k entries are the top_k first of the sorted list, in some order.  The
         // partitions and a sort of top_k entries cost a quarter of the sort of all candidates.
-        nth_element_row(key0, idx0, n0, P.top_k, key1, L);
+        nth_element_row(key0, idx0, n0, P.top_k, key1, L, done);
         sort_survivors(key0, idx0, key1, idx1, P.top_k, L);
     } else if (topp_active)
         sort_segment(key0, idx0, key1, idx1, n0, L);
@@ -1103,12 +1119,13 @@ __device__ MAKO_RARE_CALL void general_row(const mako_sample_desc& d, const Scra
 // The whole-row path for a row whose weights are already in place: key[0] of the row holds ~bits(q) of every candidate at
 // its index and ~0 elsewhere (index_weights_kernel, with a workgroup per 16 384 logits instead of one for the row).  Counts
 // and compacts the candidates in index order into the row's second buffers and goes on like general_row().  All threads
-// call; m, argidx: the row's maximum and where it is first.
-// `listed`: true when that kernel found every logit a candidate (no mask, no floor, no underflow: the usual row) and
-// has left the token ids as well, i at i in idx[0] of the row: the list is there, nothing to count or to compact.
+// call; m, argidx: the row's maximum and where it is first; n_all: its candidates.
+// When that kernel found every logit a candidate (no mask, no floor, no underflow: the usual row) it has left the token ids as
+// well, i at i in idx[0] of the row: the list is there, nothing to compact.  Rows long enough for nth_steps.h have their list
+// where the last step has left it.
 template <int SITE>
 __device__ MAKO_RARE_CALL void general_row_from_weights(const mako_sample_desc& d, const Scratch& sc, uint32_t row,
-                                                        const mako_sampling_params& P, float m, uint32_t argidx, bool listed,
+                                                        const mako_sampling_params& P, float m, uint32_t argidx, uint32_t n_all,
                                                         const FinishLds& L)
 {
     assume_lds(L);
@@ -1118,8 +1135,16 @@ __device__ MAKO_RARE_CALL void general_row_from_weights(const mako_sample_desc& 
     uint32_t* i_from = sc.idx[0] + (size_t)row * sc.vpad;
     uint32_t* k_to = sc.key[1] + (size_t)row * sc.vpad;
     uint32_t* i_to = sc.idx[1] + (size_t)row * sc.vpad;
-    uint32_t n0 = V;
-    if (!listed) { // uniform
+    uint32_t n0 = n_all;
+    bool listed = n_all == V; // in the first buffers
+    NthDone done = {0u, kNone, nullptr};
+    if (nth_steps_for(V)) { // uniform
+        const NthState s0 = *nth_state(sc.plan + row, 0u), s1 = *nth_state(sc.plan + row, 1u);
+        const bool odd = s1.seq > s0.seq;
+        const uint32_t buf = odd ? s1.buf : s0.buf;
+        done = NthDone{odd ? s1.used : s0.used, odd ? s1.len : s0.len, (odd ? s1.pre : s0.pre) ? nth_bits(sc, row, buf) : nullptr};
+        listed = buf == 0u;
+    } else if (!listed) {
         const global_ptr<const uint32_t> from = as_global(k_from);
         const global_ptr<uint32_t> kd = as_global(k_to), id = as_global(i_to);
         const uint32_t lane = lane_id(), wave = wave_id();
@@ -1189,7 +1214,7 @@ __device__ MAKO_RARE_CALL void general_row_from_weights(const mako_sample_desc& 
         return;
     }
     if (!sort_truncate_draw<SITE == 0>(d, row, P, listed ? k_from : k_to, listed ? i_from : i_to, listed ? k_to : k_from, listed ? i_to : i_from,
-                                       nullptr, n0, false, 0.0, MAKO_PATH_GENERAL, L)) {
+                                       nullptr, n0, false, 0.0, MAKO_PATH_GENERAL, L, done)) {
         __syncthreads();
         general_row<SITE>(d, sc, row, P, m, argidx, L); // (a cut too close to call: from the logits again)
     }
