@@ -28,6 +28,7 @@ struct alignas(16) CoarsePlan {
     uint2 run[kWorkers]; // entry e of that ordering, if worker w's, goes to run[w].x + e of the row's staging arrays if
                          // e < run[w].y (the share's room allows it)
     uint32_t flag, thr, n0_est;
+    uint32_t workers; // that the row's list is shared out to
     uint32_t opq_mask; // workers whose shares are left unsorted (opaque_guess())
 };
 
@@ -56,9 +57,10 @@ __device__ __forceinline__ void issue_plan_loads(const mako_sample_desc& d, cons
 // under it falls to 1 - top_p of the estimated total, less a few percent.  The list that results is checked by the
 // exact sums later: a plan that keeps too little costs a second look at the row, never a wrong answer.
 // (Every instruction here is latency of the whole pass: a workgroup's sixteen waves share four SIMDs.)
+// share_min: entries a worker is given at least, if there are as many.
 // opaque_first: the first position of the list from which a share may be left unsorted (kNone: none may).
 __device__ void coarse_plan(const Scratch& sc, uint32_t row, uint32_t slices, uint32_t n_vocab, const mako_sampling_params& P,
-                            float m, const PlanLoads& pre, bool narrow_ok, uint32_t opaque_first, CoarsePlan& pl, const uint64_t* tab)
+                            float m, const PlanLoads& pre, bool narrow_ok, uint32_t opaque_first, uint32_t share_min, CoarsePlan& pl, const uint64_t* tab)
 {
     const uint32_t tid = threadIdx.x, lane = (uint32_t)lane_id();
     MAKO_STAMP(10);
@@ -143,8 +145,9 @@ __device__ void coarse_plan(const Scratch& sc, uint32_t row, uint32_t slices, ui
     else if (n0_est > kGroup * (kMaxGroups - kWorkers))
         flag = 2; // (a list too long for the workers' group records goes to the whole-row path)
     // shares of about equal counts (a monotone estimate is all that is needed)
-    const float per_entry = flag == 1 ? (float)kWorkers / (float)max(n0_est, 1u) : 0.0f;
-    auto worker_at = [&](uint32_t excl) { return min(kWorkers - 1u, (uint32_t)((float)excl * per_entry)); };
+    const uint32_t workers = max(1u, min(kWorkers, (n0_est + share_min - 1u) / share_min));
+    const float per_entry = flag == 1 ? (float)workers / (float)max(n0_est, 1u) : 0.0f;
+    auto worker_at = [&](uint32_t excl) { return min(workers - 1u, (uint32_t)((float)excl * per_entry)); };
     const uint32_t wk = worker_at(excl_c);
     if (bin != 0 && bin < bins_end) {
         // the workers whose share starts with this bin
@@ -223,6 +226,7 @@ __device__ void coarse_plan(const Scratch& sc, uint32_t row, uint32_t slices, ui
         if (w == kWorkers - 1u) {
             pl.thr = key;
             pl.n0_est = n0_est;
+            pl.workers = workers;
             pl.mass_all = (double)all_m;
             pl.flag = (sane && upto > sc.vpad) ? 2u : flag;
             pl.opq_mask = opq_mask;

@@ -74,6 +74,13 @@ __device__ __forceinline__ int32_t log_unit(float logit, float scale)
 }
 
 constexpr uint32_t kWorkers = 32;  // workgroups that share the sort of one wide-nucleus row
+// Entries of a row's list that each of its workers is given at least, if there are as many (coarse_plan()).  A worker is a
+// workgroup with a CU to itself and takes 6.3 us for 90 entries, 11.7 for 4 400: on a large batch, which waits for all of
+// them, every row of some thousand entries cut into 32 shares costs its CUs ten times what one worker does (512 rows of a
+// decode batch: 1 820 workers, half of them with fewer than 94 entries; 225 us now, 255 in 32 shares, 240 with 5 000 entries
+// at least, which some shares overrun); on a small one the row waits for the slowest, but for more than one round of them too
+// (64 rows: 62.5 us, 65.4 in 32 shares).
+constexpr uint32_t kShareLarge = 4096, kShareSmall = 512;
 constexpr uint32_t kStageSlack = 64; // room a worker's share of the staging arrays gets beyond what the coarse counts
                                      // promise (and 1/64 of that count); the rows' arrays are sized to hold it
 constexpr uint32_t kGroup = 256;      // a sorted list is processed in groups of one wave x four entries per lane

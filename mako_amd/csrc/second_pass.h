@@ -38,7 +38,7 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
         load_penalised<VEC, KH>(d, row, lo, hi, slice_len, P, hl, pen, L.cnt, wv, [&]() {
             uint32_t n_cands, any_overflow;
             row_summary_of(pre.st, slices, m, argidx, n_cands, any_overflow);
-            coarse_plan(sc, row, slices, d.n_vocab, P, m, pre, !any_overflow && n_cands <= kSortMax, UNSORTED ? opaque_first : kNone, pl, sm.tab);
+            coarse_plan(sc, row, slices, d.n_vocab, P, m, pre, !any_overflow && n_cands <= kSortMax, UNSORTED ? opaque_first : kNone, UNSORTED ? kShareLarge : kShareSmall, pl, sm.tab);
         });
     } else {
         load_penalised<VEC, KH>(d, row, lo, hi, slice_len, P, hl, pen, L.cnt, wv);
@@ -75,13 +75,13 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
                         uint32_t at = lists.sorted_at - atomicAdd(&sc.work_n[3], collectors) - collectors;
                         for (uint32_t c = 0; c < collectors; ++c)
                             sc.work_sort[at++] = (row << 8) | (kWorkers + c);
-                        at = lists.sorted_at + atomicAdd(&sc.work_n[0], kWorkers - n_unsorted);
-                        for (uint32_t w = 0; w < kWorkers; ++w)
+                        at = lists.sorted_at + atomicAdd(&sc.work_n[0], pl.workers - n_unsorted);
+                        for (uint32_t w = 0; w < pl.workers; ++w)
                             if (!((unsorted >> w) & 1u))
                                 sc.work_sort[at++] = (row << 8) | w;
                     }
                 } else {
-                    const uint32_t work = flag == 1 ? kWorkers : 1u;
+                    const uint32_t work = flag == 1 ? pl.workers : 1u;
                     uint32_t at = atomicAdd(&sc.work_n[0], work);
                     for (uint32_t w = 0; w < work; ++w)
                         sc.work_sort[at++] = (row << 8) | w;
