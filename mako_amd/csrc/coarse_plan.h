@@ -29,6 +29,7 @@ struct alignas(16) CoarsePlan {
                          // e < run[w].y (the share's room allows it)
     uint32_t flag, thr, n0_est;
     uint32_t workers; // that the row's list is shared out to
+    uint32_t nucleus_rows; // of the batch (the large batches' instance)
     uint32_t opq_mask; // workers whose shares are left unsorted (opaque_guess())
 };
 

@@ -7,13 +7,12 @@ namespace mako {
 void launch_sort_beside(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices, uint32_t grid_rows, bool unsorted,
                         uint32_t more)
 {
-    // (a large batch's lists are sized by the batch's rows: large_batch_lists())
-    const uint32_t x = unsorted ? kSortItemsPerRow : kWorkers, rows = unsorted && grid_rows ? d.n_rows : grid_rows;
-    const dim3 grid(x, rows + (more + x - 1u) / x);
+    const uint32_t x = unsorted ? kSortItemsPerRow : kWorkers;
+    const dim3 grid(x, grid_rows + (more + x - 1u) / x);
     if (unsorted)
-        hipLaunchKernelGGL(sort_beside_kernel<true>, grid, dim3(kThreads), kSortLds, st, d, sc, slices, rows);
+        hipLaunchKernelGGL(sort_beside_kernel<true>, grid, dim3(kThreads), kSortLds, st, d, sc, slices, grid_rows);
     else
-        hipLaunchKernelGGL(sort_beside_kernel<false>, grid, dim3(kThreads), kSortLds, st, d, sc, slices, rows);
+        hipLaunchKernelGGL(sort_beside_kernel<false>, grid, dim3(kThreads), kSortLds, st, d, sc, slices, grid_rows);
 }
 
 hipError_t init_beside_sort()

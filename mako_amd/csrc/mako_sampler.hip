@@ -429,7 +429,7 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
     const uint32_t nth_steps = !any_nth ? 0u : (d.n_vocab <= 65536u ? 2u : 4u);
     const bool launch_sort = any_nucleus || any_late || beside;
     // (finish_kernel's grid: scan_kernel, which cuts the second pass up, is told of it)
-    const uint32_t finish_wgs = mako::second_pass_grid(d.n_rows, nucleus_rows, ctx->cus);
+    const uint32_t finish_wgs = mako::second_pass_grid(nucleus_rows, ctx->cus);
     // Batches with many top_k == 0 rows leave the shares of their sorted lists that need no order unsorted
     // (unsorted_shares.h): there sort_kernel is bound by the number of its workgroups, one per CU at a time, and not, as
     // on a small batch, by its slowest worker.  More than four rounds of workers; without the caller's copy of the

@@ -142,9 +142,9 @@ constexpr uint32_t kSortItemsPerRow = kWorkers + 2u;
 struct SortLists {
     uint32_t sorted_at; // first workgroup number (= entry of work_sort) of the workers that sort and the narrow rows
 };
-__host__ __device__ inline SortLists large_batch_lists(uint32_t n_rows)
+__host__ __device__ inline SortLists large_batch_lists(uint32_t nucleus_rows) // (Scratch::work_n[10])
 {
-    return SortLists{2u * n_rows};
+    return SortLists{2u * nucleus_rows};
 }
 
 constexpr uint32_t kWorkWords = 12;        // of Scratch::work_n

@@ -98,7 +98,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(VEC ? 
                                                   (cus_and_grid & kCountGeneral) != 0u);
         if (lane_id() == 0) {
             *reinterpret_cast<uint4*>(sc.work_n + 4) = make_uint4(cut.per_row, cut.piece_len, cut.busy, cut.pieces);
-            *reinterpret_cast<uint2*>(sc.work_n + 8) = make_uint2(cut.general, cut.in_order);
+            *reinterpret_cast<uint4*>(sc.work_n + 8) = make_uint4(cut.general, cut.in_order, cut.rows, 0u);
         }
     }
     // ReasoningBudget::forced's question (src/server/openai.cpp:598-602), answered in the same pass over the logits

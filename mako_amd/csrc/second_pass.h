@@ -68,7 +68,7 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
                 const uint32_t n_unsorted = (uint32_t)__popc(unsorted), collectors = (n_unsorted + (uint32_t)kWaves - 1u) / (uint32_t)kWaves;
                 if constexpr (UNSORTED) {
                     // (two lists, the costly entries in front: large_batch_lists())
-                    const SortLists lists = large_batch_lists(d.n_rows);
+                    const SortLists lists = large_batch_lists(pl.nucleus_rows);
                     if (flag == 3) {
                         sc.work_sort[lists.sorted_at + atomicAdd(&sc.work_n[0], 1u)] = row << 8;
                     } else {
@@ -302,6 +302,7 @@ __device__ __forceinline__ void finish_body(const mako_sample_desc& d_arg, const
             return;
     } else {
         const uint32_t per_xcd = (cut.z + 7u) / 8u;
+    const uint32_t nucleus_rows = UNSORTED ? sc_arg.work_n[10] : 0u;
         if (per_xcd * 8u <= n_wgs) {
             if ((wg >> 3) >= per_xcd)
                 return;
@@ -374,6 +375,8 @@ __global__ __launch_bounds__(kThreads) void finish_kernel(mako_sample_desc d_arg
     extern __shared__ __align__(16) unsigned long long s_dyn64[]; // (128-bit LDS operations need the alignment)
     __shared__ FinishShared sm;
     __shared__ ArgsLds s_args;
+    if (UNSORTED && tid == 0)
+        s_plan.nucleus_rows = nucleus_rows; // (read behind the plan's barriers)
     __shared__ CoarsePlan s_plan;
     finish_body<VEC, KH, UNSORTED>(d_arg, sc_val, slices, gridDim.y, s_dyn64, sm, s_args, s_plan);
 }

@@ -20,7 +20,7 @@ namespace mako {
 // list has room for every workgroup of the grid that it is for.)
 struct SortFirstTrip {
     ArgWords arg_words;
-    uint32_t n_work, pieces_raw, item, n_collectors;
+    uint32_t n_work, pieces_raw, item, n_collectors, nucleus_rows;
     uint64_t tab_word;
 };
 template <bool UNSORTED>
@@ -32,7 +32,8 @@ __device__ __forceinline__ void fetch_sort_entry(const mako_sample_desc& d_arg, 
     f.item = sc_arg.work_sort[entry];
     f.tab_word = k_exp2_tab[threadIdx.x & 31u];
     f.n_collectors = UNSORTED ? sc_arg.work_n[3] : 0u;
-    asm volatile("" ::"s"(f.item), "s"(f.n_work), "s"(f.n_collectors), "s"(f.pieces_raw), "v"(f.arg_words.d), "v"(f.arg_words.sc), "v"(f.tab_word));
+    f.nucleus_rows = UNSORTED ? sc_arg.work_n[10] : 0u;
+    asm volatile("" ::"s"(f.item), "s"(f.n_work), "s"(f.n_collectors), "s"(f.nucleus_rows), "s"(f.pieces_raw), "v"(f.arg_words.d), "v"(f.arg_words.sc), "v"(f.tab_word));
 }
 
 // UNSORTED: the instance for batches whose plans leave shares unsorted (unsorted_shares.h; a translation unit of its own,
@@ -49,7 +50,7 @@ __device__ __forceinline__ void sort_body(const mako_sample_desc& d_arg, const S
     if constexpr (UNSORTED) {
         // (two lists that meet at workgroup number sorted_at: large_batch_lists())
         const uint32_t n_collectors = first.n_collectors;
-        const SortLists lists = large_batch_lists(d_arg.n_rows);
+        const SortLists lists = large_batch_lists(first.nucleus_rows);
         const bool with_work = piece < lists.sorted_at ? lists.sorted_at - piece <= n_collectors : piece - lists.sorted_at < n_work;
         if (!with_work)
             return;

@@ -19,6 +19,7 @@ struct SecondPassCut {
     uint32_t pieces;    // pieces per row: workgroup g of a row takes the pieces g, g + per_row, ...
     // and of the rows of the whole-row class (index_rows.h): all of them, those in token order
     uint32_t general, in_order;
+    uint32_t rows;      // top_k == 0 rows
 };
 // finish_grid: the workgroups finish_kernel is launched with (second_pass_grid()).  count_general: the rows of the whole-row
 // class are wanted too (counted for every batch, they cost a 64-row decode batch without any 0.3 of its 66 us).
@@ -53,16 +54,19 @@ __device__ __forceinline__ SecondPassCut second_pass_cut(const mako_sample_desc&
     // to the XCDs eight at a time, see finish_kernel)
     cut.per_row = rows * cut.pieces <= cus ? cut.pieces : min(cut.pieces, max(1u, finish_grid / ((max(rows, 1u) + 7u) & ~7u)));
     cut.busy = rows * cut.per_row;
+    cut.rows = rows;
     return cut;
 }
 
-// Workgroups finish_kernel is launched with (a multiple of eight, at least a workgroup per row): one round's worth, or
-// two where the batch is expected to have more top_k == 0 rows than half a round: the CUs whose rows need little then
+// Workgroups finish_kernel is launched with (a multiple of eight, at least a workgroup per top_k == 0 row): one round's worth,
+// or two where the batch is expected to have more such rows than half a round: the CUs whose rows need little then
 // take on the second halves of those that need much (a near-flat row takes twice as long as a peaked one).  On small
 // batches the workgroups without work, which can only start once a CU is free, would lengthen the kernel instead.
-__host__ __device__ inline uint32_t second_pass_grid(uint32_t n_rows, uint32_t nucleus_rows, uint32_t cus)
+// (The rows of a large batch that are of another kind don't count: 97 of 512 rows, given four workgroups each for a grid of
+// 512, took one and a half rounds of them, 82 us; 60 to 68 with two each in one.)
+__host__ __device__ inline uint32_t second_pass_grid(uint32_t nucleus_rows, uint32_t cus)
 {
-    const uint32_t rows8 = (n_rows + 7u) & ~7u, rounds = 2u * nucleus_rows >= cus ? 2u : 1u;
+    const uint32_t rows8 = (nucleus_rows + 7u) & ~7u, rounds = 2u * nucleus_rows >= cus ? 2u : 1u;
     return rows8 > rounds * cus ? rows8 : (rounds * cus + 7u) & ~7u;
 }
 
