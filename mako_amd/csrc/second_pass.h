@@ -111,16 +111,30 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
         }
         if (lo + (VEC ? (g / 4u) * 4096u : g * (uint32_t)kThreads) < hi) {
             bool keeps[4];
+            // (the large batches' instance: a wave whose four weights a lane all underflow to zero, as those of a peaked row far
+            // below its maximum do, skips the arithmetic that would tell it so; expf_glibc() returns 0 below that bound)
+            bool any = !UNSORTED;
+            if (UNSORTED) {
+                bool under = true;
 #pragma unroll
-            for (uint32_t j = g; j < g + 4u; ++j) {
-                // (the large batches' instance: a wave whose weights all underflow to zero, as those of a peaked row far
-                // below its maximum do, skips the arithmetic that would tell it so; expf_glibc() returns 0 below that bound)
-                float q = 0.0f;
-                if (!UNSORTED || __ballot(!((wv[j] - m) * inv_t < -0x1.9fe368p6f)) != 0ull)
-                    q = weight_of(wv[j], m, inv_t, sm.tab);
-                qb[j] = (q >= floor_q && q > 0.0f) ? __float_as_uint(q) : 0u;
-                sum += qb[j] ? (double)q : 0.0;
-                keeps[j - g] = qb[j] >= thr && qb[j];
+                for (uint32_t j = g; j < g + 4u; ++j)
+                    under = under && (wv[j] - m) * inv_t < -0x1.9fe368p6f;
+                any = __ballot(!under) != 0ull; // uniform
+            }
+#pragma unroll
+            for (uint32_t j = 0; j < 4u; ++j)
+                keeps[j] = false;
+            if (any) {
+                float q[4];
+#pragma unroll
+                for (uint32_t j = 0; j < 4u; ++j)
+                    q[j] = weight_of(wv[g + j], m, inv_t, sm.tab);
+#pragma unroll
+                for (uint32_t j = 0; j < 4u; ++j) {
+                    qb[g + j] = (q[j] >= floor_q && q[j] > 0.0f) ? __float_as_uint(q[j]) : 0u;
+                    sum += (double)__uint_as_float(qb[g + j]);
+                    keeps[j] = qb[g + j] >= thr && qb[g + j];
+                }
             }
             // the worker whose range of bits(q) holds the weight (equal weights always meet in one share): the number of
             // workers whose lower edge lies above it, by bisection over the edges (the first two steps against edges held in
@@ -288,6 +302,7 @@ __device__ __forceinline__ void finish_body(const mako_sample_desc& d_arg, const
     stage_args_only(d_arg, sc_arg, s_args);
     // (pieces per row, their length, workgroups with work: the others leave at once)
     const uint4 cut = *reinterpret_cast<const uint4*>(sc_arg.work_n + 4);
+    const uint32_t nucleus_rows = UNSORTED ? sc_arg.work_n[10] : 0u;
     // Workgroups go to the eight XCDs in turn.  The shares are dealt so that an XCD's workgroups serve consecutive
     // ones: the workgroups of a row then sit on one XCD (two where a row straddles), whose L2 fetches the row's
     // coarse counts and history once for all of them.  (Only if the grid holds every workgroup the deal names.)
@@ -302,7 +317,6 @@ __device__ __forceinline__ void finish_body(const mako_sample_desc& d_arg, const
             return;
     } else {
         const uint32_t per_xcd = (cut.z + 7u) / 8u;
-    const uint32_t nucleus_rows = UNSORTED ? sc_arg.work_n[10] : 0u;
         if (per_xcd * 8u <= n_wgs) {
             if ((wg >> 3) >= per_xcd)
                 return;
@@ -361,6 +375,8 @@ __device__ __forceinline__ void finish_body(const mako_sample_desc& d_arg, const
     // penalise, and nothing here waits for the length)
     // (shares may be left unsorted from the first position that the tail neither keeps in LDS nor writes out; never on
     // verification rows, whose replay reads the list itself)
+    if (UNSORTED && tid == 0)
+        s_plan.nucleus_rows = nucleus_rows; // (read behind the plan's barriers)
     const uint32_t opaque_first = (UNSORTED && !d.draft) ? max(kHeadGroups * kGroup, (d.out_cand_idx && d.out_cand_q) ? d.cand_cap : 0u) : kNone;
     if (d.hist_tokens && !penalties_neutral(P))
         row_pieces<VEC, KH, true, UNSORTED>(d, sc, row, piece, pieces, n_pieces, piece_len, P, hl, slices, L, s_plan, opaque_first);
@@ -375,8 +391,6 @@ __global__ __launch_bounds__(kThreads) void finish_kernel(mako_sample_desc d_arg
     extern __shared__ __align__(16) unsigned long long s_dyn64[]; // (128-bit LDS operations need the alignment)
     __shared__ FinishShared sm;
     __shared__ ArgsLds s_args;
-    if (UNSORTED && tid == 0)
-        s_plan.nucleus_rows = nucleus_rows; // (read behind the plan's barriers)
     __shared__ CoarsePlan s_plan;
     finish_body<VEC, KH, UNSORTED>(d_arg, sc_val, slices, gridDim.y, s_dyn64, sm, s_args, s_plan);
 }
