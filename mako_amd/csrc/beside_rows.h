@@ -16,7 +16,7 @@ namespace mako {
 
 #ifdef MAKO_EMIT_BESIDE_FINISH
 // grid = (1, finish_wgs + workgroups for the weights)
-template <bool VEC, int KH, bool UNSORTED>
+template <bool ALIGNED, int KH, bool UNSORTED>
 __global__ __launch_bounds__(kThreads) void finish_beside_kernel(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices, uint32_t finish_wgs)
 {
     extern __shared__ __align__(16) unsigned long long s_dyn64[]; // (128-bit LDS operations need the alignment)
@@ -24,7 +24,7 @@ __global__ __launch_bounds__(kThreads) void finish_beside_kernel(mako_sample_des
     __shared__ ArgsLds s_args;
     __shared__ CoarsePlan s_plan;
     if (blockIdx.y < finish_wgs) {
-        finish_body<VEC, KH, UNSORTED>(d_arg, sc_val, slices, finish_wgs, s_dyn64, sm, s_args, s_plan);
+        finish_body<ALIGNED, KH, UNSORTED>(d_arg, sc_val, slices, finish_wgs, s_dyn64, sm, s_args, s_plan);
         return;
     }
     const uint32_t pieces = (d_arg.n_vocab + kSliceMax - 1u) / kSliceMax;
@@ -34,7 +34,7 @@ __global__ __launch_bounds__(kThreads) void finish_beside_kernel(mako_sample_des
         uint32_t row;
         if (!rows.find(d_arg, p / pieces, [](const mako_sampling_params& P) { return classify(P) == kGeneral; }, row))
             return;
-        index_weights_piece<VEC, KH, true>(d_arg, sc_val, slices, row, p % pieces, s_dyn64, sm, s_args);
+        index_weights_piece<ALIGNED, KH, true>(d_arg, sc_val, slices, row, p % pieces, s_dyn64, sm, s_args);
         __syncthreads(); // (the next piece's table of counts and arguments)
     }
 }

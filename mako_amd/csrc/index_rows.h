@@ -76,28 +76,17 @@ __device__ __forceinline__ void first_pivot(const mako_sample_desc& d, uint32_t 
     }
 }
 
-// A thread's four bits (entries as elem_index() has them, the first at `base`), whole blocks of 256 entries at a time.
-template <bool VEC>
+// A thread's four bits (of the entries from `base` on), whole blocks of 256 entries at a time.
 __device__ __forceinline__ void store_nth_bits(global_ptr<uint32_t> words, uint32_t base, uint32_t four)
 {
-    if (VEC) {
-        const uint32_t word = eight_nibbles(four);
-        if ((lane_id() & 7) == 0)
-            words[base >> 5] = word;
-    } else {
-#pragma unroll
-        for (uint32_t c = 0; c < 4; ++c) {
-            const unsigned long long m = __builtin_amdgcn_ballot_w64((four >> c) & 1u);
-            if (lane_id() == 0)
-                *(global_ptr<unsigned long long>)(words + ((base + c * (uint32_t)kThreads) >> 5)) = m;
-        }
-    }
+    const uint32_t word = eight_nibbles(four);
+    if ((lane_id() & 7) == 0)
+        words[base >> 5] = word;
 }
 
-// Piece `piece` of row `row`; of a row of another kind nothing.  (VEC: V % 4 == 0 and 16-byte aligned rows, whose
-// logits are loaded four at a time; the layout of a thread's sixteen logits is slice_load.h's either way.  STEPS: there may be
-// rows for nth_steps.h, whose bits take the registers that let two workgroups share a CU.)
-template <bool VEC, int KH, bool STEPS>
+// Piece `piece` of row `row`; of a row of another kind nothing.  (ALIGNED: as load_raw() has it.  STEPS: there may
+// be rows for nth_steps.h, whose bits take registers that the others can do without.)
+template <bool ALIGNED, int KH, bool STEPS>
 __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_arg, const Scratch& sc_val, uint32_t slices, uint32_t row, uint32_t piece,
                                                     unsigned long long* s_dyn64, FinishShared& sm, ArgsLds& s_args)
 {
@@ -133,7 +122,7 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
     float wv[16];
     // (a row for nth_steps.h: the first round's pivot if every logit should turn out to be a candidate)
     const bool steps = STEPS && !in_order && nth_steps_for(d.n_vocab); // uniform
-    load_penalised<VEC, KH>(d, row, lo, hi, kSliceMax, P, hl, pen, reinterpret_cast<uint32_t*>(s_dyn64), wv, [&]() {
+    load_penalised<ALIGNED, KH>(d, row, lo, hi, kSliceMax, P, hl, pen, reinterpret_cast<uint32_t*>(s_dyn64), wv, [&]() {
         if (steps)
             first_pivot(d, row, P, pen ? hl : 0u, m, sm);
     });
@@ -153,13 +142,13 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
 #pragma unroll
     for (uint32_t b = 0; b < 4; ++b) {
         bsum[b] = 0.0;
-        // (the thread's logits 4b .. 4b+3 lie in the piece's b-th 4 096: four in a row, or 1 024 apart)
-        const uint32_t base = elem_index<VEC>(lo, tid, 4u * b);
+        // (the thread's logits 4b .. 4b+3 lie in the piece's b-th 4 096, four in a row)
+        const uint32_t base = elem_index(lo, tid, 4u * b);
         if (lo + b * kIndexBlock < hi) { // uniform
             uint32_t k[4];
 #pragma unroll
             for (uint32_t c = 0; c < 4; ++c) {
-                const uint32_t at = elem_index<VEC>(lo, tid, 4u * b + c);
+                const uint32_t at = elem_index(lo, tid, 4u * b + c);
                 const float q = weight_of(wv[4u * b + c], m, inv_t, sm.tab);
                 const bool ok = at < hi && q >= floor_q && q > 0.0f; // src/gen/sampler.cpp:34-35
                 k[c] = ok ? __float_as_uint(q) : 0u;
@@ -167,20 +156,20 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
                 last = ok ? max(last, at + 1u) : last;
                 bsum[b] += ok ? (double)q : 0.0;
             }
-            if (VEC && base + 3u < hi) {
+            if (base + 3u < hi) {
                 *reinterpret_cast<uint4*>(key0 + base) = make_uint4(~k[0], ~k[1], ~k[2], ~k[3]);
             } else {
 #pragma unroll
                 for (uint32_t c = 0; c < 4; ++c)
-                    if (elem_index<VEC>(lo, tid, 4u * b + c) < hi)
-                        key0[elem_index<VEC>(lo, tid, 4u * b + c)] = ~k[c];
+                    if (elem_index(lo, tid, 4u * b + c) < hi)
+                        key0[elem_index(lo, tid, 4u * b + c)] = ~k[c];
             }
             if (steps) { // uniform
                 // who is a candidate, and who belongs left of the pivot: bits for nth_steps.h's first step
                 uint32_t is = 0, left = 0;
 #pragma unroll
                 for (uint32_t c = 0; c < 4; ++c) {
-                    const uint32_t at = elem_index<VEC>(lo, tid, 4u * b + c);
+                    const uint32_t at = elem_index(lo, tid, 4u * b + c);
                     // (where the pivot was, the first entry is now, token 0)
                     const bool moved = at == first.from;
                     const uint32_t key = moved ? first.first_key : ~k[c];
@@ -188,19 +177,19 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
                     is |= (k[c] ? 1u : 0u) << c;
                     left |= (at != 0u && at < hi && lighter ? 1u : 0u) << c;
                 }
-                store_nth_bits<VEC>(as_global(nth_bits(sc, row, 2u)), base, is);
-                store_nth_bits<VEC>(as_global(nth_bits(sc, row, 0u)), base, left);
+                store_nth_bits(as_global(nth_bits(sc, row, 2u)), base, is);
+                store_nth_bits(as_global(nth_bits(sc, row, 0u)), base, left);
             } else if (!in_order) { // uniform
                 // the token ids as well: with them this is the whole-row path's list of candidates when every logit turns out
                 // to be one, as the pieces' counts will tell
                 uint32_t* li = sc.idx[0] + (size_t)row * sc.vpad;
-                if (VEC && base + 3u < hi) {
+                if (base + 3u < hi) {
                     *reinterpret_cast<uint4*>(li + base) = make_uint4(base, base + 1u, base + 2u, base + 3u);
                 } else {
 #pragma unroll
                     for (uint32_t c = 0; c < 4; ++c)
-                        if (elem_index<VEC>(lo, tid, 4u * b + c) < hi)
-                            li[elem_index<VEC>(lo, tid, 4u * b + c)] = elem_index<VEC>(lo, tid, 4u * b + c);
+                        if (elem_index(lo, tid, 4u * b + c) < hi)
+                            li[elem_index(lo, tid, 4u * b + c)] = elem_index(lo, tid, 4u * b + c);
                 }
             }
         }
@@ -411,14 +400,14 @@ struct RankedRows {
 #ifdef MAKO_EMIT_INDEX_KERNELS
 // grid = (rows rounded up to a multiple of eight, ceil(V / 16384)): workgroups go to the eight XCDs in turn, so that all of
 // these kernels work on a row on the same one.
-template <bool VEC, int KH, bool STEPS>
+template <bool ALIGNED, int KH, bool STEPS>
 __global__ __launch_bounds__(kThreads) void index_weights_kernel(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices)
 {
     extern __shared__ __align__(16) unsigned long long s_dyn64[];
     __shared__ FinishShared sm;
     __shared__ ArgsLds s_args;
     if (blockIdx.x < d_arg.n_rows)
-        index_weights_piece<VEC, KH, STEPS>(d_arg, sc_val, slices, blockIdx.x, blockIdx.y, s_dyn64, sm, s_args);
+        index_weights_piece<ALIGNED, KH, STEPS>(d_arg, sc_val, slices, blockIdx.x, blockIdx.y, s_dyn64, sm, s_args);
 }
 
 // grid = (rows rounded up to a multiple of eight, ceil(V / (4096 GPW))).

@@ -4,34 +4,34 @@
 
 namespace mako {
 namespace {
-template <bool VEC, int KH, bool UNSORTED>
+template <bool ALIGNED, int KH, bool UNSORTED>
 void launch_one(uint32_t wgs, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices)
 {
-    hipLaunchKernelGGL((finish_kernel<VEC, KH, UNSORTED>), dim3(1, wgs), dim3(kThreads), kFinishLds, st, d, sc, slices);
+    hipLaunchKernelGGL((finish_kernel<ALIGNED, KH, UNSORTED>), dim3(1, wgs), dim3(kThreads), kFinishLds, st, d, sc, slices);
 }
-template <bool VEC, bool UNSORTED>
-void launch_vec(int kh, uint32_t wgs, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices)
+template <bool ALIGNED, bool UNSORTED>
+void launch_aligned(int kh, uint32_t wgs, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices)
 {
     if (kh == 2)
-        launch_one<VEC, 2, UNSORTED>(wgs, st, d, sc, slices);
+        launch_one<ALIGNED, 2, UNSORTED>(wgs, st, d, sc, slices);
     else if (kh == 8)
-        launch_one<VEC, 8, UNSORTED>(wgs, st, d, sc, slices);
+        launch_one<ALIGNED, 8, UNSORTED>(wgs, st, d, sc, slices);
     else
-        launch_one<VEC, 0, UNSORTED>(wgs, st, d, sc, slices);
+        launch_one<ALIGNED, 0, UNSORTED>(wgs, st, d, sc, slices);
 }
 } // namespace
 
-void launch_finish(bool vec, int kh, bool unsorted, uint32_t wgs, hipStream_t st, const mako_sample_desc& d, const Scratch& sc,
+void launch_finish(bool aligned, int kh, bool unsorted, uint32_t wgs, hipStream_t st, const mako_sample_desc& d, const Scratch& sc,
                    uint32_t slices)
 {
-    if (vec && unsorted)
-        launch_vec<true, true>(kh, wgs, st, d, sc, slices);
-    else if (vec)
-        launch_vec<true, false>(kh, wgs, st, d, sc, slices);
+    if (aligned && unsorted)
+        launch_aligned<true, true>(kh, wgs, st, d, sc, slices);
+    else if (aligned)
+        launch_aligned<true, false>(kh, wgs, st, d, sc, slices);
     else if (unsorted)
-        launch_vec<false, true>(kh, wgs, st, d, sc, slices);
+        launch_aligned<false, true>(kh, wgs, st, d, sc, slices);
     else
-        launch_vec<false, false>(kh, wgs, st, d, sc, slices);
+        launch_aligned<false, false>(kh, wgs, st, d, sc, slices);
 }
 
 hipError_t init_finish_kernels()

@@ -5,24 +5,24 @@
 
 namespace mako {
 namespace {
-template <bool VEC, bool STEPS>
+template <bool ALIGNED, bool STEPS>
 void launch_weights(int kh, dim3 grid, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices)
 {
     if (kh == 2)
-        hipLaunchKernelGGL((index_weights_kernel<VEC, 2, STEPS>), grid, dim3(kThreads), kDynLds, st, d, sc, slices);
+        hipLaunchKernelGGL((index_weights_kernel<ALIGNED, 2, STEPS>), grid, dim3(kThreads), kDynLds, st, d, sc, slices);
     else if (kh == 8)
-        hipLaunchKernelGGL((index_weights_kernel<VEC, 8, STEPS>), grid, dim3(kThreads), kDynLds, st, d, sc, slices);
+        hipLaunchKernelGGL((index_weights_kernel<ALIGNED, 8, STEPS>), grid, dim3(kThreads), kDynLds, st, d, sc, slices);
     else
-        hipLaunchKernelGGL((index_weights_kernel<VEC, 0, STEPS>), grid, dim3(kThreads), kDynLds, st, d, sc, slices);
+        hipLaunchKernelGGL((index_weights_kernel<ALIGNED, 0, STEPS>), grid, dim3(kThreads), kDynLds, st, d, sc, slices);
 }
 } // namespace
 
-void launch_index_weights(bool vec, int kh, bool steps, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices)
+void launch_index_weights(bool aligned, int kh, bool steps, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices)
 {
     const dim3 grid((d.n_rows + 7u) & ~7u, (d.n_vocab + kSliceMax - 1u) / kSliceMax);
-    if (vec && steps)
+    if (aligned && steps)
         launch_weights<true, true>(kh, grid, st, d, sc, slices);
-    else if (vec)
+    else if (aligned)
         launch_weights<true, false>(kh, grid, st, d, sc, slices);
     else if (steps)
         launch_weights<false, true>(kh, grid, st, d, sc, slices);

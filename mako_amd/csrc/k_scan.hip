@@ -4,41 +4,41 @@
 
 namespace mako {
 namespace {
-template <bool VEC, int KH, bool ABOVE>
+template <bool ALIGNED, int KH, bool ABOVE>
 void launch_one(dim3 grid, size_t lds, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slice_len,
                 uint32_t cus)
 {
-    hipLaunchKernelGGL((scan_kernel<VEC, KH, ABOVE>), grid, dim3(kThreads), lds, st, d, sc, slice_len, cus);
+    hipLaunchKernelGGL((scan_kernel<ALIGNED, KH, ABOVE>), grid, dim3(kThreads), lds, st, d, sc, slice_len, cus);
 }
-template <bool VEC, int KH>
+template <bool ALIGNED, int KH>
 void launch_kh(bool above, dim3 grid, size_t lds, hipStream_t st, const mako_sample_desc& d, const Scratch& sc,
                uint32_t slice_len, uint32_t cus)
 {
     if (above)
-        launch_one<VEC, KH, true>(grid, lds, st, d, sc, slice_len, cus);
+        launch_one<ALIGNED, KH, true>(grid, lds, st, d, sc, slice_len, cus);
     else
-        launch_one<VEC, KH, false>(grid, lds, st, d, sc, slice_len, cus);
+        launch_one<ALIGNED, KH, false>(grid, lds, st, d, sc, slice_len, cus);
 }
-template <bool VEC>
-void launch_vec(int kh, bool above, dim3 grid, size_t lds, hipStream_t st, const mako_sample_desc& d, const Scratch& sc,
+template <bool ALIGNED>
+void launch_aligned(int kh, bool above, dim3 grid, size_t lds, hipStream_t st, const mako_sample_desc& d, const Scratch& sc,
                 uint32_t slice_len, uint32_t cus)
 {
     if (kh == 2)
-        launch_kh<VEC, 2>(above, grid, lds, st, d, sc, slice_len, cus);
+        launch_kh<ALIGNED, 2>(above, grid, lds, st, d, sc, slice_len, cus);
     else if (kh == 8)
-        launch_kh<VEC, 8>(above, grid, lds, st, d, sc, slice_len, cus);
+        launch_kh<ALIGNED, 8>(above, grid, lds, st, d, sc, slice_len, cus);
     else
-        launch_kh<VEC, 0>(above, grid, lds, st, d, sc, slice_len, cus);
+        launch_kh<ALIGNED, 0>(above, grid, lds, st, d, sc, slice_len, cus);
 }
 } // namespace
 
-void launch_scan(bool vec, int kh, bool above, dim3 grid, size_t lds, hipStream_t st, const mako_sample_desc& d,
+void launch_scan(bool aligned, int kh, bool above, dim3 grid, size_t lds, hipStream_t st, const mako_sample_desc& d,
                  const Scratch& sc, uint32_t slice_len, uint32_t cus)
 {
-    if (vec)
-        launch_vec<true>(kh, above, grid, lds, st, d, sc, slice_len, cus);
+    if (aligned)
+        launch_aligned<true>(kh, above, grid, lds, st, d, sc, slice_len, cus);
     else
-        launch_vec<false>(kh, above, grid, lds, st, d, sc, slice_len, cus);
+        launch_aligned<false>(kh, above, grid, lds, st, d, sc, slice_len, cus);
 }
 
 hipError_t init_scan_kernels()

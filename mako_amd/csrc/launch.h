@@ -17,15 +17,15 @@ hipError_t init_plan_alone();
 hipError_t init_sort_kernels();
 hipError_t init_tail_kernels();
 
-// scan_kernel<vec, kh, above>, grid = (slices, rows), `lds` bytes of dynamic LDS
+// scan_kernel<aligned, kh, above>, grid = (slices, rows), `lds` bytes of dynamic LDS
 // (`sc`: the HOST copy of the context's record; the kernels take it by value, so that their first loads need no
 // trip to memory for the record itself)
-void launch_scan(bool vec, int kh, bool above, dim3 grid, size_t lds, hipStream_t st, const mako_sample_desc& d,
+void launch_scan(bool aligned, int kh, bool above, dim3 grid, size_t lds, hipStream_t st, const mako_sample_desc& d,
                  const Scratch& sc, uint32_t slice_len, uint32_t cus);
-// finish_kernel<vec, kh> on `wgs` workgroups
+// finish_kernel<aligned, kh> on `wgs` workgroups
 // (unsorted: the instances for batches of many top_k == 0 rows, whose plans leave shares unsorted; the kernels
 // of one batch must agree on it)
-void launch_finish(bool vec, int kh, bool unsorted, uint32_t wgs, hipStream_t st, const mako_sample_desc& d, const Scratch& sc,
+void launch_finish(bool aligned, int kh, bool unsorted, uint32_t wgs, hipStream_t st, const mako_sample_desc& d, const Scratch& sc,
                    uint32_t slices); // (host copy, by value)
 void launch_plan_alone(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices); // (host copy, by value)
 // sort_kernel's workgroup i serves entry i of the work list: `grid_rows` * kWorkers workgroups must cover the
@@ -38,7 +38,7 @@ void launch_tail(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, u
 // total and the draw
 hipError_t init_index_kernels();
 // (steps: there are rows for nth_steps.h)
-void launch_index_weights(bool vec, int kh, bool steps, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices);
+void launch_index_weights(bool aligned, int kh, bool steps, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices);
 // a step of nth_steps.h, `wgs` workgroups per row
 void launch_nth_step(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t step, uint32_t wgs);
 void launch_index_finish(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, bool in_order_rows, bool other_rows);
@@ -47,7 +47,7 @@ void launch_index_finish(hipStream_t st, const mako_sample_desc& d, const Scratc
 hipError_t init_beside_finish();
 hipError_t init_beside_sort();
 hipError_t init_beside_tail();
-void launch_finish_beside(bool vec, int kh, bool unsorted, uint32_t wgs, uint32_t more, hipStream_t st, const mako_sample_desc& d,
+void launch_finish_beside(bool aligned, int kh, bool unsorted, uint32_t wgs, uint32_t more, hipStream_t st, const mako_sample_desc& d,
                           const Scratch& sc, uint32_t slices);
 void launch_sort_beside(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices, uint32_t grid_rows, bool unsorted,
                         uint32_t more);

@@ -380,7 +380,7 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
     if (2ull * d.n_rows > kGridYMax)
         return fail(ctx, MAKO_ERR_INVALID_ARG, "sampler: more rows than one launch can index (32767)");
     const uint32_t slice_len = slice_len_for(d.n_vocab, slices);
-    const bool vec = d.n_vocab % 4 == 0 && d.logits_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(d.logits) & 15u) == 0;
+    const bool aligned = d.n_vocab % 4 == 0 && d.logits_stride % 4 == 0 && (reinterpret_cast<uintptr_t>(d.logits) & 15u) == 0;
     const size_t lds = d.hist_tokens ? (size_t)slice_len * sizeof(uint32_t) : 0;
     // (scan_kernel: with histories a row's slices share an XCD)
     const dim3 grid = d.hist_tokens ? dim3((d.n_rows + 7u) & ~7u, slices) : dim3(slices, d.n_rows);
@@ -447,7 +447,7 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
         }                                                                                                          \
     } while (0)
     MAKO_MARK(0);
-    MAKO_LAUNCH(mako::launch_scan(vec, kh, d.close_token != nullptr, grid, lds, st, d, sc, slice_len, std::min(ctx->cus, mako::kCountGeneral - 1u) | (beside ? mako::kCountGeneral : 0u) | ((finish_wgs / 8u) << 16)));
+    MAKO_LAUNCH(mako::launch_scan(aligned, kh, d.close_token != nullptr, grid, lds, st, d, sc, slice_len, std::min(ctx->cus, mako::kCountGeneral - 1u) | (beside ? mako::kCountGeneral : 0u) | ((finish_wgs / 8u) << 16)));
     MAKO_MARK(1);
     // top_k == 0 rows: planned and handed out by the second pass, sorted, cut and drawn from; the stages talk through
     // kernel boundaries (device-wide fences inside a kernel cost far more on this chip).  A batch without such rows
@@ -457,7 +457,7 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
         const uint32_t pieces = (d.n_vocab + mako::kSliceMax - 1u) / mako::kSliceMax, blocks = (d.n_vocab + mako::kIndexBlock - 1u) / mako::kIndexBlock;
         const uint32_t for_weights = (uint32_t)std::min<uint64_t>((uint64_t)index_rows * pieces, ctx->cus);
         const uint32_t for_groups = (uint32_t)std::min<uint64_t>((uint64_t)index_rows * blocks, ctx->cus);
-        MAKO_LAUNCH(mako::launch_finish_beside(vec, kh, unsorted, any_nucleus ? finish_wgs : 0u, for_weights, st, d, sc, slices));
+        MAKO_LAUNCH(mako::launch_finish_beside(aligned, kh, unsorted, any_nucleus ? finish_wgs : 0u, for_weights, st, d, sc, slices));
         MAKO_MARK(2);
         if (any_nucleus || any_in_order || any_nth || !params_host)
             MAKO_LAUNCH(mako::launch_sort_beside(st, d, sc, slices, any_nucleus ? nucleus_rows : 0u, unsorted, for_groups));
@@ -467,9 +467,9 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
         MAKO_LAUNCH(mako::launch_tail_beside(st, d, sc, slices, nucleus_rows, unsorted));
     } else {
         if (only_index)
-            MAKO_LAUNCH(mako::launch_index_weights(vec, kh, any_nth, st, d, sc, slices));
+            MAKO_LAUNCH(mako::launch_index_weights(aligned, kh, any_nth, st, d, sc, slices));
         if (any_nucleus)
-            MAKO_LAUNCH(mako::launch_finish(vec, kh, unsorted, finish_wgs, st, d, sc, slices));
+            MAKO_LAUNCH(mako::launch_finish(aligned, kh, unsorted, finish_wgs, st, d, sc, slices));
         if (!launch_sort && !only_index)
             MAKO_LAUNCH(mako::launch_plan_alone(st, d, sc, slices));
         MAKO_MARK(2);

@@ -171,7 +171,7 @@ struct Scratch {
     uint32_t* work_n;      // [kWorkWords] entries in work_sort, work_tail (zeroed by scan_kernel); [3]: the large batches' collectors; [2]: failed checks of a checked
                            // build (MAKO_CHECK); then, 16-byte aligned at [4], how the second pass is cut up
                            // (SecondPassCut; scan_kernel's first workgroup decides), and at [8], for launches that serve
-                           // them beside others, the rows of the whole-row class and those of them in token order
+                           // them beside others, the rows of the whole-row class and those of them in token order; [10]: top_k == 0 rows
     uint32_t* work_sort;   // [max_rows * kSortItemsPerRow] row << 8 | worker; appended by finish_kernel.  The large batches'
                            // instances keep two lists in it that meet, the costliest entries in front (large_batch_lists())
     uint32_t* work_tail;   // [max_rows] row; appended by finish_kernel

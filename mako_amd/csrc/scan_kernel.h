@@ -36,9 +36,10 @@ __device__ __forceinline__ uint32_t wave_kth_largest(uint32_t key, uint32_t j)
 
 // (ABOVE: the batch has close tokens, whose logits' ranks are counted on the way; a variant of its own because the
 // count takes sixteen more registers, up to the limit for two workgroups per CU, which no other batch should pay)
-// (amdgpu_waves_per_eu: the vectorised variants are held to the 64 registers that let two workgroups share a CU)
-template <bool VEC, int KH, bool ABOVE = false>
-__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(VEC ? 8 : 4))) void scan_kernel(mako_sample_desc d, Scratch sc_arg, uint32_t slice_len,
+// (amdgpu_waves_per_eu: held to the 64 registers that let two workgroups share a CU, but for rows at any address with eight
+// history entries a thread, which would spill forty)
+template <bool ALIGNED, int KH, bool ABOVE = false>
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(ALIGNED || KH < 8 ? 8 : 4))) void scan_kernel(mako_sample_desc d, Scratch sc_arg, uint32_t slice_len,
                                                         uint32_t cus_and_grid)
 {
     // (cus_and_grid: the CUs of the device, kCountGeneral, and in the upper half an eighth of finish_kernel's grid:
@@ -115,11 +116,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(VEC ? 
     uint32_t above = 0;
     float wv[16];
     if (ABOVE) {
-        load_penalised<VEC, KH>(d, row, lo, hi, slice_len, P, hl, pen, s_dyn, wv, NoOverlap(), want_above, close_v, &above);
+        load_penalised<ALIGNED, KH>(d, row, lo, hi, slice_len, P, hl, pen, s_dyn, wv, NoOverlap(), want_above, close_v, &above);
         if (want_above) // uniform
             above = __ockl_wfred_add_u32(above);
     } else {
-        load_penalised<VEC, KH>(d, row, lo, hi, slice_len, P, hl, pen, s_dyn, wv);
+        load_penalised<ALIGNED, KH>(d, row, lo, hi, slice_len, P, hl, pen, s_dyn, wv);
     }
 
     MAKO_STAMP(29);
@@ -162,7 +163,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(VEC ? 
 #pragma unroll
         for (int j = 15; j >= 0; --j)
             if (wv[j] == M)
-                first = elem_index<VEC>(lo, tid, (uint32_t)j);
+                first = elem_index(lo, tid, (uint32_t)j);
         if (first != kNone)
             atomicMin(&sm.argidx, first);
     }
@@ -211,7 +212,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(VEC ? 
                     const float w = wv[j];
                     if (w >= tau && pos < kCap) {
                         sm.cw[pos] = w;
-                        sm.ci[pos] = elem_index<VEC>(lo, tid, j);
+                        sm.ci[pos] = elem_index(lo, tid, j);
                     }
                     run += (uint32_t)__popcll(takes[j]);
                 }

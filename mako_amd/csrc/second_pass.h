@@ -18,7 +18,7 @@ namespace mako {
 // (`slices`: of scan_kernel, whose records give the row maximum)
 // (PLANNING: the workgroup's first piece, with which the plan is built; returns false when the row leaves for the
 // whole-row path and the pass has nothing more to do for it)
-template <bool VEC, int KH, bool PEN, bool PLANNING, bool UNSORTED = false>
+template <bool ALIGNED, int KH, bool PEN, bool PLANNING, bool UNSORTED = false>
 __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t row, uint32_t slice, uint32_t slice_len,
                           const mako_sampling_params& P, uint32_t hl, uint32_t slices, const FinishLds& L, CoarsePlan& pl,
                           float& m, uint32_t& argidx, uint32_t opaque_first = kNone)
@@ -35,13 +35,13 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
     if constexpr (PLANNING) {
         PlanLoads pre;
         issue_plan_loads<UNSORTED>(d, sc, row, slices, pre);
-        load_penalised<VEC, KH>(d, row, lo, hi, slice_len, P, hl, pen, L.cnt, wv, [&]() {
+        load_penalised<ALIGNED, KH>(d, row, lo, hi, slice_len, P, hl, pen, L.cnt, wv, [&]() {
             uint32_t n_cands, any_overflow;
             row_summary_of(pre.st, slices, m, argidx, n_cands, any_overflow);
             coarse_plan(sc, row, slices, d.n_vocab, P, m, pre, !any_overflow && n_cands <= kSortMax, UNSORTED ? opaque_first : kNone, UNSORTED ? kShareLarge : kShareSmall, pl, sm.tab);
         });
     } else {
-        load_penalised<VEC, KH>(d, row, lo, hi, slice_len, P, hl, pen, L.cnt, wv);
+        load_penalised<ALIGNED, KH>(d, row, lo, hi, slice_len, P, hl, pen, L.cnt, wv);
     }
     MAKO_STAMP(1);
     MAKO_STAMP(24);
@@ -109,7 +109,7 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
             qb[j] = 0u;
             slot[j] = kNone;
         }
-        if (lo + (VEC ? (g / 4u) * 4096u : g * (uint32_t)kThreads) < hi) {
+        if (lo + (g / 4u) * 4096u < hi) {
             bool keeps[4];
             // (the large batches' instance: a wave whose four weights a lane all underflow to zero, as those of a peaked row far
             // below its maximum do, skips the arithmetic that would tell it so; expf_glibc() returns 0 below that bound)
@@ -224,7 +224,7 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
 #pragma unroll
         for (uint32_t j = 0; j < 16; ++j)
             if (slot[j] != kNone)
-                buf[slot[j] & 0xffffu] = make_uint2(qb[j], elem_index<VEC>(lo, tid, j) | ((slot[j] >> 16) << kIdBits));
+                buf[slot[j] & 0xffffu] = make_uint2(qb[j], elem_index(lo, tid, j) | ((slot[j] >> 16) << kIdBits));
         if (tid < kWorkers) { // (wave 0: where each worker's run goes and where its room ends, in the workgroup's order)
             const uint32_t room = pl.cap[tid];
             pl.run[tid] = make_uint2(pl.stage_off[tid] + base_mine - lbase_mine, lbase_mine + (room > base_mine ? room - base_mine : 0u));
@@ -261,7 +261,7 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
     return true;
 }
 
-template <bool VEC, int KH, bool PEN, bool UNSORTED>
+template <bool ALIGNED, int KH, bool PEN, bool UNSORTED>
 __device__ void row_pieces(const mako_sample_desc& d, const Scratch& sc, uint32_t row, uint32_t first, uint32_t stride,
                            uint32_t n_pieces, uint32_t slice_len, const mako_sampling_params& P, uint32_t hl, uint32_t slices,
                            const FinishLds& L, CoarsePlan& pl, uint32_t opaque_first)
@@ -270,10 +270,10 @@ __device__ void row_pieces(const mako_sample_desc& d, const Scratch& sc, uint32_
     // the workgroup's pieces in turn: first, first + stride, ...
     float m = 0.0f;
     uint32_t argidx = 0;
-    if (first >= n_pieces || !one_piece<VEC, KH, PEN, true, UNSORTED>(d, sc, row, first, slice_len, P, hl, slices, L, pl, m, argidx, opaque_first))
+    if (first >= n_pieces || !one_piece<ALIGNED, KH, PEN, true, UNSORTED>(d, sc, row, first, slice_len, P, hl, slices, L, pl, m, argidx, opaque_first))
         return;
     for (uint32_t slice = first + stride; slice < n_pieces; slice += stride)
-        one_piece<VEC, KH, PEN, false, UNSORTED>(d, sc, row, slice, slice_len, P, hl, slices, L, pl, m, argidx);
+        one_piece<ALIGNED, KH, PEN, false, UNSORTED>(d, sc, row, slice, slice_len, P, hl, slices, L, pl, m, argidx);
 }
 
 // Second pass over the top_k == 0 rows.  grid = (most pieces a row can have, rows) workgroups, of which workgroup i
@@ -282,7 +282,7 @@ __device__ void row_pieces(const mako_sample_desc& d, const Scratch& sc, uint32_
 // mix of rows.
 // (UNSORTED: the instance for batches of many such rows, whose plans leave shares unsorted: unsorted_shares.h)
 // (n_wgs: workgroups of the launch that are finish_kernel's)
-template <bool VEC, int KH, bool UNSORTED>
+template <bool ALIGNED, int KH, bool UNSORTED>
 __device__ __forceinline__ void finish_body(const mako_sample_desc& d_arg, const Scratch& sc_arg, uint32_t slices, uint32_t n_wgs,
                                             unsigned long long* s_dyn64, FinishShared& sm, ArgsLds& s_args, CoarsePlan& s_plan)
 {
@@ -379,20 +379,20 @@ __device__ __forceinline__ void finish_body(const mako_sample_desc& d_arg, const
         s_plan.nucleus_rows = nucleus_rows; // (read behind the plan's barriers)
     const uint32_t opaque_first = (UNSORTED && !d.draft) ? max(kHeadGroups * kGroup, (d.out_cand_idx && d.out_cand_q) ? d.cand_cap : 0u) : kNone;
     if (d.hist_tokens && !penalties_neutral(P))
-        row_pieces<VEC, KH, true, UNSORTED>(d, sc, row, piece, pieces, n_pieces, piece_len, P, hl, slices, L, s_plan, opaque_first);
+        row_pieces<ALIGNED, KH, true, UNSORTED>(d, sc, row, piece, pieces, n_pieces, piece_len, P, hl, slices, L, s_plan, opaque_first);
     else
-        row_pieces<VEC, KH, false, UNSORTED>(d, sc, row, piece, pieces, n_pieces, piece_len, P, hl, slices, L, s_plan, opaque_first);
+        row_pieces<ALIGNED, KH, false, UNSORTED>(d, sc, row, piece, pieces, n_pieces, piece_len, P, hl, slices, L, s_plan, opaque_first);
 }
 
 // (its arguments by value: the cut is one trip to memory away, not two)
-template <bool VEC, int KH, bool UNSORTED>
+template <bool ALIGNED, int KH, bool UNSORTED>
 __global__ __launch_bounds__(kThreads) void finish_kernel(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices)
 {
     extern __shared__ __align__(16) unsigned long long s_dyn64[]; // (128-bit LDS operations need the alignment)
     __shared__ FinishShared sm;
     __shared__ ArgsLds s_args;
     __shared__ CoarsePlan s_plan;
-    finish_body<VEC, KH, UNSORTED>(d_arg, sc_val, slices, gridDim.y, s_dyn64, sm, s_args, s_plan);
+    finish_body<ALIGNED, KH, UNSORTED>(d_arg, sc_val, slices, gridDim.y, s_dyn64, sm, s_args, s_plan);
 }
 
 } // namespace mako

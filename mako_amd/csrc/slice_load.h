@@ -5,13 +5,11 @@
 
 namespace mako {
 
-// Thread t of a slice owns 16 logits: for k = 0..3 the four consecutive ones at lo + k * 4096 + 4 * t
-// (VEC), or lo + j * 1024 + t for j = 0..15 (scalar).  Either way a wavefront's loads are contiguous and
-// each logit is read once.
-template <bool VEC>
+// Thread t of a slice owns 16 logits: for k = 0..3 the four consecutive ones at lo + k * 4096 + 4 * t.  A wavefront's
+// loads are contiguous and each logit is read once.
 __device__ __forceinline__ uint32_t elem_index(uint32_t lo, uint32_t tid, uint32_t j)
 {
-    return VEC ? lo + (j >> 2) * 4096u + tid * 4u + (j & 3u) : lo + j * (uint32_t)kThreads + tid;
+    return lo + (j >> 2) * 4096u + tid * 4u + (j & 3u);
 }
 
 // accept() history -> per-token counts for [lo, hi) in LDS (src/gen/sampler.cpp:15-18); generic form used
@@ -34,96 +32,112 @@ __device__ __forceinline__ void build_counts(const mako_sample_desc& d, uint32_t
     __syncthreads();
 }
 
-// The thread's 16 logits, raw, plus the mask bits of each group of four (VEC) or of each logit (scalar).
+// The thread's 16 logits, raw, plus the mask bits of each group of four.
 // Issued before anything else so that the HBM latency overlaps the LDS work that follows.
-template <bool VEC>
+// ALIGNED: the rows are 16-byte aligned and a multiple of four long.  Of any other row a group of four is loaded the same way,
+// from a multiple of four bytes, and the row's last group from four logits in front of its end (settle_slice()).  (One logit
+// at a time, 1 024 apart, the loads take four times the instructions and twice the registers, and no two workgroups of
+// scan_kernel and index_weights_kernel shared a CU: 64 rows of 129 281 logits, temperature only, 84 us and 79 so; a decode
+// batch of 64 such rows 71 and 63; 256 top-k rows under masks 105 and 42, and 40 where the rows are aligned.)
 struct RawSlice {
     float4 v[4];
-    uint32_t bits[4]; // VEC: bit c of bits[k] = logit 4k+c allowed; scalar: bit j of bits[0] = logit j allowed
+    uint32_t bits[4]; // bit c of bits[k] = logit 4k+c allowed
 };
+typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
-template <bool VEC>
-__device__ __forceinline__ void load_raw(const mako_sample_desc& d, uint32_t row, uint32_t lo, uint32_t hi, RawSlice<VEC>& r)
+template <bool ALIGNED>
+__device__ __forceinline__ void load_raw(const mako_sample_desc& d, uint32_t row, uint32_t lo, uint32_t hi, RawSlice& r)
 {
     const uint32_t tid = threadIdx.x;
     const global_ptr<const float> lrow = as_global(d.logits) + (int64_t)row * d.logits_stride;
     const global_ptr<const uint32_t> mrow = d.mask ? as_global(d.mask) + (int64_t)row * d.mask_stride : nullptr;
-    const float nan = __uint_as_float(0x7fc00000u);
-    if (VEC) {
-        // all four loads go out back to back, from clamped addresses and without a branch between them (a branch
-        // would make the compiler wait for each load before the next); what lies past the slice is dropped after
-        uint32_t at[4];
+    // all four loads go out back to back, from clamped addresses and without a branch between them (a branch
+    // would make the compiler wait for each load before the next); what lies past the slice is dropped after
+    uint32_t at[4];
+    if (!ALIGNED && d.n_vocab < 4u) { // uniform
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            at[k] = 0u;
+            float* v = reinterpret_cast<float*>(&r.v[k]);
+#pragma unroll
+            for (uint32_t c = 0; c < 4; ++c) // (where settle_slice() expects them)
+                v[c] = lrow[c + d.n_vocab > 4u ? c + d.n_vocab - 4u : 0u];
+        }
+    } else {
 #pragma unroll
         for (uint32_t k = 0; k < 4; ++k) {
             const uint32_t i = lo + k * 4096u + tid * 4u;
-            at[k] = i < hi ? i : hi - 4u; // hi - lo is a positive multiple of 4 in this mode
-            const f32x4 x = *(global_ptr<const f32x4>)(lrow + at[k]);
+            at[k] = i < hi ? i : (hi - 1u) & ~3u;
+            f32x4 x;
+            if (ALIGNED)
+                x = *(global_ptr<const f32x4>)(lrow + at[k]);
+            else
+                x = *(global_ptr<const f32x4_any>)(lrow + min(at[k], d.n_vocab - 4u));
             r.v[k] = make_float4(x.x, x.y, x.z, x.w);
         }
-        if (mrow) {
+    }
+    if (mrow) {
 #pragma unroll
-            for (uint32_t k = 0; k < 4; ++k)
-                r.bits[k] = mrow[at[k] >> 5] >> (at[k] & 31u);
-        }
-        if (!mrow) {
+        for (uint32_t k = 0; k < 4; ++k)
+            r.bits[k] = mrow[at[k] >> 5] >> (at[k] & 31u);
+    }
+    if (!mrow) {
 #pragma unroll
-            for (uint32_t k = 0; k < 4; ++k)
-                r.bits[k] = 0xfu;
-        }
-        // (finish_slice() replaces what was read past the slice: nothing here touches the loaded values, so the
-        // loads stay in flight while the caller goes on)
-    } else {
-        float* f = reinterpret_cast<float*>(r.v);
-        uint32_t allowed = 0xffffu;
+        for (uint32_t k = 0; k < 4; ++k)
+            r.bits[k] = 0xfu;
+    }
+    // (finish_slice() replaces what was read past the slice: nothing here touches the loaded values, so the
+    // loads stay in flight while the caller goes on)
+}
+
+// The row's last group, of one to three logits, moved to the front of its four, behind it NaN.  (A slice ends behind a whole
+// group everywhere else.)
+template <bool ALIGNED>
+__device__ __forceinline__ void settle_slice(RawSlice& r, uint32_t lo, uint32_t hi)
+{
+    if (ALIGNED || (hi & 3u) == 0u) // uniform
+        return;
+    const float nan = __uint_as_float(0x7fc00000u);
 #pragma unroll
-        for (uint32_t j = 0; j < 16; ++j) {
-            const uint32_t i = lo + j * (uint32_t)kThreads + tid;
-            f[j] = nan;
-            if (i < hi) {
-                f[j] = lrow[i];
-                if (mrow && !((mrow[i >> 5] >> (i & 31u)) & 1u))
-                    allowed &= ~(1u << j);
-            }
+    for (uint32_t k = 0; k < 4; ++k) {
+        if (lo + k * 4096u + threadIdx.x * 4u == (hi & ~3u)) {
+            const uint32_t n = hi & 3u;
+            const float4 x = r.v[k];
+            r.v[k].x = n == 3u ? x.y : (n == 2u ? x.z : x.w);
+            r.v[k].y = n == 3u ? x.z : (n == 2u ? x.w : nan);
+            r.v[k].z = n == 3u ? x.w : nan;
+            r.v[k].w = nan;
         }
-        r.bits[0] = allowed;
     }
 }
 
 // How many of the thread's logits (as the sampler is given them: a token the mask clears is -inf) are strictly
 // greater than v: the count of ReasoningBudget::forced, src/server/openai.cpp:599-602.
-template <bool VEC>
-__device__ __forceinline__ uint32_t count_above(const RawSlice<VEC>& r, uint32_t lo, uint32_t hi, float v)
+__device__ __forceinline__ uint32_t count_above(const RawSlice& r, uint32_t lo, uint32_t hi, float v)
 {
     const uint32_t tid = threadIdx.x;
     uint32_t c = 0;
-    if (VEC) {
 #pragma unroll
-        for (uint32_t k = 0; k < 4; ++k) {
-            if (lo + k * 4096u + tid * 4u < hi) {
-                c += ((r.bits[k] & 1u) && r.v[k].x > v) ? 1u : 0u;
-                c += ((r.bits[k] & 2u) && r.v[k].y > v) ? 1u : 0u;
-                c += ((r.bits[k] & 4u) && r.v[k].z > v) ? 1u : 0u;
-                c += ((r.bits[k] & 8u) && r.v[k].w > v) ? 1u : 0u;
-            }
+    for (uint32_t k = 0; k < 4; ++k) {
+        if (lo + k * 4096u + tid * 4u < hi) { // (what lies behind the row's last logit in its group is NaN)
+            c += ((r.bits[k] & 1u) && r.v[k].x > v) ? 1u : 0u;
+            c += ((r.bits[k] & 2u) && r.v[k].y > v) ? 1u : 0u;
+            c += ((r.bits[k] & 4u) && r.v[k].z > v) ? 1u : 0u;
+            c += ((r.bits[k] & 8u) && r.v[k].w > v) ? 1u : 0u;
         }
-    } else {
-        const float* f = reinterpret_cast<const float*>(r.v);
-#pragma unroll
-        for (uint32_t j = 0; j < 16; ++j)
-            c += (lo + j * (uint32_t)kThreads + tid < hi && ((r.bits[0] >> j) & 1u) && f[j] > v) ? 1u : 0u;
     }
     return c;
 }
 
 // Mask and penalties (src/gen/sampler.cpp:22-28) applied to the raw logits; slots past the end of the
 // slice hold NaN, which never wins a comparison and never becomes a candidate.
-template <bool VEC>
-__device__ __forceinline__ void finish_slice(const RawSlice<VEC>& r, uint32_t lo, uint32_t hi, const mako_sampling_params& P,
+template <bool ALIGNED>
+__device__ __forceinline__ void finish_slice(const RawSlice& r, uint32_t lo, uint32_t hi, const mako_sampling_params& P,
                                              bool pen, const uint32_t* s_cnt, float (&wv)[16], bool masked)
 {
     const uint32_t tid = threadIdx.x;
-    if (VEC && !masked) { // uniform: no mask, nothing to clear
-        const float nan = __uint_as_float(0x7fc00000u);
+    const float nan = __uint_as_float(0x7fc00000u);
+    if (!masked) { // uniform: no mask, nothing to clear
 #pragma unroll
         for (uint32_t k = 0; k < 4; ++k) {
             const bool inside = lo + k * 4096u + tid * 4u < hi;
@@ -132,54 +146,38 @@ __device__ __forceinline__ void finish_slice(const RawSlice<VEC>& r, uint32_t lo
             wv[4 * k + 2] = !inside ? nan : r.v[k].z;
             wv[4 * k + 3] = !inside ? nan : r.v[k].w;
         }
-    } else if (VEC) {
+    } else {
         // (a mask bit spread over a word, then one bit-field insert: the logit where the bit is set, -inf elsewhere)
-        const float nan = __uint_as_float(0x7fc00000u);
         auto pick = [](uint32_t bits, uint32_t c, float v) {
             const uint32_t m = (uint32_t)((int32_t)(bits << (31u - c)) >> 31); // all ones if bit c is set
             return __uint_as_float((__float_as_uint(v) & m) | (0xff800000u & ~m));
         };
 #pragma unroll
         for (uint32_t k = 0; k < 4; ++k) {
-            const bool inside = lo + k * 4096u + tid * 4u < hi;
-            wv[4 * k + 0] = !inside ? nan : pick(r.bits[k], 0, r.v[k].x);
-            wv[4 * k + 1] = !inside ? nan : pick(r.bits[k], 1, r.v[k].y);
-            wv[4 * k + 2] = !inside ? nan : pick(r.bits[k], 2, r.v[k].z);
-            wv[4 * k + 3] = !inside ? nan : pick(r.bits[k], 3, r.v[k].w);
+            const uint32_t i = lo + k * 4096u + tid * 4u;
+            // (a bit behind the row's last logit may be anything)
+            auto inside = [&](uint32_t c) { return ALIGNED ? i < hi : i + c < hi; };
+            wv[4 * k + 0] = !inside(0u) ? nan : pick(r.bits[k], 0, r.v[k].x);
+            wv[4 * k + 1] = !inside(1u) ? nan : pick(r.bits[k], 1, r.v[k].y);
+            wv[4 * k + 2] = !inside(2u) ? nan : pick(r.bits[k], 2, r.v[k].z);
+            wv[4 * k + 3] = !inside(3u) ? nan : pick(r.bits[k], 3, r.v[k].w);
         }
-    } else {
-        const float* f = reinterpret_cast<const float*>(r.v);
-#pragma unroll
-        for (uint32_t j = 0; j < 16; ++j)
-            wv[j] = ((r.bits[0] >> j) & 1u) ? f[j] : -INFINITY;
     }
     if (pen) {
-        if (VEC) {
 #pragma unroll
-            for (uint32_t k = 0; k < 4; ++k) {
-                const uint32_t i = lo + k * 4096u + tid * 4u;
-                if (i < hi) {
-                    const uint4 n = *reinterpret_cast<const uint4*>(s_cnt + (i - lo));
-                    if (n.x | n.y | n.z | n.w) {
-                        if (n.x)
-                            wv[4 * k + 0] = penalize(wv[4 * k + 0], n.x, P.repetition_penalty, P.presence_penalty, P.frequency_penalty);
-                        if (n.y)
-                            wv[4 * k + 1] = penalize(wv[4 * k + 1], n.y, P.repetition_penalty, P.presence_penalty, P.frequency_penalty);
-                        if (n.z)
-                            wv[4 * k + 2] = penalize(wv[4 * k + 2], n.z, P.repetition_penalty, P.presence_penalty, P.frequency_penalty);
-                        if (n.w)
-                            wv[4 * k + 3] = penalize(wv[4 * k + 3], n.w, P.repetition_penalty, P.presence_penalty, P.frequency_penalty);
-                    }
-                }
-            }
-        } else {
-#pragma unroll
-            for (uint32_t j = 0; j < 16; ++j) {
-                const uint32_t i = lo + j * (uint32_t)kThreads + tid;
-                if (i < hi) {
-                    const uint32_t n = s_cnt[i - lo];
-                    if (n)
-                        wv[j] = penalize(wv[j], n, P.repetition_penalty, P.presence_penalty, P.frequency_penalty);
+        for (uint32_t k = 0; k < 4; ++k) {
+            const uint32_t i = lo + k * 4096u + tid * 4u;
+            if (i < hi) {
+                const uint4 n = *reinterpret_cast<const uint4*>(s_cnt + (i - lo));
+                if (n.x | n.y | n.z | n.w) {
+                    if (n.x)
+                        wv[4 * k + 0] = penalize(wv[4 * k + 0], n.x, P.repetition_penalty, P.presence_penalty, P.frequency_penalty);
+                    if (n.y)
+                        wv[4 * k + 1] = penalize(wv[4 * k + 1], n.y, P.repetition_penalty, P.presence_penalty, P.frequency_penalty);
+                    if (n.z)
+                        wv[4 * k + 2] = penalize(wv[4 * k + 2], n.z, P.repetition_penalty, P.presence_penalty, P.frequency_penalty);
+                    if (n.w)
+                        wv[4 * k + 3] = penalize(wv[4 * k + 3], n.w, P.repetition_penalty, P.presence_penalty, P.frequency_penalty);
                 }
             }
         }
@@ -202,7 +200,7 @@ struct NoOverlap {
 
 // `overlap` runs right after the slice's loads have been issued: work that does not depend on them hides
 // behind their latency.  It must be reached by the whole workgroup or by none of it.
-template <bool VEC, int KH, typename Overlap = NoOverlap>
+template <bool ALIGNED, int KH, typename Overlap = NoOverlap>
 __device__ __forceinline__ void load_penalised(const mako_sample_desc& d, uint32_t row, uint32_t lo, uint32_t hi,
                                                uint32_t slice_len, const mako_sampling_params& P, uint32_t hl, bool pen,
                                                uint32_t* s_cnt, float (&wv)[16], Overlap overlap = Overlap(),
@@ -231,18 +229,26 @@ __device__ __forceinline__ void load_penalised(const mako_sample_desc& d, uint32
                 cnt[k] = hc[min(tid + (uint32_t)k * kThreads, last)];
         }
     }
-    RawSlice<VEC> raw;
-    load_raw<VEC>(d, row, lo, hi, raw);
+    RawSlice raw;
+    load_raw<ALIGNED>(d, row, lo, hi, raw);
     overlap();
-    if (want_above) // uniform
-        *above = count_above<VEC>(raw, lo, hi, close_v);
+    if (want_above) { // uniform
+        settle_slice<ALIGNED>(raw, lo, hi);
+        *above = count_above(raw, lo, hi, close_v);
+    }
+    auto settle = [&]() {
+        if (!want_above)
+            settle_slice<ALIGNED>(raw, lo, hi);
+    };
     if (!pen) {
-        finish_slice<VEC>(raw, lo, hi, P, false, s_cnt, wv, d.mask != nullptr);
+        settle();
+        finish_slice<ALIGNED>(raw, lo, hi, P, false, s_cnt, wv, d.mask != nullptr);
         return;
     }
     if (KH == 0) {
         build_counts(d, row, hl, lo, hi, slice_len, s_cnt);
-        finish_slice<VEC>(raw, lo, hi, P, true, s_cnt, wv, d.mask != nullptr);
+        settle();
+        finish_slice<ALIGNED>(raw, lo, hi, P, true, s_cnt, wv, d.mask != nullptr);
         return;
     }
 #pragma unroll
@@ -280,31 +286,21 @@ __device__ __forceinline__ void load_penalised(const mako_sample_desc& d, uint32
             cnt[k] = s_cnt[tok[k] - lo]; // occurrences of the token in the whole history
     lds_barrier(); // (the slots are about to be overwritten)
     MAKO_STAMP(22);
-    finish_slice<VEC>(raw, lo, hi, P, false, s_cnt, wv, d.mask != nullptr);
+    settle();
+    finish_slice<ALIGNED>(raw, lo, hi, P, false, s_cnt, wv, d.mask != nullptr);
     MAKO_STAMP(23);
     // owners: a logit whose slot is taken goes into the slot (its bits); `moved` remembers which of the sixteen
     uint32_t moved = 0;
-    if (VEC) {
 #pragma unroll
-        for (uint32_t k = 0; k < 4; ++k) {
-            const uint32_t i = lo + k * 4096u + tid * 4u;
-            if (i < hi) {
-                uint4* slot = reinterpret_cast<uint4*>(s_cnt + (i - lo));
-                const uint4 n = *slot;
-                if (n.x | n.y | n.z | n.w) {
-                    *slot = make_uint4(n.x ? __float_as_uint(wv[4 * k + 0]) : 0u, n.y ? __float_as_uint(wv[4 * k + 1]) : 0u,
-                                       n.z ? __float_as_uint(wv[4 * k + 2]) : 0u, n.w ? __float_as_uint(wv[4 * k + 3]) : 0u);
-                    moved |= ((n.x ? 1u : 0u) | (n.y ? 2u : 0u) | (n.z ? 4u : 0u) | (n.w ? 8u : 0u)) << (4u * k);
-                }
-            }
-        }
-    } else {
-#pragma unroll
-        for (uint32_t j = 0; j < 16; ++j) {
-            const uint32_t i = lo + j * (uint32_t)kThreads + tid;
-            if (i < hi && s_cnt[i - lo]) {
-                s_cnt[i - lo] = __float_as_uint(wv[j]);
-                moved |= 1u << j;
+    for (uint32_t k = 0; k < 4; ++k) {
+        const uint32_t i = lo + k * 4096u + tid * 4u;
+        if (i < hi) {
+            uint4* slot = reinterpret_cast<uint4*>(s_cnt + (i - lo));
+            const uint4 n = *slot;
+            if (n.x | n.y | n.z | n.w) {
+                *slot = make_uint4(n.x ? __float_as_uint(wv[4 * k + 0]) : 0u, n.y ? __float_as_uint(wv[4 * k + 1]) : 0u,
+                                   n.z ? __float_as_uint(wv[4 * k + 2]) : 0u, n.w ? __float_as_uint(wv[4 * k + 3]) : 0u);
+                moved |= ((n.x ? 1u : 0u) | (n.y ? 2u : 0u) | (n.z ? 4u : 0u) | (n.w ? 8u : 0u)) << (4u * k);
             }
         }
     }
@@ -318,22 +314,15 @@ __device__ __forceinline__ void load_penalised(const mako_sample_desc& d, uint32
         }
     lds_barrier();
     if (moved) {
-        if (VEC) {
 #pragma unroll
-            for (uint32_t k = 0; k < 4; ++k)
-                if ((moved >> (4u * k)) & 0xfu) {
-                    const uint4 v = *reinterpret_cast<const uint4*>(s_cnt + (lo + k * 4096u + tid * 4u - lo));
-                    wv[4 * k + 0] = (moved >> (4u * k)) & 1u ? __uint_as_float(v.x) : wv[4 * k + 0];
-                    wv[4 * k + 1] = (moved >> (4u * k)) & 2u ? __uint_as_float(v.y) : wv[4 * k + 1];
-                    wv[4 * k + 2] = (moved >> (4u * k)) & 4u ? __uint_as_float(v.z) : wv[4 * k + 2];
-                    wv[4 * k + 3] = (moved >> (4u * k)) & 8u ? __uint_as_float(v.w) : wv[4 * k + 3];
-                }
-        } else {
-#pragma unroll
-            for (uint32_t j = 0; j < 16; ++j)
-                if ((moved >> j) & 1u)
-                    wv[j] = __uint_as_float(s_cnt[j * (uint32_t)kThreads + tid]);
-        }
+        for (uint32_t k = 0; k < 4; ++k)
+            if ((moved >> (4u * k)) & 0xfu) {
+                const uint4 v = *reinterpret_cast<const uint4*>(s_cnt + (k * 4096u + tid * 4u));
+                wv[4 * k + 0] = (moved >> (4u * k)) & 1u ? __uint_as_float(v.x) : wv[4 * k + 0];
+                wv[4 * k + 1] = (moved >> (4u * k)) & 2u ? __uint_as_float(v.y) : wv[4 * k + 1];
+                wv[4 * k + 2] = (moved >> (4u * k)) & 4u ? __uint_as_float(v.z) : wv[4 * k + 2];
+                wv[4 * k + 3] = (moved >> (4u * k)) & 8u ? __uint_as_float(v.w) : wv[4 * k + 3];
+            }
     }
 }
 
