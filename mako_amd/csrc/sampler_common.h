@@ -75,7 +75,7 @@ __device__ __forceinline__ int32_t log_unit(float logit, float scale)
 
 constexpr uint32_t kWorkers = 32;  // workgroups that share the sort of one wide-nucleus row
 // Entries of a row's list that each of its workers is given at least, if there are as many (coarse_plan()).  A worker is a
-// workgroup with a CU to itself and takes 6.3 us for 90 entries, 11.7 for 4 400: on a large batch, which waits for all of
+// workgroup with a CU to itself and takes 6.3 us for 90 entries, 9.7 for 4 400: on a large batch, which waits for all of
 // them, every row of some thousand entries cut into 32 shares costs its CUs ten times what one worker does (512 rows of a
 // decode batch: 1 820 workers, half of them with fewer than 94 entries; 225 us now, 255 in 32 shares, 240 with 5 000 entries
 // at least, which some shares overrun); on a small one the row waits for the slowest, but for more than one round of them too
@@ -87,10 +87,10 @@ constexpr uint32_t kGroup = 256;      // a sorted list is processed in groups of
 constexpr uint32_t kMaxGroups = 1024; // groups per list
 constexpr uint32_t kSegCap = 6144;    // entries a worker sorts in LDS
 constexpr uint32_t kFine = 2048;      // value buckets of that sort
-// dynamic LDS of sort_kernel: the entries, the entries again in the order of their buckets, the buckets, and a copy
-// of the sorted weights for the group records
-constexpr uint32_t kSortLds = kSegCap * 8u + kSegCap * 8u + (kFine + 4u) * 4u + kSegCap * 4u;
-constexpr uint32_t kSortedCopyAt = kSegCap * 8u + kSegCap * 8u + (kFine + 4u) * 4u; // byte offset of that copy
+// dynamic LDS of sort_kernel: the entries in the order of their buckets (and four more), the buckets, and a copy of the sorted
+// weights for the group records
+constexpr uint32_t kSortedCopyAt = (kSegCap + 4u) * 8u + (kFine + 4u) * 4u; // byte offset of that copy
+constexpr uint32_t kSortLds = (kSortedCopyAt + kSegCap * 4u) > kTailLds ? (kSortedCopyAt + kSegCap * 4u) : kTailLds;
 
 // Work order for a top_k == 0 row, written by the second pass (every workgroup of the row derives the same one from
 // scan_kernel's coarse counts, see coarse_plan(); the row's first piece stores it): the weights with bits(q) >= thr

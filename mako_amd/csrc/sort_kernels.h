@@ -200,14 +200,34 @@ __device__ __forceinline__ void sort_body(const mako_sample_desc& d_arg, const S
         return;
     }
     if (cnt) {
+        // (the guess of the running sum before the share: the plan's estimate, in the exact total's units; the walk starts
+        // from u * (the nucleus' fp32 total), which is top_p * total64 and at most one weight more.  In scalar registers while
+        // the share is sorted)
+        const double r0_raw = (double)u_row * ((double)s_args.P.top_p * total64);
+        const double r0 = readlane_f64(r0_raw == r0_raw ? r0_raw : 0.0, 0);
+        const double before = readlane_f64(mass_all > 0.0 ? readlane_f64(mass_l, w) * (total64 / mass_all) : 0.0, 0);
         MAKO_STAMP(10);
         MAKO_COUNT(31, threadIdx.x == 0 && cnt > kSegCap ? 1 : 0);
         MAKO_COUNT(21, threadIdx.x == 0 ? cnt : 0);
         uint32_t* sorted_copy = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(s_dyn64) + kSortedCopyAt);
         const FinishLds L = finish_lds_views(sm, s_dyn64);
-        const bool sorted = in_lds
-                                ? lds_sort_staged(share, key_lo, key_hi, cnt, key0 + off, idx0 + off, s_dyn64, sm, sorted_copy)
-                                : lds_sort_staged_runs(key1 + stage, idx1 + stage, key_lo, key_hi, cnt, key0 + off, idx0 + off, s_dyn64, sm);
+        // (one sort of the share, or of one run of it after the other)
+        const uint32_t runs = in_lds ? 1u : plan_runs(key1 + stage, key_lo, key_hi, cnt, s_dyn64, sm);
+        bool sorted = runs != 0u;
+        for (uint32_t r = 0; sorted && r < runs; ++r) { // uniform
+            uint32_t lo_r = key_lo, hi_r = key_hi, at = 0, n = cnt;
+            if (!in_lds) {
+                // keys of buckets [b0, b1): (key_hi - 1 - k) >> shift in [b0, b1)
+                const uint32_t range = key_hi - key_lo, shift = range > kFine ? 32u - (uint32_t)__clz((range - 1u) >> 11) : 0u;
+                const uint32_t b0 = uniform_u32(sm.hist[r]), b1 = uniform_u32(sm.hist[64u + r]);
+                at = uniform_u32(sm.run[r]);
+                n = uniform_u32(sm.run[64u + r]);
+                hi_r = key_hi - (b0 << shift);
+                lo_r = ((unsigned long long)b1 << shift) >= range ? key_lo : key_hi - (b1 << shift);
+                sorted = collect_run(key1 + stage, idx1 + stage, key_lo, key_hi, cnt, lo_r, hi_r, n, s_dyn64, sm, share);
+            }
+            sorted = sorted && lds_sort_staged(share, lo_r, hi_r, n, key0 + off + at, idx0 + off + at, s_dyn64, sm, in_lds ? sorted_copy : nullptr);
+        }
         if (cnt > kSegCap)
             MAKO_STAMP(18);
         if (!sorted) {
@@ -225,12 +245,7 @@ __device__ __forceinline__ void sort_body(const mako_sample_desc& d_arg, const S
             sort_segment(key0 + off, idx0 + off, key1 + stage, idx1 + stage, cnt, L);
         }
         MAKO_STAMP(11);
-        // (the guess of the running sum before the share: the plan's estimate, in the exact total's units)
-        const double mass_w = readlane_f64(mass_l, w);
-        // (the walk starts from u * (the nucleus' fp32 total), which is top_p * total64 and at most one weight more)
-        const double r0 = (double)u_row * ((double)s_args.P.top_p * total64);
-        worker_groups(key0, off, cnt, sc.gt + t_row + gbase, mass_all > 0.0 ? mass_w * (total64 / mass_all) : 0.0, L,
-                      (in_lds && sorted) ? sorted_copy : nullptr, r0 == r0 ? r0 : 0.0);
+        worker_groups(key0, off, cnt, sc.gt + t_row + gbase, before, L, (in_lds && sorted) ? sorted_copy : nullptr, r0);
         MAKO_STAMP(12);
     }
 }

@@ -7,39 +7,37 @@
 
 namespace mako {
 
-__device__ bool lds_bucket_sort(uint32_t n, uint32_t key_lo, uint32_t key_hi, uint32_t* kout, uint32_t* iout,
-                                unsigned long long* dyn, FinishShared& sm, uint32_t* sorted_lds = nullptr);
-
-// The workers' sort in LDS: the n entries (bits(q), idx) in LDS at A, all with key_lo <= bits(q) < key_hi,
-// are dropped into kFine value buckets (descending), and every entry finds its place by counting the entries of its
-// own bucket that precede it under (q desc, idx asc); they go to kout / iout as ~bits(q) and token id.  Returns false
-// when a bucket is too crowded to be ranked by counting.  hist must be zero and sm.flag 0 on entry.
+// The workers' sort in LDS: up to kSegCap entries (bits(q), idx), entry t * 1024 + tid in this thread's k[t] / id[t], all with
+// key_lo <= bits(q) < key_hi, are dropped into kFine value buckets (descending), and every entry finds its place by counting
+// the entries of its own bucket that precede it under (q desc, idx asc); they go to kout / iout as ~bits(q) and token id.
+// Returns false when a bucket is too crowded to be ranked by counting.  hist must be zero and sm.flag 0 on entry, behind a
+// barrier.
 // sorted_lds (optional, n words of LDS outside the sort's own): receives the sorted ~bits(q) as well, and the
 // function then returns behind a barrier that orders LDS only: the caller goes on from the copy instead of waiting
 // for the stores to kout and reading them back.
-__device__ bool lds_bucket_sort(uint32_t n, uint32_t key_lo, uint32_t key_hi, uint32_t* kout, uint32_t* iout,
-                                unsigned long long* dyn, FinishShared& sm, uint32_t* sorted_lds)
+// (An entry moves as one 64-bit value, the weight above the complement of its token id, so that one comparison orders two of
+// them; and whoever counts may read past the bucket's end, where all there is is smaller.  With the two halves compared and the
+// reads held inside the bucket the counting took 4.3 of a worker's 11.7 us for 4 400 entries; 2.2 of 9.7 so.)
+constexpr uint32_t kSortPer = kSegCap / (uint32_t)kThreads;
+__device__ bool lds_bucket_sort(const uint32_t (&k)[kSortPer], const uint32_t (&id)[kSortPer], uint32_t n, uint32_t key_lo, uint32_t key_hi,
+                                uint32_t* kout, uint32_t* iout, unsigned long long* dyn, FinishShared& sm, uint32_t* sorted_lds = nullptr)
 {
-    uint2* A = reinterpret_cast<uint2*>(dyn);
-    uint2* A2 = A + kSegCap; // the entries again, bucket after bucket (any order inside a bucket)
-    uint32_t* hist = reinterpret_cast<uint32_t*>(A2 + kSegCap);
+    typedef unsigned long long u64;
+    constexpr uint32_t kTrip = 4;
+    const lds_ptr<u64> A = as_lds(dyn); // [kSegCap + kTrip] bucket after bucket (any order inside a bucket)
+    const lds_ptr<uint32_t> hist = (lds_ptr<uint32_t>)(A + kSegCap + kTrip);
     const uint32_t tid = threadIdx.x;
-    // 2. buckets by value, heaviest first
+    // 1. buckets by value, heaviest first
     const uint32_t range = key_hi - key_lo; // > 0
     const uint32_t shift = range > kFine ? 32u - (uint32_t)__clz((range - 1u) >> 11) : 0u; // (range - 1) >> shift < kFine
-    constexpr uint32_t kPer = kSegCap / kThreads;
-    uint32_t bucket[kPer], pib[kPer];
+    uint32_t pib[kSortPer];
 #pragma unroll
-    for (uint32_t t = 0; t < kPer; ++t) {
-        const uint32_t e = t * kThreads + tid;
-        bucket[t] = kNone;
+    for (uint32_t t = 0; t < kSortPer; ++t) {
         pib[t] = 0;
-        if (e < n) {
-            bucket[t] = (key_hi - 1u - A[e].x) >> shift;
-            pib[t] = atomicAdd(&hist[bucket[t]], 1u);
-        }
+        if (t * kThreads + tid < n)
+            pib[t] = __hip_atomic_fetch_add(&hist[(key_hi - 1u - k[t]) >> shift], 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
     }
-    __syncthreads();
+    lds_barrier();
     {
         const uint32_t c0 = hist[2u * tid], c1 = hist[2u * tid + 1u];
         if (max(c0, c1) > 64u)
@@ -51,41 +49,41 @@ __device__ bool lds_bucket_sort(uint32_t n, uint32_t key_lo, uint32_t key_hi, ui
         if (tid == 0)
             hist[kFine] = total;
     }
-    __syncthreads();
+    lds_barrier();
     MAKO_STAMP(14);
     if (sm.flag)
         return false;
-    // (the entries themselves move, not their numbers: whoever ranks an entry reads its bucket's entries in one
-    // trip to LDS each instead of two)
 #pragma unroll
-    for (uint32_t t = 0; t < kPer; ++t)
-        if (bucket[t] != kNone)
-            A2[hist[bucket[t]] + pib[t]] = A[t * kThreads + tid];
-    __syncthreads();
+    for (uint32_t t = 0; t < kSortPer; ++t)
+        if (t * kThreads + tid < n)
+            A[hist[(key_hi - 1u - k[t]) >> shift] + pib[t]] = ((u64)k[t] << 32) | (u64)~id[t];
+    if (tid < kTrip)
+        A[n + tid] = 0ull;
+    lds_barrier();
     MAKO_STAMP(15);
-    // 3. rank inside the bucket, and out
+    // 2. rank inside the bucket, and out
 #pragma unroll
-    for (uint32_t t = 0; t < kPer; ++t) {
+    for (uint32_t t = 0; t < kSortPer; ++t) {
         const uint32_t s = t * kThreads + tid;
         if (s < n) {
-            const uint2 me = A2[s];
-            const uint32_t b = (key_hi - 1u - me.x) >> shift;
+            const u64 me = A[s];
+            const uint32_t b = (key_hi - 1u - (uint32_t)(me >> 32)) >> shift;
             const uint32_t lo = hist[b], hi = hist[b + 1u];
-            // (four of the bucket's entries per trip, from clamped positions: a bucket rarely holds more)
-            uint32_t r = 0;
-            for (uint32_t x = lo; x < hi; x += 4u) {
-                uint2 o[4];
+            // (four entries per trip: a bucket rarely holds more)
+            uint32_t at = lo;
+            for (uint32_t x = lo; x < hi; x += kTrip) {
+                u64 o[kTrip];
 #pragma unroll
-                for (uint32_t u = 0; u < 4; ++u)
-                    o[u] = A2[min(x + u, hi - 1u)];
+                for (uint32_t u = 0; u < kTrip; ++u)
+                    o[u] = A[x + u]; // (x + u < n + kTrip)
 #pragma unroll
-                for (uint32_t u = 0; u < 4; ++u)
-                    r += (x + u < hi && ((o[u].x > me.x) || (o[u].x == me.x && o[u].y < me.y))) ? 1u : 0u;
+                for (uint32_t u = 0; u < kTrip; ++u)
+                    at += o[u] > me ? 1u : 0u;
             }
-            kout[lo + r] = ~me.x;
-            iout[lo + r] = me.y;
+            kout[at] = ~(uint32_t)(me >> 32);
+            iout[at] = ~(uint32_t)me;
             if (sorted_lds)
-                sorted_lds[lo + r] = ~me.x;
+                sorted_lds[at] = ~(uint32_t)(me >> 32);
         }
     }
     if (sorted_lds) // uniform
@@ -99,58 +97,54 @@ __device__ bool lds_bucket_sort(uint32_t n, uint32_t key_lo, uint32_t key_hi, ui
 // order): asked for with fetch_staged_share() (the loads stay in flight while the caller goes on), sorted into
 // kout / iout by lds_sort_staged().
 struct StagedShare {
-    uint32_t k[kSegCap / kThreads], id[kSegCap / kThreads];
+    uint32_t k[kSortPer], id[kSortPer];
 };
 __device__ __forceinline__ void fetch_staged_share(const uint32_t* ks, const uint32_t* is, uint32_t cnt, StagedShare& s)
 {
     const GlobalKeys gk{ks}, gi{is};
 #pragma unroll
-    for (uint32_t t = 0; t < kSegCap / kThreads; ++t) { // (all loads first, from clamped positions; cnt > 0)
+    for (uint32_t t = 0; t < kSortPer; ++t) { // (all loads first, from clamped positions; cnt > 0)
         const uint32_t e = min(t * kThreads + threadIdx.x, cnt - 1u);
         s.k[t] = gk[e];
         s.id[t] = gi[e];
     }
 }
-__device__ __forceinline__ bool lds_sort_staged(const StagedShare& s, uint32_t key_lo, uint32_t key_hi, uint32_t cnt,
+__device__ __forceinline__ bool lds_sort_staged(StagedShare& s, uint32_t key_lo, uint32_t key_hi, uint32_t cnt,
                                                 uint32_t* kout, uint32_t* iout, unsigned long long* dyn, FinishShared& sm,
                                                 uint32_t* sorted_lds = nullptr)
 {
-    uint2* A = reinterpret_cast<uint2*>(dyn);
-    uint32_t* hist = reinterpret_cast<uint32_t*>(A + 2u * kSegCap); // (behind lds_bucket_sort()'s second copy)
+    uint32_t* hist = reinterpret_cast<uint32_t*>(dyn + kSegCap + 4u); // (lds_bucket_sort()'s)
     const uint32_t tid = threadIdx.x;
     for (uint32_t b = tid; b <= kFine; b += kThreads)
         hist[b] = 0;
     if (tid == 0)
         sm.flag = 0;
+    lds_barrier();
 #pragma unroll
-    for (uint32_t t = 0; t < kSegCap / kThreads; ++t) {
-        const uint32_t e = t * kThreads + tid;
+    for (uint32_t t = 0; t < kSortPer; ++t) {
         uint32_t k = s.k[t];
         asm volatile("" : "+v"(k)); // (used here and not before: the loads are to be waited for no earlier)
-        if (e < cnt)
-            A[e] = make_uint2(min(max(k, key_lo), key_hi - 1u), s.id[t]); // (clamped: a bucket index is always valid)
+        s.k[t] = min(max(k, key_lo), key_hi - 1u); // (clamped: a bucket index is always valid)
     }
-    __syncthreads();
     MAKO_STAMP(13);
-    return lds_bucket_sort(cnt, key_lo, key_hi, kout, iout, dyn, sm, sorted_lds);
+    return lds_bucket_sort(s.k, s.id, cnt, key_lo, key_hi, kout, iout, dyn, sm, sorted_lds);
 }
 
 // A share too large for one LDS sort is cut by value into runs that fit: one counting sweep over the share (the
-// same kFine buckets as the sort uses) finds run boundaries at bucket edges, then each run is collected from the
-// share and sorted on its own.  Returns false (the caller falls back to the radix sort through global memory)
-// when a single bucket holds more than fits.
-__device__ bool lds_sort_staged_runs(const uint32_t* ks, const uint32_t* is, uint32_t key_lo, uint32_t key_hi, uint32_t cnt,
-                                     uint32_t* kout, uint32_t* iout, unsigned long long* dyn, FinishShared& sm)
+// same kFine buckets as the sort uses) finds run boundaries at bucket edges (plan_runs()), then each run is collected from
+// the share and sorted on its own.  Returns the runs, 0 (the caller falls back to the radix sort through global memory)
+// when a single bucket holds more than fits.  Run r covers buckets [sm.hist[r], sm.hist[64 + r]) = entries
+// [sm.run[r], sm.run[r] + sm.run[64 + r]) of the sorted share.
+__device__ uint32_t plan_runs(const uint32_t* ks, uint32_t key_lo, uint32_t key_hi, uint32_t cnt, unsigned long long* dyn, FinishShared& sm)
 {
-    uint2* A = reinterpret_cast<uint2*>(dyn);
-    uint32_t* hist = reinterpret_cast<uint32_t*>(A + 2u * kSegCap); // (behind lds_bucket_sort()'s second copy) // [kFine + 1]
-    const uint32_t tid = threadIdx.x, lane = lane_id();
+    uint32_t* hist = reinterpret_cast<uint32_t*>(dyn + kSegCap + 4u); // [kFine + 1] (lds_bucket_sort()'s)
+    const uint32_t tid = threadIdx.x;
     const uint32_t range = key_hi - key_lo;
     const uint32_t shift = range > kFine ? 32u - (uint32_t)__clz((range - 1u) >> 11) : 0u;
     for (uint32_t b = tid; b <= kFine; b += kThreads)
         hist[b] = 0;
     __syncthreads();
-    constexpr uint32_t kTrip = 8; // loads in flight per thread: the sweeps below are bound by memory latency
+    constexpr uint32_t kTrip = 8; // loads in flight per thread: the sweep is bound by memory latency
     for (uint32_t base = 0; base < cnt; base += kTrip * kThreads) {
         uint32_t k[kTrip];
 #pragma unroll
@@ -169,19 +163,17 @@ __device__ bool lds_sort_staged_runs(const uint32_t* ks, const uint32_t* is, uin
     __syncthreads();
     hist[2u * tid] = ex;
     hist[2u * tid + 1u] = ex + c0;
-    if (tid == 0) {
+    if (tid == 0)
         hist[kFine] = total;
-        sm.flag = 0;
-    }
     __syncthreads();
-    // runs: greedily as many whole buckets as fit (thread 0; a handful of runs).  Run r covers buckets
-    // [sm.hist[r], sm.hist[64 + r]) = entries [sm.run[r], sm.run[r] + sm.run[64 + r]) of the sorted share.
+    // runs: greedily as many whole buckets as fit (thread 0; a handful of runs)
     if (tid == 0) {
         uint32_t runs = 0, b0 = 0;
         while (b0 < kFine && runs < 64u) {
             uint32_t b1 = b0 + 1u;
             if (hist[b1] - hist[b0] > kSegCap) { // one bucket alone is too much
-                runs = 0xffffffffu;
+                runs = 0;
+                b0 = kFine;
                 break;
             }
             { // the last bucket edge within reach: the bucket starts never decrease, so bisect
@@ -204,68 +196,69 @@ __device__ bool lds_sort_staged_runs(const uint32_t* ks, const uint32_t* is, uin
             }
             b0 = b1;
         }
-        if (runs != 0xffffffffu && b0 < kFine)
-            runs = 0xffffffffu;
-        sm.ticket = runs;
+        sm.ticket = b0 < kFine ? 0u : runs;
     }
     __syncthreads();
     const uint32_t runs = sm.ticket;
-    if (runs == 0xffffffffu)
-        return false;
-    for (uint32_t r = 0; r < runs; ++r) {
-        const uint32_t b0 = sm.hist[r], b1 = sm.hist[64u + r];
-        const uint32_t at = sm.run[r], n = sm.run[64u + r];
-        // keys of buckets [b0, b1): (key_hi - 1 - k) >> shift in [b0, b1)
-        const uint32_t hi_r = key_hi - (b0 << shift);
-        const uint32_t lo_r = ((unsigned long long)b1 << shift) >= range ? key_lo : key_hi - (b1 << shift);
-        __syncthreads();
-        for (uint32_t b = tid; b <= kFine; b += kThreads)
-            hist[b] = 0;
-        if (tid == 0) {
-            sm.ticket = 0;
-            sm.flag = 0;
+    __syncthreads();
+    return runs;
+}
+
+// Run r's n entries, those of the share with lo_r <= bits(q) < hi_r, as fetch_staged_share() leaves a whole share.
+__device__ bool collect_run(const uint32_t* ks, const uint32_t* is, uint32_t key_lo, uint32_t key_hi, uint32_t cnt, uint32_t lo_r, uint32_t hi_r,
+                            uint32_t n, unsigned long long* dyn, FinishShared& sm, StagedShare& s)
+{
+    uint2* A = reinterpret_cast<uint2*>(dyn);
+    const uint32_t tid = threadIdx.x, lane = lane_id();
+    __syncthreads();
+    if (tid == 0)
+        sm.ticket = 0;
+    __syncthreads();
+    constexpr uint32_t kTrip = 6;
+    const unsigned long long lower = (1ull << lane) - 1ull;
+    for (uint32_t base = 0; base < cnt; base += kTrip * kThreads) {
+        uint32_t k[kTrip], id[kTrip];
+#pragma unroll
+        for (uint32_t u = 0; u < kTrip; ++u) {
+            const uint32_t e = min(base + u * kThreads + tid, cnt - 1u);
+            k[u] = ks[e];
+            id[u] = is[e];
         }
-        __syncthreads();
-        const unsigned long long lower = (1ull << lane) - 1ull;
-        for (uint32_t base = 0; base < cnt; base += kTrip * kThreads) {
-            uint32_t k[kTrip], id[kTrip];
+        // slots for the whole trip from one LDS atomic per wave
+        bool mine[kTrip];
+        uint32_t before = 0, wave_total = 0;
 #pragma unroll
-            for (uint32_t u = 0; u < kTrip; ++u) {
-                const uint32_t e = min(base + u * kThreads + tid, cnt - 1u);
-                k[u] = ks[e];
-                id[u] = is[e];
-            }
-            // slots for the whole trip from one LDS atomic per wave
-            bool mine[kTrip];
-            uint32_t before = 0, wave_total = 0;
-#pragma unroll
-            for (uint32_t u = 0; u < kTrip; ++u) {
-                k[u] = min(max(k[u], key_lo), key_hi - 1u);
-                mine[u] = base + u * kThreads + tid < cnt && k[u] >= lo_r && k[u] < hi_r;
-                const unsigned long long bal = __ballot(mine[u]);
-                before += (uint32_t)__popcll(bal & lower);
-                wave_total += (uint32_t)__popcll(bal);
-            }
-            if (wave_total) { // uniform
-                uint32_t slot = 0;
-                if (lane == 0)
-                    slot = atomicAdd(&sm.ticket, wave_total);
-                slot = uniform_u32(slot) + before;
-#pragma unroll
-                for (uint32_t u = 0; u < kTrip; ++u)
-                    if (mine[u]) {
-                        if (slot < kSegCap)
-                            A[slot] = make_uint2(k[u], id[u]);
-                        ++slot;
-                    }
-            }
+        for (uint32_t u = 0; u < kTrip; ++u) {
+            k[u] = min(max(k[u], key_lo), key_hi - 1u);
+            mine[u] = base + u * kThreads + tid < cnt && k[u] >= lo_r && k[u] < hi_r;
+            const unsigned long long bal = __ballot(mine[u]);
+            before += (uint32_t)__popcll(bal & lower);
+            wave_total += (uint32_t)__popcll(bal);
         }
-        __syncthreads();
-        if (sm.ticket != n) // (cannot happen: the same keys were counted above)
-            return false;
-        if (!lds_bucket_sort(n, lo_r, hi_r, kout + at, iout + at, dyn, sm))
-            return false; // (a crowded bucket: ties)
+        if (wave_total) { // uniform
+            uint32_t slot = 0;
+            if (lane == 0)
+                slot = atomicAdd(&sm.ticket, wave_total);
+            slot = uniform_u32(slot) + before;
+#pragma unroll
+            for (uint32_t u = 0; u < kTrip; ++u)
+                if (mine[u]) {
+                    if (slot < kSegCap)
+                        A[slot] = make_uint2(k[u], id[u]);
+                    ++slot;
+                }
+        }
     }
+    __syncthreads();
+    if (sm.ticket != n) // (cannot happen: the same keys were counted by plan_runs())
+        return false;
+#pragma unroll
+    for (uint32_t t = 0; t < kSortPer; ++t) {
+        const uint2 x = A[min(t * kThreads + tid, n - 1u)];
+        s.k[t] = x.x;
+        s.id[t] = x.y;
+    }
+    __syncthreads(); // (the sort puts the entries there again, in the order of their buckets)
     return true;
 }
 
