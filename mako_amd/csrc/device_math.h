@@ -29,8 +29,9 @@ __device__ const uint64_t k_exp2_tab[32] = {
 // the conversion at the end rounds to the same value, infinity, the least subnormal or zero (all 2^32 arguments compared), and
 // nothing branches: with a branch per special case every call waited for its own table entry and its own chain, with none the
 // four calls side by side overlap (the second pass over 256 rows of 151 552
-// logits 123 -> 114 us, the weights of 64 rows in token order 19.7 -> 18.3).
-__device__ __forceinline__ float expf_glibc(float x, const uint64_t* tab)
+// logits 123 -> 114 us, the weights of 64 rows in token order 19.7 -> 17.9).
+// (exp_moved(): NaN is moved to the lower bound.)
+__device__ __forceinline__ float exp_moved(float x, const uint64_t* tab)
 {
     const double inv_ln2_n = 0x1.71547652b82fep+0 * 32.0;
     const double shift = 0x1.8p+52;
@@ -39,16 +40,20 @@ __device__ __forceinline__ float expf_glibc(float x, const uint64_t* tab)
     const double c2 = 0x1.62e42ff0c52d6p-1 / 32;
     const double xd = (double)__builtin_amdgcn_fmed3f(x, -104.0f, 89.0f);
     double kd = fma(inv_ln2_n, xd, shift);
-    const uint64_t ki = (uint64_t)__double_as_longlong(kd);
+    const uint32_t ki = (uint32_t)__double_as_longlong(kd);
     kd -= shift;
     const double r = fma(inv_ln2_n, xd, -kd);
-    const double s = __longlong_as_double((long long)(tab[ki & 31] + (ki << 47)));
+    const uint64_t t = tab[ki & 31u]; // (+ ki << 47, which the lower word has no part in)
+    const double s = __longlong_as_double((long long)(((uint64_t)((uint32_t)(t >> 32) + (ki << 15)) << 32) | (uint32_t)t));
     const double z = fma(c0, r, c1);
     const double r2 = r * r;
     double y = fma(c2, r, 1.0);
     y = fma(z, r2, y);
-    const float q = (float)(y * s);
-    return x == x ? q : x + x;
+    return (float)(y * s);
+}
+__device__ __forceinline__ float expf_glibc(float x, const uint64_t* tab)
+{
+    return x == x ? exp_moved(x, tab) : x + x;
 }
 
 // The three penalties of src/gen/sampler.cpp:25-27 for a token seen n times.
@@ -61,12 +66,13 @@ __device__ __forceinline__ float penalize(float l, uint32_t n, float rep, float 
     return l - dec;
 }
 
-// q = exp((w - m) * inv_t), src/gen/sampler.cpp:33: subtract, multiply, expf.
+// q = exp((w - m) * inv_t), src/gen/sampler.cpp:33: subtract, multiply, expf.  (0 where that is NaN: neither is a candidate,
+// src/gen/sampler.cpp:34.)
 __device__ __forceinline__ float weight_of(float w, float m, float inv_t, const uint64_t* tab)
 {
     const float diff = w - m;
     const float x = diff * inv_t;
-    return expf_glibc(x, tab);
+    return exp_moved(x, tab);
 }
 
 } // namespace mako

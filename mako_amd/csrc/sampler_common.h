@@ -25,7 +25,7 @@ constexpr uint32_t kTopKFast = 128;  // largest top_k resolved from the per-slic
 constexpr uint32_t kSortMax = 4096;  // candidates the finisher sorts in LDS
 constexpr uint32_t kSmall = 256;     // lists of up to this many entries are ordered by counting ranks
 constexpr uint32_t kDynLds = 65536;  // dynamic LDS that the penalty table of a slice takes
-constexpr uint32_t kFinishLds = kSliceMax * 8u; // and of the second pass's kernels, which put all a piece keeps in order there
+constexpr uint32_t kFinishLds = (kSliceMax + 128u) * 8u; // and of the second pass's kernels, which put all a piece keeps in order there
 constexpr uint32_t kHeadGroups = 32; // groups at the head of a sorted list that tail code keeps in LDS as floats
 constexpr uint32_t kTailLds = kDynLds + (kHeadGroups - 8u) * 1024u; // dynamic LDS of the kernels that cut and draw
 constexpr uint32_t kFlagFirstNan = 1u; // element 0 of the row is NaN (slice 0 only)

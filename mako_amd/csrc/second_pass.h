@@ -14,14 +14,18 @@ namespace mako {
 // The plan (coarse_plan()) is built while the first piece's logits are on their way; every workgroup of the row
 // arrives at the same one, and the one with the row's first piece stores it for the kernels that follow and enters
 // the row in their lists.
+// The large batches' instance, whose workgroups go through several pieces, asks for a piece's logits ahead of the hand-over of
+// the piece before it (AHEAD; where their registers are to be had: not with eight history entries a thread, and not beside
+// other rows).
+// `loads`: the piece's own where they have been asked for ahead, then those of piece `next` (kNone: there is none).
 // (PEN: the row has penalties to apply; a compile-time fact so that each case gets straight-line code of its own.)
 // (`slices`: of scan_kernel, whose records give the row maximum)
 // (PLANNING: the workgroup's first piece, with which the plan is built; returns false when the row leaves for the
 // whole-row path and the pass has nothing more to do for it)
-template <bool ALIGNED, int KH, bool PEN, bool PLANNING, bool UNSORTED = false>
+template <bool ALIGNED, int KH, bool PEN, bool PLANNING, bool UNSORTED, bool AHEAD>
 __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t row, uint32_t slice, uint32_t slice_len,
                           const mako_sampling_params& P, uint32_t hl, uint32_t slices, const FinishLds& L, CoarsePlan& pl,
-                          float& m, uint32_t& argidx, uint32_t opaque_first = kNone)
+                          float& m, uint32_t& argidx, uint32_t opaque_first, SliceLoads<KH>& loads, uint32_t next)
 {
     assume_lds(L);
     FinishShared& sm = *L.sm;
@@ -35,14 +39,19 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
     if constexpr (PLANNING) {
         PlanLoads pre;
         issue_plan_loads<UNSORTED>(d, sc, row, slices, pre);
-        load_penalised<ALIGNED, KH>(d, row, lo, hi, slice_len, P, hl, pen, L.cnt, wv, [&]() {
+        issue_slice<ALIGNED, KH>(d, row, lo, hi, loads);
+        clear_counts<KH>(d, slice_len, L.cnt);
+        {
             uint32_t n_cands, any_overflow;
             row_summary_of(pre.st, slices, m, argidx, n_cands, any_overflow);
             coarse_plan(sc, row, slices, d.n_vocab, P, m, pre, !any_overflow && n_cands <= kSortMax, UNSORTED ? opaque_first : kNone, UNSORTED ? kShareLarge : kShareSmall, pl, sm.tab);
-        });
+        }
     } else {
-        load_penalised<ALIGNED, KH>(d, row, lo, hi, slice_len, P, hl, pen, L.cnt, wv);
+        if (!AHEAD)
+            issue_slice<ALIGNED, KH>(d, row, lo, hi, loads);
+        clear_counts<KH>(d, slice_len, L.cnt);
     }
+    finish_penalised<ALIGNED, KH>(d, row, lo, hi, slice_len, P, hl, pen, L.cnt, loads, wv);
     MAKO_STAMP(1);
     MAKO_STAMP(24);
     const uint32_t flag = pl.flag;
@@ -94,8 +103,9 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
     if (flag == 2) // the whole-row path starts from the logits again
         return false;
     const float inv_t = 1.0f / P.temperature;
-    const float floor_q = (1.0f < P.min_p) ? 1.0f : P.min_p;
-    const uint32_t thr = pl.thr;
+    // (a weight of zero is below either)
+    const float floor_p = (1.0f < P.min_p) ? 1.0f : P.min_p, floor_q = floor_p < 0x1p-149f ? 0x1p-149f : floor_p;
+    const uint32_t thr = max(pl.thr, 1u);
     const uint32_t edge7 = uniform_u32(pl.key_lo[7]), edge15 = uniform_u32(pl.key_lo[15]), edge23 = uniform_u32(pl.key_lo[23]);
     double sum = 0;
     uint32_t qb[16];   // bits(q), 0 where q is not a candidate
@@ -110,7 +120,6 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
             slot[j] = kNone;
         }
         if (lo + (g / 4u) * 4096u < hi) {
-            bool keeps[4];
             // (the large batches' instance: a wave whose four weights a lane all underflow to zero, as those of a peaked row far
             // below its maximum do, skips the arithmetic that would tell it so; expf_glibc() returns 0 below that bound)
             bool any = !UNSORTED;
@@ -118,54 +127,59 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
                 bool under = true;
 #pragma unroll
                 for (uint32_t j = g; j < g + 4u; ++j)
-                    under = under && (wv[j] - m) * inv_t < -0x1.9fe368p6f;
+                    under = under & ((wv[j] - m) * inv_t < -0x1.9fe368p6f);
                 any = __ballot(!under) != 0ull; // uniform
             }
-#pragma unroll
-            for (uint32_t j = 0; j < 4u; ++j)
-                keeps[j] = false;
             if (any) {
                 float q[4];
+                bool keeps[4];
 #pragma unroll
-                for (uint32_t j = 0; j < 4u; ++j)
+                for (uint32_t j = 0; j < 4; ++j)
                     q[j] = weight_of(wv[g + j], m, inv_t, sm.tab);
 #pragma unroll
-                for (uint32_t j = 0; j < 4u; ++j) {
-                    qb[g + j] = (q[j] >= floor_q && q[j] > 0.0f) ? __float_as_uint(q[j]) : 0u;
-                    sum += (double)__uint_as_float(qb[g + j]);
-                    keeps[j] = qb[g + j] >= thr && qb[g + j];
-                }
-            }
-            // the worker whose range of bits(q) holds the weight (equal weights always meet in one share): the number of
-            // workers whose lower edge lies above it, by bisection over the edges (the first two steps against edges held in
-            // scalar registers, the other three from LDS), and a place among the workgroup's entries for it.
-            // (Four logits side by side: one after the other, each with its own branch, they wait for three reads and an
-            // atomic's answer every time.  A flat row's piece of 16 384: 6.2 -> 4.6 us.)
-            if (__ballot(keeps[0] || keeps[1] || keeps[2] || keeps[3]) != 0ull) { // uniform
-                static_assert(kWorkers == 32, "five steps");
-                uint32_t w[4], place[4];
-#pragma unroll
                 for (uint32_t j = 0; j < 4; ++j) {
-                    w[j] = qb[g + j] < edge15 ? 16u : 0u;
-                    w[j] += qb[g + j] < (w[j] ? edge23 : edge7) ? 8u : 0u;
-                    place[j] = 0u;
+                    qb[g + j] = q[j] >= floor_q ? __float_as_uint(q[j]) : 0u;
+                    sum += (double)__uint_as_float(qb[g + j]);
+                    keeps[j] = qb[g + j] >= thr;
                 }
+                // the worker whose range of bits(q) holds the weight (equal weights always meet in one share): the number of
+                // workers whose lower edge lies above it, by bisection over the edges (the first two steps against edges held
+                // in scalar registers, the other three from LDS), and a place among the workgroup's entries for it.
+                // (Four logits side by side: one after the other, each with its own branch, they wait for three reads and an
+                // atomic's answer every time.  The worker's number is kept as an offset into its words in LDS.  A flat row's
+                // piece of 16 384, weights and all: 7.1 -> 6.0 us.)
+                if (__ballot(keeps[0] | keeps[1] | keeps[2] | keeps[3]) != 0ull) { // uniform
+                    static_assert(kWorkers == 32, "five steps");
+                    const lds_ptr<const char> edges = (lds_ptr<const char>)as_lds(pl.key_lo), counts = (lds_ptr<const char>)as_lds(pl.count);
+                    uint32_t w[4], place[4];
 #pragma unroll
-                for (uint32_t step = 4u; step; step >>= 1)
+                    for (uint32_t j = 0; j < 4; ++j) {
+                        w[j] = qb[g + j] < edge15 ? 64u : 0u;
+                        w[j] |= qb[g + j] < (qb[g + j] < edge15 ? edge23 : edge7) ? 32u : 0u;
+                        place[j] = 0u;
+                    }
+#pragma unroll
+                    for (uint32_t step = 4u; step; step >>= 1)
+#pragma unroll
+                        for (uint32_t j = 0; j < 4; ++j)
+                            w[j] += qb[g + j] < *(lds_ptr<const uint32_t>)(edges + w[j] + 4u * (step - 1u)) ? 4u * step : 0u;
+                    __builtin_amdgcn_sched_barrier(0); // (the four counters are asked for one behind the other)
 #pragma unroll
                     for (uint32_t j = 0; j < 4; ++j)
-                        w[j] += qb[g + j] < pl.key_lo[w[j] + step - 1u] ? step : 0u;
+                        if (keeps[j])
+                            place[j] = __hip_atomic_fetch_add((lds_ptr<uint32_t>)(counts + w[j]), 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
 #pragma unroll
-                for (uint32_t j = 0; j < 4; ++j)
-                    if (keeps[j])
-                        place[j] = atomicAdd(&pl.count[w[j]], 1u);
-#pragma unroll
-                for (uint32_t j = 0; j < 4; ++j)
-                    slot[g + j] = keeps[j] ? (w[j] << 16) | place[j] : kNone;
+                    for (uint32_t j = 0; j < 4; ++j)
+                        slot[g + j] = keeps[j] ? (w[j] << 14) | place[j] : kNone;
+                }
             }
         }
     }
     MAKO_STAMP(25);
+    if (AHEAD)
+        __builtin_amdgcn_sched_barrier(0); // (not among the weights, whose registers these take)
+    if (AHEAD && next != kNone) // uniform
+        issue_slice<ALIGNED, KH>(d, row, next * slice_len, min(d.n_vocab, next * slice_len + slice_len), loads);
     // the piece's sum: wave reductions, then the sixteen waves' results in order
     {
         const double sw = __ockl_wfred_add_f64(sum);
@@ -175,14 +189,14 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
     lds_barrier();
     MAKO_STAMP(26);
     // One run per worker in its share of the row's staging arrays, reserved with a single atomic.  The kept weights
-    // are first put in LDS (the penalty table's block, free by now) in the order of their workers, so that the runs
-    // go out as contiguous stores.
+    // are first put in LDS (the penalty table's block, free by now) in the order of their workers, each worker's from a
+    // multiple of four on, so that the runs go out as contiguous stores, four entries at a time.
     // (the reservations' answers take a trip to device memory: the entries are put in LDS order under it)
     uint32_t mine = 0, lbase_mine = 0, base_mine = 0;
     if (wave_id() == 0) {
         mine = tid < kWorkers ? pl.count[tid] : 0u;
-        const uint32_t upto = __ockl_wfscan_add_u32(mine, true);
-        lbase_mine = upto - mine;
+        const uint32_t padded = (mine + 3u) & ~3u, upto = __ockl_wfscan_add_u32(padded, true);
+        lbase_mine = upto - padded;
         if (tid < kWorkers) {
             pl.lbase[tid] = lbase_mine;
             if (mine)
@@ -199,8 +213,8 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
     const global_ptr<uint32_t> istage = as_global(sc.idx[1]) + (size_t)row * sc.vpad;
     // (room for all a piece can hold: with half as much, a flat row's pieces, which keep nearly everything, went through
     // it twice, 2 us more each, and the workgroup has its CU to itself anyway)
-    uint2* buf = reinterpret_cast<uint2*>(L.cnt); // [kSliceMax] (weight, token id)
-    static_assert(kFinishLds >= kSliceMax * sizeof(uint2), "");
+    uint2* buf = reinterpret_cast<uint2*>(L.cnt); // [kSliceMax + 3 kWorkers] (weight, token id)
+    static_assert(kFinishLds >= (kSliceMax + 3u * kWorkers) * sizeof(uint2), "");
     const uint32_t kept = pl.lbase[kWorkers];
     // (an entry's worker travels in the upper bits of its token id)
     constexpr uint32_t kIdBits = 27;
@@ -225,24 +239,38 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
         for (uint32_t j = 0; j < 16; ++j)
             if (slot[j] != kNone)
                 buf[slot[j] & 0xffffu] = make_uint2(qb[j], elem_index(lo, tid, j) | ((slot[j] >> 16) << kIdBits));
-        if (tid < kWorkers) { // (wave 0: where each worker's run goes and where its room ends, in the workgroup's order)
-            const uint32_t room = pl.cap[tid];
-            pl.run[tid] = make_uint2(pl.stage_off[tid] + base_mine - lbase_mine, lbase_mine + (room > base_mine ? room - base_mine : 0u));
+        if (tid < kWorkers) { // (wave 0: where each worker's run goes and where it, or its room, ends in the workgroup's order)
+            const uint32_t room = pl.cap[tid], left = room > base_mine ? room - base_mine : 0u;
+            pl.run[tid] = make_uint2(pl.stage_off[tid] + base_mine - lbase_mine, lbase_mine + min(mine, left));
+            dropped = mine > left;
         }
         lds_barrier();
-#pragma unroll 4 // (fully unrolled, the unaligned variants spill dozens of registers for no gain)
-        for (uint32_t e = tid; e < kept; e += kThreads) { // (uniform per wave but for the last trip)
-            const uint2 x = buf[e];
-            const uint32_t w = x.y >> kIdBits;
+        typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(4)));
+        const uint32_t id_mask = (1u << kIdBits) - 1u;
+        // (a share that is only summed has no use for the token ids)
+        auto wants_ids = [&](uint32_t w) { return !UNSORTED || !((unsorted_mask >> w) & 1u); };
+        for (uint32_t e = 4u * tid; e < kept; e += 4u * kThreads) { // (uniform per wave but for the last trip)
+            const uint4 x0 = *reinterpret_cast<const uint4*>(buf + e), x1 = *reinterpret_cast<const uint4*>(buf + e + 2u);
+            const uint32_t w = x0.y >> kIdBits;
             const uint2 run = pl.run[w];
+            if (e + 4u <= run.y) {
+                MAKO_CHECK(sc, kCheckStage, (uint64_t)(run.x + e) + 3u < sc.vpad && run.x + e >= pl.stage_off[w] &&
+                                                run.x + e + 4u <= pl.stage_off[w] + pl.cap[w]);
+                *(global_ptr<u32x4_any>)(kstage + run.x + e) = u32x4_any{x0.x, x0.z, x1.x, x1.z};
+                if (wants_ids(w))
+                    *(global_ptr<u32x4_any>)(istage + run.x + e) = u32x4_any{x0.y & id_mask, x0.w & id_mask, x1.y & id_mask, x1.w & id_mask};
+            }
+        }
+        if (tid < 4u * kWorkers) { // each run's last entries, fewer than four
+            const uint32_t w = tid >> 2, first = pl.lbase[w];
+            const uint2 run = pl.run[w];
+            const uint32_t e = first + ((run.y - first) & ~3u) + (tid & 3u);
             if (e < run.y) {
-                MAKO_CHECK(sc, kCheckStage, (uint64_t)(run.x + e) < sc.vpad && run.x + e >= pl.stage_off[w] &&
-                                                run.x + e < pl.stage_off[w] + pl.cap[w]);
+                const uint2 x = buf[e];
+                MAKO_CHECK(sc, kCheckStage, (uint64_t)(run.x + e) < sc.vpad && run.x + e >= pl.stage_off[w] && run.x + e < pl.stage_off[w] + pl.cap[w]);
                 kstage[run.x + e] = x.x;
-                if (!UNSORTED || !((unsorted_mask >> w) & 1u)) // (a share that is only summed has no use for the token ids)
-                    istage[run.x + e] = x.y & ((1u << kIdBits) - 1u);
-            } else {
-                dropped = true;
+                if (wants_ids(w))
+                    istage[run.x + e] = x.y & id_mask;
             }
         }
         lds_barrier();
@@ -261,7 +289,7 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
     return true;
 }
 
-template <bool ALIGNED, int KH, bool PEN, bool UNSORTED>
+template <bool ALIGNED, int KH, bool PEN, bool UNSORTED, bool AHEAD>
 __device__ void row_pieces(const mako_sample_desc& d, const Scratch& sc, uint32_t row, uint32_t first, uint32_t stride,
                            uint32_t n_pieces, uint32_t slice_len, const mako_sampling_params& P, uint32_t hl, uint32_t slices,
                            const FinishLds& L, CoarsePlan& pl, uint32_t opaque_first)
@@ -270,10 +298,13 @@ __device__ void row_pieces(const mako_sample_desc& d, const Scratch& sc, uint32_
     // the workgroup's pieces in turn: first, first + stride, ...
     float m = 0.0f;
     uint32_t argidx = 0;
-    if (first >= n_pieces || !one_piece<ALIGNED, KH, PEN, true, UNSORTED>(d, sc, row, first, slice_len, P, hl, slices, L, pl, m, argidx, opaque_first))
+    SliceLoads<KH> loads;
+    auto behind = [&](uint32_t slice) { return slice + stride < n_pieces ? slice + stride : kNone; };
+    if (first >= n_pieces || !one_piece<ALIGNED, KH, PEN, true, UNSORTED, AHEAD>(d, sc, row, first, slice_len, P, hl, slices, L, pl, m, argidx, opaque_first, loads,
+                                                                         behind(first)))
         return;
     for (uint32_t slice = first + stride; slice < n_pieces; slice += stride)
-        one_piece<ALIGNED, KH, PEN, false, UNSORTED>(d, sc, row, slice, slice_len, P, hl, slices, L, pl, m, argidx);
+        one_piece<ALIGNED, KH, PEN, false, UNSORTED, AHEAD>(d, sc, row, slice, slice_len, P, hl, slices, L, pl, m, argidx, kNone, loads, behind(slice));
 }
 
 // Second pass over the top_k == 0 rows.  grid = (most pieces a row can have, rows) workgroups, of which workgroup i
@@ -282,7 +313,7 @@ __device__ void row_pieces(const mako_sample_desc& d, const Scratch& sc, uint32_
 // mix of rows.
 // (UNSORTED: the instance for batches of many such rows, whose plans leave shares unsorted: unsorted_shares.h)
 // (n_wgs: workgroups of the launch that are finish_kernel's)
-template <bool ALIGNED, int KH, bool UNSORTED>
+template <bool ALIGNED, int KH, bool UNSORTED, bool AHEAD>
 __device__ __forceinline__ void finish_body(const mako_sample_desc& d_arg, const Scratch& sc_arg, uint32_t slices, uint32_t n_wgs,
                                             unsigned long long* s_dyn64, FinishShared& sm, ArgsLds& s_args, CoarsePlan& s_plan)
 {
@@ -379,9 +410,9 @@ __device__ __forceinline__ void finish_body(const mako_sample_desc& d_arg, const
         s_plan.nucleus_rows = nucleus_rows; // (read behind the plan's barriers)
     const uint32_t opaque_first = (UNSORTED && !d.draft) ? max(kHeadGroups * kGroup, (d.out_cand_idx && d.out_cand_q) ? d.cand_cap : 0u) : kNone;
     if (d.hist_tokens && !penalties_neutral(P))
-        row_pieces<ALIGNED, KH, true, UNSORTED>(d, sc, row, piece, pieces, n_pieces, piece_len, P, hl, slices, L, s_plan, opaque_first);
+        row_pieces<ALIGNED, KH, true, UNSORTED, AHEAD>(d, sc, row, piece, pieces, n_pieces, piece_len, P, hl, slices, L, s_plan, opaque_first);
     else
-        row_pieces<ALIGNED, KH, false, UNSORTED>(d, sc, row, piece, pieces, n_pieces, piece_len, P, hl, slices, L, s_plan, opaque_first);
+        row_pieces<ALIGNED, KH, false, UNSORTED, AHEAD>(d, sc, row, piece, pieces, n_pieces, piece_len, P, hl, slices, L, s_plan, opaque_first);
 }
 
 // (its arguments by value: the cut is one trip to memory away, not two)
@@ -392,7 +423,7 @@ __global__ __launch_bounds__(kThreads) void finish_kernel(mako_sample_desc d_arg
     __shared__ FinishShared sm;
     __shared__ ArgsLds s_args;
     __shared__ CoarsePlan s_plan;
-    finish_body<ALIGNED, KH, UNSORTED>(d_arg, sc_val, slices, gridDim.y, s_dyn64, sm, s_args, s_plan);
+    finish_body<ALIGNED, KH, UNSORTED, UNSORTED && KH <= 2>(d_arg, sc_val, slices, gridDim.y, s_dyn64, sm, s_args, s_plan);
 }
 
 } // namespace mako

@@ -198,13 +198,14 @@ struct NoOverlap {
     __device__ __forceinline__ void operator()() const {}
 };
 
-// `overlap` runs right after the slice's loads have been issued: work that does not depend on them hides
-// behind their latency.  It must be reached by the whole workgroup or by none of it.
-template <bool ALIGNED, int KH, typename Overlap = NoOverlap>
-__device__ __forceinline__ void load_penalised(const mako_sample_desc& d, uint32_t row, uint32_t lo, uint32_t hi,
-                                               uint32_t slice_len, const mako_sampling_params& P, uint32_t hl, bool pen,
-                                               uint32_t* s_cnt, float (&wv)[16], Overlap overlap = Overlap(),
-                                               bool want_above = false, float close_v = 0.0f, uint32_t* above = nullptr)
+// A slice's loads on their way: the thread's logits and history entries (KH > 0).
+template <int KH>
+struct SliceLoads {
+    RawSlice raw;
+    uint32_t tok[KH > 0 ? KH : 1], cnt[KH > 0 ? KH : 1];
+};
+template <bool ALIGNED, int KH>
+__device__ __forceinline__ void issue_slice(const mako_sample_desc& d, uint32_t row, uint32_t lo, uint32_t hi, SliceLoads<KH>& s)
 {
     const uint32_t tid = threadIdx.x;
     // My history entries go first: loads return in the order they were issued, so whatever waits for these does not
@@ -212,33 +213,46 @@ __device__ __forceinline__ void load_penalised(const mako_sample_desc& d, uint32
     // (Loads from clamped positions, issued without branches between them; what was not wanted is dropped
     // afterwards: a branch around each load would make every load wait for the one before.)
     // Whether they are asked for depends on the kernel's arguments alone, not on the row's parameters or its history
-    // length (`hl`, `pen`): a caller may still be waiting for those when these loads and the logits' go out.
-    const bool may_penalise = KH > 0 && d.hist_tokens != nullptr && d.hist_stride > 0; // uniform
-    const global_ptr<const int32_t> ht = as_global(d.hist_tokens) + (int64_t)row * d.hist_stride;
-    const global_ptr<const uint32_t> hc = d.hist_counts ? as_global(d.hist_counts) + (int64_t)row * d.hist_stride : nullptr;
-    uint32_t tok[KH > 0 ? KH : 1], cnt[KH > 0 ? KH : 1];
-    bool have[KH > 0 ? KH : 1];
-    if (may_penalise) {
+    // length: a caller may still be waiting for those when these loads and the logits' go out.
+    if (KH > 0 && d.hist_tokens != nullptr && d.hist_stride > 0) { // uniform
+        const global_ptr<const int32_t> ht = as_global(d.hist_tokens) + (int64_t)row * d.hist_stride;
         const uint32_t last = (uint32_t)d.hist_stride - 1u; // (entries past the row's length are read and dropped)
 #pragma unroll
         for (int k = 0; k < KH; ++k)
-            tok[k] = (uint32_t)ht[min(tid + (uint32_t)k * kThreads, last)];
-        if (hc) {
+            s.tok[k] = (uint32_t)ht[min(tid + (uint32_t)k * kThreads, last)];
+        if (d.hist_counts) {
+            const global_ptr<const uint32_t> hc = as_global(d.hist_counts) + (int64_t)row * d.hist_stride;
 #pragma unroll
             for (int k = 0; k < KH; ++k)
-                cnt[k] = hc[min(tid + (uint32_t)k * kThreads, last)];
+                s.cnt[k] = hc[min(tid + (uint32_t)k * kThreads, last)];
         }
     }
-    RawSlice raw;
-    load_raw<ALIGNED>(d, row, lo, hi, raw);
-    // (the table of counts is cleared while the loads are on their way, whether the row will need it or not: behind them it
-    // took 1.5 of the 7.7 us that a workgroup of a 512-row decode batch has for its slice)
-    if (may_penalise) {
+    load_raw<ALIGNED>(d, row, lo, hi, s.raw);
+}
+// (the table of counts is cleared while the loads are on their way, whether the row will need it or not: behind them it
+// took 1.5 of the 7.7 us that a workgroup of a 512-row decode batch has for its slice)
+template <int KH>
+__device__ __forceinline__ void clear_counts(const mako_sample_desc& d, uint32_t slice_len, uint32_t* s_cnt)
+{
+    if (KH > 0 && d.hist_tokens != nullptr && d.hist_stride > 0) { // uniform
         uint4* z = reinterpret_cast<uint4*>(s_cnt); // slice_len is a multiple of 4
-        for (uint32_t i = tid; i < slice_len / 4; i += kThreads)
+        for (uint32_t i = threadIdx.x; i < slice_len / 4; i += kThreads)
             z[i] = make_uint4(0, 0, 0, 0);
     }
-    overlap();
+}
+
+// The rest, on what issue_slice() has asked for; the table is clear.
+template <bool ALIGNED, int KH>
+__device__ __forceinline__ void finish_penalised(const mako_sample_desc& d, uint32_t row, uint32_t lo, uint32_t hi, uint32_t slice_len,
+                                                 const mako_sampling_params& P, uint32_t hl, bool pen, uint32_t* s_cnt, SliceLoads<KH>& s,
+                                                 float (&wv)[16], bool want_above = false, float close_v = 0.0f, uint32_t* above = nullptr)
+{
+    const uint32_t tid = threadIdx.x;
+    RawSlice& raw = s.raw;
+    uint32_t (&tok)[KH > 0 ? KH : 1] = s.tok;
+    uint32_t (&cnt)[KH > 0 ? KH : 1] = s.cnt;
+    const bool hc = d.hist_counts != nullptr;
+    bool have[KH > 0 ? KH : 1];
     if (want_above) { // uniform
         settle_slice<ALIGNED>(raw, lo, hi);
         *above = count_above(raw, lo, hi, close_v);
@@ -328,6 +342,21 @@ __device__ __forceinline__ void load_penalised(const mako_sample_desc& d, uint32
                 wv[4 * k + 3] = (moved >> (4u * k)) & 8u ? __uint_as_float(v.w) : wv[4 * k + 3];
             }
     }
+}
+
+// `overlap` runs right after the slice's loads have been issued: work that does not depend on them hides
+// behind their latency.  It must be reached by the whole workgroup or by none of it.
+template <bool ALIGNED, int KH, typename Overlap = NoOverlap>
+__device__ __forceinline__ void load_penalised(const mako_sample_desc& d, uint32_t row, uint32_t lo, uint32_t hi,
+                                               uint32_t slice_len, const mako_sampling_params& P, uint32_t hl, bool pen,
+                                               uint32_t* s_cnt, float (&wv)[16], Overlap overlap = Overlap(),
+                                               bool want_above = false, float close_v = 0.0f, uint32_t* above = nullptr)
+{
+    SliceLoads<KH> s;
+    issue_slice<ALIGNED, KH>(d, row, lo, hi, s);
+    clear_counts<KH>(d, slice_len, s_cnt);
+    overlap();
+    finish_penalised<ALIGNED, KH>(d, row, lo, hi, slice_len, P, hl, pen, s_cnt, s, wv, want_above, close_v, above);
 }
 
 } // namespace mako
