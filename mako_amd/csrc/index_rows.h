@@ -137,6 +137,15 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
     // (~bits(q), at the token's own position)
     uint32_t* key0 = sc.key[0] + (size_t)row * sc.vpad;
     MAKO_CHECK(sc, kCheckStage, (uint64_t)hi <= sc.vpad);
+    // (a wide row: its weights counted by value)
+    const bool wide = STEPS && wide_row(P0) && nth_picks_for(d.n_vocab); // uniform
+    uint32_t* const bins = reinterpret_cast<uint32_t*>(s_dyn64) + 1024u; // [kNthBins], behind the sums below
+    if (wide) {
+        lds_barrier(); // (the penalty table is done with)
+        if (tid < kNthBins)
+            bins[tid] = 0u;
+        lds_barrier();
+    }
     uint32_t cnt = 0, last = 0;
     double bsum[4];
 #pragma unroll
@@ -155,6 +164,8 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
                 cnt += ok ? 1u : 0u;
                 last = ok ? max(last, at + 1u) : last;
                 bsum[b] += ok ? (double)q : 0.0;
+                if (wide && ok)
+                    atomicAdd(&bins[nth_bin(k[c])], 1u);
             }
             if (base + 3u < hi) {
                 *reinterpret_cast<uint4*>(key0 + base) = make_uint4(~k[0], ~k[1], ~k[2], ~k[3]);
@@ -215,6 +226,8 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
         wcnt[kWaves + wave_id()] = last;
     }
     __syncthreads();
+    if (wide && tid < kNthBins)
+        nth_hist(sc, row, piece)[tid] = bins[tid];
     if (tid < 4u && lo + tid * kIndexBlock < hi) { // (a sum per 4 096 entries: index_groups_kernel's workgroups may be that small)
         double s = 0.0;
         for (int w = 0; w < kWaves; ++w)
@@ -234,7 +247,7 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
         plan->key_lo[piece] = last;
         if (piece == 0) {
             if (STEPS) {
-                nth_state(plan, 0u)->seq = nth_state(plan, 1u)->seq = 0u;
+                nth_state(plan, 0u)->seq = nth_state(plan, 1u)->seq = plan->cap[kNthCursor] = 0u;
                 *nth_first(plan) = first;
             }
             plan->flag = kIndexClaimed;

@@ -32,7 +32,8 @@ void launch_index_weights(bool aligned, int kh, bool steps, hipStream_t st, cons
 
 void launch_nth_step(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t step, uint32_t wgs)
 {
-    hipLaunchKernelGGL(nth_step_kernel, dim3((d.n_rows + 7u) & ~7u, wgs), dim3(kThreads), kNthChunk * 8u + (d.n_vocab + 63u) / 64u * 12u + 64u, st, d, sc, step);
+    const uint32_t rounds = kNthChunk * 8u + (d.n_vocab + 63u) / 64u * 12u + 64u, picking = step == 1u ? kNthPickedMax * 8u + 64u : 0u;
+    hipLaunchKernelGGL(nth_step_kernel, dim3((d.n_rows + 7u) & ~7u, wgs), dim3(kThreads), rounds > picking ? rounds : picking, st, d, sc, step);
 }
 
 void launch_index_finish(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, bool in_order_rows, bool other_rows)

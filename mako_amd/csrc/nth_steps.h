@@ -12,6 +12,10 @@
 //   step 1                 such a row: the first round.  Any other: the candidates moved together.
 //   step 2, 3, ...         a round each, until what is left fits a workgroup's registers (kNthUntil), where the row's one
 //                          workgroup goes on in the last launch.
+// A top-k before a top-p (wide_row()) needs no rounds: its survivors end up sorted, so only which candidates they are matters.
+// index_weights_kernel counts the weights by value, and step 1 picks those from the bin that holds the k-th on, which the last
+// launch sorts.  (64 rows of 129 280, top_k 200 to 1 000: 183 us with the rounds, 75 so.)  Where the bin is too crowded, as on a
+// grid of few weights, the rounds are made.
 // A step writes the list it makes beside the old one, with the next round's pivot already swapped to the front; its workgroups
 // take 4 096 entries of the new list at a time.  An entry that belongs left and lies in front of the cut stays where it is; a
 // hole's filler comes through LDS: the holes of 4 096 places in a row are filled from one stretch of the old list, from its
@@ -31,11 +35,14 @@ constexpr uint32_t kNthLds = kNthChunk * 8u + kNthWords * 12u + 64u;
 
 // Where a row stands: two records in turn in the row's plan (a step reads one and writes the other), in the words its workers
 // would use.  seq: steps made, 0: none yet.  len entries of key[buf] / idx[buf] are what is left of the list, `used` rounds
-// behind them.  pre: the next round's pivot is at the front and its bits are in place.
+// behind them.  pre: kNthBits: the next round's pivot is at the front and its bits are in place; kNthPicked: the list is what a
+// wide row keeps, and more, in any order, and `used` the least bits(q) it may hold.
 struct alignas(4) NthState {
     uint32_t seq, len, pre, used, buf;
 };
-static_assert(2u * sizeof(NthState) <= sizeof(BigPlan::cap), "");
+constexpr uint32_t kNthBits = 1, kNthPicked = 2;
+constexpr uint32_t kNthCursor = 16; // the word of the plan's `cap` that counts what step 1 picks
+static_assert(2u * sizeof(NthState) <= kNthCursor * 4u && sizeof(BigPlan::cap) > kNthCursor * 4u, "");
 // The first pivot of a row that is its own list, where it came from, and the key of its first entry.
 struct NthFirst {
     uint32_t pivot_key, pivot_id, from, first_key;
@@ -55,7 +62,7 @@ __device__ __forceinline__ uint32_t* nth_bits(const Scratch& sc, uint32_t row, u
     return reinterpret_cast<uint32_t*>(sc.wbuf + (size_t)row * sc.vpad) + buf * (uint32_t)(sc.vpad / 32u + 256u);
 }
 // Is the row one of these?  (The others of its class stay in token order: index_rows.h.)
-__device__ __forceinline__ bool nth_row(const mako_sampling_params& P)
+__host__ __device__ __forceinline__ bool nth_row(const mako_sampling_params& P)
 {
     return classify(P) == kGeneral && P.top_k != 0u;
 }
@@ -63,6 +70,38 @@ __device__ __forceinline__ bool nth_row(const mako_sampling_params& P)
 __host__ __device__ __forceinline__ bool nth_steps_for(uint32_t n_vocab)
 {
     return n_vocab > kNthUntil && n_vocab <= kNthMaxVocab;
+}
+
+// ... and of those, a top-k before a top-p?
+__host__ __device__ __forceinline__ bool wide_row(const mako_sampling_params& P)
+{
+    return nth_row(P) && P.top_p < 1.0f;
+}
+// Are a wide row's picked, of so many logits?  (16 000 of them: 89 us with the rounds in one workgroup's registers, 48 so.)
+__host__ __device__ __forceinline__ bool nth_picks_for(uint32_t n_vocab)
+{
+    return n_vocab > 2048u && n_vocab <= kNthMaxVocab;
+}
+// A wide row's weights counted by value, a table per 16 384 logits, behind the bits: 64 bins a binade for the four heaviest
+// binades, where a flat row has all of its weights, four a binade below.
+constexpr uint32_t kNthBins = 768, kNthFine = 256;
+constexpr uint32_t kNthPickedMax = kSegCap; // entries that step 1 may pick: what one sort in LDS holds
+static_assert(kNthPickedMax * 8u + 64u <= kNthLds, "");
+__device__ __forceinline__ uint32_t nth_bin(uint32_t q_bits) // (heaviest first)
+{
+    static_assert(kNthFine + ((0x3f800000u - (kNthFine << 17)) >> 21) < kNthBins, "weights are at most 1");
+    const uint32_t d = 0x3f800000u - q_bits;
+    return d < kNthFine << 17 ? d >> 17 : kNthFine + ((d - (kNthFine << 17)) >> 21);
+}
+__device__ __forceinline__ uint32_t nth_bin_edge(uint32_t bin) // the bits of the lightest weight in it
+{
+    const uint32_t d = (bin < kNthFine ? (bin + 1u) << 17 : (kNthFine << 17) + ((bin + 1u - kNthFine) << 21)) - 1u;
+    return d < 0x3f800000u ? 0x3f800000u - d : 1u;
+}
+__device__ __forceinline__ uint32_t* nth_hist(const Scratch& sc, uint32_t row, uint32_t piece)
+{
+    static_assert(3u * (kNthUntil / 32u + 256u) + kNthMaxVocab / kSliceMax * kNthBins <= kNthUntil, "a row's bits and tables in the place of its logits");
+    return nth_bits(sc, row, 3u) + piece * kNthBins;
 }
 
 __device__ __forceinline__ uint32_t mask_rank(unsigned long long m)
@@ -89,7 +128,70 @@ __device__ __forceinline__ uint32_t eight_nibbles(uint32_t nibble)
     return v;
 }
 
-// One step of row `row`, by workgroup w of W.  lds: kNthLds bytes (what the row's bits take of it).  All threads call.
+// What a wide row keeps, by workgroup w of W (step 1): the entries from the bin that holds the nth-heaviest on, in any
+// order, to key[1] / idx[1].  Returns how many that is in all, kNone if it is too many (or nothing is cut off): then nothing has been written.  All threads call.
+__device__ __forceinline__ uint32_t nth_pick(const mako_sample_desc& d, const Scratch& sc, uint32_t row, uint32_t w, uint32_t W, uint32_t n0, uint32_t nth,
+                                             uint32_t& from, unsigned long long* lds_dyn, BlockScratch& bs)
+{
+    typedef unsigned long long u64;
+    const uint32_t tid = threadIdx.x;
+    if (nth >= n0) // uniform
+        return kNone;
+    const lds_ptr<u64> kept = as_lds(lds_dyn);                                        // [kNthPickedMax]
+    const lds_ptr<uint32_t> found = (lds_ptr<uint32_t>)(kept + kNthPickedMax);        // the bin, the entries from it on, this workgroup's, their place
+    // (thread t: bin t)
+    const uint32_t pieces = (d.n_vocab + kSliceMax - 1u) / kSliceMax;
+    uint32_t c = 0;
+    if (tid < kNthBins)
+        for (uint32_t p = 0; p < pieces; ++p)
+            c += as_global(nth_hist(sc, row, p))[tid];
+    uint32_t all;
+    const uint32_t above = block_excl_scan_u32(c, all, bs);
+    if (above < nth && above + c >= nth) {
+        found[0] = tid;
+        found[1] = above + c;
+        found[2] = 0u;
+    }
+    __syncthreads();
+    from = nth_bin_edge(uniform_u32(found[0]));
+    const uint32_t n = uniform_u32(found[1]);
+    if (n > kNthPickedMax) // uniform
+        return kNone;
+    const global_ptr<const uint32_t> key = as_global(sc.key[0]) + (size_t)row * sc.vpad;
+    constexpr uint32_t kTrip = 4;
+    for (uint32_t c0 = w; c0 * kNthChunk < d.n_vocab; c0 += W * kTrip) { // uniform
+        u32x4 k[kTrip];
+#pragma unroll
+        for (uint32_t u = 0; u < kTrip; ++u) // (rows' arrays are a multiple of 1 024 long)
+            k[u] = *(global_ptr<const u32x4>)(key + min((c0 + u * W) * kNthChunk + 4u * tid, (d.n_vocab - 1u) & ~3u));
+#pragma unroll
+        for (uint32_t u = 0; u < kTrip; ++u)
+#pragma unroll
+            for (uint32_t j = 0; j < 4; ++j) {
+                const uint32_t i = (c0 + u * W) * kNthChunk + 4u * tid + j;
+                if (i < d.n_vocab && ~k[u][j] >= from && k[u][j] != ~0u) { // (few)
+                    const uint32_t at = __hip_atomic_fetch_add(found + 2, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+                    if (at < kNthPickedMax)
+                        kept[at] = ((u64)k[u][j] << 32) | (u64)i;
+                }
+            }
+    }
+    __syncthreads();
+    const uint32_t mine = min(uniform_u32(found[2]), kNthPickedMax);
+    if (tid == 0)
+        found[3] = mine ? __hip_atomic_fetch_add(as_global(&sc.plan[row].cap[kNthCursor]), mine, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) : 0u;
+    __syncthreads();
+    const uint32_t base = uniform_u32(found[3]);
+    const global_ptr<uint32_t> kout = as_global(sc.key[1]) + (size_t)row * sc.vpad, iout = as_global(sc.idx[1]) + (size_t)row * sc.vpad;
+    for (uint32_t e = tid; e < mine && base + e < kNthPickedMax; e += (uint32_t)kThreads) {
+        MAKO_CHECK(sc, kCheckCompact, base + e < n);
+        kout[base + e] = (uint32_t)(kept[e] >> 32);
+        iout[base + e] = (uint32_t)kept[e];
+    }
+    return n;
+}
+
+// One step of row `row`, by workgroup w of W.  lds: kNthLds bytes, or what the row's bits, and the first step's picks, take of it.  All threads call.
 __device__ __forceinline__ void nth_step(const mako_sample_desc& d, const Scratch& sc, uint32_t row, uint32_t w, uint32_t W, uint32_t step,
                                          unsigned long long* lds_dyn, BlockScratch& bs)
 {
@@ -113,14 +215,27 @@ __device__ __forceinline__ void nth_step(const mako_sample_desc& d, const Scratc
     };
     load_bits(usual, words_max);
     const uint32_t nth = P.top_k;
-    if (!nth_row(P) || flag != kIndexClaimed) // uniform (a row of another kind; one whose token is forced)
+    const bool picks = step == 1u && wide_row(P) && nth_picks_for(d.n_vocab);
+    if (!nth_row(P) || flag != kIndexClaimed || !(picks || nth_steps_for(d.n_vocab))) // uniform (a row of another kind; one whose token is forced)
         return;
     bool compact = false;
     if (step == 1u) {
         const uint32_t n0 = uniform_u32(__ockl_wfred_add_u32(lane < pieces ? counted : 0u));
         compact = n0 != d.n_vocab;
         // (a whole list that nothing is cut off stays as it is)
-        now = NthState{0u, d.n_vocab, compact || nth < n0 ? 1u : 0u, 0u, 0u};
+        now = NthState{0u, d.n_vocab, compact || nth < n0 ? kNthBits : 0u, 0u, 0u};
+        if (picks) { // uniform
+            uint32_t from = 0;
+            const uint32_t picked = nth_pick(d, sc, row, w, W, n0, nth, from, lds_dyn, bs);
+            if (picked != kNone) {
+                if (w == 0u && tid == 0u)
+                    *nth_state(plan, 1u) = NthState{1u, picked, kNthPicked, from, 1u};
+                return;
+            }
+            if (!nth_steps_for(d.n_vocab))
+                return;
+            __syncthreads();
+        }
     }
     const uint32_t len = uniform_u32(now.len), from_buf = uniform_u32(now.buf), used = now.used;
     auto leave = [&](uint32_t n, uint32_t pre, uint32_t rounds, uint32_t in) {
@@ -140,7 +255,7 @@ __device__ __forceinline__ void nth_step(const mako_sample_desc& d, const Scratc
     const uint32_t to_buf = from_buf ^ 1u;
     const global_ptr<const uint32_t> kin = as_global(sc.key[from_buf]) + (size_t)row * sc.vpad, iin = as_global(sc.idx[from_buf]) + (size_t)row * sc.vpad;
     const global_ptr<uint32_t> kout = as_global(sc.key[to_buf]) + (size_t)row * sc.vpad, iout = as_global(sc.idx[to_buf]) + (size_t)row * sc.vpad;
-    bool go = uniform_u32(now.pre) != 0u;
+    bool go = uniform_u32(now.pre) == kNthBits;
     uint32_t smalls = 0;
     if (go) { // uniform
         if (compact || from_buf != usual) // uniform
@@ -325,7 +440,7 @@ __device__ __forceinline__ void nth_step(const mako_sample_desc& d, const Scratc
         }
         __syncthreads(); // (the fillers' buffer)
     }
-    leave(out_len, goes_on ? 1u : 0u, used + (compact ? 0u : 1u), to_buf);
+    leave(out_len, goes_on ? kNthBits : 0u, used + (compact ? 0u : 1u), to_buf);
 }
 
 } // namespace mako

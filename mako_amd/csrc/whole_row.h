@@ -1,6 +1,7 @@
 // The whole-row path: exact for every parameter combination, one workgroup per row.
 #pragma once
 
+#include "lds_sort.h"
 #include "nth_steps.h"
 #include "sorted_tail.h"
 
@@ -102,6 +103,7 @@ __device__ bool radix_pass(const uint32_t* ksrc, const uint32_t* isrc, uint32_t*
 
 __device__ void sort_segment(uint32_t* k0, uint32_t* i0, uint32_t* k1, uint32_t* i1, uint32_t n, const FinishLds& L);
 __device__ void sort_survivors(uint32_t* k0, uint32_t* i0, uint32_t* k1, uint32_t* i1, uint32_t n, const FinishLds& L);
+__device__ void sort_picked(uint32_t* k0, uint32_t* i0, uint32_t* k1, uint32_t* i1, uint32_t n, uint32_t key_lo, const FinishLds& L);
 
 // libstdc++'s __heap_select(first, nth + 1, last) followed by iter_swap(first, nth) (bits/stl_algo.h:1956-1960,
 // stl_heap.h): where introselect ends up when its depth limit is spent.  The arrangement it leaves is the library's,
@@ -678,14 +680,16 @@ __device__ __forceinline__ bool nth_rounds_wave(lds_ptr<unsigned long long> rang
 }
 
 // What other workgroups have done of it (nth_steps.h): `used` rounds, which left `len` entries; `ready` as for
-// nth_rounds_memory().
+// nth_rounds_memory().  picked: the list is what a wide row keeps, and more, none with less bits(q) than `used`.
 struct NthDone {
     uint32_t used, len;
     const uint32_t* ready;
+    bool picked;
 };
+constexpr NthDone kNthNothing = {0u, kNone, nullptr, false};
 // The row's candidates in device memory (key[i], idx[i]; far: n / 32 words of it that are free), n of them to begin with.  All threads call.
 __device__ MAKO_RARE_CALL void nth_element_row(uint32_t* key_p, uint32_t* idx_p, uint32_t n, uint32_t nth, uint32_t* far, const FinishLds& L,
-                                               NthDone done = NthDone{0u, kNone, nullptr})
+                                               NthDone done = kNthNothing)
 {
     assume_lds(L);
     typedef unsigned long long u64;
@@ -814,7 +818,7 @@ __device__ MAKO_RARE_CALL void compact_candidates(const uint32_t* qb, uint32_t V
 template <bool TOPK_ALONE>
 __device__ bool sort_truncate_draw(const mako_sample_desc& d, uint32_t row, const mako_sampling_params& P, uint32_t* key0, uint32_t* idx0,
                                    uint32_t* key1, uint32_t* idx1, const uint32_t* qk, uint32_t n0, bool have_total, double total64,
-                                   uint32_t path, const FinishLds& L, NthDone done = NthDone{0u, kNone, nullptr})
+                                   uint32_t path, const FinishLds& L, NthDone done = kNthNothing)
 {
     assume_lds(L);
     FinishShared& sm = *L.sm;
@@ -826,7 +830,9 @@ __device__ bool sort_truncate_draw(const mako_sample_desc& d, uint32_t row, cons
     const bool nth_order = TOPK_ALONE && topk_active && !topp_active;
     if (nth_order)
         nth_element_row(key0, idx0, n0, P.top_k, key1, L, done);
-    else if (topk_active) {
+    else if (topk_active && done.picked) {
+        sort_picked(key0, idx0, key1, idx1, min(done.len, kNthPickedMax), done.used, L);
+    } else if (topk_active) {
         // a top-p follows: the survivors are sorted, so only which candidates they are matters, and `desc` is a total
         // order: nth_element's first top_k entries are the top_k first of the sorted list, in some order.  The
         // partitions and a sort of top_k entries cost a quarter of the sort of all candidates.
@@ -979,6 +985,36 @@ __device__ void sort_survivors(uint32_t* k0, uint32_t* i0, uint32_t* k1, uint32_
     else
         sort(std::integral_constant<int, 4>());
     __syncthreads();
+}
+
+// The n <= kNthPickedMax entries that nth_pick() has left at (k0, i0), none with less bits(q) than key_lo, by key, then id, both
+// ascending; (k1, i1): a second buffer.
+__device__ void sort_picked(uint32_t* k0, uint32_t* i0, uint32_t* k1, uint32_t* i1, uint32_t n, uint32_t key_lo, const FinishLds& L)
+{
+    assume_lds(L);
+    FinishShared& sm = *L.sm;
+    const uint32_t tid = threadIdx.x;
+    const uint32_t key_hi = 0x3f800001u; // (just above 1.0)
+    static_assert((kSegCap + 4u) * 8u + (kFine + 4u) * 4u <= kTailLds, "the sort's buckets");
+    uint32_t* hist = reinterpret_cast<uint32_t*>(L.sortk + kSegCap + 4u); // (lds_bucket_sort()'s)
+    const global_ptr<const uint32_t> k = as_global(k0), i = as_global(i0);
+    uint32_t key[kSortPer], id[kSortPer];
+    __syncthreads();
+#pragma unroll
+    for (uint32_t t = 0; t < kSortPer; ++t) {
+        const uint32_t e = min(t * kThreads + tid, n - 1u);
+        key[t] = min(max(~k[e], key_lo), key_hi - 1u);
+        id[t] = i[e];
+    }
+    for (uint32_t b = tid; b <= kFine; b += kThreads)
+        hist[b] = 0;
+    if (tid == 0)
+        sm.flag = 0;
+    __syncthreads(); // (everything has been read)
+    if (!lds_bucket_sort(key, id, n, key_lo, key_hi, k0, i0, L.sortk, sm)) {
+        __syncthreads();
+        sort_survivors(k0, i0, k1, i1, n, L); // (a crowded bucket; nothing has been moved)
+    }
 }
 
 // Whole-row path: exact for every parameter combination.  One workgroup rebuilds the penalised
@@ -1137,12 +1173,13 @@ __device__ MAKO_RARE_CALL void general_row_from_weights(const mako_sample_desc& 
     uint32_t* i_to = sc.idx[1] + (size_t)row * sc.vpad;
     uint32_t n0 = n_all;
     bool listed = n_all == V; // in the first buffers
-    NthDone done = {0u, kNone, nullptr};
-    if (nth_steps_for(V)) { // uniform
+    NthDone done = kNthNothing;
+    if ((nth_steps_for(V) || (wide_row(P) && nth_picks_for(V))) && nth_state(sc.plan + row, 0u)->seq + nth_state(sc.plan + row, 1u)->seq != 0u) { // uniform
         const NthState s0 = *nth_state(sc.plan + row, 0u), s1 = *nth_state(sc.plan + row, 1u);
         const bool odd = s1.seq > s0.seq;
         const uint32_t buf = odd ? s1.buf : s0.buf;
-        done = NthDone{odd ? s1.used : s0.used, odd ? s1.len : s0.len, (odd ? s1.pre : s0.pre) ? nth_bits(sc, row, buf) : nullptr};
+        const uint32_t pre = odd ? s1.pre : s0.pre;
+        done = NthDone{odd ? s1.used : s0.used, odd ? s1.len : s0.len, pre == kNthBits ? nth_bits(sc, row, buf) : nullptr, pre == kNthPicked};
         listed = buf == 0u;
     } else if (!listed) {
         const global_ptr<const uint32_t> from = as_global(k_from);

@@ -87,3 +87,31 @@ def test_steps_forced_and_verified(vocab):
                 assert (g["tokens"][r], bool(g["accepted"][r])) == (t, bool(tr["accepted"])), (r, hinted)
     finally:
         ctx.close()
+
+
+# (the bin that holds the k-th heaviest: a few entries more than k, thousands, more than one sort in LDS holds)
+@pytest.mark.parametrize("vocab", [2048, 2049, 9001, 16381, 40000, 131072, 151553])
+@pytest.mark.parametrize("sigma", [3.0, 0.5, 0.02])
+def test_wide_top_k_before_a_top_p(vocab, sigma):
+    rng = np.random.Generator(np.random.PCG64([vocab, int(sigma * 100)]))
+    top_ks = [k for k in (129, 200, 500, 1000, 4096, 6143, 6144, 6145, 9000) if k < vocab] + [vocab - 1, vocab]
+    rows = len(top_ks)
+    x = (rng.standard_normal((rows, vocab)) * sigma).astype(np.float32)
+    x[1::3] = np.round(x[1::3] * 16.0) / np.float32(16.0)
+    p = api.make_params(rows, 1.0, 0, 0.95)
+    p["top_k"] = top_ks
+    p["top_p"][::2] = np.float32(0.9999)
+    p["min_p"][3] = np.float32(0.5)
+    w = dict(name="wide V=%d" % vocab, logits=x, params=p, u=rng.random(rows).astype(np.float32))
+    ctx = api.SamplerContext(max_rows=rows, max_vocab=vocab)
+    try:
+        for masked in (False, True):
+            if masked:
+                w["mask"] = rng.integers(0, 2**32, (rows, (vocab + 31) // 32), dtype=np.uint64).astype(np.uint32)
+            for hinted in (True, False):
+                assert_parity(ctx, w, cap=300, hinted=hinted)
+        p["top_k"][0], p["top_p"][0] = 0, 0.9  # (beside a nucleus)
+        for hinted in (True, False):
+            assert_parity(ctx, w, cap=300, hinted=hinted)
+    finally:
+        ctx.close()
