@@ -122,7 +122,7 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
     float wv[16];
     // (a row for nth_steps.h: the first round's pivot if every logit should turn out to be a candidate)
     const bool steps = STEPS && !in_order && nth_steps_for(d.n_vocab); // uniform
-    load_penalised<ALIGNED, KH>(d, row, lo, hi, kSliceMax, P, hl, pen, reinterpret_cast<uint32_t*>(s_dyn64), wv, [&]() {
+    load_penalised<ALIGNED, KH>(d, row, lo, hi, kSliceMax, P, pen, hl, pen, reinterpret_cast<uint32_t*>(s_dyn64), wv, [&]() {
         if (steps)
             first_pivot(d, row, P, pen ? hl : 0u, m, sm);
     });

@@ -72,7 +72,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(ALIGNE
     const RowClass cls = classify(P);
     // Greedy rows ignore the penalties (src/gen/sampler.cpp:77-78).
     const uint32_t hl = cls != kGreedy ? hl_row : 0u;
-    const bool pen = hl > 0 && !penalties_neutral(P);
+    const bool penalised = cls != kGreedy && !penalties_neutral(P), pen = hl > 0 && penalised;
     if (tid == 0) {
         sm.argidx = kNone;
         sm.emit_n = 0;
@@ -116,11 +116,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(ALIGNE
     uint32_t above = 0;
     float wv[16];
     if (ABOVE) {
-        load_penalised<ALIGNED, KH>(d, row, lo, hi, slice_len, P, hl, pen, s_dyn, wv, NoOverlap(), want_above, close_v, &above);
+        load_penalised<ALIGNED, KH>(d, row, lo, hi, slice_len, P, penalised, hl, pen, s_dyn, wv, NoOverlap(), want_above, close_v, &above);
         if (want_above) // uniform
             above = __ockl_wfred_add_u32(above);
     } else {
-        load_penalised<ALIGNED, KH>(d, row, lo, hi, slice_len, P, hl, pen, s_dyn, wv);
+        load_penalised<ALIGNED, KH>(d, row, lo, hi, slice_len, P, penalised, hl, pen, s_dyn, wv);
     }
 
     MAKO_STAMP(29);

@@ -40,7 +40,7 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
         PlanLoads pre;
         issue_plan_loads<UNSORTED>(d, sc, row, slices, pre);
         issue_slice<ALIGNED, KH>(d, row, lo, hi, loads);
-        clear_counts<KH>(d, slice_len, L.cnt);
+        clear_counts<KH>(d, pen, slice_len, L.cnt);
         {
             uint32_t n_cands, any_overflow;
             row_summary_of(pre.st, slices, m, argidx, n_cands, any_overflow);
@@ -49,7 +49,7 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
     } else {
         if (!AHEAD)
             issue_slice<ALIGNED, KH>(d, row, lo, hi, loads);
-        clear_counts<KH>(d, slice_len, L.cnt);
+        clear_counts<KH>(d, pen, slice_len, L.cnt);
     }
     finish_penalised<ALIGNED, KH>(d, row, lo, hi, slice_len, P, hl, pen, L.cnt, loads, wv);
     MAKO_STAMP(1);

@@ -229,12 +229,12 @@ __device__ __forceinline__ void issue_slice(const mako_sample_desc& d, uint32_t 
     }
     load_raw<ALIGNED>(d, row, lo, hi, s.raw);
 }
-// (the table of counts is cleared while the loads are on their way, whether the row will need it or not: behind them it
-// took 1.5 of the 7.7 us that a workgroup of a 512-row decode batch has for its slice)
+// (the table of counts is cleared while the loads are on their way, also for a row that may turn out to have no history;
+// `penalised`: it has penalties, and a use for them)
 template <int KH>
-__device__ __forceinline__ void clear_counts(const mako_sample_desc& d, uint32_t slice_len, uint32_t* s_cnt)
+__device__ __forceinline__ void clear_counts(const mako_sample_desc& d, bool penalised, uint32_t slice_len, uint32_t* s_cnt)
 {
-    if (KH > 0 && d.hist_tokens != nullptr && d.hist_stride > 0) { // uniform
+    if (KH > 0 && penalised && d.hist_tokens != nullptr && d.hist_stride > 0) { // uniform
         uint4* z = reinterpret_cast<uint4*>(s_cnt); // slice_len is a multiple of 4
         for (uint32_t i = threadIdx.x; i < slice_len / 4; i += kThreads)
             z[i] = make_uint4(0, 0, 0, 0);
@@ -348,13 +348,13 @@ __device__ __forceinline__ void finish_penalised(const mako_sample_desc& d, uint
 // behind their latency.  It must be reached by the whole workgroup or by none of it.
 template <bool ALIGNED, int KH, typename Overlap = NoOverlap>
 __device__ __forceinline__ void load_penalised(const mako_sample_desc& d, uint32_t row, uint32_t lo, uint32_t hi,
-                                               uint32_t slice_len, const mako_sampling_params& P, uint32_t hl, bool pen,
+                                               uint32_t slice_len, const mako_sampling_params& P, bool penalised, uint32_t hl, bool pen,
                                                uint32_t* s_cnt, float (&wv)[16], Overlap overlap = Overlap(),
                                                bool want_above = false, float close_v = 0.0f, uint32_t* above = nullptr)
 {
     SliceLoads<KH> s;
     issue_slice<ALIGNED, KH>(d, row, lo, hi, s);
-    clear_counts<KH>(d, slice_len, s_cnt);
+    clear_counts<KH>(d, penalised, slice_len, s_cnt);
     overlap();
     finish_penalised<ALIGNED, KH>(d, row, lo, hi, slice_len, P, hl, pen, s_cnt, s, wv, want_above, close_v, above);
 }
