@@ -63,7 +63,7 @@ __global__ __launch_bounds__(kThreads) void sort_beside_kernel(mako_sample_desc 
     const uint32_t all = in_order * blocks;
     const uint32_t me = (blockIdx.y - sort_rows) * gridDim.x + blockIdx.x, wgs = (gridDim.y - sort_rows) * gridDim.x;
     // (nth_steps.h's first step, as many workgroups a row as there are; the groups' workgroups are counted from the other end)
-    const uint32_t nth_rows = nth_picks_for(d_arg.n_vocab) ? general - in_order : 0u;
+    const uint32_t nth_rows = nth_steps_for(d_arg.n_vocab) ? general - in_order : 0u;
     if (nth_rows) { // uniform
         const uint32_t per_row = min(max(wgs / nth_rows, 1u), (d_arg.n_vocab + kNthChunk - 1u) / kNthChunk);
         RankedRows rows;

@@ -37,7 +37,7 @@ void launch_tail(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, u
 // the three kernels of a batch with none but rows of the whole-row class (index_rows.h): the weights, the group records, the
 // total and the draw
 hipError_t init_index_kernels();
-// (steps: there are rows for nth_steps.h)
+// (steps: there are rows for nth_steps.h, its steps or its picks)
 void launch_index_weights(bool aligned, int kh, bool steps, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices);
 // a step of nth_steps.h, `wgs` workgroups per row
 void launch_nth_step(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t step, uint32_t wgs);

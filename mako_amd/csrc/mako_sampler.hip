@@ -423,13 +423,13 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
         beside = n_index != 0 && !only_index;
         index_rows = n_index;
     }
-    const bool any_nth = any_unordered && (mako::nth_steps_for(d.n_vocab) || (any_wide && mako::nth_picks_for(d.n_vocab)));
+    const bool any_nth = any_unordered && mako::nth_steps_for(d.n_vocab), any_bits = any_nth || (any_wide && mako::nth_picks_for(d.n_vocab));
     // (their steps: a launch each, of about two workgroups per CU.  Beside other rows the sort's launch has the first.  A launch
     // costs 8 to 10 us and leaves 0.44 of a row: as many as bring the 64 rows' unluckiest near what a workgroup takes into its
     // registers.  64 rows of 129 280: 185 us with two, 172, 164, 162, 168 with six; of 40 000: 104 with two, 105, 110)
     const uint32_t nth_wgs = std::min(std::max(2u * ctx->cus / ((d.n_rows + 7u) & ~7u), 1u), (d.n_vocab + mako::kNthChunk - 1u) / mako::kNthChunk);
     // (rows of a top-k before a top-p alone have no use for more than the first)
-    const uint32_t nth_steps = !any_nth ? 0u : (!any_rounds || !mako::nth_steps_for(d.n_vocab) ? 1u : (d.n_vocab <= 65536u ? 2u : 4u));
+    const uint32_t nth_steps = !any_nth ? 0u : (!any_rounds ? 1u : (d.n_vocab <= 65536u ? 2u : 4u));
     const bool launch_sort = any_nucleus || any_late || beside;
     // (finish_kernel's grid: scan_kernel, which cuts the second pass up, is told of it)
     const uint32_t finish_wgs = mako::second_pass_grid(nucleus_rows, ctx->cus);
@@ -470,7 +470,7 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
         MAKO_LAUNCH(mako::launch_tail_beside(st, d, sc, slices, nucleus_rows, unsorted));
     } else {
         if (only_index)
-            MAKO_LAUNCH(mako::launch_index_weights(aligned, kh, any_nth, st, d, sc, slices));
+            MAKO_LAUNCH(mako::launch_index_weights(aligned, kh, any_bits, st, d, sc, slices));
         if (any_nucleus)
             MAKO_LAUNCH(mako::launch_finish(aligned, kh, unsorted, finish_wgs, st, d, sc, slices));
         if (!launch_sort && !only_index)

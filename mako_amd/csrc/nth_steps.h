@@ -66,10 +66,12 @@ __host__ __device__ __forceinline__ bool nth_row(const mako_sampling_params& P)
 {
     return classify(P) == kGeneral && P.top_k != 0u;
 }
-// Are there steps for rows of this many logits?
+// Are there steps for rows of this many logits?  (Below, a round in device memory takes a workgroup 12 us at most, and a step's
+// launch 8, and all of its rows may be masked down to a few candidates: 64 rows of 19 392, half of them masked, 82 us without
+// steps, 91 with two.)
 __host__ __device__ __forceinline__ bool nth_steps_for(uint32_t n_vocab)
 {
-    return n_vocab > kNthUntil && n_vocab <= kNthMaxVocab;
+    return n_vocab > 32768u && n_vocab <= kNthMaxVocab;
 }
 
 // ... and of those, a top-k before a top-p?
@@ -77,7 +79,8 @@ __host__ __device__ __forceinline__ bool wide_row(const mako_sampling_params& P)
 {
     return nth_row(P) && P.top_p < 1.0f;
 }
-// Are a wide row's picked, of so many logits?  (16 000 of them: 89 us with the rounds in one workgroup's registers, 48 so.)
+// Are a wide row's picked, of so many logits?  Where there are steps, by the first of them, else by the row's one workgroup in the
+// last launch.  (16 000 of them: 89 us with the rounds in that workgroup's registers, 45 so; 48 with a step.)
 __host__ __device__ __forceinline__ bool nth_picks_for(uint32_t n_vocab)
 {
     return n_vocab > 2048u && n_vocab <= kNthMaxVocab;
@@ -215,8 +218,7 @@ __device__ __forceinline__ void nth_step(const mako_sample_desc& d, const Scratc
     };
     load_bits(usual, words_max);
     const uint32_t nth = P.top_k;
-    const bool picks = step == 1u && wide_row(P) && nth_picks_for(d.n_vocab);
-    if (!nth_row(P) || flag != kIndexClaimed || !(picks || nth_steps_for(d.n_vocab))) // uniform (a row of another kind; one whose token is forced)
+    if (!nth_row(P) || flag != kIndexClaimed) // uniform (a row of another kind; one whose token is forced)
         return;
     bool compact = false;
     if (step == 1u) {
@@ -224,7 +226,7 @@ __device__ __forceinline__ void nth_step(const mako_sample_desc& d, const Scratc
         compact = n0 != d.n_vocab;
         // (a whole list that nothing is cut off stays as it is)
         now = NthState{0u, d.n_vocab, compact || nth < n0 ? kNthBits : 0u, 0u, 0u};
-        if (picks) { // uniform
+        if (wide_row(P)) { // uniform
             uint32_t from = 0;
             const uint32_t picked = nth_pick(d, sc, row, w, W, n0, nth, from, lds_dyn, bs);
             if (picked != kNone) {
@@ -232,8 +234,6 @@ __device__ __forceinline__ void nth_step(const mako_sample_desc& d, const Scratc
                     *nth_state(plan, 1u) = NthState{1u, picked, kNthPicked, from, 1u};
                 return;
             }
-            if (!nth_steps_for(d.n_vocab))
-                return;
             __syncthreads();
         }
     }

@@ -103,7 +103,7 @@ __device__ bool radix_pass(const uint32_t* ksrc, const uint32_t* isrc, uint32_t*
 
 __device__ void sort_segment(uint32_t* k0, uint32_t* i0, uint32_t* k1, uint32_t* i1, uint32_t n, const FinishLds& L);
 __device__ void sort_survivors(uint32_t* k0, uint32_t* i0, uint32_t* k1, uint32_t* i1, uint32_t n, const FinishLds& L);
-__device__ void sort_picked(uint32_t* k0, uint32_t* i0, uint32_t* k1, uint32_t* i1, uint32_t n, uint32_t key_lo, const FinishLds& L);
+__device__ MAKO_RARE_CALL bool sort_picked(uint32_t* k0, uint32_t* i0, uint32_t n, uint32_t key_lo, const FinishLds& L);
 
 // libstdc++'s __heap_select(first, nth + 1, last) followed by iter_swap(first, nth) (bits/stl_algo.h:1956-1960,
 // stl_heap.h): where introselect ends up when its depth limit is spent.  The arrangement it leaves is the library's,
@@ -831,7 +831,11 @@ __device__ bool sort_truncate_draw(const mako_sample_desc& d, uint32_t row, cons
     if (nth_order)
         nth_element_row(key0, idx0, n0, P.top_k, key1, L, done);
     else if (topk_active && done.picked) {
-        sort_picked(key0, idx0, key1, idx1, min(done.len, kNthPickedMax), done.used, L);
+        const uint32_t n = min(done.len, kNthPickedMax);
+        if (!sort_picked(key0, idx0, n, done.used, L)) { // (a crowded bucket: what was picked is cut to what is kept first)
+            nth_element_row(key0, idx0, n, P.top_k, key1, L);
+            sort_survivors(key0, idx0, key1, idx1, P.top_k, L);
+        }
     } else if (topk_active) {
         // a top-p follows: the survivors are sorted, so only which candidates they are matters, and `desc` is a total
         // order: nth_element's first top_k entries are the top_k first of the sorted list, in some order.  The
@@ -988,8 +992,8 @@ __device__ void sort_survivors(uint32_t* k0, uint32_t* i0, uint32_t* k1, uint32_
 }
 
 // The n <= kNthPickedMax entries that nth_pick() has left at (k0, i0), none with less bits(q) than key_lo, by key, then id, both
-// ascending; (k1, i1): a second buffer.
-__device__ void sort_picked(uint32_t* k0, uint32_t* i0, uint32_t* k1, uint32_t* i1, uint32_t n, uint32_t key_lo, const FinishLds& L)
+// ascending.  Returns false, and has moved nothing, where they crowd few of the sort's buckets.
+__device__ MAKO_RARE_CALL bool sort_picked(uint32_t* k0, uint32_t* i0, uint32_t n, uint32_t key_lo, const FinishLds& L)
 {
     assume_lds(L);
     FinishShared& sm = *L.sm;
@@ -1011,10 +1015,9 @@ __device__ void sort_picked(uint32_t* k0, uint32_t* i0, uint32_t* k1, uint32_t* 
     if (tid == 0)
         sm.flag = 0;
     __syncthreads(); // (everything has been read)
-    if (!lds_bucket_sort(key, id, n, key_lo, key_hi, k0, i0, L.sortk, sm)) {
-        __syncthreads();
-        sort_survivors(k0, i0, k1, i1, n, L); // (a crowded bucket; nothing has been moved)
-    }
+    const bool sorted = lds_bucket_sort(key, id, n, key_lo, key_hi, k0, i0, L.sortk, sm);
+    __syncthreads();
+    return sorted;
 }
 
 // Whole-row path: exact for every parameter combination.  One workgroup rebuilds the penalised
@@ -1174,7 +1177,16 @@ __device__ MAKO_RARE_CALL void general_row_from_weights(const mako_sample_desc& 
     uint32_t n0 = n_all;
     bool listed = n_all == V; // in the first buffers
     NthDone done = kNthNothing;
-    if ((nth_steps_for(V) || (wide_row(P) && nth_picks_for(V))) && nth_state(sc.plan + row, 0u)->seq + nth_state(sc.plan + row, 1u)->seq != 0u) { // uniform
+    if (!nth_steps_for(V) && wide_row(P) && nth_picks_for(V)) { // uniform
+        uint32_t from = 0;
+        const uint32_t picked = nth_pick(d, sc, row, 0u, 1u, n0, P.top_k, from, L.sortk, sm.bs);
+        if (picked != kNone)
+            done = NthDone{from, picked, nullptr, true};
+        __syncthreads();
+    }
+    if (done.picked) {
+        listed = false; // (in the second buffers)
+    } else if (nth_steps_for(V)) { // uniform
         const NthState s0 = *nth_state(sc.plan + row, 0u), s1 = *nth_state(sc.plan + row, 1u);
         const bool odd = s1.seq > s0.seq;
         const uint32_t buf = odd ? s1.buf : s0.buf;
