@@ -43,7 +43,7 @@ __global__ __launch_bounds__(kThreads) void finish_beside_kernel(mako_sample_des
 #ifdef MAKO_EMIT_BESIDE_SORT
 // grid = (as sort_kernel's, sort_rows + rows of workgroups for the groups)
 template <bool UNSORTED>
-__global__ __launch_bounds__(kThreads) void sort_beside_kernel(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices, uint32_t sort_rows)
+__global__ __launch_bounds__(kThreads) void sort_beside_kernel(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices, uint32_t sort_rows, uint32_t cus)
 {
     extern __shared__ __align__(16) unsigned long long s_dyn64[]; // (128-bit LDS operations need the alignment)
     __shared__ FinishShared sm;
@@ -62,26 +62,27 @@ __global__ __launch_bounds__(kThreads) void sort_beside_kernel(mako_sample_desc 
     const uint32_t blocks = (d_arg.n_vocab + kIndexBlock - 1u) / kIndexBlock;
     const uint32_t all = in_order * blocks;
     const uint32_t me = (blockIdx.y - sort_rows) * gridDim.x + blockIdx.x, wgs = (gridDim.y - sort_rows) * gridDim.x;
-    // (nth_steps.h's first step, as many workgroups a row as there are; the groups' workgroups are counted from the other end)
-    const uint32_t nth_rows = nth_steps_for(d_arg.n_vocab) ? general - in_order : 0u;
-    if (nth_rows) { // uniform
-        const uint32_t per_row = min(max(wgs / nth_rows, 1u), (d_arg.n_vocab + kNthChunk - 1u) / kNthChunk);
-        RankedRows rows;
-        for (uint32_t p = me; p < nth_rows * per_row; p += wgs) {
-            uint32_t row;
-            if (!rows.find(d_arg, p / per_row, [](const mako_sampling_params& P) { return nth_row(P); }, row))
-                break;
-            nth_step(d_arg, sc_val, row, p % per_row, per_row, 1u, s_dyn64, sm.bs);
-            __syncthreads();
-        }
-    }
     RankedRows rows;
     for (uint32_t p = wgs - 1u - me; p < all; p += wgs) {
         uint32_t row;
         if (!rows.find(d_arg, p / blocks, [](const mako_sampling_params& P) { return index_order_row(P); }, row))
-            return;
+            break;
         index_groups_block<1u>(d_arg, sc_val, row, p % blocks, reinterpret_cast<double*>(s_dyn64));
         __syncthreads();
+    }
+    // (nth_steps.h's steps, by as many workgroups a row as there are CUs for, since they wait for each other.  Behind the groups,
+    // whose workgroups are counted from the other end)
+    const uint32_t nth_rows = nth_steps_for(d_arg.n_vocab) ? general - in_order : 0u;
+    if (nth_rows) { // uniform
+        const uint32_t per_row = min(max(min(wgs, cus) / nth_rows, 1u), (d_arg.n_vocab + kNthChunk - 1u) / kNthChunk);
+        for (uint32_t p = me; p < nth_rows * per_row; p += wgs) {
+            RankedRows ranked;
+            uint32_t row;
+            if (!ranked.find(d_arg, p / per_row, [](const mako_sampling_params& P) { return nth_row(P); }, row))
+                break;
+            nth_steps_at_once(d_arg, sc_val, row, p % per_row, per_row, s_dyn64, sm.bs);
+            __syncthreads();
+        }
     }
 }
 #endif

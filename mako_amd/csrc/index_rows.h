@@ -247,7 +247,7 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
         plan->key_lo[piece] = last;
         if (piece == 0) {
             if (STEPS) {
-                nth_state(plan, 0u)->seq = nth_state(plan, 1u)->seq = plan->cap[kNthCursor] = 0u;
+                plan->cap[kNthCursor] = plan->cap[kNthMet] = plan->cap[kNthMade] = 0u;
                 *nth_first(plan) = first;
             }
             plan->flag = kIndexClaimed;
@@ -439,8 +439,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_num_sgpr(80))) void
 {
     extern __shared__ __align__(16) unsigned long long s_dyn64[];
     __shared__ BlockScratch s_bs;
-    if (blockIdx.x < d_arg.n_rows)
-        nth_step(d_arg, sc_val, blockIdx.x, blockIdx.y, gridDim.y, step, s_dyn64, s_bs);
+    if (blockIdx.x < d_arg.n_rows) {
+        const NthMadeOf made = nth_step(d_arg, sc_val, blockIdx.x, blockIdx.y, gridDim.y, step, s_dyn64, s_bs);
+        if (made != kNthNone && blockIdx.y == 0u && threadIdx.x == 0u)
+            sc_val.plan[blockIdx.x].cap[kNthMade] = step;
+    }
 }
 
 // grid = (1, rows).

@@ -5,14 +5,14 @@
 
 namespace mako {
 void launch_sort_beside(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices, uint32_t grid_rows, bool unsorted,
-                        uint32_t more)
+                        uint32_t more, uint32_t cus)
 {
     const uint32_t x = unsorted ? kSortItemsPerRow : kWorkers;
     const dim3 grid(x, grid_rows + (more + x - 1u) / x);
     if (unsorted)
-        hipLaunchKernelGGL(sort_beside_kernel<true>, grid, dim3(kThreads), kSortLds, st, d, sc, slices, grid_rows);
+        hipLaunchKernelGGL(sort_beside_kernel<true>, grid, dim3(kThreads), kSortLds, st, d, sc, slices, grid_rows, cus);
     else
-        hipLaunchKernelGGL(sort_beside_kernel<false>, grid, dim3(kThreads), kSortLds, st, d, sc, slices, grid_rows);
+        hipLaunchKernelGGL(sort_beside_kernel<false>, grid, dim3(kThreads), kSortLds, st, d, sc, slices, grid_rows, cus);
 }
 
 hipError_t init_beside_sort()

@@ -50,6 +50,6 @@ hipError_t init_beside_tail();
 void launch_finish_beside(bool aligned, int kh, bool unsorted, uint32_t wgs, uint32_t more, hipStream_t st, const mako_sample_desc& d,
                           const Scratch& sc, uint32_t slices);
 void launch_sort_beside(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices, uint32_t grid_rows, bool unsorted,
-                        uint32_t more);
+                        uint32_t more, uint32_t cus);
 void launch_tail_beside(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices, uint32_t tail_cap, bool unsorted);
 } // namespace mako

@@ -424,7 +424,7 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
         index_rows = n_index;
     }
     const bool any_nth = any_unordered && mako::nth_steps_for(d.n_vocab), any_bits = any_nth || (any_wide && mako::nth_picks_for(d.n_vocab));
-    // (their steps: a launch each, of about two workgroups per CU.  Beside other rows the sort's launch has the first.  A launch
+    // (their steps: a launch each, of about two workgroups per CU.  Beside other rows the sort's launch has them all.  A launch
     // costs 8 to 10 us and leaves 0.44 of a row: as many as bring the 64 rows' unluckiest near what a workgroup takes into its
     // registers.  64 rows of 129 280: 185 us with two, 172, 164, 162, 168 with six; of 40 000: 104 with two, 105, 110)
     const uint32_t nth_wgs = std::min(std::max(2u * ctx->cus / ((d.n_rows + 7u) & ~7u), 1u), (d.n_vocab + mako::kNthChunk - 1u) / mako::kNthChunk);
@@ -463,10 +463,8 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
         MAKO_LAUNCH(mako::launch_finish_beside(aligned, kh, unsorted, any_nucleus ? finish_wgs : 0u, for_weights, st, d, sc, slices));
         MAKO_MARK(2);
         if (any_nucleus || any_in_order || any_nth || !params_host)
-            MAKO_LAUNCH(mako::launch_sort_beside(st, d, sc, slices, any_nucleus ? nucleus_rows : 0u, unsorted, for_groups));
+            MAKO_LAUNCH(mako::launch_sort_beside(st, d, sc, slices, any_nucleus ? nucleus_rows : 0u, unsorted, for_groups, ctx->cus));
         MAKO_MARK(3);
-        for (uint32_t step = 2u; params_host && step <= nth_steps; ++step)
-            MAKO_LAUNCH(mako::launch_nth_step(st, d, sc, step, nth_wgs));
         MAKO_LAUNCH(mako::launch_tail_beside(st, d, sc, slices, nucleus_rows, unsorted));
     } else {
         if (only_index)

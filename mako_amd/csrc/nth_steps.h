@@ -16,6 +16,10 @@
 // index_weights_kernel counts the weights by value, and step 1 picks those from the bin that holds the k-th on, which the last
 // launch sorts.  (64 rows of 129 280, top_k 200 to 1 000: 183 us with the rounds, 75 so.)  Where the bin is too crowded, as on a
 // grid of few weights, the rounds are made.
+// Beside rows of other kinds, where a launch that no row needs would be paid for all the same, the sort's launch makes all steps:
+// a row's workgroups, as many as there are CUs for, meet after each (nth_steps_at_once()).  (Of 24 rows of 151 553 of all
+// kinds 205 us with the first step alone there, 140 so; top-k alone, 8 rows of 129 280: 157 and 121, 100 rows: 294 and 276.  A
+// batch of such rows alone keeps its launches: two workgroups share a CU there, and 64 rows take 162 us instead of 172.)
 // A step writes the list it makes beside the old one, with the next round's pivot already swapped to the front; its workgroups
 // take 4 096 entries of the new list at a time.  An entry that belongs left and lies in front of the cut stays where it is; a
 // hole's filler comes through LDS: the holes of 4 096 places in a row are filled from one stretch of the old list, from its
@@ -34,15 +38,17 @@ constexpr uint32_t kNthWords = kNthMaxVocab / 64u; // of a row's bits
 constexpr uint32_t kNthLds = kNthChunk * 8u + kNthWords * 12u + 64u;
 
 // Where a row stands: two records in turn in the row's plan (a step reads one and writes the other), in the words its workers
-// would use.  seq: steps made, 0: none yet.  len entries of key[buf] / idx[buf] are what is left of the list, `used` rounds
+// would use.  len entries of key[buf] / idx[buf] are what is left of the list, `used` rounds
 // behind them.  pre: kNthBits: the next round's pivot is at the front and its bits are in place; kNthPicked: the list is what a
 // wide row keeps, and more, in any order, and `used` the least bits(q) it may hold.
 struct alignas(4) NthState {
-    uint32_t seq, len, pre, used, buf;
+    uint32_t len, pre, used, buf;
 };
 constexpr uint32_t kNthBits = 1, kNthPicked = 2;
-constexpr uint32_t kNthCursor = 16; // the word of the plan's `cap` that counts what step 1 picks
-static_assert(2u * sizeof(NthState) <= kNthCursor * 4u && sizeof(BigPlan::cap) > kNthCursor * 4u, "");
+// (words of the plan's `cap`: what step 1 has picked; the row's workgroups that have made a step, all steps together (nth_meet());
+// the steps that all of them have made)
+constexpr uint32_t kNthCursor = 16, kNthMet = 17, kNthMade = 18;
+static_assert(2u * sizeof(NthState) <= kNthCursor * 4u && sizeof(BigPlan::cap) > kNthMade * 4u, "");
 // The first pivot of a row that is its own list, where it came from, and the key of its first entry.
 struct NthFirst {
     uint32_t pivot_key, pivot_id, from, first_key;
@@ -195,7 +201,9 @@ __device__ __forceinline__ uint32_t nth_pick(const mako_sample_desc& d, const Sc
 }
 
 // One step of row `row`, by workgroup w of W.  lds: kNthLds bytes, or what the row's bits, and the first step's picks, take of it.  All threads call.
-__device__ __forceinline__ void nth_step(const mako_sample_desc& d, const Scratch& sc, uint32_t row, uint32_t w, uint32_t W, uint32_t step,
+// Returns (the same to all of the row's workgroups) kNthNone if the row is none of these, kNthLast, or kNthMore if there is a next step.
+enum NthMadeOf : uint32_t { kNthNone, kNthLast, kNthMore };
+__device__ __forceinline__ NthMadeOf nth_step(const mako_sample_desc& d, const Scratch& sc, uint32_t row, uint32_t w, uint32_t W, uint32_t step,
                                          unsigned long long* lds_dyn, BlockScratch& bs)
 {
     typedef unsigned long long u64;
@@ -219,35 +227,33 @@ __device__ __forceinline__ void nth_step(const mako_sample_desc& d, const Scratc
     load_bits(usual, words_max);
     const uint32_t nth = P.top_k;
     if (!nth_row(P) || flag != kIndexClaimed) // uniform (a row of another kind; one whose token is forced)
-        return;
-    bool compact = false;
-    if (step == 1u) {
-        const uint32_t n0 = uniform_u32(__ockl_wfred_add_u32(lane < pieces ? counted : 0u));
-        compact = n0 != d.n_vocab;
-        // (a whole list that nothing is cut off stays as it is)
-        now = NthState{0u, d.n_vocab, compact || nth < n0 ? kNthBits : 0u, 0u, 0u};
-        if (wide_row(P)) { // uniform
-            uint32_t from = 0;
-            const uint32_t picked = nth_pick(d, sc, row, w, W, n0, nth, from, lds_dyn, bs);
-            if (picked != kNone) {
-                if (w == 0u && tid == 0u)
-                    *nth_state(plan, 1u) = NthState{1u, picked, kNthPicked, from, 1u};
-                return;
-            }
-            __syncthreads();
-        }
-    }
-    const uint32_t len = uniform_u32(now.len), from_buf = uniform_u32(now.buf), used = now.used;
+        return kNthNone;
     auto leave = [&](uint32_t n, uint32_t pre, uint32_t rounds, uint32_t in) {
         if (w == 0u && tid == 0u) {
             NthState* s = nth_state(plan, step & 1u);
-            s->seq = step;
             s->len = n;
             s->pre = pre;
             s->used = rounds;
             s->buf = in;
         }
     };
+    bool compact = false;
+    if (step == 1u) {
+        const uint32_t n0 = uniform_u32(__ockl_wfred_add_u32(lane < pieces ? counted : 0u));
+        compact = n0 != d.n_vocab;
+        // (a whole list that nothing is cut off stays as it is)
+        now = NthState{d.n_vocab, compact || nth < n0 ? kNthBits : 0u, 0u, 0u};
+        if (wide_row(P)) { // uniform
+            uint32_t from = 0;
+            const uint32_t picked = nth_pick(d, sc, row, w, W, n0, nth, from, lds_dyn, bs);
+            if (picked != kNone) {
+                leave(picked, kNthPicked, from, 1u);
+                return kNthLast;
+            }
+            __syncthreads();
+        }
+    }
+    const uint32_t len = uniform_u32(now.len), from_buf = uniform_u32(now.buf), used = now.used;
     const lds_ptr<u64> buf = as_lds(lds_dyn);                // [kNthChunk] fillers
     const lds_ptr<u64> bits = buf + kNthChunk;               // [words]
     const uint32_t words = (len + 63u) / 64u;
@@ -288,7 +294,7 @@ __device__ __forceinline__ void nth_step(const mako_sample_desc& d, const Scratc
                 ids[i] = i;
         }
         leave(len, step == 1u ? 0u : now.pre, used, from_buf);
-        return;
+        return kNthLast;
     }
     const bool goes_on = out_len > kNthUntil && nth < out_len; // uniform
     // the entry at i of the old list; a row that is its own list has no token ids, and its first entry has yet to change places
@@ -441,6 +447,77 @@ __device__ __forceinline__ void nth_step(const mako_sample_desc& d, const Scratc
         __syncthreads(); // (the fillers' buffer)
     }
     leave(out_len, goes_on ? kNthBits : 0u, used + (compact ? 0u : 1u), to_buf);
+    return goes_on ? kNthMore : kNthLast;
+}
+
+// The row's workgroups meet behind step `step` (without `wait` they only count).  Returns whether they go on with the next.  They
+// don't where one has waited `polls` times: the others may have to wait for a CU themselves, behind another stream's work, and
+// nothing may depend on that.  Whoever gives up says so and the rest follow, each at its next meeting at the latest; the row's
+// one workgroup in the last launch goes on from the last step that all W have made, whose list no later step has touched (two
+// lists, two records and two rows of bits, in turn).  All threads of all of the row's W workgroups call.
+__device__ __forceinline__ bool nth_meet(BigPlan* plan, uint32_t step, uint32_t W, bool wait, uint32_t polls, BlockScratch& bs)
+{
+    constexpr uint32_t kGivenUp = 0x80000000u;
+    const global_ptr<uint32_t> met = as_global(plan->cap + kNthMet);
+    if (wait) // uniform: the wave's stores have arrived where the fence finds them
+        asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
+    __syncthreads();
+    if (threadIdx.x == 0) {
+        if (wait)
+            __builtin_amdgcn_fence(__ATOMIC_RELEASE, "agent");
+        const uint32_t upto = W * step;
+        bool all = ((__hip_atomic_fetch_add(met, 1u, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) + 1u) & ~kGivenUp) == upto;
+        if (all) // (the last of them; of different steps' last, the later step counts)
+            __hip_atomic_fetch_max(as_global(plan->cap + kNthMade), step, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        for (uint32_t i = 0; wait && !all; ++i) {
+            const uint32_t v = __hip_atomic_load(met, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+            all = (v & ~kGivenUp) >= upto;
+            if (all || (v & kGivenUp))
+                break;
+            if (i >= polls) {
+                __hip_atomic_fetch_or(met, kGivenUp, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+                break;
+            }
+            __builtin_amdgcn_s_sleep(2);
+        }
+        if (wait)
+            __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent");
+        bs.bcast = all ? 1u : 0u;
+    }
+    if (!wait) // uniform
+        return false;
+    __syncthreads();
+    const bool go = bs.bcast != 0u;
+    __syncthreads();
+    return go;
+}
+
+// All of a row's steps by the same workgroups, in one launch that has other work besides (sort_beside_kernel).  All threads call.
+__device__ __forceinline__ void nth_steps_at_once(const mako_sample_desc& d, const Scratch& sc, uint32_t row, uint32_t w, uint32_t W,
+                                                  unsigned long long* lds_dyn, BlockScratch& bs)
+{
+    constexpr uint32_t kStepsMax = 12; // (of the 30 rounds and more before the depth limit)
+    // (140 us: twice what all steps of 24 rows of 151 553 take.  A checked build's even rows don't wait at all.)
+#ifdef MAKO_CHECKED
+    const uint32_t polls = (row & 1u) ? 400u : 0u;
+#else
+    constexpr uint32_t polls = 400u;
+#endif
+    // (the first step apart, which has no token ids to read: one workgroup takes 97 us for it, 117 otherwise)
+    NthMadeOf made = nth_step(d, sc, row, w, W, 1u, lds_dyn, bs);
+    if (made == kNthNone)
+        return;
+    if (made == kNthLast || W == 1u) { // uniform; all of them make the first
+        if (w == 0u && threadIdx.x == 0u)
+            sc.plan[row].cap[kNthMade] = 1u;
+        return;
+    }
+    for (uint32_t step = 1; nth_meet(sc.plan + row, step, W, made == kNthMore && step < kStepsMax, polls, bs);) {
+        // (one step's addresses are not kept for the next: the scalar registers do not suffice)
+        uint32_t r = uniform_u32(row), wr = uniform_u32(w), Wr = uniform_u32(W);
+        asm volatile("" : "+s"(r), "+s"(wr), "+s"(Wr));
+        made = nth_step(d, sc, r, wr, Wr, ++step, lds_dyn, bs);
+    }
 }
 
 } // namespace mako

@@ -1188,7 +1188,7 @@ __device__ MAKO_RARE_CALL void general_row_from_weights(const mako_sample_desc& 
         listed = false; // (in the second buffers)
     } else if (nth_steps_for(V)) { // uniform
         const NthState s0 = *nth_state(sc.plan + row, 0u), s1 = *nth_state(sc.plan + row, 1u);
-        const bool odd = s1.seq > s0.seq;
+        const bool odd = (sc.plan[row].cap[kNthMade] & 1u) != 0u;
         const uint32_t buf = odd ? s1.buf : s0.buf;
         const uint32_t pre = odd ? s1.pre : s0.pre;
         done = NthDone{odd ? s1.used : s0.used, odd ? s1.len : s0.len, pre == kNthBits ? nth_bits(sc, row, buf) : nullptr, pre == kNthPicked};

@@ -115,3 +115,31 @@ def test_wide_top_k_before_a_top_p(vocab, sigma):
             assert_parity(ctx, w, cap=300, hinted=hinted)
     finally:
         ctx.close()
+
+
+# (beside other rows a row's workgroups make all steps in one launch and wait for each other in between; in the checked build
+# those of every other row don't, and leave the rest to the last launch)
+@pytest.mark.parametrize("checked", [False, True])
+@pytest.mark.parametrize("vocab, copies", [(32769, 1), (32769, 8), (40000, 34), (151553, 1)])
+def test_steps_in_one_launch(vocab, copies, checked):
+    ctx = api.SamplerContext(max_rows=9 * copies, max_vocab=vocab, lib_path=api.CHECKED_LIB_PATH if checked else None)
+    try:
+        for gaps in ("none", "mask"):
+            w = _batch(vocab, gaps, 5, False)
+            if copies > 1:  # (the same rows again; many have one workgroup each)
+                w = {k: v if k == "name" else np.concatenate([v] * copies) for k, v in w.items()}
+            one = oracle_rows({k: v if k == "name" else v[:9] for k, v in w.items()}, cap=64)
+            if checked:
+                ctx.failed_checks()
+            for _ in range(3):
+                g = gpu_rows(ctx, w, cap=64, hinted=False)
+                for r in range(9 * copies):
+                    t, tr = one[r % 9]
+                    n = min(64, tr["n_cand"])
+                    assert (g["tokens"][r], g["n_cand"][r]) == (t, tr["n_cand"]), (r, gaps)
+                    assert np.array_equal(g["cand_idx"][r, :n], tr["cand_idx"][:n]), (r, gaps)
+                    assert np.float32(g["total"][r]).view(np.uint32) == np.float32(tr["total"]).view(np.uint32), (r, gaps)
+            if checked:
+                assert ctx.failed_checks() == 1 << 31
+    finally:
+        ctx.close()
