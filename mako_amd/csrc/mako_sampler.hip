@@ -11,6 +11,7 @@
 #include <mutex>
 #include <new>
 #include <string>
+#include <type_traits>
 
 #include "../../include/mako_sampler.h"
 #include "host_stage.h"
@@ -603,12 +604,35 @@ int mako_sampler_sample_host(mako_sampler_ctx* ctx, const float* logits, int64_t
     }
     d.logits = reinterpret_cast<const float*>(ctx->st_dev + stage.put_rows(logits, (size_t)logits_stride * 4, (size_t)n_vocab * 4, (size_t)stride * 4, n_rows));
     d.logits_stride = stride;
-    if (const int e = stage.send())
+    // What would be a single copy (a MiB at most) is left where it is if no row's logits are read a second time: the kernels
+    // then read it over the bus, 14 us for a row of 129 280 logits in place of a copy's 17 and 7 from device memory.  (One
+    // top-k row: 48.1 us with the copy, 44.9 so; of 8 000 logits 33.4 and 29.9; seven rows of 32 000 63.0 and 58.2.  A nucleus
+    // row, whose logits the second pass reads again: 72.7 and 79.4.)
+    bool once = ctx->st_pinned && stage.sent == 0 && stage.status == 0;
+    for (uint32_t r = 0; once && r < n_rows; ++r) {
+        const mako::RowClass c = mako::classify(params[r]);
+        once = c == mako::kGreedy || c == mako::kTopK;
+    }
+    if (once) {
+        auto in_place = [&](auto& p) {
+            if (p)
+                p = reinterpret_cast<std::remove_reference_t<decltype(p)>>(ctx->st_host + (reinterpret_cast<uintptr_t>(p) - reinterpret_cast<uintptr_t>(ctx->st_dev)));
+        };
+        in_place(d.params);
+        in_place(d.u);
+        in_place(d.mask);
+        in_place(d.hist_tokens);
+        in_place(d.hist_counts);
+        in_place(d.hist_len);
+        in_place(d.draft);
+        in_place(d.u2);
+        in_place(d.logits);
+    } else if (const int e = stage.send())
         return fail(ctx, MAKO_ERR_HIP, std::string("sampler: copying a call's inputs: ") + (e > 0 ? hipGetErrorString((hipError_t)e) : "they do not fit"));
     d.out_tokens = reinterpret_cast<int32_t*>(out);
     // (the caller's parameters are in host memory: the call looks at them and leaves out what no row needs)
     const int rc = mako_sampler_sample_batch_hinted(ctx, &d, params, nullptr);
-    MAKO_HIP(ctx, hipStreamSynchronize(nullptr)); // (also behind a failed launch: the copies read the pinned memory)
+    MAKO_HIP(ctx, hipStreamSynchronize(nullptr)); // (also behind a failed launch: the copies, or the kernels, read the pinned memory)
     if (rc != MAKO_OK)
         return rc;
     if (ctx->st_pinned) {

@@ -51,3 +51,30 @@ def test_same_as_the_device_call(rows, vocab, apart, verify, lib):
             whole[:] = np.roll(whole, 1, axis=1)
     finally:
         ctx.close()
+
+
+# (top-k and greedy rows whose inputs would be one copy are read where they were put together: also where the candidates don't
+# settle a row, whose logits are then read again, and on either side of a MiB)
+@pytest.mark.parametrize("rows,vocab", [(1, 8), (1, 129280), (4, 32000), (1, 261800), (1, 262100), (1, 262200)])
+def test_inputs_left_in_place(rows, vocab):
+    rng = np.random.Generator(np.random.PCG64([rows, vocab]))
+    tokens = np.full(rows, -1, np.int32)
+    ctx = api.SamplerContext(max_rows=rows, max_vocab=vocab)
+
+    def at(a):
+        return ctypes.c_void_p(a.ctypes.data)
+
+    try:
+        for top_k, top_p, levels in ((40, 0.95, 0), (40, 0.95, 1), (128, 0.999, 3), (0, 0.9, 0)):
+            x = (rng.standard_normal((rows, vocab)) * 3.0).astype(np.float32)
+            if levels:
+                x = np.floor(x.clip(0, levels - 0.5))
+            p = api.make_params(rows, 0.8, top_k, top_p)
+            p["temperature"][1:2] = 0.0
+            u = rng.random(rows).astype(np.float32)
+            rc = ctx.lib.mako_sampler_sample_host(ctypes.c_void_p(ctx.ptr), at(x), vocab, rows, vocab, at(p), at(u), None, 0, None, None, 0, None, None,
+                                                  None, None, at(tokens))
+            assert rc == api.MAKO_OK, ctx.last_error()
+            assert np.array_equal(tokens, gpu_rows(ctx, dict(logits=x, params=p, u=u))["tokens"]), (top_k, levels)
+    finally:
+        ctx.close()
