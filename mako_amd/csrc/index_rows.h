@@ -16,6 +16,8 @@
 // `r < q` is never true for it.  The list ends behind the row's last candidate, which is where the reference's walk
 // ends when it runs off its list.  Verification works on the same list: the draft's weight is entry `draft`, and a
 // rejected draft is redrawn with that entry taken as 0.0f (sorted_tail's UNORDERED instance).
+// A row with up to 256 candidates (a min-p on a peaked row, a grammar's mask) needs no records: each piece leaves its candidates'
+// token ids in order, and few_candidates_row() finishes the row from those.
 // The other rows of the whole-row class (top-k without top-p, top-k beyond the candidate lists) only get their weights
 // here (into the array general_row_from_weights() starts from), the first rounds of their nth_element (nth_steps.h), and one
 // workgroup each in the last launch for the rest of the whole-row path.
@@ -30,6 +32,7 @@ namespace mako {
 
 constexpr uint32_t kIndexBlock = 4096;                   // entries whose fp64 sum index_weights_kernel leaves as one number
 constexpr uint32_t kIndexMaxVocab = kMaxGroups * kGroup; // the group records of a row
+constexpr uint32_t kIndexFewMax = kGroup;                // candidates that a row may have to be finished from a list of them
 static_assert(kIndexMaxVocab / kSliceMax <= kWorkers && kIndexMaxVocab / kIndexBlock <= kMaxSlices && kIndexMaxVocab / kIndexBlock <= (uint32_t)kWave &&
                   kSliceMax == 4u * kIndexBlock && kIndexBlock == (uint32_t)kWaves * kGroup,
               "a piece's count and last candidate travel in the plan's per-worker words, the blocks' sums in the row's part_sum, a lane each");
@@ -146,7 +149,7 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
             bins[tid] = 0u;
         lds_barrier();
     }
-    uint32_t cnt = 0, last = 0;
+    uint32_t is_cand = 0; // bit j: the thread's logit j is a candidate
     double bsum[4];
 #pragma unroll
     for (uint32_t b = 0; b < 4; ++b) {
@@ -161,8 +164,7 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
                 const float q = weight_of(wv[4u * b + c], m, inv_t, sm.tab);
                 const bool ok = at < hi && q >= floor_q && q > 0.0f; // src/gen/sampler.cpp:34-35
                 k[c] = ok ? __float_as_uint(q) : 0u;
-                cnt += ok ? 1u : 0u;
-                last = ok ? max(last, at + 1u) : last;
+                is_cand |= (ok ? 1u : 0u) << (4u * b + c);
                 bsum[b] += ok ? (double)q : 0.0;
                 if (wide && ok)
                     atomicAdd(&bins[nth_bin(k[c])], 1u);
@@ -219,8 +221,8 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
         if (lane_id() == 0)
             wsum[b * kWaves + wave_id()] = s;
     }
-    cnt = __ockl_wfred_add_u32(cnt);
-    last = __ockl_wfred_max_u32(last);
+    uint32_t cnt = __ockl_wfred_add_u32((uint32_t)__popc(is_cand));
+    uint32_t last = __ockl_wfred_max_u32(is_cand ? elem_index(lo, tid, 31u - (uint32_t)__clz((int)is_cand)) + 1u : 0u);
     if (lane_id() == 0) {
         wcnt[wave_id()] = cnt;
         wcnt[kWaves + wave_id()] = last;
@@ -228,6 +230,38 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
     __syncthreads();
     if (wide && tid < kNthBins)
         nth_hist(sc, row, piece)[tid] = bins[tid];
+    if (in_order) { // uniform
+        // few candidates: their token ids in order (in the piece's part of idx[1]; few_candidates_row())
+        const uint32_t all = __ockl_wfred_add_u32((uint32_t)lane_id() < (uint32_t)kWaves ? wcnt[min((uint32_t)lane_id(), (uint32_t)kWaves - 1u)] : 0u);
+        if (all <= kIndexFewMax) { // uniform
+            uint32_t* const in_front = wcnt + 2 * kWaves; // [4][kWaves] of the piece's b-th 4 096, by wave
+            uint32_t mine[2], upto[2]; // (two counts a word)
+#pragma unroll
+            for (uint32_t h = 0; h < 2; ++h) {
+                mine[h] = (uint32_t)__popc((is_cand >> (8u * h)) & 15u) | ((uint32_t)__popc((is_cand >> (8u * h + 4u)) & 15u) << 16);
+                upto[h] = __ockl_wfscan_add_u32(mine[h], true);
+                if (lane_id() == kWave - 1) {
+                    in_front[2u * h * kWaves + wave_id()] = upto[h] & 0xffffu;
+                    in_front[(2u * h + 1u) * kWaves + wave_id()] = upto[h] >> 16;
+                }
+            }
+            lds_barrier();
+            static_assert(4 * kWaves == kWave, "a count per lane");
+            const uint32_t n = in_front[lane_id()], before = __ockl_wfscan_add_u32(n, true) - n;
+            uint32_t* ids = sc.idx[1] + (size_t)row * sc.vpad + lo;
+#pragma unroll
+            for (uint32_t b = 0; b < 4; ++b) {
+                uint32_t at = (uint32_t)__builtin_amdgcn_readlane((int)before, (int)uniform_u32(b * (uint32_t)kWaves + wave_id())) +
+                              (((upto[b / 2u] - mine[b / 2u]) >> (16u * (b & 1u))) & 0xffffu);
+#pragma unroll
+                for (uint32_t c = 0; c < 4; ++c)
+                    if ((is_cand >> (4u * b + c)) & 1u) {
+                        MAKO_CHECK(sc, kCheckCompact, at < all && (uint64_t)lo + at < sc.vpad);
+                        ids[at++] = elem_index(lo, tid, 4u * b + c);
+                    }
+            }
+        }
+    }
     if (tid < 4u && lo + tid * kIndexBlock < hi) { // (a sum per 4 096 entries: index_groups_kernel's workgroups may be that small)
         double s = 0.0;
         for (int w = 0; w < kWaves; ++w)
@@ -289,9 +323,9 @@ __device__ __forceinline__ void index_groups_block(const mako_sample_desc& d_arg
         plan->total64 = total64;
         plan->thr = n_cand;
         const bool gaps_matter = n_cand < n_list && d_arg.out_cand_idx && d_arg.out_cand_q && d_arg.cand_cap;
-        plan->flag = n_cand == 0u ? kIndexEmpty : (gaps_matter ? kIndexWhole : kIndexReady);
+        plan->flag = n_cand == 0u ? kIndexEmpty : (gaps_matter ? kIndexWhole : (n_cand <= kIndexFewMax ? kIndexFew : kIndexReady));
     }
-    if (n_cand == 0u || p * kSpan >= n_list) // uniform
+    if (n_cand <= kIndexFewMax || p * kSpan >= n_list) // uniform
         return;
     const uint32_t off = p * kSpan, cnt = min(kSpan, n_list - off);
     const uint32_t groups = (cnt + kGroup - 1u) / kGroup; // <= 16 GPW <= 64
@@ -332,6 +366,36 @@ __device__ __forceinline__ void index_groups_block(const mako_sample_desc& d_arg
     }
 }
 
+// A row with few candidates, n_cand of them (a min-p leaves a peaked row a few dozen): the pieces' lists one after the other are
+// the row's, in token order, which one wave adds up and walks.  All threads call.
+// (64 rows of 129 280 with a min-p of 0.02 to 0.1: 68 us over the group records of every logit, 51 so; one row 31
+// and 25; 400 rows 235 and 183; 24 of 151 553 without the caller's copy of the parameters 79 and 70.)
+__device__ MAKO_RARE_CALL void few_candidates_row(const mako_sample_desc& d, const Scratch& sc, uint32_t row, const mako_sampling_params& P, uint32_t n_cand,
+                                                  double total64, const FinishLds& L)
+{
+    assume_lds(L);
+    const uint32_t tid = threadIdx.x, lane = lane_id(), pieces = (d.n_vocab + kSliceMax - 1u) / kSliceMax;
+    const uint32_t upto = __ockl_wfscan_add_u32(lane < pieces ? sc.plan[row].cursor[min(lane, kWorkers - 1u)] : 0u, true);
+    uint32_t piece = 0, before = 0;
+    for (uint32_t k = 0; k < pieces; ++k) { // uniform
+        const uint32_t to = (uint32_t)__builtin_amdgcn_readlane((int)upto, (int)k);
+        if (tid >= to) {
+            piece = k + 1u;
+            before = to;
+        }
+    }
+    const size_t at = (size_t)row * sc.vpad;
+    uint32_t* kf = sc.key[1] + at;
+    uint32_t* jf = sc.idx[0] + at;
+    if (tid < n_cand) { // (at most kIndexFewMax)
+        const uint32_t id = min(sc.idx[1][at + min(piece, pieces - 1u) * kSliceMax + (tid - before)], d.n_vocab - 1u);
+        kf[tid] = sc.key[0][at + id];
+        jf[tid] = id;
+    }
+    __syncthreads();
+    sorted_tail<false, true>(d, row, P, kf, jf, n_cand, true, total64, MAKO_PATH_INDEXED, L);
+}
+
 // What these kernels have left of a row of theirs (flag: of its plan, which is zero again behind this), by one workgroup: the
 // rest of the whole-row path, or the total and the draw.  All threads call; sm.tab must hold the exp2 table.  ALL_KINDS: rows
 // that are not in token order are among them (their code costs the others' kernel scratch memory, 0.7 of 78 us on 64 rows).
@@ -361,6 +425,10 @@ __device__ __forceinline__ void finish_index_row_here(const mako_sample_desc& d,
     }
     if (flag == kIndexEmpty) {
         fallback_row(d, row, argidx);
+        return;
+    }
+    if (flag == kIndexFew) {
+        few_candidates_row(d, sc, row, P, n_cand, total64, L);
         return;
     }
     if (flag == kIndexReady) {

@@ -259,6 +259,7 @@ constexpr uint32_t kIndexClaimed = 6; // index_weights_kernel has the row: the k
 constexpr uint32_t kIndexReady = 7;   // the group records are in place
 constexpr uint32_t kIndexWhole = 8;   // the whole-row path is wanted (candidates to be written out from a list with gaps)
 constexpr uint32_t kIndexEmpty = 9;   // no candidate survived
+constexpr uint32_t kIndexFew = 10;    // so few did that they are a list of their own
 
 __device__ __forceinline__ bool penalties_neutral(const mako_sampling_params& p)
 {
