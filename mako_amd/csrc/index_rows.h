@@ -366,16 +366,16 @@ __device__ __forceinline__ void index_groups_block(const mako_sample_desc& d_arg
     }
 }
 
-// A row with few candidates, n_cand of them (a min-p leaves a peaked row a few dozen): the pieces' lists one after the other are
+// A row with few candidates (a min-p leaves a peaked row a few dozen): the pieces' lists one after the other are
 // the row's, in token order, which one wave adds up and walks.  All threads call.
-// (64 rows of 129 280 with a min-p of 0.02 to 0.1: 68 us over the group records of every logit, 51 so; one row 31
+// (64 rows of 129 280 with a min-p of 0.02 to 0.1: 68 us over the group records of every logit, 54 so; one row 31
 // and 25; 400 rows 235 and 183; 24 of 151 553 without the caller's copy of the parameters 79 and 70.)
-__device__ MAKO_RARE_CALL void few_candidates_row(const mako_sample_desc& d, const Scratch& sc, uint32_t row, const mako_sampling_params& P, uint32_t n_cand,
-                                                  double total64, const FinishLds& L)
+__device__ MAKO_RARE_CALL void few_candidates_row(const mako_sample_desc& d, const Scratch& sc, uint32_t row, const mako_sampling_params& P, const FinishLds& L)
 {
     assume_lds(L);
     const uint32_t tid = threadIdx.x, lane = lane_id(), pieces = (d.n_vocab + kSliceMax - 1u) / kSliceMax;
     const uint32_t upto = __ockl_wfscan_add_u32(lane < pieces ? sc.plan[row].cursor[min(lane, kWorkers - 1u)] : 0u, true);
+    const uint32_t n_cand = min((uint32_t)__builtin_amdgcn_readlane((int)upto, kWave - 1), kIndexFewMax);
     uint32_t piece = 0, before = 0;
     for (uint32_t k = 0; k < pieces; ++k) { // uniform
         const uint32_t to = (uint32_t)__builtin_amdgcn_readlane((int)upto, (int)k);
@@ -387,20 +387,23 @@ __device__ MAKO_RARE_CALL void few_candidates_row(const mako_sample_desc& d, con
     const size_t at = (size_t)row * sc.vpad;
     uint32_t* kf = sc.key[1] + at;
     uint32_t* jf = sc.idx[0] + at;
-    if (tid < n_cand) { // (at most kIndexFewMax)
+    if (tid < n_cand) {
         const uint32_t id = min(sc.idx[1][at + min(piece, pieces - 1u) * kSliceMax + (tid - before)], d.n_vocab - 1u);
         kf[tid] = sc.key[0][at + id];
         jf[tid] = id;
     }
     __syncthreads();
-    sorted_tail<false, true>(d, row, P, kf, jf, n_cand, true, total64, MAKO_PATH_INDEXED, L);
+    // (the instance that general_row() calls as well: tail_beside_kernel has the one for short lists inline, for its top-k rows, and a
+    // second caller would make it a call there, with scratch memory: 510 such rows 16.6 us, 45 so)
+    sorted_tail(d, row, P, kf, jf, n_cand, true, sc.plan[row].total64, MAKO_PATH_INDEXED, L);
 }
 
 // What these kernels have left of a row of theirs (flag: of its plan, which is zero again behind this), by one workgroup: the
 // rest of the whole-row path, or the total and the draw.  All threads call; sm.tab must hold the exp2 table.  ALL_KINDS: rows
 // that are not in token order are among them (their code costs the others' kernel scratch memory, 0.7 of 78 us on 64 rows).
+// Returns whether the row is one for few_candidates_row(), which the caller calls (from here it would be deeper in the stack).
 template <bool ALL_KINDS = true>
-__device__ __forceinline__ void finish_index_row_here(const mako_sample_desc& d, const Scratch& sc, const mako_sampling_params& P, uint32_t row,
+__device__ __forceinline__ bool finish_index_row_here(const mako_sample_desc& d, const Scratch& sc, const mako_sampling_params& P, uint32_t row,
                                                       const FinishLds& L)
 {
     const uint32_t tid = threadIdx.x;
@@ -419,18 +422,18 @@ __device__ __forceinline__ void finish_index_row_here(const mako_sample_desc& d,
     if (!index_order_row(P)) {
         // the whole-row path from the weights index_weights_kernel left (the group records' kernel has not touched the row)
         if constexpr (ALL_KINDS)
-            if (flag == kIndexClaimed)
-                general_row_from_weights<0>(d, sc, row, P, m, argidx, uniform_u32(counted), L);
-        return;
+            if (flag == kIndexClaimed && !general_row_from_weights<0>(d, sc, row, P, m, argidx, uniform_u32(counted), L)) { // uniform
+                __syncthreads();
+                general_row<0>(d, sc, row, P, m, argidx, L);
+            }
+        return false;
     }
     if (flag == kIndexEmpty) {
         fallback_row(d, row, argidx);
-        return;
+        return false;
     }
-    if (flag == kIndexFew) {
-        few_candidates_row(d, sc, row, P, n_cand, total64, L);
-        return;
-    }
+    if (flag == kIndexFew)
+        return true;
     if (flag == kIndexReady) {
         const uint32_t* kf = sc.key[0] + (size_t)row * sc.vpad;
         // (entry i of the list is token i: no array of token ids)
@@ -440,17 +443,23 @@ __device__ __forceinline__ void finish_index_row_here(const mako_sample_desc& d,
             // (the list's length counts the gaps; the candidates are what the reference counts)
             if (tid == 0 && d.out_n_cand)
                 d.out_n_cand[row] = n_cand;
-            return;
+            return false;
         }
     }
     if (flag == kIndexReady || flag == kIndexWhole)
         general_row<0>(d, sc, row, P, m, argidx, L);
+    return false;
 }
-__device__ MAKO_RARE_CALL void finish_index_row(const mako_sample_desc& d, const Scratch& sc, const mako_sampling_params& P, uint32_t row,
+__device__ MAKO_RARE_CALL bool finish_index_row_call(const mako_sample_desc& d, const Scratch& sc, const mako_sampling_params& P, uint32_t row,
                                                 const FinishLds& L)
 {
     assume_lds(L);
-    finish_index_row_here(d, sc, P, row, L);
+    return finish_index_row_here(d, sc, P, row, L);
+}
+__device__ __forceinline__ void finish_index_row(const mako_sample_desc& d, const Scratch& sc, const mako_sampling_params& P, uint32_t row, const FinishLds& L)
+{
+    if (finish_index_row_call(d, sc, P, row, L)) // uniform
+        few_candidates_row(d, sc, row, P, L);
 }
 
 // Rows of the kind that `want` says (kGeneral, or those of them that are in token order) by their rank among them, for ranks that
@@ -529,7 +538,8 @@ __global__ __launch_bounds__(kThreads) void index_tail_kernel(mako_sample_desc d
         sm.tab[threadIdx.x] = k_exp2_tab[threadIdx.x];
     stage_args(d_arg, sc_val, row, s_args);
     const FinishLds views = finish_lds_views(sm, s_dyn64);
-    finish_index_row_here<ALL_KINDS>(s_args.d, s_args.sc, s_args.P, row, views);
+    if (finish_index_row_here<ALL_KINDS>(s_args.d, s_args.sc, s_args.P, row, views)) // uniform
+        few_candidates_row(s_args.d, s_args.sc, row, s_args.P, views);
 }
 #endif // MAKO_EMIT_INDEX_KERNELS
 

@@ -1162,8 +1162,9 @@ __device__ MAKO_RARE_CALL void general_row(const mako_sample_desc& d, const Scra
 // When that kernel found every logit a candidate (no mask, no floor, no underflow: the usual row) it has left the token ids as
 // well, i at i in idx[0] of the row: the list is there, nothing to compact.  Rows long enough for nth_steps.h have their list
 // where the last step has left it.
+// Returns false where a cut is too close to call: general_row() has to look at the row again, from the logits on.
 template <int SITE>
-__device__ MAKO_RARE_CALL void general_row_from_weights(const mako_sample_desc& d, const Scratch& sc, uint32_t row,
+__device__ MAKO_RARE_CALL bool general_row_from_weights(const mako_sample_desc& d, const Scratch& sc, uint32_t row,
                                                         const mako_sampling_params& P, float m, uint32_t argidx, uint32_t n_all,
                                                         const FinishLds& L)
 {
@@ -1260,13 +1261,10 @@ __device__ MAKO_RARE_CALL void general_row_from_weights(const mako_sample_desc& 
     }
     if (n0 == 0) {
         fallback_row(d, row, argidx);
-        return;
+        return true;
     }
-    if (!sort_truncate_draw<SITE == 0>(d, row, P, listed ? k_from : k_to, listed ? i_from : i_to, listed ? k_to : k_from, listed ? i_to : i_from,
-                                       nullptr, n0, false, 0.0, MAKO_PATH_GENERAL, L, done)) {
-        __syncthreads();
-        general_row<SITE>(d, sc, row, P, m, argidx, L); // (a cut too close to call: from the logits again)
-    }
+    return sort_truncate_draw<SITE == 0>(d, row, P, listed ? k_from : k_to, listed ? i_from : i_to, listed ? k_to : k_from, listed ? i_to : i_from,
+                                       nullptr, n0, false, 0.0, MAKO_PATH_GENERAL, L, done);
 }
 
 } // namespace mako
