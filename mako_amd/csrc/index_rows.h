@@ -292,7 +292,7 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
     }
 }
 
-// Workgroup p of a row leaves the records of the groups of its 4096 GPW entries.  Wave w
+// Workgroup p of a row leaves the records of the groups of its 4096 GPW entries, or none if few_candidates_row() does without.  Wave w
 // takes the groups w, w + 16, ... (GPW of them): their entries in one trip to memory, their fp64 sums to LDS, and once
 // every wave has the sums before each group, the increments from the entries it still holds.  (GPW = 4 where there are rows
 // enough to fill the chip, 1 on a small batch, which waits for one workgroup's chain of dependent steps.)

@@ -454,7 +454,7 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
     MAKO_LAUNCH(mako::launch_scan(aligned, kh, d.close_token != nullptr, grid, lds, st, d, sc, slice_len, std::min(ctx->cus, mako::kCountGeneral - 1u) | (beside ? mako::kCountGeneral : 0u) | ((finish_wgs / 8u) << 16)));
     MAKO_MARK(1);
     // top_k == 0 rows: planned and handed out by the second pass, sorted, cut and drawn from; the stages talk through
-    // kernel boundaries (device-wide fences inside a kernel cost far more on this chip).  A batch without such rows
+    // kernel boundaries (device-wide fences cost far more on this chip where hundreds of workgroups make one).  A batch without such rows
     // (and without rows for the whole-row path) ends with plan_kernel instead.
     if (beside) {
         // (workgroups for the rows of index_rows.h: a round of them at most, each takes several pieces in turn)
