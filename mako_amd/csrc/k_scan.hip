@@ -4,20 +4,22 @@
 
 namespace mako {
 namespace {
-template <bool ALIGNED, int KH, bool ABOVE>
+template <bool ALIGNED, int KH, bool ABOVE, bool SHORT>
 void launch_one(dim3 grid, size_t lds, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slice_len,
                 uint32_t cus)
 {
-    hipLaunchKernelGGL((scan_kernel<ALIGNED, KH, ABOVE>), grid, dim3(kThreads), lds, st, d, sc, slice_len, cus);
+    hipLaunchKernelGGL((scan_kernel<ALIGNED, KH, ABOVE, SHORT>), grid, dim3(kThreads), lds, st, d, sc, slice_len, cus);
 }
 template <bool ALIGNED, int KH>
 void launch_kh(bool above, dim3 grid, size_t lds, hipStream_t st, const mako_sample_desc& d, const Scratch& sc,
                uint32_t slice_len, uint32_t cus)
 {
-    if (above)
-        launch_one<ALIGNED, KH, true>(grid, lds, st, d, sc, slice_len, cus);
+    if (short_slice(slice_len)) // (a row of one slice)
+        launch_one<ALIGNED, KH, true, true>(grid, lds, st, d, sc, slice_len, cus);
+    else if (above)
+        launch_one<ALIGNED, KH, true, false>(grid, lds, st, d, sc, slice_len, cus);
     else
-        launch_one<ALIGNED, KH, false>(grid, lds, st, d, sc, slice_len, cus);
+        launch_one<ALIGNED, KH, false, false>(grid, lds, st, d, sc, slice_len, cus);
 }
 template <bool ALIGNED>
 void launch_aligned(int kh, bool above, dim3 grid, size_t lds, hipStream_t st, const mako_sample_desc& d, const Scratch& sc,
@@ -48,7 +50,10 @@ hipError_t init_scan_kernels()
                              (const void*)scan_kernel<true, 8, false>, (const void*)scan_kernel<false, 8, false>,
                              (const void*)scan_kernel<true, 0, true>,  (const void*)scan_kernel<false, 0, true>,
                              (const void*)scan_kernel<true, 2, true>,  (const void*)scan_kernel<false, 2, true>,
-                             (const void*)scan_kernel<true, 8, true>,  (const void*)scan_kernel<false, 8, true>};
+                             (const void*)scan_kernel<true, 8, true>,  (const void*)scan_kernel<false, 8, true>,
+                             (const void*)scan_kernel<true, 0, true, true>, (const void*)scan_kernel<false, 0, true, true>,
+                             (const void*)scan_kernel<true, 2, true, true>, (const void*)scan_kernel<false, 2, true, true>,
+                             (const void*)scan_kernel<true, 8, true, true>, (const void*)scan_kernel<false, 8, true, true>};
     for (const void* k : kernels) {
         const hipError_t e = hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kDynLds);
         if (e != hipSuccess)

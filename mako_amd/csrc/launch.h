@@ -17,7 +17,7 @@ hipError_t init_plan_alone();
 hipError_t init_sort_kernels();
 hipError_t init_tail_kernels();
 
-// scan_kernel<aligned, kh, above>, grid = (slices, rows), `lds` bytes of dynamic LDS
+// scan_kernel<aligned, kh, above, short_slice(slice_len)>, grid = (slices, rows), `lds` bytes of dynamic LDS
 // (`sc`: the HOST copy of the context's record; the kernels take it by value, so that their first loads need no
 // trip to memory for the record itself)
 void launch_scan(bool aligned, int kh, bool above, dim3 grid, size_t lds, hipStream_t st, const mako_sample_desc& d,
