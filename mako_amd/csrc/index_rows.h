@@ -16,7 +16,7 @@
 // `r < q` is never true for it.  The list ends behind the row's last candidate, which is where the reference's walk
 // ends when it runs off its list.  Verification works on the same list: the draft's weight is entry `draft`, and a
 // rejected draft is redrawn with that entry taken as 0.0f (sorted_tail's UNORDERED instance).
-// A row with up to 256 candidates (a min-p on a peaked row, a grammar's mask) needs no records: each piece leaves its candidates'
+// A row of some length with up to 256 candidates (a min-p on a peaked row, a grammar's mask) needs no records: each piece leaves its candidates'
 // token ids in order, and few_candidates_row() finishes the row from those.
 // The other rows of the whole-row class (top-k without top-p, top-k beyond the candidate lists) only get their weights
 // here (into the array general_row_from_weights() starts from), the first rounds of their nth_element (nth_steps.h), and one
@@ -33,6 +33,13 @@ namespace mako {
 constexpr uint32_t kIndexBlock = 4096;                   // entries whose fp64 sum index_weights_kernel leaves as one number
 constexpr uint32_t kIndexMaxVocab = kMaxGroups * kGroup; // the group records of a row
 constexpr uint32_t kIndexFewMax = kGroup;                // candidates that a row may have to be finished from a list of them
+// ... and how long it has to be for that.  (30 rows with a min-p: of 172 logits 23.9 us from a list of the candidates and 21.5
+// from the records, of 359 24.6 and 23.4, of 511 24.6 and 24.3, of 700 24.1 and 24.8, of 1 500 24.2 and 29.5.)
+constexpr uint32_t kIndexFewFrom = 640;
+__device__ __forceinline__ bool index_few(uint32_t n_cand, uint32_t n_vocab)
+{
+    return n_cand <= kIndexFewMax && n_vocab > kIndexFewFrom;
+}
 static_assert(kIndexMaxVocab / kSliceMax <= kWorkers && kIndexMaxVocab / kIndexBlock <= kMaxSlices && kIndexMaxVocab / kIndexBlock <= (uint32_t)kWave &&
                   kSliceMax == 4u * kIndexBlock && kIndexBlock == (uint32_t)kWaves * kGroup,
               "a piece's count and last candidate travel in the plan's per-worker words, the blocks' sums in the row's part_sum, a lane each");
@@ -233,7 +240,7 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
     if (in_order) { // uniform
         // few candidates: their token ids in order (in the piece's part of idx[1]; few_candidates_row())
         const uint32_t all = __ockl_wfred_add_u32((uint32_t)lane_id() < (uint32_t)kWaves ? wcnt[min((uint32_t)lane_id(), (uint32_t)kWaves - 1u)] : 0u);
-        if (all <= kIndexFewMax) { // uniform
+        if (index_few(all, d.n_vocab)) { // uniform
             uint32_t* const in_front = wcnt + 2 * kWaves; // [4][kWaves] of the piece's b-th 4 096, by wave
             uint32_t mine[2], upto[2]; // (two counts a word)
 #pragma unroll
@@ -323,9 +330,9 @@ __device__ __forceinline__ void index_groups_block(const mako_sample_desc& d_arg
         plan->total64 = total64;
         plan->thr = n_cand;
         const bool gaps_matter = n_cand < n_list && d_arg.out_cand_idx && d_arg.out_cand_q && d_arg.cand_cap;
-        plan->flag = n_cand == 0u ? kIndexEmpty : (gaps_matter ? kIndexWhole : (n_cand <= kIndexFewMax ? kIndexFew : kIndexReady));
+        plan->flag = n_cand == 0u ? kIndexEmpty : (gaps_matter ? kIndexWhole : (index_few(n_cand, d_arg.n_vocab) ? kIndexFew : kIndexReady));
     }
-    if (n_cand <= kIndexFewMax || p * kSpan >= n_list) // uniform
+    if (n_cand == 0u || index_few(n_cand, d_arg.n_vocab) || p * kSpan >= n_list) // uniform
         return;
     const uint32_t off = p * kSpan, cnt = min(kSpan, n_list - off);
     const uint32_t groups = (cnt + kGroup - 1u) / kGroup; // <= 16 GPW <= 64

@@ -52,3 +52,32 @@ def test_few_candidates(vocab):
                     assert (v["tokens"][r], bool(v["accepted"][r])) == (verified[r][0], bool(verified[r][1]["accepted"])), (r, hinted)
     finally:
         ctx.close()
+
+
+# (rows too short for a list of their candidates to pay, and the shortest that have one)
+@pytest.mark.parametrize("vocab", [2, 255, 256, 257, 512, 513, 640, 641, 20000])
+def test_few_candidates_of_short_rows(vocab):
+    rng = np.random.Generator(np.random.PCG64([9, vocab]))
+    ends = [e for e in (1, 255, 256, 257, 511, 512, 513, vocab) if e <= vocab]
+    counts = [c for c in (1, 2, 100, 255, 256, 257, 500) if c <= vocab]
+    x = np.full((len(ends) * len(counts), vocab), -np.inf, np.float32)
+    for r, (end, n) in enumerate((e, c) for e in ends for c in counts):
+        at = np.append(rng.permutation(end - 1)[: n - 1], end - 1)
+        x[r, at] = rng.standard_normal(len(at)) * 0.5
+    rows = len(x)
+    p = api.make_params(rows, 0.8, 0, 1.0)
+    u = np.resize(np.float32([0.0, 0.3, 0.7, 1.0 - 2.0**-24]), rows)
+    w = dict(name="few, short, V=%d" % vocab, logits=x, params=p, u=u)
+    draft, u2 = np.argmax(x, 1).astype(np.int32), rng.random(rows).astype(np.float32)
+    ctx = api.SamplerContext(max_rows=rows, max_vocab=vocab)
+    try:
+        ref, verified = oracle_rows(w), oracle_rows(w, draft=draft, u2=u2)
+        for hinted in (True, False):
+            g, v = gpu_rows(ctx, w, hinted=hinted), gpu_rows(ctx, w, draft=draft, u2=u2, hinted=hinted)
+            for r in range(rows):
+                t, tr = ref[r]
+                assert (g["tokens"][r], g["n_cand"][r]) == (t, tr["n_cand"]), (r, hinted)
+                assert np.float32(g["total"][r]).view(np.uint32) == np.float32(tr["total"]).view(np.uint32), (r, hinted)
+                assert (v["tokens"][r], bool(v["accepted"][r])) == (verified[r][0], bool(verified[r][1]["accepted"])), (r, hinted)
+    finally:
+        ctx.close()
