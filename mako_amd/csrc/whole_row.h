@@ -3,6 +3,7 @@
 
 #include "lds_sort.h"
 #include "nth_steps.h"
+#include "slice_load.h"
 #include "sorted_tail.h"
 
 namespace mako {
@@ -1026,6 +1027,35 @@ __device__ MAKO_RARE_CALL bool sort_picked(uint32_t* k0, uint32_t* i0, uint32_t 
     return sorted;
 }
 
+// The row's logits, -inf where the mask says so, to wbuf.  All threads call.
+// (Sixteen logits a thread and trip, all asked for before anything is waited for: they may be in host memory, a trip over the bus
+// away.  One row of 129 280 equal logits through the host call: 339 us with one logit a thread and trip from device memory, 433
+// from host memory, 333 from there so; 64 such rows 360 us, 339 so.)
+__device__ MAKO_RARE_CALL void copy_masked_row(const mako_sample_desc& d, uint32_t row, const mako_sampling_params& P, float* wbuf)
+{
+    const uint32_t tid = threadIdx.x;
+    for (uint32_t lo = 0; lo < d.n_vocab; lo += kSliceMax) {
+        const uint32_t hi = min(d.n_vocab, lo + kSliceMax);
+        RawSlice raw;
+        load_raw<false>(d, row, lo, hi, raw);
+        settle_slice<false>(raw, lo, hi);
+        float w[16];
+        finish_slice<false>(raw, lo, hi, P, false, nullptr, w, d.mask != nullptr);
+#pragma unroll
+        for (uint32_t k = 0; k < 4; ++k) {
+            const uint32_t i = elem_index(lo, tid, 4u * k);
+            if (i + 3u < hi) {
+                *reinterpret_cast<float4*>(wbuf + i) = make_float4(w[4 * k], w[4 * k + 1], w[4 * k + 2], w[4 * k + 3]);
+            } else {
+#pragma unroll
+                for (uint32_t c = 0; c < 4; ++c)
+                    if (i + c < hi)
+                        wbuf[i + c] = w[4 * k + c];
+            }
+        }
+    }
+}
+
 // Whole-row path: exact for every parameter combination.  One workgroup rebuilds the penalised
 // row in scratch, keeps the candidates, sorts them by (q desc, idx asc) when top-k or top-p is
 // active, truncates, and draws.  src/gen/sampler.cpp:20-62.
@@ -1043,16 +1073,9 @@ __device__ MAKO_RARE_CALL void general_row(const mako_sample_desc& d, const Scra
     uint32_t* cnt = sc.cnt + (size_t)row * sc.vpad;
     uint32_t* key0 = sc.key[0] + (size_t)row * sc.vpad;
     uint32_t* idx0 = sc.idx[0] + (size_t)row * sc.vpad;
-    const float* lrow = d.logits + (int64_t)row * d.logits_stride;
-    const uint32_t* mrow = d.mask ? d.mask + (int64_t)row * d.mask_stride : nullptr;
 
     // 1. masked copy, then the penalties once per distinct history token
-    for (uint32_t i = tid; i < V; i += kThreads) {
-        float v = lrow[i];
-        if (mrow && !((mrow[i >> 5] >> (i & 31u)) & 1u))
-            v = -INFINITY;
-        wbuf[i] = v;
-    }
+    copy_masked_row(d, row, P, wbuf);
     __syncthreads();
     const uint32_t hl = d.hist_tokens ? d.hist_len[row] : 0u;
     if (hl > 0 && !penalties_neutral(P)) {
