@@ -261,7 +261,7 @@ constexpr uint32_t kIndexWhole = 8;   // the whole-row path is wanted (candidate
 constexpr uint32_t kIndexEmpty = 9;   // no candidate survived
 constexpr uint32_t kIndexFew = 10;    // so few did that they are a list of their own
 
-__device__ __forceinline__ bool penalties_neutral(const mako_sampling_params& p)
+__host__ __device__ __forceinline__ bool penalties_neutral(const mako_sampling_params& p)
 {
     return p.repetition_penalty == 1.0f && p.presence_penalty == 0.0f && p.frequency_penalty == 0.0f;
 }

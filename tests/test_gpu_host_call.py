@@ -78,3 +78,38 @@ def test_inputs_left_in_place(rows, vocab):
             assert np.array_equal(tokens, gpu_rows(ctx, dict(logits=x, params=p, u=u))["tokens"]), (top_k, levels)
     finally:
         ctx.close()
+
+
+# (rows whose histories are long enough to be read in trips go through a copy, and greedy rows and rows without penalties, which have
+# no use for theirs, don't: around the 8 192 entries that a slice's threads hold in registers, with rows that are read again)
+@pytest.mark.parametrize("entries", [1, 8191, 8192, 8193, 20000])
+@pytest.mark.parametrize("vocab", [9000, 40001])
+def test_long_histories(vocab, entries):
+    rows = 3
+    rng = np.random.Generator(np.random.PCG64([vocab, entries]))
+    tokens = np.full(rows, -1, np.int32)
+    ctx = api.SamplerContext(max_rows=rows, max_vocab=vocab, max_hist=20000)
+
+    def at(a):
+        return ctypes.c_void_p(a.ctypes.data)
+
+    try:
+        for levels in (0, 2):
+            x = (rng.standard_normal((rows, vocab)) * 3.0).astype(np.float32)
+            if levels:
+                x = np.floor(x.clip(0, levels - 0.5))
+            p = api.make_params(rows, 0.8, 40, 0.95)
+            hist = rng.integers(0, vocab, (rows, entries)).astype(np.int32)
+            counts = rng.integers(1, 4, (rows, entries)).astype(np.uint32)
+            length = np.array([entries, entries // 2, entries], np.uint32)
+            u = rng.random(rows).astype(np.float32)
+            for penalised in ((), (0,), (0, 1, 2)):
+                p["repetition_penalty"][list(penalised)], p["frequency_penalty"][list(penalised)] = 1.3, 0.2
+                p["temperature"][2] = 0.0 if len(penalised) == 1 else 0.8
+                rc = ctx.lib.mako_sampler_sample_host(ctypes.c_void_p(ctx.ptr), at(x), vocab, rows, vocab, at(p), at(u), None, 0, at(hist),
+                                                      at(counts), entries, at(length), None, None, None, at(tokens))
+                assert rc == api.MAKO_OK, ctx.last_error()
+                w = dict(logits=x, params=p, u=u, hist=hist, hist_len=length)
+                assert np.array_equal(tokens, gpu_rows(ctx, w, hist_counts=counts)["tokens"]), (levels, penalised)
+    finally:
+        ctx.close()
