@@ -403,7 +403,7 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
     const bool index_served = d.n_vocab <= mako::kIndexMaxVocab;
     // (any_unordered: those of the class that are not in token order, of nth_steps.h: a top-k alone, which takes rounds, or wide)
     bool any_nucleus = true, any_late = true, only_index = false, any_in_order = false, beside = index_served, any_unordered = index_served, any_rounds = index_served, any_wide = index_served;
-    uint32_t nucleus_rows = d.n_rows, index_rows = d.n_rows;
+    uint32_t nucleus_rows = d.n_rows, index_rows = d.n_rows, least_top_k = ~0u; // (least_top_k: of the rows that take rounds)
     if (params_host) {
         any_nucleus = any_late = any_unordered = any_rounds = any_wide = false;
         uint32_t n_nucleus = 0, n_index = 0;
@@ -416,7 +416,10 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
             any_in_order |= index_row && mako::index_order_row(params_host[r]);
             any_unordered |= index_row && !mako::index_order_row(params_host[r]);
             any_wide |= index_row && mako::wide_row(params_host[r]);
-            any_rounds |= index_row && !(params_host[r].top_p < 1.0f);
+            if (index_row && params_host[r].top_k != 0u && !(params_host[r].top_p < 1.0f)) {
+                any_rounds = true;
+                least_top_k = std::min(least_top_k, params_host[r].top_k);
+            }
             n_nucleus += c == mako::kNucleus;
         }
         nucleus_rows = std::max(n_nucleus, 1u);
@@ -425,12 +428,10 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
         index_rows = n_index;
     }
     const bool any_nth = any_unordered && mako::nth_steps_for(d.n_vocab), any_bits = any_nth || (any_wide && mako::nth_picks_for(d.n_vocab));
-    // (their steps: a launch each, of about two workgroups per CU.  Beside other rows the sort's launch has them all.  A launch
-    // costs 8 to 10 us and leaves 0.44 of a row: as many as bring the 64 rows' unluckiest near what a workgroup takes into its
-    // registers.  64 rows of 129 280: 185 us with two, 172, 164, 162, 168 with six; of 40 000: 104 with two, 105, 110)
+    // (their steps: a launch each, of about two workgroups per CU.  Beside other rows the sort's launch has them all.  Rows of a
+    // top-k before a top-p alone have no use for more than the first)
     const uint32_t nth_wgs = std::min(std::max(2u * ctx->cus / ((d.n_rows + 7u) & ~7u), 1u), (d.n_vocab + mako::kNthChunk - 1u) / mako::kNthChunk);
-    // (rows of a top-k before a top-p alone have no use for more than the first)
-    const uint32_t nth_steps = !any_nth ? 0u : (!any_rounds ? 1u : (d.n_vocab <= 65536u ? 2u : 4u));
+    const uint32_t nth_steps = !any_nth ? 0u : (!any_rounds ? 1u : mako::nth_launches(d.n_vocab, least_top_k));
     const bool launch_sort = any_nucleus || any_late || beside;
     // (finish_kernel's grid: scan_kernel, which cuts the second pass up, is told of it)
     const uint32_t finish_wgs = mako::second_pass_grid(nucleus_rows, ctx->cus);

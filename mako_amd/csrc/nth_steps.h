@@ -80,6 +80,21 @@ __host__ __device__ __forceinline__ bool nth_steps_for(uint32_t n_vocab)
     return n_vocab > 32768u && n_vocab <= kNthMaxVocab;
 }
 
+// How many launches of their own, of rows the least of whose top_k is this?  Each costs 8 to 10 us and leaves 0.44 of the list: as
+// many as bring the 64 rows' unluckiest near what a workgroup takes into its registers (64 rows of 129 280, top_k 40: 185 us with
+// two, 172, 164, 162, 168 with six; of 40 000: 104 with two, 105, 110), but none for a list that is expected to be less than twice
+// top_k long, since a row is done with steps once its cut lies in front of its top_k.  (64 rows of 129 280, one to four launches:
+// top_k 1 293 260 us, 239, 230, 234; 6 464 315, 318, 330, 341; 25 856 468, 484, 496, 507; 64 640 637, 653, 659, 664; 129 280 580,
+// 582, 585, 589; one row, top_k 6 464: 188, 184, 184, 186.)
+inline uint32_t nth_launches(uint32_t n_vocab, uint32_t least_top_k)
+{
+    const uint32_t most = n_vocab <= 65536u ? 2u : 4u;
+    uint32_t n = 1;
+    for (float left = 0.44f * (float)n_vocab; n < most && left > 2.0f * (float)least_top_k; left *= 0.44f)
+        ++n;
+    return n;
+}
+
 // ... and of those, a top-k before a top-p?
 __host__ __device__ __forceinline__ bool wide_row(const mako_sampling_params& P)
 {
