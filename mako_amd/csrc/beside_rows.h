@@ -75,8 +75,8 @@ __global__ __launch_bounds__(kThreads) void sort_beside_kernel(mako_sample_desc 
     const uint32_t nth_rows = nth_steps_for(d_arg.n_vocab) ? general - in_order : 0u;
     if (nth_rows) { // uniform
         const uint32_t per_row = min(max(min(wgs, cus) / nth_rows, 1u), (d_arg.n_vocab + kNthChunk - 1u) / kNthChunk);
+        RankedRows ranked;
         for (uint32_t p = me; p < nth_rows * per_row; p += wgs) {
-            RankedRows ranked;
             uint32_t row;
             if (!ranked.find(d_arg, p / per_row, [](const mako_sampling_params& P) { return nth_row(P); }, row))
                 break;
