@@ -184,8 +184,7 @@ __device__ void coarse_plan(const Scratch& sc, uint32_t row, uint32_t slices, ui
                 break;
             edge = below;
         }
-        const float qe = weight_of(edge, m, inv_t, tab);
-        uint32_t key = qe == qe ? __float_as_uint(qe) : 0u; // (positive floats order like their bits)
+        uint32_t key = __float_as_uint(weight_of(edge, m, inv_t, tab)); // (no NaN; positive floats order like their bits)
         for (uint32_t o = 1; o < kWorkers; o <<= 1) { // the edges never rise from one worker to the next
             const uint32_t t = (uint32_t)__shfl_up((int)key, o);
             if (lane >= o)

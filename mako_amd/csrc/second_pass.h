@@ -121,7 +121,7 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
         }
         if (lo + (g / 4u) * 4096u < hi) {
             // (the large batches' instance: a wave whose four weights a lane all underflow to zero, as those of a peaked row far
-            // below its maximum do, skips the arithmetic that would tell it so; expf_glibc() returns 0 below that bound)
+            // below its maximum do, skips the arithmetic that would tell it so; exp_moved() returns 0 below that bound)
             bool any = !UNSORTED;
             if (UNSORTED) {
                 bool under = true;
