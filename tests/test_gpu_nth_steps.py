@@ -46,6 +46,8 @@ def _batch(vocab, gaps, seed, ties, hist=0):
     return w
 
 
+# (there are no steps up to 32 768 logits: rows of 16 381 and 20 002 take the same rounds in the last launch alone, more than its
+# registers hold and no more)
 @pytest.mark.parametrize("gaps", ["none", "mask", "min_p", "underflow", "one"])
 @pytest.mark.parametrize("vocab", [16381, 20002, 65537, 131072, 151553])
 def test_steps(vocab, gaps):
@@ -87,6 +89,27 @@ def test_steps_forced_and_verified(vocab):
                 assert (g["tokens"][r], bool(g["accepted"][r])) == (t, bool(tr["accepted"])), (r, hinted)
     finally:
         ctx.close()
+
+
+# (launches of their own with two steps at most, of rows with and without gaps, whose first pivots are penalised or not; and the
+# longest rows without steps and with two)
+@pytest.mark.parametrize("gaps", ["none", "mask", "min_p", "underflow", "one"])
+@pytest.mark.parametrize("vocab", [32768, 32769, 40000, 50001, 65536])
+def test_two_steps(vocab, gaps):
+    test_steps(vocab, gaps)
+    w = _batch(vocab, gaps, 6, False, hist=30)  # (the least top_k of a batch says how many launches it takes)
+    ctx = api.SamplerContext(max_rows=len(w["u"]), max_vocab=vocab, max_hist=64)
+    try:
+        for first in (4, 5, 7):
+            part = {k: v if k == "name" else v[first:] for k, v in w.items()}
+            assert_parity(ctx, part, cap=64, hinted=True)
+    finally:
+        ctx.close()
+
+
+@pytest.mark.parametrize("vocab", [32769, 40000, 65536])
+def test_two_steps_forced_and_verified(vocab):
+    test_steps_forced_and_verified(vocab)
 
 
 # (the bin that holds the k-th heaviest: a few entries more than k, thousands, more than one sort in LDS holds)
