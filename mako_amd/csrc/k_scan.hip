@@ -14,8 +14,10 @@ template <bool ALIGNED, int KH>
 void launch_kh(bool above, dim3 grid, size_t lds, hipStream_t st, const mako_sample_desc& d, const Scratch& sc,
                uint32_t slice_len, uint32_t cus)
 {
-    if (short_slice(slice_len)) // (a row of one slice)
+    if (short_slice(slice_len) && above) // (a row of one slice)
         launch_one<ALIGNED, KH, true, true>(grid, lds, st, d, sc, slice_len, cus);
+    else if (short_slice(slice_len))
+        launch_one<ALIGNED, KH, false, true>(grid, lds, st, d, sc, slice_len, cus);
     else if (above)
         launch_one<ALIGNED, KH, true, false>(grid, lds, st, d, sc, slice_len, cus);
     else
@@ -51,6 +53,9 @@ hipError_t init_scan_kernels()
                              (const void*)scan_kernel<true, 0, true>,  (const void*)scan_kernel<false, 0, true>,
                              (const void*)scan_kernel<true, 2, true>,  (const void*)scan_kernel<false, 2, true>,
                              (const void*)scan_kernel<true, 8, true>,  (const void*)scan_kernel<false, 8, true>,
+                             (const void*)scan_kernel<true, 0, false, true>, (const void*)scan_kernel<false, 0, false, true>,
+                             (const void*)scan_kernel<true, 2, false, true>, (const void*)scan_kernel<false, 2, false, true>,
+                             (const void*)scan_kernel<true, 8, false, true>, (const void*)scan_kernel<false, 8, false, true>,
                              (const void*)scan_kernel<true, 0, true, true>, (const void*)scan_kernel<false, 0, true, true>,
                              (const void*)scan_kernel<true, 2, true, true>, (const void*)scan_kernel<false, 2, true, true>,
                              (const void*)scan_kernel<true, 8, true, true>, (const void*)scan_kernel<false, 8, true, true>};
