@@ -16,7 +16,7 @@
 // `r < q` is never true for it.  The list ends behind the row's last candidate, which is where the reference's walk
 // ends when it runs off its list.  Verification works on the same list: the draft's weight is entry `draft`, and a
 // rejected draft is redrawn with that entry taken as 0.0f (sorted_tail's UNORDERED instance).
-// A row of some length with up to 256 candidates (a min-p on a peaked row, a grammar's mask) needs no records: each piece leaves its candidates'
+// A row with up to 256 candidates (a min-p on a peaked row, a grammar's mask) needs no records: each piece leaves its candidates'
 // token ids in order, and few_candidates_row() finishes the row from those.
 // The other rows of the whole-row class (top-k without top-p, top-k beyond the candidate lists) only get their weights
 // here (into the array general_row_from_weights() starts from), the first rounds of their nth_element (nth_steps.h), and one
@@ -33,13 +33,6 @@ namespace mako {
 constexpr uint32_t kIndexBlock = 4096;                   // entries whose fp64 sum index_weights_kernel leaves as one number
 constexpr uint32_t kIndexMaxVocab = kMaxGroups * kGroup; // the group records of a row
 constexpr uint32_t kIndexFewMax = kGroup;                // candidates that a row may have to be finished from a list of them
-// ... and how long it has to be for that.  (30 rows with a min-p: of 172 logits 23.9 us from a list of the candidates and 21.5
-// from the records, of 359 24.6 and 23.4, of 511 24.6 and 24.3, of 700 24.1 and 24.8, of 1 500 24.2 and 29.5.)
-constexpr uint32_t kIndexFewFrom = 640;
-__device__ __forceinline__ bool index_few(uint32_t n_cand, uint32_t n_vocab)
-{
-    return n_cand <= kIndexFewMax && n_vocab > kIndexFewFrom;
-}
 static_assert(kIndexMaxVocab / kSliceMax <= kWorkers && kIndexMaxVocab / kIndexBlock <= kMaxSlices && kIndexMaxVocab / kIndexBlock <= (uint32_t)kWave &&
                   kSliceMax == 4u * kIndexBlock && kIndexBlock == (uint32_t)kWaves * kGroup,
               "a piece's count and last candidate travel in the plan's per-worker words, the blocks' sums in the row's part_sum, a lane each");
@@ -240,7 +233,7 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
     if (in_order) { // uniform
         // few candidates: their token ids in order (in the piece's part of idx[1]; few_candidates_row())
         const uint32_t all = __ockl_wfred_add_u32((uint32_t)lane_id() < (uint32_t)kWaves ? wcnt[min((uint32_t)lane_id(), (uint32_t)kWaves - 1u)] : 0u);
-        if (index_few(all, d.n_vocab)) { // uniform
+        if (all <= kIndexFewMax) { // uniform
             uint32_t* const in_front = wcnt + 2 * kWaves; // [4][kWaves] of the piece's b-th 4 096, by wave
             uint32_t mine[2], upto[2]; // (two counts a word)
 #pragma unroll
@@ -330,9 +323,9 @@ __device__ __forceinline__ void index_groups_block(const mako_sample_desc& d_arg
         plan->total64 = total64;
         plan->thr = n_cand;
         const bool gaps_matter = n_cand < n_list && d_arg.out_cand_idx && d_arg.out_cand_q && d_arg.cand_cap;
-        plan->flag = n_cand == 0u ? kIndexEmpty : (gaps_matter ? kIndexWhole : (index_few(n_cand, d_arg.n_vocab) ? kIndexFew : kIndexReady));
+        plan->flag = n_cand == 0u ? kIndexEmpty : (gaps_matter ? kIndexWhole : (n_cand <= kIndexFewMax ? kIndexFew : kIndexReady));
     }
-    if (n_cand == 0u || index_few(n_cand, d_arg.n_vocab) || p * kSpan >= n_list) // uniform
+    if (n_cand <= kIndexFewMax || p * kSpan >= n_list) // uniform
         return;
     const uint32_t off = p * kSpan, cnt = min(kSpan, n_list - off);
     const uint32_t groups = (cnt + kGroup - 1u) / kGroup; // <= 16 GPW <= 64
@@ -375,9 +368,12 @@ __device__ __forceinline__ void index_groups_block(const mako_sample_desc& d_arg
 
 // A row with few candidates (a min-p leaves a peaked row a few dozen): the pieces' lists one after the other are
 // the row's, in token order, which one wave adds up and walks.  All threads call.
-// (64 rows of 129 280 with a min-p of 0.02 to 0.1: 68 us over the group records of every logit, 54 so; one row 31
-// and 25; 400 rows 235 and 183; 24 of 151 553 without the caller's copy of the parameters 79 and 70.)
-__device__ MAKO_RARE_CALL void few_candidates_row(const mako_sample_desc& d, const Scratch& sc, uint32_t row, const mako_sampling_params& P, const FinishLds& L)
+// In line in the kernel, or at most one call away, and the tail for short lists in line here: where the tail was a called function,
+// and this another, sixteen waves stored and fetched their registers at each entry for what one wave does, and from 128 rows on that
+// took longer than the records.  (Peaked rows with a min-p of 0.02 to 0.1, over the group records, with the calls, and so: one of
+// 129 280 31.7 us, 26.2 and 22.1, 64 of them 66, 44 and 37, 512 rows of 700 40.6, 61.0 and 28.4; without the caller's copy of the
+// parameters 24 rows of 151 553 71, 48 and 41, 512 of 700 119, 147 and 111.)
+__device__ __forceinline__ void few_candidates_row(const mako_sample_desc& d, const Scratch& sc, uint32_t row, const mako_sampling_params& P, const FinishLds& L)
 {
     assume_lds(L);
     const uint32_t tid = threadIdx.x, lane = lane_id(), pieces = (d.n_vocab + kSliceMax - 1u) / kSliceMax;
@@ -400,9 +396,7 @@ __device__ MAKO_RARE_CALL void few_candidates_row(const mako_sample_desc& d, con
         jf[tid] = id;
     }
     __syncthreads();
-    // (the instance that general_row() calls as well: tail_beside_kernel has the one for short lists inline, for its top-k rows, and a
-    // second caller would make it a call there, with scratch memory: 510 such rows 16.6 us, 45 so)
-    sorted_tail(d, row, P, kf, jf, n_cand, true, sc.plan[row].total64, MAKO_PATH_INDEXED, L);
+    [[clang::always_inline]] sorted_tail<false, true>(d, row, P, kf, jf, n_cand, true, sc.plan[row].total64, MAKO_PATH_INDEXED, L);
 }
 
 // What these kernels have left of a row of theirs (flag: of its plan, which is zero again behind this), by one workgroup: the
@@ -459,16 +453,12 @@ __device__ __forceinline__ bool finish_index_row_here(const mako_sample_desc& d,
         general_row<0>(d, sc, row, P, m, argidx, L);
     return false;
 }
-__device__ MAKO_RARE_CALL bool finish_index_row_call(const mako_sample_desc& d, const Scratch& sc, const mako_sampling_params& P, uint32_t row,
+// (those of few_candidates_row() apart)
+__device__ MAKO_RARE_CALL void finish_index_row(const mako_sample_desc& d, const Scratch& sc, const mako_sampling_params& P, uint32_t row,
                                                 const FinishLds& L)
 {
     assume_lds(L);
-    return finish_index_row_here(d, sc, P, row, L);
-}
-__device__ __forceinline__ void finish_index_row(const mako_sample_desc& d, const Scratch& sc, const mako_sampling_params& P, uint32_t row, const FinishLds& L)
-{
-    if (finish_index_row_call(d, sc, P, row, L)) // uniform
-        few_candidates_row(d, sc, row, P, L);
+    (void)finish_index_row_here(d, sc, P, row, L);
 }
 
 // Rows of the kind that `want` says (kGeneral, or those of them that are in token order) by their rank among them, for ranks that

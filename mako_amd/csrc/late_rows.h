@@ -94,6 +94,17 @@ __device__ MAKO_RARE_CALL bool late_plain_row(const mako_sample_desc& d, const S
     return false;
 }
 
+// A row of index_rows.h with few candidates.  (Called from the kernel itself: a call that it were deeper in the stack stores the
+// registers of sixteen waves, for what one of them does.)
+__device__ MAKO_RARE_CALL void late_few_row(const mako_sample_desc& d, const Scratch& sc, const mako_sampling_params& P, uint32_t row, const FinishLds& L)
+{
+    assume_lds(L);
+    __syncthreads(); // (the plan's flag has been read)
+    if (threadIdx.x == 0)
+        sc.plan[row].flag = 0;
+    few_candidates_row(d, sc, row, P, L);
+}
+
 // What the earlier kernels leave of row `row`, by one workgroup (all threads call; sm.tab must hold the exp2 table):
 // rows whose token is forced, greedy rows, top-k rows, rows for the whole-row path, second looks.
 // BESIDE: the rows that the launches before have begun for index_rows.h are finished here too.
@@ -106,8 +117,11 @@ __device__ MAKO_RARE_CALL void finish_late_row(const mako_sample_desc& d, const 
     if ((d.force_token || d.close_token || cls == kGreedy) && late_plain_row(d, sc, cls, row, slices))
         return;
     if constexpr (BESIDE)
-        if (cls == kGeneral && sc.plan[row].flag != 0u) { // uniform
-            finish_index_row(d, sc, P, row, L);
+        if (cls == kGeneral && sc.plan[row].flag != 0u) { // uniform (of a batch that may have forced tokens)
+            if (sc.plan[row].flag == kIndexFew)
+                late_few_row(d, sc, P, row, L);
+            else
+                finish_index_row(d, sc, P, row, L);
             return;
         }
     if (cls == kNucleus) {

@@ -70,6 +70,18 @@ __device__ __forceinline__ void tail_body(const mako_sample_desc& d_arg, const S
         // (the views handed on by reference live in scratch memory, 32 bytes per thread: made here, where only the
         // rows that take the call store them)
         const FinishLds late_views = finish_lds_views(sm, s_dyn64);
+        // (the rows of index_rows.h with one call less than through finish_late_row())
+        if (BESIDE && late_cls == kGeneral && !plain) { // uniform
+            const uint32_t late_flag = sc_arg.plan[r].flag;
+            if (late_flag == kIndexFew) {
+                late_few_row(s_args.d, s_args.sc, s_args.P, r, late_views);
+                return;
+            }
+            if (late_flag != 0u) {
+                finish_index_row(s_args.d, s_args.sc, s_args.P, r, late_views);
+                return;
+            }
+        }
         finish_late_row<BESIDE>(s_args.d, s_args.sc, s_args.P, r, slices, late_views);
         return;
     }

@@ -283,7 +283,9 @@ __device__ __forceinline__ void topk_row(const mako_sample_desc& d, const Scratc
     // (sampler.cpp:40-43; at most top_k <= kTopKFast <= kGroup entries.  A top-p cut too close to call is left to the
     // whole-row path, which can sum in the reference's order.)
     static_assert(kTopKFast <= kGroup, "top-k rows end in sorted_tail's short-list path");
-    if (ok && sorted_tail<false, true>(d, row, P, kf, jf, min(P.top_k, n_valid), false, 0.0, MAKO_PATH_TOPK, L))
+    if (ok)
+        [[clang::always_inline]] ok = sorted_tail<false, true>(d, row, P, kf, jf, min(P.top_k, n_valid), false, 0.0, MAKO_PATH_TOPK, L);
+    if (ok)
         return;
     __syncthreads(); // (the lists in LDS are done with)
     // (where the whole-row path is a called function the views it receives by reference live in scratch memory: a copy

@@ -54,7 +54,7 @@ def test_few_candidates(vocab):
         ctx.close()
 
 
-# (rows too short for a list of their candidates to pay, and the shortest that have one)
+# (rows of a few groups of 256, for which records would be as short as the list)
 @pytest.mark.parametrize("vocab", [2, 255, 256, 257, 512, 513, 640, 641, 20000])
 def test_few_candidates_of_short_rows(vocab):
     rng = np.random.Generator(np.random.PCG64([9, vocab]))
