@@ -13,6 +13,7 @@ namespace mako {
 constexpr size_t kStageAlign = 256;
 constexpr size_t kStagePinned = (size_t)16 << 20; // staging memory kept per context, at most
 constexpr size_t kStageCopy = (size_t)1 << 20;    // bytes per copy: a copy costs 8 us and a MiB's transfer 20, putting it together 12
+constexpr size_t kStageSmall = (size_t)16 << 10; // bytes that the runtime copies for 5 us less than one more
 
 // Arrays are put one after the other, each at a multiple of kStageAlign, into staging memory on the host, from where every
 // kStageCopy bytes are copied to the same places of the context's block of device memory.

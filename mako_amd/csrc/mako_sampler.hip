@@ -605,14 +605,16 @@ int mako_sampler_sample_host(mako_sampler_ctx* ctx, const float* logits, int64_t
     }
     d.logits = reinterpret_cast<const float*>(ctx->st_dev + stage.put_rows(logits, (size_t)logits_stride * 4, (size_t)n_vocab * 4, (size_t)stride * 4, n_rows));
     d.logits_stride = stride;
-    // What would be a single copy (a MiB at most) is left where it is if no row's logits are sure to be read a second time: the
+    // What would be a single copy (of 16 KiB to a MiB) is left where it is if no row's logits are sure to be read a second time: the
     // kernels then read it over the bus, 14 us for a row of 129 280 logits in place of a copy's 17 and 7 from device memory.  (One
     // top-k row: 48.1 us with the copy, 44.9 so; of 8 000 logits 33.4 and 29.9; seven rows of 32 000 63.0 and 58.2.  A nucleus
     // row, whose logits the second pass reads again: 72.7 and 79.4.)  A top-k row that its candidates do not settle is read again
     // (one of 129 280 equal logits: 339 and 333; with the counts of 7 300 tokens 851 and 878), and its history once per slice, which
     // is as fast as long as a thread holds its share of it in registers: eight entries.  Behind that it is read in trips, each over the bus.  (32 000 logits, 31 000 tokens
     // with their counts: 47.4 and 52.4; 129 280 and 8 100: 52.8 and 46.9, 9 900: 55.8 and 56.9.)
-    bool once = ctx->st_pinned && stage.sent == 0 && stage.status == 0;
+    // Smaller calls are copied: a greedy row of 3 000 logits 19.6 us, 20.3 over the bus, with a mask and a draft 19.5 and 21.9; of
+    // 4 000 24.5 and 20.4.
+    bool once = ctx->st_pinned && stage.sent == 0 && stage.status == 0 && stage.at > mako::kStageSmall;
     for (uint32_t r = 0; once && r < n_rows; ++r) {
         const mako::RowClass c = mako::classify(params[r]);
         const bool history = d.hist_stride > 8 * (int64_t)mako::kThreads && !mako::penalties_neutral(params[r]);

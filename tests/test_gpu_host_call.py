@@ -80,6 +80,12 @@ def test_inputs_left_in_place(rows, vocab):
         ctx.close()
 
 
+# (on either side of the 16 KiB up to which a call is copied all the same)
+@pytest.mark.parametrize("rows,vocab", [(1, 3964), (1, 3968), (1, 3969), (1, 3972), (16, 200), (16, 260)])
+def test_small_calls(rows, vocab):
+    test_inputs_left_in_place(rows, vocab)
+
+
 # (rows whose histories are long enough to be read in trips go through a copy, and greedy rows and rows without penalties, which have
 # no use for theirs, don't: around the 8 192 entries that a slice's threads hold in registers, with rows that are read again)
 @pytest.mark.parametrize("entries", [1, 8191, 8192, 8193, 20000])
