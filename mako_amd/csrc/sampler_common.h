@@ -211,6 +211,12 @@ enum CheckBit {
 #ifndef MAKO_RARE_CALL
 #define MAKO_RARE_CALL
 #endif
+// (at a call: not to be made part of the caller, there)
+#ifdef MAKO_REAL_CALLS
+#define MAKO_CALL [[clang::noinline]]
+#else
+#define MAKO_CALL
+#endif
 
 // The reference adds a row's weights one after the other in fp64 (src/gen/sampler.cpp:46-48 in candidate order,
 // :55-56 in sorted order); the sums here associate differently (per thread, wave and workgroup; bin masses).  An

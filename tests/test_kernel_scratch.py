@@ -20,7 +20,8 @@ def _code_objects(data):
     at = data.find(b"\x7fELF", 4)
     while at >= 0:
         if struct.unpack_from("<H", data, at + 18)[0] == 224:  # EM_AMDGPU
-            yield data[at:]
+            size = struct.unpack_from("<Q", data, at + 40)[0] + struct.unpack_from("<H", data, at + 60)[0] * struct.unpack_from("<H", data, at + 58)[0]
+            yield data[at:at + size]
         at = data.find(b"\x7fELF", at + 4)
 
 
@@ -50,3 +51,15 @@ def test_kernels_of_many_workgroups_use_no_scratch_memory():
     many = {k: v for k, v in found.items() if NONE.search(k)}
     assert len(many) > 20, sorted(found)
     assert not {k: v for k, v in many.items() if v}, {k: v for k, v in many.items() if v}
+
+
+def test_the_tail_of_the_whole_row_path_is_a_call():
+    # (in line, the path to it is a call longer, and a third slower for rows with few survivors)
+    if not os.path.exists(api.LIB_PATH):
+        pytest.skip("the library is not built")
+    with open(api.LIB_PATH, "rb") as f:
+        elves = [e for e in _code_objects(f.read()) if any("index_tail_kernel" in k for k in _kernels(e))]
+    assert elves
+    for elf in elves:
+        assert b"\0_ZN4mako11sorted_tailILb0ELb0ELb0ELb0ELb0EEE" in elf
+        assert b"\0_ZN4mako18sort_truncate_drawILb1EEE" not in elf
