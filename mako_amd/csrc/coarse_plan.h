@@ -52,7 +52,7 @@ __device__ __forceinline__ void issue_plan_loads(const mako_sample_desc& d, cons
 }
 
 // Builds the row's plan in `pl` (all threads call; barriers order LDS only, the logits' loads stay in flight).
-// `m`: the row's maximum.  narrow_ok: a narrow nucleus may be left to the candidate lists.
+// `m`: the row's maximum.  narrow_max: the longest list that may be left to the candidate lists.
 // The slices' counts are moved into the frame of the row's maximum (exactly: units are absolute), each bin's mass is
 // estimated from the middle of the units it covers, and the threshold is put one bin below where the estimated mass
 // under it falls to 1 - top_p of the estimated total, less a few percent.  The list that results is checked by the
@@ -61,7 +61,7 @@ __device__ __forceinline__ void issue_plan_loads(const mako_sample_desc& d, cons
 // share_min: entries a worker is given at least, if there are as many.
 // opaque_first: the first position of the list from which a share may be left unsorted (kNone: none may).
 __device__ void coarse_plan(const Scratch& sc, uint32_t row, uint32_t slices, uint32_t n_vocab, const mako_sampling_params& P,
-                            float m, const PlanLoads& pre, bool narrow_ok, uint32_t opaque_first, uint32_t share_min, CoarsePlan& pl, const uint64_t* tab)
+                            float m, const PlanLoads& pre, uint32_t narrow_max, uint32_t opaque_first, uint32_t share_min, CoarsePlan& pl, const uint64_t* tab)
 {
     const uint32_t tid = threadIdx.x, lane = (uint32_t)lane_id();
     MAKO_STAMP(10);
@@ -141,7 +141,7 @@ __device__ void coarse_plan(const Scratch& sc, uint32_t row, uint32_t slices, ui
     uint32_t flag = 1;
     if (!sane)
         flag = 2;
-    else if (narrow_ok && n0_est <= kSmall)
+    else if (n0_est <= narrow_max)
         flag = 3;
     else if (n0_est > kGroup * (kMaxGroups - kWorkers))
         flag = 2; // (a list too long for the workers' group records goes to the whole-row path)

@@ -18,59 +18,27 @@ struct alignas(16) ScanShared {
     uint32_t log_hist[kLogBins + kWave]; // top_k == 0 rows (and one slot per lane for what is not counted)
 };
 
-// A lower bound, tight to 2^-9 relative, of the j-th largest of the wavefront's order keys, one or more per lane (j >= 1): the
-// largest v with at least j keys >= v, built bit by bit from the top down to bit 14 (the low fourteen bits stay zero: whoever
-// uses the result as a threshold keeps at least j keys, and a handful more at most).  One vector compare per key and bit;
+// A lower bound, tight to 2^-9 relative, of the j-th largest of the wavefront's 64 order keys (j >= 1): the largest
+// v with at least j keys >= v, built bit by bit from the top down to bit 14 (the low fourteen bits stay zero: whoever
+// uses the result as a threshold keeps at least j keys, and a handful more at most).  One vector compare per bit;
 // the rest is scalar.
-template <typename... Keys>
-__device__ __forceinline__ uint32_t wave_kth_largest(uint32_t j, Keys... keys)
+__device__ __forceinline__ uint32_t wave_kth_largest(uint32_t key, uint32_t j)
 {
     uint32_t prefix = 0;
 #pragma unroll
     for (int b = 31; b >= 14; --b) {
         const uint32_t cand = prefix | (1u << b);
-        const uint32_t c = ((uint32_t)__popcll(__ballot(keys >= cand)) + ...);
+        const uint32_t c = (uint32_t)__popcll(__ballot(key >= cand));
         prefix = c >= j ? cand : prefix;
     }
     return prefix;
-}
-
-// A slice too short for all waves to hold logits, and too long for a list of all of it: each of the n waves that hold some takes
-// the ceil(K/n)-th largest (the last one is left out where that is a larger part of its few logits than of the others' 256), the
-// others a key above every logit's.  A nucleus row is to have kSmall logits in its list, the most that a narrow nucleus may have,
-// and takes the larger of every two logits for it instead of every four; a list that overflows leaves the row to the workers.
-// (With the waves that hold none every logit was a candidate, the list overflowed and the row was left to the whole-row path:
-// one top-k row of 1 003 logits 40 us, 12 so; 147 of 2 899 with histories 101 and 16.
-// A kernel of its own: with the branch in everybody's, 512 rows of a decode batch took 0.6 % longer.)
-__host__ __device__ inline bool short_slice(uint32_t len) // (len: as slice_len, rounded up to a multiple of four)
-{
-    return len < 4u * (uint32_t)kThreads && len > kCap;
-}
-__device__ __forceinline__ uint32_t short_slice_kth(const float (&wv)[16], uint32_t len, bool nucleus, uint32_t top_k)
-{
-    static_assert(kCap >= 2u * kGroup && kTopKFast <= 2u * (uint32_t)kWave && kSmall <= 4u * (uint32_t)kWave, "no wave is asked for more than it has");
-    const uint32_t K = nucleus ? kSmall : top_k;
-    // (ceil(K / n): the quotient with half a unit more is never as close to a whole number as the reciprocal is inexact)
-    auto share = [K](uint32_t n) { return (uint32_t)__builtin_amdgcn_readfirstlane((int)(((float)(K + n) - 0.5f) * __builtin_amdgcn_rcpf((float)n))); };
-    const uint32_t full = len / kGroup, rest = len % kGroup; // (full > 1)
-    const uint32_t without = share(full), with = share(full + 1u);
-    const bool rest_too = with * kGroup <= without * rest;
-    const uint32_t j = rest_too ? with : without;
-    // (NaN is no candidate)
-    const uint32_t a = order_key(fmaxf(fmaxf(wv[0], wv[1]), -INFINITY)), b = order_key(fmaxf(fmaxf(wv[2], wv[3]), -INFINITY));
-    uint32_t kth;
-    if (nucleus) // uniform
-        kth = wave_kth_largest(j, a, b);
-    else
-        kth = wave_kth_largest(j, max(a, b));
-    return (uint32_t)wave_id() < full + (rest_too ? 1u : 0u) ? kth : 0xffffffffu;
 }
 
 // (ABOVE: the batch has close tokens, whose logits' ranks are counted on the way; a variant of its own because the
 // count takes sixteen more registers, up to the limit for two workgroups per CU, which no other batch should pay)
 // (amdgpu_waves_per_eu: held to the 64 registers that let two workgroups share a CU, but for rows at any address with eight
 // history entries a thread, which would spill forty)
-// (SHORT: short_slice() slices)
+// (SHORT: short_slice() slices.  A kernel of its own: with a branch in everybody's, 512 rows of a decode batch took 0.6 % longer)
 template <bool ALIGNED, int KH, bool ABOVE = false, bool SHORT = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(ALIGNED || KH < 8 ? 8 : 4))) void scan_kernel(mako_sample_desc d, Scratch sc_arg, uint32_t slice_len,
                                                         uint32_t cus_and_grid)
@@ -149,11 +117,11 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(ALIGNE
     uint32_t above = 0;
     float wv[16];
     if (ABOVE) {
-        load_penalised<ALIGNED, KH>(d, row, lo, hi, slice_len, P, penalised, hl, pen, s_dyn, wv, NoOverlap(), want_above, close_v, &above);
+        load_penalised<ALIGNED, KH, SHORT>(d, row, lo, hi, slice_len, P, penalised, hl, pen, s_dyn, wv, NoOverlap(), want_above, close_v, &above);
         if (want_above) // uniform
             above = __ockl_wfred_add_u32(above);
     } else {
-        load_penalised<ALIGNED, KH>(d, row, lo, hi, slice_len, P, penalised, hl, pen, s_dyn, wv);
+        load_penalised<ALIGNED, KH, SHORT>(d, row, lo, hi, slice_len, P, penalised, hl, pen, s_dyn, wv);
     }
 
     MAKO_STAMP(29);
@@ -171,10 +139,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(ALIGNE
         // takes the ceil(K/16)-th largest of its per-thread maxima; at least K logits of the slice are >= the
         // smallest of those 16 values, which becomes the emission threshold.
         const uint32_t K = cls == kTopK ? P.top_k : kTopKFast;
-        if (SHORT)
-            wkth = short_slice_kth(wv, hi - lo, cls == kNucleus, P.top_k);
-        else
-            wkth = wave_kth_largest((K + kWaves - 1) / kWaves, bkey);
+        wkth = wave_kth_largest(bkey, (K + kWaves - 1) / kWaves);
     }
     if (lane_id() == 0) {
         sm.wave_max[wave_id()] = wmax;
@@ -199,7 +164,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(ALIGNE
 #pragma unroll
         for (int j = 15; j >= 0; --j)
             if (wv[j] == M)
-                first = elem_index(lo, tid, (uint32_t)j);
+                first = elem_index(lo, slice_thread<SHORT>(), (uint32_t)j);
         if (first != kNone)
             atomicMin(&sm.argidx, first);
     }
@@ -248,7 +213,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(ALIGNE
                     const float w = wv[j];
                     if (w >= tau && pos < kCap) {
                         sm.cw[pos] = w;
-                        sm.ci[pos] = elem_index(lo, tid, j);
+                        sm.ci[pos] = elem_index(lo, slice_thread<SHORT>(), j);
                     }
                     run += (uint32_t)__popcll(takes[j]);
                 }

@@ -11,6 +11,26 @@ __device__ __forceinline__ uint32_t elem_index(uint32_t lo, uint32_t tid, uint32
 {
     return lo + (j >> 2) * 4096u + tid * 4u + (j & 3u);
 }
+// The t that a thread is there.  MIXED: a wave has sixteen logits of every 256, in place of 256 of every 4 096.
+template <bool MIXED>
+__device__ __forceinline__ uint32_t slice_thread()
+{
+    const uint32_t tid = threadIdx.x;
+    return MIXED ? (tid & 3u) | ((tid >> 6) << 2) | ((tid & 0x3cu) << 4) : tid;
+}
+
+// A slice that scan_kernel takes MIXED: too long for a candidate list of all of it, and so short that the waves have 256 logits in
+// a row each, or none.  The smallest of the waves' thresholds is the slice's, so that a single wave whose logits are not like the
+// others' makes the list overflow: one without logits, whose threshold is -inf, or the first tokens', which a long history
+// penalises most.  The row is then left to the whole-row path.  (Flat rows with penalties over histories of 5 000 tokens, mixed and
+// not: six of 2 067 33 us and 74, 17 of 4 101 17.9 and 86; a top-k row of 1 003 12.1 and 39.  From 5 120 on the waves that
+// hold the first tokens have others besides: 17 of 5 125 17.6 either way.)
+__host__ __device__ inline bool short_slice(uint32_t len) // (len: as slice_len, rounded up to a multiple of four)
+{
+    // (128 groups of four at least, eight a wave, as many as a top_k of kTopKFast asks each for)
+    static_assert(kTopKFast <= (kCap / 4u / (uint32_t)kWaves) * (uint32_t)kWaves, "no wave is asked for more logits than it has");
+    return len < 5u * (uint32_t)kThreads && len > kCap;
+}
 
 // accept() history -> per-token counts for [lo, hi) in LDS (src/gen/sampler.cpp:15-18); generic form used
 // when a row's history is too long for the register-resident scheme of load_penalised().
@@ -45,10 +65,10 @@ struct RawSlice {
 };
 typedef float f32x4_any __attribute__((ext_vector_type(4), aligned(4)));
 
-template <bool ALIGNED>
+template <bool ALIGNED, bool MIXED = false>
 __device__ __forceinline__ void load_raw(const mako_sample_desc& d, uint32_t row, uint32_t lo, uint32_t hi, RawSlice& r)
 {
-    const uint32_t tid = threadIdx.x;
+    const uint32_t tid = slice_thread<MIXED>();
     const global_ptr<const float> lrow = as_global(d.logits) + (int64_t)row * d.logits_stride;
     const global_ptr<const uint32_t> mrow = d.mask ? as_global(d.mask) + (int64_t)row * d.mask_stride : nullptr;
     // all four loads go out back to back, from clamped addresses and without a branch between them (a branch
@@ -92,7 +112,7 @@ __device__ __forceinline__ void load_raw(const mako_sample_desc& d, uint32_t row
 
 // The row's last group, of one to three logits, moved to the front of its four, behind it NaN.  (A slice ends behind a whole
 // group everywhere else.)
-template <bool ALIGNED>
+template <bool ALIGNED, bool MIXED = false>
 __device__ __forceinline__ void settle_slice(RawSlice& r, uint32_t lo, uint32_t hi)
 {
     if (ALIGNED || (hi & 3u) == 0u) // uniform
@@ -100,7 +120,7 @@ __device__ __forceinline__ void settle_slice(RawSlice& r, uint32_t lo, uint32_t 
     const float nan = __uint_as_float(0x7fc00000u);
 #pragma unroll
     for (uint32_t k = 0; k < 4; ++k) {
-        if (lo + k * 4096u + threadIdx.x * 4u == (hi & ~3u)) {
+        if (lo + k * 4096u + slice_thread<MIXED>() * 4u == (hi & ~3u)) {
             const uint32_t n = hi & 3u;
             const float4 x = r.v[k];
             r.v[k].x = n == 3u ? x.y : (n == 2u ? x.z : x.w);
@@ -113,9 +133,10 @@ __device__ __forceinline__ void settle_slice(RawSlice& r, uint32_t lo, uint32_t 
 
 // How many of the thread's logits (as the sampler is given them: a token the mask clears is -inf) are strictly
 // greater than v: the count of ReasoningBudget::forced, src/server/openai.cpp:599-602.
+template <bool MIXED>
 __device__ __forceinline__ uint32_t count_above(const RawSlice& r, uint32_t lo, uint32_t hi, float v)
 {
-    const uint32_t tid = threadIdx.x;
+    const uint32_t tid = slice_thread<MIXED>();
     uint32_t c = 0;
 #pragma unroll
     for (uint32_t k = 0; k < 4; ++k) {
@@ -131,11 +152,11 @@ __device__ __forceinline__ uint32_t count_above(const RawSlice& r, uint32_t lo, 
 
 // Mask and penalties (src/gen/sampler.cpp:22-28) applied to the raw logits; slots past the end of the
 // slice hold NaN, which never wins a comparison and never becomes a candidate.
-template <bool ALIGNED>
+template <bool ALIGNED, bool MIXED = false>
 __device__ __forceinline__ void finish_slice(const RawSlice& r, uint32_t lo, uint32_t hi, const mako_sampling_params& P,
                                              bool pen, const uint32_t* s_cnt, float (&wv)[16], bool masked)
 {
-    const uint32_t tid = threadIdx.x;
+    const uint32_t tid = slice_thread<MIXED>();
     const float nan = __uint_as_float(0x7fc00000u);
     if (!masked) { // uniform: no mask, nothing to clear
 #pragma unroll
@@ -204,7 +225,7 @@ struct SliceLoads {
     RawSlice raw;
     uint32_t tok[KH > 0 ? KH : 1], cnt[KH > 0 ? KH : 1];
 };
-template <bool ALIGNED, int KH>
+template <bool ALIGNED, int KH, bool MIXED = false>
 __device__ __forceinline__ void issue_slice(const mako_sample_desc& d, uint32_t row, uint32_t lo, uint32_t hi, SliceLoads<KH>& s)
 {
     const uint32_t tid = threadIdx.x;
@@ -227,7 +248,7 @@ __device__ __forceinline__ void issue_slice(const mako_sample_desc& d, uint32_t 
                 s.cnt[k] = hc[min(tid + (uint32_t)k * kThreads, last)];
         }
     }
-    load_raw<ALIGNED>(d, row, lo, hi, s.raw);
+    load_raw<ALIGNED, MIXED>(d, row, lo, hi, s.raw);
 }
 // (the table of counts is cleared while the loads are on their way, also for a row that may turn out to have no history;
 // `penalised`: it has penalties, and a use for them)
@@ -242,34 +263,34 @@ __device__ __forceinline__ void clear_counts(const mako_sample_desc& d, bool pen
 }
 
 // The rest, on what issue_slice() has asked for; the table is clear.
-template <bool ALIGNED, int KH>
+template <bool ALIGNED, int KH, bool MIXED = false>
 __device__ __forceinline__ void finish_penalised(const mako_sample_desc& d, uint32_t row, uint32_t lo, uint32_t hi, uint32_t slice_len,
                                                  const mako_sampling_params& P, uint32_t hl, bool pen, uint32_t* s_cnt, SliceLoads<KH>& s,
                                                  float (&wv)[16], bool want_above = false, float close_v = 0.0f, uint32_t* above = nullptr)
 {
-    const uint32_t tid = threadIdx.x;
+    const uint32_t tid = threadIdx.x, mine = slice_thread<MIXED>();
     RawSlice& raw = s.raw;
     uint32_t (&tok)[KH > 0 ? KH : 1] = s.tok;
     uint32_t (&cnt)[KH > 0 ? KH : 1] = s.cnt;
     const bool hc = d.hist_counts != nullptr;
     bool have[KH > 0 ? KH : 1];
     if (want_above) { // uniform
-        settle_slice<ALIGNED>(raw, lo, hi);
-        *above = count_above(raw, lo, hi, close_v);
+        settle_slice<ALIGNED, MIXED>(raw, lo, hi);
+        *above = count_above<MIXED>(raw, lo, hi, close_v);
     }
     auto settle = [&]() {
         if (!want_above)
-            settle_slice<ALIGNED>(raw, lo, hi);
+            settle_slice<ALIGNED, MIXED>(raw, lo, hi);
     };
     if (!pen) {
         settle();
-        finish_slice<ALIGNED>(raw, lo, hi, P, false, s_cnt, wv, d.mask != nullptr);
+        finish_slice<ALIGNED, MIXED>(raw, lo, hi, P, false, s_cnt, wv, d.mask != nullptr);
         return;
     }
     if (KH == 0) {
         build_counts(d, row, hl, lo, hi, slice_len, s_cnt);
         settle();
-        finish_slice<ALIGNED>(raw, lo, hi, P, true, s_cnt, wv, d.mask != nullptr);
+        finish_slice<ALIGNED, MIXED>(raw, lo, hi, P, true, s_cnt, wv, d.mask != nullptr);
         return;
     }
 #pragma unroll
@@ -305,13 +326,13 @@ __device__ __forceinline__ void finish_penalised(const mako_sample_desc& d, uint
     lds_barrier(); // (the slots are about to be overwritten)
     MAKO_STAMP(22);
     settle();
-    finish_slice<ALIGNED>(raw, lo, hi, P, false, s_cnt, wv, d.mask != nullptr);
+    finish_slice<ALIGNED, MIXED>(raw, lo, hi, P, false, s_cnt, wv, d.mask != nullptr);
     MAKO_STAMP(23);
     // owners: a logit whose slot is taken goes into the slot (its bits); `moved` remembers which of the sixteen
     uint32_t moved = 0;
 #pragma unroll
     for (uint32_t k = 0; k < 4; ++k) {
-        const uint32_t i = lo + k * 4096u + tid * 4u;
+        const uint32_t i = lo + k * 4096u + mine * 4u;
         if (i < hi) {
             uint4* slot = reinterpret_cast<uint4*>(s_cnt + (i - lo));
             const uint4 n = *slot;
@@ -335,7 +356,7 @@ __device__ __forceinline__ void finish_penalised(const mako_sample_desc& d, uint
 #pragma unroll
         for (uint32_t k = 0; k < 4; ++k)
             if ((moved >> (4u * k)) & 0xfu) {
-                const uint4 v = *reinterpret_cast<const uint4*>(s_cnt + (k * 4096u + tid * 4u));
+                const uint4 v = *reinterpret_cast<const uint4*>(s_cnt + (k * 4096u + mine * 4u));
                 wv[4 * k + 0] = (moved >> (4u * k)) & 1u ? __uint_as_float(v.x) : wv[4 * k + 0];
                 wv[4 * k + 1] = (moved >> (4u * k)) & 2u ? __uint_as_float(v.y) : wv[4 * k + 1];
                 wv[4 * k + 2] = (moved >> (4u * k)) & 4u ? __uint_as_float(v.z) : wv[4 * k + 2];
@@ -346,17 +367,17 @@ __device__ __forceinline__ void finish_penalised(const mako_sample_desc& d, uint
 
 // `overlap` runs right after the slice's loads have been issued: work that does not depend on them hides
 // behind their latency.  It must be reached by the whole workgroup or by none of it.
-template <bool ALIGNED, int KH, typename Overlap = NoOverlap>
+template <bool ALIGNED, int KH, bool MIXED = false, typename Overlap = NoOverlap>
 __device__ __forceinline__ void load_penalised(const mako_sample_desc& d, uint32_t row, uint32_t lo, uint32_t hi,
                                                uint32_t slice_len, const mako_sampling_params& P, bool penalised, uint32_t hl, bool pen,
                                                uint32_t* s_cnt, float (&wv)[16], Overlap overlap = Overlap(),
                                                bool want_above = false, float close_v = 0.0f, uint32_t* above = nullptr)
 {
     SliceLoads<KH> s;
-    issue_slice<ALIGNED, KH>(d, row, lo, hi, s);
+    issue_slice<ALIGNED, KH, MIXED>(d, row, lo, hi, s);
     clear_counts<KH>(d, penalised, slice_len, s_cnt);
     overlap();
-    finish_penalised<ALIGNED, KH>(d, row, lo, hi, slice_len, P, hl, pen, s_cnt, s, wv, want_above, close_v, above);
+    finish_penalised<ALIGNED, KH, MIXED>(d, row, lo, hi, slice_len, P, hl, pen, s_cnt, s, wv, want_above, close_v, above);
 }
 
 } // namespace mako

@@ -1,5 +1,5 @@
-"""GPU parity of rows that one workgroup's waves do not all hold logits of, and that are too long for a candidate list of all of
-their logits (513 to 4 092): top-k rows of any such length are finished from their candidates, aligned or not."""
+"""GPU parity of rows of few logits per wave that are too long for a candidate list of all of them (513 to 5 116): top-k rows of any
+such length are finished from their candidates, aligned or not, whatever their histories penalise."""
 import numpy as np
 import pytest
 
@@ -22,8 +22,9 @@ def _batch(vocab, seed):
     return dict(name="short V=%d" % vocab, logits=x, params=p, u=rng.random(rows).astype(np.float32))
 
 
-# (512: the longest row whose list may hold all of it; the last wave's first logit, a few and all of them; 4 096: no wave without)
-@pytest.mark.parametrize("vocab", [511, 512, 513, 600, 681, 767, 768, 769, 1003, 2048, 2049, 3001, 3840, 3841, 3845, 3899, 4092, 4093, 4096, 4097])
+# (512: the longest row whose list may hold all of it; around whole groups of 256, and of 4 096; 5 116: the longest
+# of these rows)
+@pytest.mark.parametrize("vocab", [511, 512, 513, 600, 681, 767, 768, 769, 1003, 2048, 2049, 3001, 3840, 3841, 3845, 3899, 4092, 4093, 4096, 4097, 5115, 5116, 5117, 5121])
 def test_short_rows(vocab):
     w = _batch(vocab, 1)
     ctx = api.SamplerContext(max_rows=16, max_vocab=vocab, max_hist=64)
@@ -44,5 +45,28 @@ def test_short_rows(vocab):
         w["hist_len"] = np.full(len(w["u"]), 50, np.uint32)
         for hinted in (True, False):
             assert_parity(ctx, w, cap=600, hinted=hinted)
+    finally:
+        ctx.close()
+
+
+# (a history that names the first tokens most often, on rows as flat as they come: those tokens' logits are no one's candidates)
+@pytest.mark.parametrize("vocab", [600, 901, 2067, 2068, 3068, 4101, 4352, 5116])
+@pytest.mark.parametrize("hist", [1000, 2048, 5000, 9000])
+def test_short_rows_with_long_histories(vocab, hist):
+    rows = 5
+    rng = np.random.Generator(np.random.PCG64([vocab, hist]))
+    p = api.make_params(rows, 0.7, 40, 0.95)
+    p["top_k"][1], p["top_k"][4], p["top_p"][4] = 20, 0, 0.9
+    for name, v in (("repetition_penalty", 1.1), ("frequency_penalty", 0.2), ("presence_penalty", 0.3)):
+        p[name] = np.float32(v)
+    cdf = np.cumsum(np.arange(1, vocab + 1) ** -1.1)
+    w = dict(name="V=%d hist=%d" % (vocab, hist), params=p, logits=(rng.standard_normal((rows, vocab)) * 0.1).astype(np.float32),
+             u=rng.random(rows).astype(np.float32), hist_len=np.full(rows, hist, np.uint32),
+             hist=np.minimum(np.searchsorted(cdf, rng.random((rows, hist)) * cdf[-1]), vocab - 1).astype(np.int32))
+    ctx = api.SamplerContext(max_rows=rows, max_vocab=vocab, max_hist=hist)
+    try:
+        for hinted in (True, False):
+            g = assert_parity(ctx, w, cap=600, hinted=hinted)
+            assert (g["path"][:4] == api.PATH_TOPK).all(), g["path"]
     finally:
         ctx.close()
