@@ -401,9 +401,9 @@ __device__ __forceinline__ void few_candidates_row(const mako_sample_desc& d, co
 
 // What these kernels have left of a row of theirs (flag: of its plan, which is zero again behind this), by one workgroup: the
 // rest of the whole-row path, or the total and the draw.  All threads call; sm.tab must hold the exp2 table.  ALL_KINDS: rows
-// that are not in token order are among them.  (With their code in it the kernel spills twice as many registers on its way into
-// every row; both need as much scratch memory.  With a min-p, without it and with it: one row of 16 000 24.4 us and 25.1, 256 rows
-// of 1 000 38.0 and 39.0; 64 rows of 129 280, temperature only, 76.6 and 76.9.)
+// that are not in token order are among them.  (Without their code, and with it, as much scratch memory either way.  With a min-p: one
+// row of 129 280 21.8 us and 22.2, 64 of them 37.2 and 37.6, 512 rows of 700 28.4 and 29.0; temperature only, one row 39.1 and 39.6,
+// 64 76.2 and 76.5.)
 // Returns whether the row is one for few_candidates_row(), which the caller calls (from here it would be deeper in the stack).
 template <bool ALL_KINDS = true>
 __device__ __forceinline__ bool finish_index_row_here(const mako_sample_desc& d, const Scratch& sc, const mako_sampling_params& P, uint32_t row,

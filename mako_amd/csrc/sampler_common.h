@@ -87,8 +87,9 @@ constexpr uint32_t kGroup = 256;      // a sorted list is processed in groups of
 constexpr uint32_t kMaxGroups = 1024; // groups per list
 constexpr uint32_t kSegCap = 6144;    // entries a worker sorts in LDS
 constexpr uint32_t kFine = 2048;      // value buckets of that sort
-// dynamic LDS of sort_kernel: the entries in the order of their buckets (and four more), the buckets, and a copy of the sorted
-// weights for the group records
+// dynamic LDS of sort_kernel: for the sort the entries in the order of their buckets (and four more), the buckets, and a copy of the
+// sorted weights for the group records, 81 968 bytes; for a narrow row the lists that its tail works on, kTailLds, 90 112 bytes, which
+// is what the launch asks for.  With its 100 vector registers a workgroup has a CU to itself either way.
 constexpr uint32_t kSortedCopyAt = (kSegCap + 4u) * 8u + (kFine + 4u) * 4u; // byte offset of that copy
 constexpr uint32_t kSortLds = (kSortedCopyAt + kSegCap * 4u) > kTailLds ? (kSortedCopyAt + kSegCap * 4u) : kTailLds;
 
