@@ -55,6 +55,14 @@ __device__ __forceinline__ lds_ptr<T> as_lds(T* p)
 {
     return (lds_ptr<T>)p;
 }
+// An address that is the same in all lanes, in scalar registers.
+template <typename T>
+__device__ __forceinline__ global_ptr<T> uniform_ptr(global_ptr<T> p)
+{
+    const unsigned long long a = (unsigned long long)p;
+    const uint32_t lo = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)a), hi = (uint32_t)__builtin_amdgcn_readfirstlane((int)(uint32_t)(a >> 32));
+    return (global_ptr<T>)(((unsigned long long)hi << 32) | (unsigned long long)lo);
+}
 typedef uint32_t u32x4 __attribute__((ext_vector_type(4))); // (plain vector types: they load from any address space)
 typedef float f32x4 __attribute__((ext_vector_type(4)));
 

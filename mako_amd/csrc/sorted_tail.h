@@ -120,7 +120,7 @@ __device__ bool sorted_tail(const mako_sample_desc& d, uint32_t row, const mako_
     };
     const GroupLds G = group_lds(L);
     const bool topp_active = P.top_p < 1.0f;
-    if (!PLANNED && n1 > kGroup * kMaxGroups) {
+    if (!PLANNED && !SHORT_ONLY && n1 > kGroup * kMaxGroups) {
         // oversized lists take the generic windowed replay
         uint32_t n = n1;
         if (topp_active) {
@@ -171,7 +171,8 @@ __device__ bool sorted_tail(const mako_sample_desc& d, uint32_t row, const mako_
         }
         if (need_cut && !(q_bound < qat(n - 1)))
             return false;
-        draw_from_list(d, row, qat, idat, n, path, sm);
+        // (a call: so long a list is rare, and the code for it, in line, costs every other list registers)
+        MAKO_CALL draw_from_list(d, row, qat, idat, n, path, sm);
         return true;
     }
 

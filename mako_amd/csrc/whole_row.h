@@ -882,10 +882,16 @@ __device__ bool sort_truncate_draw(const mako_sample_desc& d, uint32_t row, cons
         return true;
     }
     // nth_element's order (long lists), or neither top-k nor top-p: the candidates stay in index order
-    const uint32_t* kf = ks;
-    const uint32_t* jf = is;
-    draw_from_list(
-        d, row, [=](uint32_t i) { return __uint_as_float(~kf[i]); }, [=](uint32_t i) { return jf[i]; }, n1, path, sm);
+    // (qk: general_row(), whose long lists gain from addresses in scalar registers; general_row_from_weights(), whose registers
+    // those are short of, loses by them: 64 rows, top_k 200 to 1 000, 71.4 us and 72.3)
+    auto draw = [&](auto kf, auto jf) {
+        draw_from_list(
+            d, row, [=](uint32_t i) { return __uint_as_float(~kf[i]); }, [=](uint32_t i) { return jf[i]; }, n1, path, sm);
+    };
+    if (qk) // uniform
+        draw(uniform_ptr(as_global(ks)), uniform_ptr(as_global(is)));
+    else
+        draw(GlobalKeys{ks}, GlobalKeys{is});
     return true;
 }
 
@@ -1110,6 +1116,11 @@ __device__ MAKO_RARE_CALL void general_row(const mako_sample_desc& d, const Scra
     const float inv_t = 1.0f / P.temperature;
     const float floor_q = (1.0f < P.min_p) ? 1.0f : P.min_p; // std::min(min_p, 1.0f)
     uint32_t* qb = reinterpret_cast<uint32_t*>(wbuf);
+    // (The arrays by typed addresses in scalar registers, for the draw too: in vector registers they are spilled, and fetched from
+    // scratch memory again for every 256 logits.  Rows in token order with gaps whose candidates are written out: three of 136 640
+    // logits 500 us, 430 so; 39 of 34 688 325 and 282.  One row of 300 000 1 016 and 925.)
+    const global_ptr<float> wg = uniform_ptr(as_global(wbuf));
+    const global_ptr<uint32_t> qg = (global_ptr<uint32_t>)wg, kg = uniform_ptr(as_global(key0)), ig = uniform_ptr(as_global(idx0));
     const uint32_t lane = lane_id(), wave = wave_id();
     const uint32_t chunk = ((V + kThreads * 4u - 1u) / (kThreads * 4u)) * kGroup;
     const uint32_t beg = min(V, wave * chunk), end = min(V, beg + chunk);
@@ -1119,13 +1130,13 @@ __device__ MAKO_RARE_CALL void general_row(const mako_sample_desc& d, const Scra
         float w[4] = {0.0f, 0.0f, 0.0f, 0.0f};
         const bool whole = i + 3u < end;
         if (whole) {
-            const float4 x = *reinterpret_cast<const float4*>(wbuf + i);
+            const f32x4 x = *(global_ptr<const f32x4>)(wg + i);
             w[0] = x.x, w[1] = x.y, w[2] = x.z, w[3] = x.w;
         } else {
 #pragma unroll
             for (uint32_t j = 0; j < 4; ++j)
                 if (i + j < end)
-                    w[j] = wbuf[i + j];
+                    w[j] = wg[i + j];
         }
         uint32_t k[4];
 #pragma unroll
@@ -1135,12 +1146,12 @@ __device__ MAKO_RARE_CALL void general_row(const mako_sample_desc& d, const Scra
             mine += k[j] ? 1u : 0u;
         }
         if (whole) {
-            *reinterpret_cast<uint4*>(qb + i) = make_uint4(k[0], k[1], k[2], k[3]);
+            *(global_ptr<u32x4>)(qg + i) = u32x4{k[0], k[1], k[2], k[3]};
         } else {
 #pragma unroll
             for (uint32_t j = 0; j < 4; ++j)
                 if (i + j < end)
-                    qb[i + j] = k[j];
+                    qg[i + j] = k[j];
         }
     }
     mine = __ockl_wfred_add_u32(mine);
@@ -1158,13 +1169,13 @@ __device__ MAKO_RARE_CALL void general_row(const mako_sample_desc& d, const Scra
         const uint32_t i = base + lane * 4u;
         uint32_t k[4] = {0u, 0u, 0u, 0u};
         if (i + 3u < end) {
-            const uint4 x = *reinterpret_cast<const uint4*>(qb + i);
+            const u32x4 x = *(global_ptr<const u32x4>)(qg + i);
             k[0] = x.x, k[1] = x.y, k[2] = x.z, k[3] = x.w;
         } else {
 #pragma unroll
             for (uint32_t j = 0; j < 4; ++j)
                 if (i + j < end)
-                    k[j] = qb[i + j];
+                    k[j] = qg[i + j];
         }
         const uint32_t c = (k[0] ? 1u : 0u) + (k[1] ? 1u : 0u) + (k[2] ? 1u : 0u) + (k[3] ? 1u : 0u);
         const uint32_t incl = __ockl_wfscan_add_u32(c, true);
@@ -1173,8 +1184,8 @@ __device__ MAKO_RARE_CALL void general_row(const mako_sample_desc& d, const Scra
         for (uint32_t j = 0; j < 4; ++j)
             if (k[j]) {
                 MAKO_CHECK(sc, kCheckCompact, pos < n0 && (uint64_t)pos < sc.vpad);
-                key0[pos] = ~k[j];
-                idx0[pos] = i + j;
+                kg[pos] = ~k[j];
+                ig[pos] = i + j;
                 ++pos;
             }
         at += (uint32_t)__builtin_amdgcn_readlane((int)incl, kWave - 1);
