@@ -1,4 +1,4 @@
-// Workgroup-wide primitives for 1024-thread workgroups of 64-wide wavefronts.
+// Workgroup-wide primitives for workgroups of kThreads threads and 64-wide wavefronts.
 // Every function must be reached by all threads of the workgroup.
 #pragma once
 
@@ -20,7 +20,11 @@ extern "C" __device__ float __ockl_wfscan_add_f32(float, bool inclusive);
 
 namespace mako {
 
-constexpr int kThreads = 1024;
+// Threads of a workgroup: 1024, but for a translation unit that says otherwise (mako_amd/build.py).
+#ifndef MAKO_THREADS
+#define MAKO_THREADS 1024
+#endif
+constexpr int kThreads = MAKO_THREADS;
 constexpr int kWave = 64;
 constexpr int kWaves = kThreads / kWave;
 

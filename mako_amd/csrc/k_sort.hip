@@ -1,7 +1,8 @@
 // sort_kernel: the wide rows' shares sorted by their workers; narrow nuclei finished by one worker.
+#define MAKO_THREADS 512
 #define MAKO_EMIT_SORT_KERNELS
 #include "launch.h"
-#include "sampler_kernels.h"
+#include "sort_kernels.h"
 
 namespace mako {
 void launch_sort_unsorted(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices, uint32_t grid_rows);
@@ -17,7 +18,6 @@ void launch_sort(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, u
 hipError_t init_sort_unsorted();
 hipError_t init_sort_kernels()
 {
-    static_assert(kSortLds >= kTailLds, "sort_kernel's tail uses the finishing kernels' LDS layout");
     const hipError_t e = hipFuncSetAttribute((const void*)sort_kernel, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kSortLds);
     return e != hipSuccess ? e : init_sort_unsorted();
 }

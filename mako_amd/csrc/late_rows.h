@@ -5,7 +5,7 @@
 
 #include "row_records.h"
 #include "sorted_tail.h"
-#include "topk_candidates.h"
+#include "topk_row.h"
 #include "whole_row.h"
 #include "index_rows.h"
 

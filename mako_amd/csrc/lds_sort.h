@@ -5,7 +5,7 @@
 
 namespace mako {
 
-// The sort of a worker's share, and of what a wide top-k keeps, in LDS: up to kSegCap entries (bits(q), idx), entry t * 1024 + tid in this thread's k[t] / id[t], all with
+// The sort of a worker's share, and of what a wide top-k keeps, in LDS: up to kSegCap entries (bits(q), idx), entry t * kThreads + tid in this thread's k[t] / id[t], all with
 // key_lo <= bits(q) < key_hi, are dropped into kFine value buckets (descending), and every entry finds its place by counting
 // the entries of its own bucket that precede it under (q desc, idx asc); they go to kout / iout as ~bits(q) and token id.
 // Returns false when a bucket is too crowded to be ranked by counting.  hist must be zero and sm.flag 0 on entry, behind a
@@ -17,6 +17,8 @@ namespace mako {
 // them; and whoever counts may read past the bucket's end, where all there is is smaller.  With the two halves compared and the
 // reads held inside the bucket the counting took 4.3 of a worker's 11.7 us for 4 400 entries; 2.2 of 9.7 so.)
 constexpr uint32_t kSortPer = kSegCap / (uint32_t)kThreads;
+constexpr uint32_t kFinePer = kFine / (uint32_t)kThreads; // buckets a thread
+static_assert(kSegCap % (uint32_t)kThreads == 0 && kFine % (uint32_t)kThreads == 0, "whole rounds of the workgroup");
 __device__ bool lds_bucket_sort(const uint32_t (&k)[kSortPer], const uint32_t (&id)[kSortPer], uint32_t n, uint32_t key_lo, uint32_t key_hi,
                                 uint32_t* kout, uint32_t* iout, unsigned long long* dyn, FinishShared& sm, uint32_t* sorted_lds = nullptr)
 {
@@ -37,13 +39,22 @@ __device__ bool lds_bucket_sort(const uint32_t (&k)[kSortPer], const uint32_t (&
     }
     lds_barrier();
     {
-        const uint32_t c0 = hist[2u * tid], c1 = hist[2u * tid + 1u];
-        if (max(c0, c1) > 64u)
+        uint32_t c[kFinePer], mine = 0, most = 0;
+#pragma unroll
+        for (uint32_t j = 0; j < kFinePer; ++j) {
+            c[j] = hist[kFinePer * tid + j];
+            mine += c[j];
+            most = max(most, c[j]);
+        }
+        if (most > 64u)
             sm.flag = 1;
         uint32_t total;
-        const uint32_t ex = block_excl_scan_u32(c0 + c1, total, sm.bs); // (barriers: all counts are read before)
-        hist[2u * tid] = ex;
-        hist[2u * tid + 1u] = ex + c0;
+        uint32_t ex = block_excl_scan_u32(mine, total, sm.bs); // (barriers: all counts are read before)
+#pragma unroll
+        for (uint32_t j = 0; j < kFinePer; ++j) {
+            hist[kFinePer * tid + j] = ex;
+            ex += c[j];
+        }
         if (tid == 0)
             hist[kFine] = total;
     }

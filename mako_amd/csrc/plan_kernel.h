@@ -1,7 +1,7 @@
 // plan_kernel: one workgroup per row of a batch that needs neither the second pass nor the sort.
 #pragma once
 
-#include "topk_candidates.h"
+#include "topk_row.h"
 
 namespace mako {
 

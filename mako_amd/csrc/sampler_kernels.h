@@ -29,6 +29,7 @@
 #include "worker_sort.h"
 #include "row_records.h"
 #include "topk_candidates.h"
+#include "topk_row.h"
 #include "second_pass.h"
 #include "plan_kernel.h"
 #include "sort_kernels.h"

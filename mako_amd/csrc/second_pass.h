@@ -76,9 +76,9 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
             const uint32_t unsorted = (UNSORTED && flag == 1) ? pl.opq_mask : 0u;
             plan->opq_mask = unsorted;
             if (flag == 1 || flag == 3) {
-                // sort_kernel's work: a workgroup per worker that sorts, and up to kCollectors whose waves take one of the
-                // row's unsorted shares each (work items kWorkers + c)
-                const uint32_t n_unsorted = (uint32_t)__popc(unsorted), collectors = (n_unsorted + (uint32_t)kWaves - 1u) / (uint32_t)kWaves;
+                // sort_kernel's work: a workgroup per worker that sorts, and up to kCollectors whose waves take the row's
+                // unsorted shares, a share at a time (work items kWorkers + c)
+                const uint32_t n_unsorted = (uint32_t)__popc(unsorted), collectors = (n_unsorted + kCollected - 1u) / kCollected;
                 if constexpr (UNSORTED) {
                     // (two lists, the costly entries in front: large_batch_lists())
                     const SortLists lists = large_batch_lists(pl.nucleus_rows);

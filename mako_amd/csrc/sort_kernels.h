@@ -169,19 +169,21 @@ __device__ __forceinline__ void sort_body(const mako_sample_desc& d_arg, const S
     const uint32_t gbase = (uint32_t)__builtin_amdgcn_readlane((int)(grp_upto - grp_l), (int)w);
     const size_t t_row = (size_t)row * sc.g_cap;
     if (UNSORTED && w >= kWorkers) {
-        // One of the row's collectors: each of its waves takes one of the shares that are left unsorted (collector c the
-        // shares 16 c .. 16 c + 15 of them) and leaves its record.  (The binades of the increments from the plan's estimates in
+        // One of the row's collectors: each of its waves takes one of the shares that are left unsorted, or two (collector c
+        // the shares 16 c .. 16 c + 15 of them), and leaves its record.  (The binades of the increments from the plan's estimates in
         // the exact total's units; any guess is safe, the tail tests what it applies.  A verification row has no such
         // shares.)
         MAKO_WG_TAG(0xc0000000u);
         const double r0_raw = (double)u_row * ((double)s_args.P.top_p * total64);
         const double r0 = r0_raw == r0_raw ? r0_raw : 0.0, scale = mass_all > 0.0 ? total64 / mass_all : 0.0;
         uint32_t* wave_lds = reinterpret_cast<uint32_t*>(s_dyn64) + (uint32_t)wave_id() * (kOpaqueLdsWords + 2u);
-        const uint32_t mine = (w - kWorkers) * (uint32_t)kWaves + (uint32_t)wave_id();
+        uint32_t mine = (w - kWorkers) * kCollected + (uint32_t)wave_id();
+        const uint32_t end = (w - kWorkers + 1u) * kCollected;
         uint32_t rank = 0;
         for (uint32_t v = 0; v + 1u < kWorkers; ++v) { // (uniform)
-            if (!((opq_mask >> v) & 1u) || rank++ != mine)
+            if (!((opq_mask >> v) & 1u) || rank++ != mine || mine >= end)
                 continue;
+            mine += (uint32_t)kWaves;
             const uint32_t cnt_v = (uint32_t)__builtin_amdgcn_readlane((int)cnt_l, (int)v);
             const uint32_t stage_v = (uint32_t)__builtin_amdgcn_readlane((int)stage_l, (int)v);
             const uint32_t off_v = (uint32_t)__builtin_amdgcn_readlane((int)(cnt_upto - cnt_l), (int)v);
@@ -250,8 +252,14 @@ __device__ __forceinline__ void sort_body(const mako_sample_desc& d_arg, const S
     }
 }
 #ifdef MAKO_EMIT_SORT_KERNELS // (not templates: defined by the one translation unit that launches them)
+// Workgroups of 512, two to a CU (four waves a SIMD: 128 registers).  A worker is three dependent trips to memory, some twenty
+// barriers and vector instructions for 40 % of the time in between: with 1 024 threads, alone on its CU, it leaves it idle for most of
+// that, and two workgroups that have nothing to do with each other fill each other's gaps.  (256 rows of 151 552 logits, half of
+// them flat: the kernel 100 -> 66 us, the batch 289 -> 255; 97 nucleus rows of 512 189 -> 186.)  On a small batch, where a worker
+// has a CU to itself either way, half the waves start and meet sooner (one row 43.8 -> 42.9 us, 64 rows 58.0 -> 57.3).
+// (sort_beside_kernel has 1 024, as the groups and steps in it want.)
 #ifdef MAKO_SORT_UNSORTED
-__global__ __launch_bounds__(kThreads) void sort_kernel_unsorted(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices)
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void sort_kernel_unsorted(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices)
 {
     extern __shared__ __align__(16) unsigned long long s_dyn64[]; // (128-bit LDS operations need the alignment)
     __shared__ FinishShared sm;
@@ -261,7 +269,7 @@ __global__ __launch_bounds__(kThreads) void sort_kernel_unsorted(mako_sample_des
     sort_body<true>(d_arg, sc_val, slices, first, s_dyn64, sm, s_args);
 }
 #else
-__global__ __launch_bounds__(kThreads) void sort_kernel(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices)
+__global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void sort_kernel(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices)
 {
     extern __shared__ __align__(16) unsigned long long s_dyn64[]; // (128-bit LDS operations need the alignment)
     __shared__ FinishShared sm;

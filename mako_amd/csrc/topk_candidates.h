@@ -1,8 +1,7 @@
-// Top-k rows (and narrow nuclei) resolved from the candidate lists scan_kernel left.
+// The candidate lists scan_kernel left of a row: their weights, and the heaviest of them in order.
 #pragma once
 
 #include "row_records.h"
-#include "whole_row.h"
 
 namespace mako {
 
@@ -12,7 +11,7 @@ namespace mako {
 #ifndef MAKO_TOPK_PART
 #define MAKO_TOPK_PART
 #endif
-// Keys (bits(q) << 32 | ~token id, 0 = not a candidate) of candidates t * 1024 + tid of the row's flattened
+// Keys (bits(q) << 32 | ~token id, 0 = not a candidate) of candidates t * kThreads + tid of the row's flattened
 // candidate list (all slices; sm.soff holds the slices' offsets), t < ITEMS.  Positions first, then every load
 // from a clamped position with no branch in between (a branch around each load would make it wait for the one
 // before), then the weights of the candidates that exist.
@@ -25,7 +24,7 @@ __device__ __forceinline__ void candidate_keys(const Scratch& sc, uint32_t row, 
     size_t at[ITEMS];
 #pragma unroll
     for (uint32_t t = 0; t < (uint32_t)ITEMS; ++t) {
-        const uint32_t c = t * 1024u + tid < n_cands ? t * 1024u + tid : 0u; // (past the end: candidate 0, a short search)
+        const uint32_t e = t * (uint32_t)kThreads + tid, c = e < n_cands ? e : 0u; // (past the end: candidate 0, a short search)
         uint32_t s = 0;
         while (s + 1 < slices && c >= sm.soff[s + 1]) // slice holding candidate c
             ++s;
@@ -44,20 +43,21 @@ __device__ __forceinline__ void candidate_keys(const Scratch& sc, uint32_t row, 
 #pragma unroll
     for (uint32_t t = 0; t < (uint32_t)ITEMS; ++t) {
         key[t] = 0;
-        if (t * 1024u < n_cands) { // uniform: whole trips past the end of the list are skipped
+        if (t * (uint32_t)kThreads < n_cands) { // uniform: whole trips past the end of the list are skipped
             const float q = weight_of(w[t], m, inv_t, sm.tab);
-            if (t * 1024u + tid < n_cands && q >= floor_q && q > 0.0f)
+            if (t * (uint32_t)kThreads + tid < n_cands && q >= floor_q && q > 0.0f)
                 key[t] = ((unsigned long long)__float_as_uint(q) << 32) | (unsigned long long)(kNone - id[t]);
         }
     }
 }
 
 // The same keys from the candidate lists read as SLOTS: thread tid takes entries (tid % 128) + 128 t, t < 4, of slice
-// tid / 128, whether or not the slice emitted that many.  Where the lists end is not needed to ask for them, so the
+// tid / 128 (in a workgroup of 1024; an eighth of the threads to a slice in any), whether or not the slice emitted that many.  Where the lists end is not needed to ask for them, so the
 // loads go out together with the loads of the slices' records instead of one trip to memory behind them; and
 // since every slice's list starts at t = 0, the trips past the longest list are skipped by whole waves.
 // For rows of at most eight slices.
-constexpr int kPrefetchItems = 4;
+constexpr uint32_t kSlotThreads = (uint32_t)kThreads / 8u;
+constexpr int kPrefetchItems = (int)(kCap / kSlotThreads);
 struct CandSlots {
     float w[kPrefetchItems];
     uint32_t id[kPrefetchItems];
@@ -65,27 +65,27 @@ struct CandSlots {
 __device__ __forceinline__ bool slots_cover(uint32_t slices) { return slices <= 8u; }
 __device__ __forceinline__ void fetch_candidate_slots(const Scratch& sc, uint32_t row, uint32_t slices, CandSlots& c)
 {
-    static_assert(kCap == (uint32_t)kPrefetchItems * 128u && kThreads == 1024, "eight slices of 128 threads, four entries each");
-    const uint32_t sl = min(threadIdx.x >> 7, slices - 1u), i0 = threadIdx.x & 127u;
+    static_assert(kCap == (uint32_t)kPrefetchItems * kSlotThreads && kSortMax == (uint32_t)(kPrefetchItems * kThreads), "eight slices' lists, one entry after the other");
+    const uint32_t sl = min(threadIdx.x / kSlotThreads, slices - 1u), i0 = threadIdx.x % kSlotThreads;
     const size_t base = ((size_t)row * sc.slices_cap + sl) * kCap + i0;
     const global_ptr<const float> cand_w = as_global(sc.cand_w);
     const global_ptr<const uint32_t> cand_i = as_global(sc.cand_i);
 #pragma unroll
     for (uint32_t t = 0; t < (uint32_t)kPrefetchItems; ++t) {
-        c.w[t] = cand_w[base + 128u * t];
-        c.id[t] = cand_i[base + 128u * t];
+        c.w[t] = cand_w[base + kSlotThreads * t];
+        c.id[t] = cand_i[base + kSlotThreads * t];
     }
 }
 // (sm.soff as candidate_bound() leaves it)
 __device__ __forceinline__ void keys_from_slots(const CandSlots& c, uint32_t slices, float m, float inv_t, float floor_q,
                                                 const FinishShared& sm, unsigned long long (&key)[kPrefetchItems])
 {
-    const uint32_t sl = min(threadIdx.x >> 7, slices - 1u), i0 = threadIdx.x & 127u;
-    const uint32_t emitted = (threadIdx.x >> 7) < slices ? sm.soff[sl + 1] - sm.soff[sl] : 0u;
+    const uint32_t sl = min(threadIdx.x / kSlotThreads, slices - 1u), i0 = threadIdx.x % kSlotThreads;
+    const uint32_t emitted = threadIdx.x / kSlotThreads < slices ? sm.soff[sl + 1] - sm.soff[sl] : 0u;
 #pragma unroll
     for (uint32_t t = 0; t < (uint32_t)kPrefetchItems; ++t) {
         key[t] = 0;
-        if (i0 + 128u * t < emitted) {
+        if (i0 + kSlotThreads * t < emitted) {
             const float q = weight_of(c.w[t], m, inv_t, sm.tab);
             if (q >= floor_q && q > 0.0f)
                 key[t] = ((unsigned long long)__float_as_uint(q) << 32) | (unsigned long long)(kNone - c.id[t]);
@@ -93,30 +93,7 @@ __device__ __forceinline__ void keys_from_slots(const CandSlots& c, uint32_t sli
     }
 }
 
-// The row's candidates (all slices) weighted, sorted by (q desc, idx asc) and left in LDS as kf[i] = ~bits(q_i),
-// jf[i] = token id, invalid ones (q not a candidate) last.  Returns the number of valid candidates.
-template <int ITEMS>
-__device__ MAKO_TOPK_PART uint32_t sort_candidates(const Scratch& sc, uint32_t row, uint32_t slices, uint32_t n_cands, float m, float inv_t,
-                                    float floor_q, uint32_t* kf, uint32_t* jf, const FinishLds& L)
-{
-    assume_lds(L);
-    FinishShared& sm = *L.sm;
-    const uint32_t tid = threadIdx.x;
-    unsigned long long key[ITEMS];
-    candidate_keys<ITEMS>(sc, row, slices, n_cands, m, inv_t, floor_q, sm, key);
-    bitonic_sort_regs<ITEMS>(key, as_lds(L.sortk));
-    uint32_t nv = 0;
-#pragma unroll
-    for (uint32_t t = 0; t < (uint32_t)ITEMS; ++t) {
-        kf[t * 1024u + tid] = ~(uint32_t)(key[t] >> 32);
-        jf[t * 1024u + tid] = kNone - (uint32_t)key[t];
-        nv += key[t] != 0;
-    }
-    return block_sum_u32(nv, sm.bs); // (its barriers publish kf / jf)
-}
-
-
-// Fast route for rows that need only a few of their candidates.  Every thread weights up to four candidates;
+// Fast route for rows that need only a few of their candidates.  Every thread weights up to kPrefetchItems candidates;
 // those at or above a weight threshold (at most kSmall of them) are ordered by (q desc, idx asc) by counting, for
 // each, the entries that precede it, and left in LDS as kf[i] = ~bits(q_i), jf[i] = token id.
 //   top_k > 0:  the threshold is the lower edge of the quarter-binade bin that holds the top_k-th largest weight
@@ -144,18 +121,18 @@ __device__ MAKO_TOPK_PART uint32_t small_candidates(const Scratch& sc, uint32_t 
         rank[tid] = 0;
     if (tid == 0)
         *counter = 0;
-    unsigned long long key[4];
-    static_assert(kPrefetchItems == 4, "one key array for both routes");
+    constexpr uint32_t kItems = (uint32_t)kPrefetchItems;
+    unsigned long long key[kItems];
     if (have_pre) // uniform
         keys_from_slots(pre, slices, m, inv_t, floor_q, sm, key);
     else
-        candidate_keys<4>(sc, row, slices, n_cands, m, inv_t, floor_q, sm, key);
+        candidate_keys<kPrefetchItems>(sc, row, slices, n_cands, m, inv_t, floor_q, sm, key);
     MAKO_STAMP(17);
     lds_barrier();
     uint32_t n_list;
     if (top_k > 0) {
 #pragma unroll
-        for (uint32_t t = 0; t < 4; ++t)
+        for (uint32_t t = 0; t < kItems; ++t)
             if (key[t])
                 atomicAdd(&hist[min((uint32_t)(key[t] >> 53), 511u)], 1u);
         lds_barrier();
@@ -194,7 +171,7 @@ __device__ MAKO_TOPK_PART uint32_t small_candidates(const Scratch& sc, uint32_t 
     } else {
         uint32_t mine = 0, ge = 0;
 #pragma unroll
-        for (uint32_t t = 0; t < 4; ++t) {
+        for (uint32_t t = 0; t < kItems; ++t) {
             mine += key[t] != 0;
             ge += key[t] != 0 && (uint32_t)(key[t] >> 32) >= thr_bits;
         }
@@ -208,7 +185,7 @@ __device__ MAKO_TOPK_PART uint32_t small_candidates(const Scratch& sc, uint32_t 
     // compaction in any order: the keys are distinct, the ranks below put them in place
     const unsigned long long lower = (1ull << lane_id()) - 1ull;
 #pragma unroll
-    for (uint32_t t = 0; t < 4; ++t) {
+    for (uint32_t t = 0; t < kItems; ++t) {
         const bool keep = key[t] != 0 && (uint32_t)(key[t] >> 32) >= thr_bits;
         const unsigned long long bal = __ballot(keep);
         if (bal) {
@@ -223,10 +200,11 @@ __device__ MAKO_TOPK_PART uint32_t small_candidates(const Scratch& sc, uint32_t 
     __syncthreads();
     MAKO_STAMP(19);
     {
-        const uint32_t e = tid & (kSmall - 1u), part = tid / kSmall; // four threads share the comparisons of an entry
+        const uint32_t e = tid & (kSmall - 1u), part = tid / kSmall; // kParts threads share the comparisons of an entry
+        constexpr uint32_t kParts = (uint32_t)kThreads / kSmall;
         const unsigned long long my = e < n_list ? sel[e] : ~0ull;
-        // each of the four takes a quarter of the list; waves whose entries lie past its end have nothing to count
-        const uint32_t chunk = (n_list + 3u) / 4u, jb = part * chunk, je = min(n_list, jb + chunk);
+        // each of them takes its part of the list; waves whose entries lie past its end have nothing to count
+        const uint32_t chunk = (n_list + kParts - 1u) / kParts, jb = part * chunk, je = min(n_list, jb + chunk);
         uint32_t r = 0;
         if ((e & ~(kWave - 1u)) < n_list) {
 #pragma unroll 4
@@ -244,54 +222,6 @@ __device__ MAKO_TOPK_PART uint32_t small_candidates(const Scratch& sc, uint32_t 
     }
     __syncthreads();
     return n_list;
-}
-
-// A top-k row (top_k <= kTopKFast) from the candidates scan_kernel left: weights of the candidates, the top_k-th
-// weight's neighbourhood ordered by (q desc, idx asc) in LDS, the certificate that nothing left behind in a slice can
-// reach the top_k-th weight, then top-p, total and draw by one wave.  A row that cannot be certified takes the
-// whole-row path: here and now (INLINE_GENERAL), or through sort_kernel's work list.
-#ifndef MAKO_TOPK_GENERAL_SITE
-#define MAKO_TOPK_GENERAL_SITE 1 // (the general_row instance a top-k row falls back to: 0 where one exists anyway)
-#endif
-__device__ __forceinline__ void topk_row(const mako_sample_desc& d, const Scratch& sc, uint32_t row, uint32_t slices,
-                                         const mako_sampling_params& P, float m, uint32_t argidx, uint32_t n_cands,
-                                         const SliceStat& lane_stat, const FinishLds& L, bool have_pre = false,
-                                         const CandSlots& pre = CandSlots{})
-{
-    assume_lds(L);
-    FinishShared& sm = *L.sm;
-    // ---- top-k rows: weights of the row's candidates, sorted by (q desc, idx asc) in LDS ----
-    const float inv_t = 1.0f / P.temperature;
-    const float floor_q = (1.0f < P.min_p) ? 1.0f : P.min_p;
-    const float q_bound = candidate_bound(lane_stat, slices, m, inv_t, floor_q, sm);
-    MAKO_STAMP(3);
-    uint32_t* kf = reinterpret_cast<uint32_t*>(L.sortk + kSortMax); // upper half of the dynamic block
-    uint32_t* jf = kf + kSortMax;
-    uint32_t n_valid = 0;
-    // the top_k-th weight's neighbourhood only
-    uint32_t n_list = small_candidates(sc, row, slices, n_cands, m, inv_t, floor_q, P.top_k, 0u, kf, jf, n_valid, L, have_pre, pre);
-    if (n_list == kNone)
-        n_valid = n_cands <= 1024u ? sort_candidates<1>(sc, row, slices, n_cands, m, inv_t, floor_q, kf, jf, L)
-                                   : sort_candidates<4>(sc, row, slices, n_cands, m, inv_t, floor_q, kf, jf, L);
-    MAKO_STAMP(4);
-    // top-k of the row = top-k of the candidates, provided nothing left behind can tie with or beat the k-th
-    bool ok = n_valid >= P.top_k ? q_bound < __uint_as_float(~kf[P.top_k - 1]) : q_bound == 0.0f;
-    if (ok && n_valid == 0) {
-        fallback_row(d, row, argidx);
-        return;
-    }
-    // (sampler.cpp:40-43; at most top_k <= kTopKFast <= kGroup entries.  A top-p cut too close to call is left to the
-    // whole-row path, which can sum in the reference's order.)
-    static_assert(kTopKFast <= kGroup, "top-k rows end in sorted_tail's short-list path");
-    if (ok)
-        [[clang::always_inline]] ok = sorted_tail<false, true>(d, row, P, kf, jf, min(P.top_k, n_valid), false, 0.0, MAKO_PATH_TOPK, L);
-    if (ok)
-        return;
-    __syncthreads(); // (the lists in LDS are done with)
-    // (where the whole-row path is a called function the views it receives by reference live in scratch memory: a copy
-    // made here, so that only the rows that come this way store one)
-    const FinishLds views = L;
-    general_row<MAKO_TOPK_GENERAL_SITE>(d, sc, row, P, m, argidx, views);
 }
 
 } // namespace mako

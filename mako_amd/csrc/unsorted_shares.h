@@ -27,8 +27,9 @@ namespace mako {
 // kHeadGroups groups of a list, and the list's entries at its positions are not written.)
 constexpr int kOpaqueShift = 11;     // the share's largest weight lies at least this many binades below the sum and r
 constexpr uint32_t kOpaqueTies = 16; // exact ties a share may hold (expected: entries * 2^-kOpaqueShift <= 3)
-constexpr uint32_t kCollectors = 2;  // workgroups of sort_kernel that take a row's unsorted shares, one share per wave (work items kWorkers + c)
-static_assert(kCollectors * (uint32_t)kWaves + 1u >= kWorkers, "a wave for every share but the last, which is never left unsorted");
+constexpr uint32_t kCollectors = 2;  // workgroups of sort_kernel that take a row's unsorted shares, a share per wave at a time (work items kWorkers + c)
+constexpr uint32_t kCollected = 16;  // shares that one of them takes
+static_assert(kCollectors * kCollected + 1u >= kWorkers, "every share but the last, which is never left unsorted");
 constexpr double kOpaqueMu = 0.01;   // what the estimates of the mass above a share are trusted to ...
 constexpr double kOpaqueMuCut = 0.03; // ... and of the mass below it
 

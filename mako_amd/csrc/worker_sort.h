@@ -2,8 +2,8 @@
 #pragma once
 
 #include "lds_sort.h"
+#include "radix_sort.h"
 #include "sorted_tail.h"
-#include "whole_row.h"
 #include "unsorted_shares.h"
 
 namespace mako {
@@ -73,11 +73,19 @@ __device__ uint32_t plan_runs(const uint32_t* ks, uint32_t key_lo, uint32_t key_
     __syncthreads();
     // bucket starts (exclusive scan), kept in sm.hist / sm.run as run boundaries below
     uint32_t total;
-    const uint32_t c0 = hist[2u * tid], c1 = hist[2u * tid + 1u];
-    const uint32_t ex = block_excl_scan_u32(c0 + c1, total, sm.bs);
+    uint32_t c[kFinePer], mine = 0;
+#pragma unroll
+    for (uint32_t j = 0; j < kFinePer; ++j) {
+        c[j] = hist[kFinePer * tid + j];
+        mine += c[j];
+    }
+    uint32_t ex = block_excl_scan_u32(mine, total, sm.bs);
     __syncthreads();
-    hist[2u * tid] = ex;
-    hist[2u * tid + 1u] = ex + c0;
+#pragma unroll
+    for (uint32_t j = 0; j < kFinePer; ++j) {
+        hist[kFinePer * tid + j] = ex;
+        ex += c[j];
+    }
     if (tid == 0)
         hist[kFine] = total;
     __syncthreads();
