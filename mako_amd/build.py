@@ -7,7 +7,7 @@ HERE = os.path.dirname(os.path.abspath(__file__))
 CSRC = os.path.join(HERE, "csrc")
 # the C ABI, and one translation unit per kernel family (a kernel's register allocation then does not depend on
 # which other kernels exist; they also compile side by side)
-SOURCES = ["mako_sampler.hip", "k_scan.hip", "k_finish.hip", "k_plan_alone.hip", "k_sort.hip", "k_sort_unsorted.hip", "k_tail.hip", "k_tail_unsorted.hip", "k_index.hip",
+SOURCES = ["mako_sampler.hip", "k_scan.hip", "k_finish.hip", "k_finish_halves.hip", "k_plan_alone.hip", "k_sort.hip", "k_sort_unsorted.hip", "k_tail.hip", "k_tail_unsorted.hip", "k_index.hip",
            "k_beside_finish.hip", "k_beside_sort.hip", "k_beside_tail.hip"]
 OBJ_DIR = os.path.join(HERE, "csrc", "_obj")
 OUT = os.path.join(HERE, "libmako_sampler.so")
@@ -52,7 +52,7 @@ SOURCE_FLAGS = {
 # pass), for the test that expects the oracle's results all the same, through rows given up to the whole-row path; and
 # without pinned memory (-DMAKO_NO_PINNED, the C ABI), for the host-pointer call's way round it
 OUT_RASH = os.path.join(HERE, "libmako_sampler_rash.so")
-RASH_FLAGS = {"k_finish.hip": ["-DMAKO_RASH_PLANS=1"], "k_beside_finish.hip": ["-DMAKO_RASH_PLANS=1"],
+RASH_FLAGS = {"k_finish.hip": ["-DMAKO_RASH_PLANS=1"], "k_finish_halves.hip": ["-DMAKO_RASH_PLANS=1"], "k_beside_finish.hip": ["-DMAKO_RASH_PLANS=1"],
               "mako_sampler.hip": ["-DMAKO_NO_PINNED=1"]}
 
 

@@ -59,6 +59,10 @@ __device__ __forceinline__ lds_ptr<T> as_lds(T* p)
 {
     return (lds_ptr<T>)p;
 }
+__device__ __forceinline__ uint32_t uniform_u32(uint32_t v)
+{
+    return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
+}
 // An address that is the same in all lanes, in scalar registers.
 template <typename T>
 __device__ __forceinline__ global_ptr<T> uniform_ptr(global_ptr<T> p)

@@ -7,6 +7,9 @@
 namespace mako {
 
 constexpr uint32_t kPlanSlices = 12; // slices whose counts are asked for ahead of the logits (the rest: one more trip)
+constexpr uint32_t kBinsPer = kLogBins / (uint32_t)kThreads; // bins a thread: one, or two that lie next to each other
+static_assert(kBinsPer * (uint32_t)kThreads == kLogBins && kBinsPer <= 2u, "a thread's counts of a slice are one load");
+using BinCounts = std::conditional_t<kBinsPer == 1u, uint16_t, uint32_t>;
 
 // Every workgroup of a row builds the same plan (same inputs, same instructions); LDS of its own, beside the
 // penalty table that the logits' loads work on meanwhile.
@@ -45,10 +48,10 @@ __device__ __forceinline__ void issue_plan_loads(const mako_sample_desc& d, cons
 {
     pre.u = WITH_U ? as_global(d.u)[row] : 0.0f;
     pre.st = load_slice_stat(sc.stats, (size_t)row * kMaxSlices + min((uint32_t)lane_id(), slices - 1u));
-    const global_ptr<const uint16_t> lh = as_global(sc.log_hist) + (size_t)row * sc.slices_cap * kLogBins + threadIdx.x;
+    const global_ptr<const BinCounts> lh = (global_ptr<const BinCounts>)(as_global(sc.log_hist) + (size_t)row * sc.slices_cap * kLogBins) + threadIdx.x;
 #pragma unroll
     for (uint32_t t = 0; t < kPlanSlices; ++t)
-        pre.v[t] = lh[(size_t)min(t, slices - 1u) * kLogBins]; // (clamped, not skipped: no branch between the loads)
+        pre.v[t] = lh[(size_t)min(t, slices - 1u) * (uint32_t)kThreads]; // (clamped, not skipped: no branch between the loads)
 }
 
 // Builds the row's plan in `pl` (all threads call; barriers order LDS only, the logits' loads stay in flight).
@@ -69,7 +72,9 @@ __device__ void coarse_plan(const Scratch& sc, uint32_t row, uint32_t slices, ui
     const float inv_t = 1.0f / P.temperature;
     constexpr float kPerUnit = -1.0f / (float)kLogUnitsPerOctave;
     const int32_t k_top = log_unit(m, scale);
-    pl.cnt[tid] = 0;
+#pragma unroll
+    for (uint32_t i = 0; i < kBinsPer; ++i)
+        pl.cnt[tid + i * (uint32_t)kThreads] = 0;
     if (tid <= kWorkers)
         pl.first_bin[tid] = 0; // (0: no bin opens the worker; worker 0 starts at bin 0 anyway)
     if (tid < kWorkers)
@@ -83,27 +88,38 @@ __device__ void coarse_plan(const Scratch& sc, uint32_t row, uint32_t slices, ui
         if (!v)
             return;
         // (the slice's maximum in a scalar register: what depends on it alone is scalar arithmetic)
-        const uint32_t b = log_bin_moved(tid, (int32_t)__builtin_amdgcn_readfirstlane(pl.slice_top[s]), k_top);
-        if (b < kLogBins - 1u)
-            atomicAdd(&pl.cnt[b], v);
+        const int32_t s_top = (int32_t)__builtin_amdgcn_readfirstlane(pl.slice_top[s]);
+#pragma unroll
+        for (uint32_t i = 0; i < kBinsPer; ++i) {
+            const uint32_t b = log_bin_moved(tid * kBinsPer + i, s_top, k_top), n = kBinsPer == 1u ? v : (i ? v >> 16 : v & 0xffffu);
+            if (b < kLogBins - 1u)
+                atomicAdd(&pl.cnt[b], n);
+        }
     };
 #pragma unroll
     for (uint32_t t = 0; t < kPlanSlices; ++t)
         if (t < slices)
             add(t, pre.v[t]);
     for (uint32_t s = kPlanSlices; s < slices; ++s)
-        add(s, as_global(sc.log_hist)[((size_t)row * sc.slices_cap + s) * kLogBins + tid]);
+        add(s, ((global_ptr<const BinCounts>)(as_global(sc.log_hist) + ((size_t)row * sc.slices_cap + s) * kLogBins))[tid]);
     lds_barrier();
     MAKO_STAMP(3);
-    // Running mass and count from the LOWEST bin up (thread t takes bin kLogBins - 1 - t): the mass below a bin, which
-    // is what the threshold is about, is then a sum of small terms and as accurate as they are, however close to one
-    // top_p is.  Wave scans, then one scan of the sixteen waves' totals by every wave for itself.
-    const uint32_t bin = kLogBins - 1u - tid;
-    const uint32_t c = pl.cnt[bin];
+    // Running mass and count from the LOWEST bin up (thread t takes bin kLogBins - 1 - t, or the two from there down to
+    // kLogBins - 2 - 2 t): the mass below a bin, which is what the threshold is about, is then a sum of small terms and as
+    // accurate as they are, however close to one top_p is.  Wave scans, then one scan of the waves' totals by every wave for itself.
+    uint32_t bin[kBinsPer], c[kBinsPer], c_all = 0;
+    float mass[kBinsPer], mass_all = 0.0f;
     const float top_frac = fminf(fmaxf(m * scale, -1.0e9f), 1.0e9f) - (float)k_top; // the maximum inside its unit
-    const float mass = (float)c * __builtin_amdgcn_exp2f((log_bin_middle(bin, k_top) + top_frac) * kPerUnit);
-    const float mass_w = __ockl_wfscan_add_f32(mass, true);
-    const uint32_t cnt_w = __ockl_wfscan_add_u32(c, true);
+#pragma unroll
+    for (uint32_t i = 0; i < kBinsPer; ++i) {
+        bin[i] = kLogBins - 1u - (tid * kBinsPer + i);
+        c[i] = pl.cnt[bin[i]];
+        mass[i] = (float)c[i] * __builtin_amdgcn_exp2f((log_bin_middle(bin[i], k_top) + top_frac) * kPerUnit);
+        c_all += c[i];
+        mass_all += mass[i];
+    }
+    const float mass_w = __ockl_wfscan_add_f32(mass_all, true);
+    const uint32_t cnt_w = __ockl_wfscan_add_u32(c_all, true);
     if (lane == kWave - 1) {
         pl.wave_mass[wave_id()] = mass_w;
         pl.wave_cnt[wave_id()] = cnt_w;
@@ -116,19 +132,36 @@ __device__ void coarse_plan(const Scratch& sc, uint32_t row, uint32_t slices, ui
     const uint32_t wc_upto = __ockl_wfscan_add_u32(wc, true);
     const float all_m = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wm_upto), kWaves - 1));
     const uint32_t all_c = (uint32_t)__builtin_amdgcn_readlane((int)wc_upto, kWaves - 1);
-    const float below_m = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wm_upto - wm), wave_id())) + mass_w - mass; // mass under the bin
-    const uint32_t from_c = (uint32_t)__builtin_amdgcn_readlane((int)(wc_upto - wc), wave_id()) + cnt_w; // logits in it and under it
-    const uint32_t excl_c = all_c - from_c, incl_c = excl_c + c; // logits above the bin; and with it
-    pl.incl[bin] = incl_c;
+    float below_m[kBinsPer];     // mass under the bin
+    uint32_t excl_c[kBinsPer];   // logits above it
+    below_m[0] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wm_upto - wm), wave_id())) + mass_w - mass_all;
+    excl_c[0] = all_c - ((uint32_t)__builtin_amdgcn_readlane((int)(wc_upto - wc), wave_id()) + cnt_w - c_all) - c[0];
+#pragma unroll
+    for (uint32_t i = 1; i < kBinsPer; ++i) {
+        below_m[i] = below_m[i - 1u] + mass[i - 1u];
+        excl_c[i] = excl_c[i - 1u] - c[i];
+    }
+#pragma unroll
+    for (uint32_t i = 0; i < kBinsPer; ++i)
+        pl.incl[bin[i]] = excl_c[i] + c[i]; // logits above the bin and in it
     // the nucleus ends where what lies below it is 1 - top_p of the total; the estimates of both are good to a few
     // percent of themselves (the bins' widths), whatever top_p is
     // (what the bins do not cover, masked and far-off logits alike, is taken at the weight where the bins end)
     const float tail_allowed = (1.0f - P.top_p) * all_m * 0.9f -
                                (float)(n_vocab - min(all_c, n_vocab)) * __builtin_amdgcn_exp2f((log_bin_middle(kLogBins - 2u, k_top) + top_frac) * kPerUnit);
     {
-        const unsigned long long bal = __ballot(c != 0 && below_m <= tail_allowed);
-        if (lane == 0) // (the highest such bin: the last such thread)
-            pl.wave_hit[wave_id()] = bal ? kLogBins - 1u - ((uint32_t)wave_id() * kWave + 63u - (uint32_t)__clzll((long long)bal)) : kNone;
+        // (the highest such bin: the last such thread's)
+        unsigned long long bal = 0ull;
+        uint32_t hit = 0;
+#pragma unroll
+        for (uint32_t i = 0; i < kBinsPer; ++i) {
+            const unsigned long long b = __ballot(c[i] != 0 && below_m[i] <= tail_allowed);
+            const uint32_t at = ((uint32_t)wave_id() * kWave + 63u - (uint32_t)__clzll((long long)b)) * kBinsPer + i;
+            hit = b ? max(hit, at) : hit;
+            bal |= b;
+        }
+        if (lane == 0)
+            pl.wave_hit[wave_id()] = bal ? kLogBins - 1u - hit : kNone;
     }
     lds_barrier();
     MAKO_STAMP(5);
@@ -149,13 +182,16 @@ __device__ void coarse_plan(const Scratch& sc, uint32_t row, uint32_t slices, ui
     const uint32_t workers = max(1u, min(kWorkers, (n0_est + share_min - 1u) / share_min));
     const float per_entry = flag == 1 ? (float)workers / (float)max(n0_est, 1u) : 0.0f;
     auto worker_at = [&](uint32_t excl) { return min(workers - 1u, (uint32_t)((float)excl * per_entry)); };
-    const uint32_t wk = worker_at(excl_c);
-    if (bin != 0 && bin < bins_end) {
-        // the workers whose share starts with this bin
-        const uint32_t c_prev = pl.cnt[bin - 1u];
-        for (uint32_t w = worker_at(excl_c - c_prev) + 1u; w <= wk; ++w) {
-            pl.first_bin[w] = bin;
-            pl.mass_above[w] = (double)(all_m - below_m - mass);
+#pragma unroll
+    for (uint32_t i = 0; i < kBinsPer; ++i) {
+        const uint32_t wk = worker_at(excl_c[i]);
+        if (bin[i] != 0 && bin[i] < bins_end) {
+            // the workers whose share starts with this bin
+            const uint32_t c_prev = i + 1u < kBinsPer ? c[min(i + 1u, kBinsPer - 1u)] : pl.cnt[bin[i] - 1u];
+            for (uint32_t w = worker_at(excl_c[i] - c_prev) + 1u; w <= wk; ++w) {
+                pl.first_bin[w] = bin[i];
+                pl.mass_above[w] = (double)(all_m - below_m[i] - mass[i]);
+            }
         }
     }
     if (tid == 0)

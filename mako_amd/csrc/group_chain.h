@@ -16,11 +16,6 @@ __device__ __forceinline__ double readlane_f64(double v, uint32_t lane)
     return __longlong_as_double((long long)(((unsigned long long)hi << 32) | lo));
 }
 
-__device__ __forceinline__ uint32_t uniform_u32(uint32_t v)
-{
-    return (uint32_t)__builtin_amdgcn_readfirstlane((int)v);
-}
-
 __device__ __forceinline__ float readlane_f32(float v, uint32_t lane)
 {
     return __uint_as_float((uint32_t)__builtin_amdgcn_readlane((int)__float_as_uint(v), (int)lane));

@@ -47,6 +47,6 @@ hipError_t init_finish_kernels()
         if (e != hipSuccess)
             return e;
     }
-    return hipSuccess;
+    return init_finish_halves();
 }
 } // namespace mako

@@ -27,6 +27,9 @@ void launch_scan(bool aligned, int kh, bool above, dim3 grid, size_t lds, hipStr
 // of one batch must agree on it)
 void launch_finish(bool aligned, int kh, bool unsorted, uint32_t wgs, hipStream_t st, const mako_sample_desc& d, const Scratch& sc,
                    uint32_t slices); // (host copy, by value)
+// the large batches' instance of 512 threads, two workgroups to a CU (second_pass_halves(); histories of up to 2 048 entries)
+hipError_t init_finish_halves();
+void launch_finish_halves(bool aligned, uint32_t wgs, hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices);
 void launch_plan_alone(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices); // (host copy, by value)
 // sort_kernel's workgroup i serves entry i of the work list: `grid_rows` * kWorkers workgroups must cover the
 // longest list the batch can produce (kWorkers entries per top_k == 0 row); tail_kernel takes one workgroup per possible wide row.  Workgroups beyond the lists leave at once, but each

@@ -433,14 +433,15 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
     const uint32_t nth_wgs = std::min(std::max(2u * ctx->cus / ((d.n_rows + 7u) & ~7u), 1u), (d.n_vocab + mako::kNthChunk - 1u) / mako::kNthChunk);
     const uint32_t nth_steps = !any_nth ? 0u : (!any_rounds ? 1u : mako::nth_launches(d.n_vocab, least_top_k));
     const bool launch_sort = any_nucleus || any_late || beside;
-    // (finish_kernel's grid: scan_kernel, which cuts the second pass up, is told of it)
-    const uint32_t finish_wgs = mako::second_pass_grid(nucleus_rows, ctx->cus);
     // Batches with many top_k == 0 rows leave the shares of their sorted lists that need no order unsorted
     // (unsorted_shares.h): there sort_kernel is bound by the number of its workgroups, one per CU at a time, and not, as
     // on a small batch, by its slowest worker.  More than four rounds of workers; without the caller's copy of the
     // parameters, from twice as many rows.
     const bool unsorted = params_host ? (uint64_t)nucleus_rows * mako::kWorkers > 4ull * ctx->cus
                                       : (uint64_t)d.n_rows * mako::kWorkers > 8ull * ctx->cus;
+    // (finish_kernel's grid: scan_kernel, which cuts the second pass up, is told of it)
+    const bool halves = !beside && mako::second_pass_halves(d.n_vocab, kh, unsorted);
+    const uint32_t finish_wgs = mako::second_pass_grid(nucleus_rows, ctx->cus, halves);
     // (a launch that fails stops the batch there: the kernels after it would work on what it did not write)
 #define MAKO_LAUNCH(call)                                                                                          \
     do {                                                                                                           \
@@ -452,7 +453,7 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
         }                                                                                                          \
     } while (0)
     MAKO_MARK(0);
-    MAKO_LAUNCH(mako::launch_scan(aligned, kh, d.close_token != nullptr, grid, lds, st, d, sc, slice_len, std::min(ctx->cus, mako::kCountGeneral - 1u) | (beside ? mako::kCountGeneral : 0u) | ((finish_wgs / 8u) << 16)));
+    MAKO_LAUNCH(mako::launch_scan(aligned, kh, d.close_token != nullptr, grid, lds, st, d, sc, slice_len, std::min(ctx->cus, mako::kHalfPieces - 1u) | (halves ? mako::kHalfPieces : 0u) | (beside ? mako::kCountGeneral : 0u) | ((finish_wgs / 8u) << 16)));
     MAKO_MARK(1);
     // top_k == 0 rows: planned and handed out by the second pass, sorted, cut and drawn from; the stages talk through
     // kernel boundaries (device-wide fences cost far more on this chip where hundreds of workgroups make one).  A batch without such rows
@@ -471,7 +472,9 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
     } else {
         if (only_index)
             MAKO_LAUNCH(mako::launch_index_weights(aligned, kh, any_bits, st, d, sc, slices));
-        if (any_nucleus)
+        if (any_nucleus && halves)
+            MAKO_LAUNCH(mako::launch_finish_halves(aligned, finish_wgs, st, d, sc, slices));
+        else if (any_nucleus)
             MAKO_LAUNCH(mako::launch_finish(aligned, kh, unsorted, finish_wgs, st, d, sc, slices));
         if (!launch_sort && !only_index)
             MAKO_LAUNCH(mako::launch_plan_alone(st, d, sc, slices));

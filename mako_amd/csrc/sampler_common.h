@@ -19,13 +19,15 @@ namespace mako {
 constexpr uint32_t kNone = 0xffffffffu;
 
 constexpr uint32_t kSliceMax = 16384; // elements per slice: 16 per thread
+constexpr uint32_t kSliceThreads = kSliceMax / 16u; // of scan_kernel
+constexpr uint32_t kPieceMax = 16u * (uint32_t)kThreads; // elements that a workgroup of this translation unit takes at once
 constexpr uint32_t kMaxSlices = 64;
 constexpr uint32_t kCap = 512;       // candidates kept per slice
 constexpr uint32_t kTopKFast = 128;  // largest top_k resolved from the per-slice candidates
 constexpr uint32_t kSortMax = 4096;  // candidates the finisher sorts in LDS
 constexpr uint32_t kSmall = 256;     // lists of up to this many entries are ordered by counting ranks
 constexpr uint32_t kDynLds = 65536;  // dynamic LDS that the penalty table of a slice takes
-constexpr uint32_t kFinishLds = (kSliceMax + 128u) * 8u; // and of the second pass's kernels, which put all a piece keeps in order there
+constexpr uint32_t kFinishLds = (kPieceMax + 128u) * 8u; // and of the second pass's kernels, which put all a piece keeps in order there
 constexpr uint32_t kHeadGroups = 32; // groups at the head of a sorted list that tail code keeps in LDS as floats
 constexpr uint32_t kTailLds = kDynLds + (kHeadGroups - 8u) * 1024u; // dynamic LDS of the kernels that cut and draw
 constexpr uint32_t kFlagFirstNan = 1u; // element 0 of the row is NaN (slice 0 only)
@@ -151,6 +153,7 @@ __host__ __device__ inline SortLists large_batch_lists(uint32_t nucleus_rows) //
 }
 
 constexpr uint32_t kWorkWords = 12;        // of Scratch::work_n
+constexpr uint32_t kHalfPieces = 0x4000u;   // scan_kernel: finish_kernel's workgroups have 512 threads (second_pass_halves())
 constexpr uint32_t kCountGeneral = 0x8000u; // scan_kernel: leave the number of rows of the whole-row class (beside_rows.h)
 struct Scratch {
     SliceStat* stats;  // [max_rows][kMaxSlices]

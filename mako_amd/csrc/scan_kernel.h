@@ -43,7 +43,7 @@ template <bool ALIGNED, int KH, bool ABOVE = false, bool SHORT = false>
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(ALIGNED || KH < 8 ? 8 : 4))) void scan_kernel(mako_sample_desc d, Scratch sc_arg, uint32_t slice_len,
                                                         uint32_t cus_and_grid)
 {
-    // (cus_and_grid: the CUs of the device, kCountGeneral, and in the upper half an eighth of finish_kernel's grid:
+    // (cus_and_grid: the CUs of the device, kCountGeneral, kHalfPieces, and in the upper half an eighth of finish_kernel's grid:
     // second_pass_cut())
     // (scan_kernel takes the context's record by value: its first loads then need no trip to memory for a pointer)
     const Scratch& sc = sc_arg;
@@ -96,8 +96,8 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(ALIGNE
         }
     }
     if (row == 0 && slice == 0 && wave_id() == 1) { // how the second pass will be cut up
-        const SecondPassCut cut = second_pass_cut(d, n_slices, slice_len, cus_and_grid & (kCountGeneral - 1u), (cus_and_grid >> 16) * 8u,
-                                                  (cus_and_grid & kCountGeneral) != 0u);
+        const SecondPassCut cut = second_pass_cut(d, n_slices, slice_len, cus_and_grid & (kHalfPieces - 1u), (cus_and_grid >> 16) * 8u,
+                                                  (cus_and_grid & kCountGeneral) != 0u, (cus_and_grid & kHalfPieces) != 0u);
         if (lane_id() == 0) {
             *reinterpret_cast<uint4*>(sc.work_n + 4) = make_uint4(cut.per_row, cut.piece_len, cut.busy, cut.pieces);
             *reinterpret_cast<uint4*>(sc.work_n + 8) = make_uint4(cut.general, cut.in_order, cut.rows, 0u);

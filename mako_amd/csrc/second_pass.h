@@ -123,7 +123,7 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
             qb[j] = 0u;
             slot[j] = kNone;
         }
-        if (lo + (g / 4u) * 4096u < hi) {
+        if (lo + (g / 4u) * kBlock < hi) {
             // (the large batches' instance: a wave whose four weights a lane all underflow to zero, as those of a peaked row far
             // below its maximum do, skips the arithmetic that would tell it so; exp_moved() returns 0 below that bound)
             bool any = !UNSORTED;
@@ -217,8 +217,8 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
     const global_ptr<uint32_t> istage = as_global(sc.idx[1]) + (size_t)row * sc.vpad;
     // (room for all a piece can hold: with half as much, a flat row's pieces, which keep nearly everything, went through
     // it twice, 2 us more each, and the workgroup has its CU to itself anyway)
-    uint2* buf = reinterpret_cast<uint2*>(L.cnt); // [kSliceMax + 3 kWorkers] (weight, token id)
-    static_assert(kFinishLds >= (kSliceMax + 3u * kWorkers) * sizeof(uint2), "");
+    uint2* buf = reinterpret_cast<uint2*>(L.cnt); // [kPieceMax + 3 kWorkers] (weight, token id)
+    static_assert(kFinishLds >= (kPieceMax + 3u * kWorkers) * sizeof(uint2), "");
     const uint32_t kept = pl.lbase[kWorkers];
     // (an entry's worker travels in the upper bits of its token id)
     constexpr uint32_t kIdBits = 27;
@@ -420,8 +420,8 @@ __device__ __forceinline__ void finish_body(const mako_sample_desc& d_arg, const
 }
 
 // (its arguments by value: the cut is one trip to memory away, not two)
-template <bool ALIGNED, int KH, bool UNSORTED>
-__global__ __launch_bounds__(kThreads) void finish_kernel(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices)
+template <bool ALIGNED, int KH, bool UNSORTED, int THREADS = kThreads>
+__global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) void finish_kernel(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices)
 {
     extern __shared__ __align__(16) unsigned long long s_dyn64[]; // (128-bit LDS operations need the alignment)
     __shared__ FinishShared sm;

@@ -5,11 +5,12 @@
 
 namespace mako {
 
-// Thread t of a slice owns 16 logits: for k = 0..3 the four consecutive ones at lo + k * 4096 + 4 * t.  A wavefront's
+// Thread t of a slice owns 16 logits: for k = 0..3 the four consecutive ones at lo + k * kBlock + 4 * t.  A wavefront's
 // loads are contiguous and each logit is read once.
+constexpr uint32_t kBlock = 4u * (uint32_t)kThreads;
 __device__ __forceinline__ uint32_t elem_index(uint32_t lo, uint32_t tid, uint32_t j)
 {
-    return lo + (j >> 2) * 4096u + tid * 4u + (j & 3u);
+    return lo + (j >> 2) * kBlock + tid * 4u + (j & 3u);
 }
 // The t that a thread is there.  MIXED: a wave has sixteen logits of every 256, in place of 256 of every 4 096.
 template <bool MIXED>
@@ -28,8 +29,8 @@ __device__ __forceinline__ uint32_t slice_thread()
 __host__ __device__ inline bool short_slice(uint32_t len) // (len: as slice_len, rounded up to a multiple of four)
 {
     // (128 groups of four at least, eight a wave, as many as a top_k of kTopKFast asks each for)
-    static_assert(kTopKFast <= (kCap / 4u / (uint32_t)kWaves) * (uint32_t)kWaves, "no wave is asked for more logits than it has");
-    return len < 5u * (uint32_t)kThreads && len > kCap;
+    static_assert(kTopKFast <= (kCap / 4u / (kSliceThreads / 64u)) * (kSliceThreads / 64u), "no wave is asked for more logits than it has");
+    return len < 5u * kSliceThreads && len > kCap;
 }
 
 // accept() history -> per-token counts for [lo, hi) in LDS (src/gen/sampler.cpp:15-18); generic form used
@@ -86,7 +87,7 @@ __device__ __forceinline__ void load_raw(const mako_sample_desc& d, uint32_t row
     } else {
 #pragma unroll
         for (uint32_t k = 0; k < 4; ++k) {
-            const uint32_t i = lo + k * 4096u + tid * 4u;
+            const uint32_t i = lo + k * kBlock + tid * 4u;
             at[k] = i < hi ? i : (hi - 1u) & ~3u;
             f32x4 x;
             if (ALIGNED)
@@ -120,7 +121,7 @@ __device__ __forceinline__ void settle_slice(RawSlice& r, uint32_t lo, uint32_t 
     const float nan = __uint_as_float(0x7fc00000u);
 #pragma unroll
     for (uint32_t k = 0; k < 4; ++k) {
-        if (lo + k * 4096u + slice_thread<MIXED>() * 4u == (hi & ~3u)) {
+        if (lo + k * kBlock + slice_thread<MIXED>() * 4u == (hi & ~3u)) {
             const uint32_t n = hi & 3u;
             const float4 x = r.v[k];
             r.v[k].x = n == 3u ? x.y : (n == 2u ? x.z : x.w);
@@ -140,7 +141,7 @@ __device__ __forceinline__ uint32_t count_above(const RawSlice& r, uint32_t lo, 
     uint32_t c = 0;
 #pragma unroll
     for (uint32_t k = 0; k < 4; ++k) {
-        if (lo + k * 4096u + tid * 4u < hi) { // (what lies behind the row's last logit in its group is NaN)
+        if (lo + k * kBlock + tid * 4u < hi) { // (what lies behind the row's last logit in its group is NaN)
             c += ((r.bits[k] & 1u) && r.v[k].x > v) ? 1u : 0u;
             c += ((r.bits[k] & 2u) && r.v[k].y > v) ? 1u : 0u;
             c += ((r.bits[k] & 4u) && r.v[k].z > v) ? 1u : 0u;
@@ -161,7 +162,7 @@ __device__ __forceinline__ void finish_slice(const RawSlice& r, uint32_t lo, uin
     if (!masked) { // uniform: no mask, nothing to clear
 #pragma unroll
         for (uint32_t k = 0; k < 4; ++k) {
-            const bool inside = lo + k * 4096u + tid * 4u < hi;
+            const bool inside = lo + k * kBlock + tid * 4u < hi;
             wv[4 * k + 0] = !inside ? nan : r.v[k].x;
             wv[4 * k + 1] = !inside ? nan : r.v[k].y;
             wv[4 * k + 2] = !inside ? nan : r.v[k].z;
@@ -175,7 +176,7 @@ __device__ __forceinline__ void finish_slice(const RawSlice& r, uint32_t lo, uin
         };
 #pragma unroll
         for (uint32_t k = 0; k < 4; ++k) {
-            const uint32_t i = lo + k * 4096u + tid * 4u;
+            const uint32_t i = lo + k * kBlock + tid * 4u;
             // (a bit behind the row's last logit may be anything)
             auto inside = [&](uint32_t c) { return ALIGNED ? i < hi : i + c < hi; };
             wv[4 * k + 0] = !inside(0u) ? nan : pick(r.bits[k], 0, r.v[k].x);
@@ -187,7 +188,7 @@ __device__ __forceinline__ void finish_slice(const RawSlice& r, uint32_t lo, uin
     if (pen) {
 #pragma unroll
         for (uint32_t k = 0; k < 4; ++k) {
-            const uint32_t i = lo + k * 4096u + tid * 4u;
+            const uint32_t i = lo + k * kBlock + tid * 4u;
             if (i < hi) {
                 const uint4 n = *reinterpret_cast<const uint4*>(s_cnt + (i - lo));
                 if (n.x | n.y | n.z | n.w) {
@@ -332,7 +333,7 @@ __device__ __forceinline__ void finish_penalised(const mako_sample_desc& d, uint
     uint32_t moved = 0;
 #pragma unroll
     for (uint32_t k = 0; k < 4; ++k) {
-        const uint32_t i = lo + k * 4096u + mine * 4u;
+        const uint32_t i = lo + k * kBlock + mine * 4u;
         if (i < hi) {
             uint4* slot = reinterpret_cast<uint4*>(s_cnt + (i - lo));
             const uint4 n = *slot;
@@ -356,7 +357,7 @@ __device__ __forceinline__ void finish_penalised(const mako_sample_desc& d, uint
 #pragma unroll
         for (uint32_t k = 0; k < 4; ++k)
             if ((moved >> (4u * k)) & 0xfu) {
-                const uint4 v = *reinterpret_cast<const uint4*>(s_cnt + (k * 4096u + mine * 4u));
+                const uint4 v = *reinterpret_cast<const uint4*>(s_cnt + (k * kBlock + mine * 4u));
                 wv[4 * k + 0] = (moved >> (4u * k)) & 1u ? __uint_as_float(v.x) : wv[4 * k + 0];
                 wv[4 * k + 1] = (moved >> (4u * k)) & 2u ? __uint_as_float(v.y) : wv[4 * k + 1];
                 wv[4 * k + 2] = (moved >> (4u * k)) & 4u ? __uint_as_float(v.z) : wv[4 * k + 2];

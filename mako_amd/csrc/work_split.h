@@ -12,6 +12,7 @@ namespace mako {
 // many workgroups per row as keeps it to one round; each of them goes through its share of the row's pieces in turn
 // (and builds the row's plan once, not once per piece).  Worked out from the rows' parameters by one wave of
 // scan_kernel's first workgroup and left in Scratch::work_n.
+// (halves: finish_kernel's workgroups have half the threads and take half the logits at once, two to a CU)
 struct SecondPassCut {
     uint32_t per_row;   // workgroups per top_k == 0 row
     uint32_t piece_len;
@@ -24,7 +25,7 @@ struct SecondPassCut {
 // finish_grid: the workgroups finish_kernel is launched with (second_pass_grid()).  count_general: the rows of the whole-row
 // class are wanted too (counted for every batch, they cost a 64-row decode batch without any 0.3 of its 66 us).
 __device__ __forceinline__ SecondPassCut second_pass_cut(const mako_sample_desc& d, uint32_t slices, uint32_t slice_len,
-                                                         uint32_t cus, uint32_t finish_grid, bool count_general)
+                                                         uint32_t cus, uint32_t finish_grid, bool count_general, bool halves)
 {
     uint32_t rows = 0; // top_k == 0 rows of the batch (every lane ends up with the count)
     SecondPassCut cut;
@@ -39,12 +40,13 @@ __device__ __forceinline__ SecondPassCut second_pass_cut(const mako_sample_desc&
             cut.in_order += (uint32_t)__popcll(__ballot(r < d.n_rows && index_order_row(P)));
         }
     }
-    cut.piece_len = slice_len;
-    cut.pieces = slices;
+    const uint32_t block = halves ? kSliceMax / 8u : kSliceMax / 4u, slots = halves ? 2u * cus : cus;
+    cut.piece_len = halves ? min(slice_len, 4u * block) : slice_len;
+    cut.pieces = halves ? (d.n_vocab + cut.piece_len - 1u) / cut.piece_len : slices;
     for (uint32_t blocks = 1; blocks < 4u; ++blocks) {
-        const uint32_t len = blocks * 4096u;
+        const uint32_t len = blocks * block;
         const uint32_t n = (d.n_vocab + len - 1u) / len;
-        if (len < slice_len && n <= kMaxSlices && rows * n <= cus) {
+        if (len < cut.piece_len && n <= kMaxSlices && rows * n <= slots) {
             cut.piece_len = len;
             cut.pieces = n;
             break;
@@ -52,7 +54,7 @@ __device__ __forceinline__ SecondPassCut second_pass_cut(const mako_sample_desc&
     }
     // (more pieces than one round of workgroups: as many workgroups per row as the grid allows when the rows are dealt
     // to the XCDs eight at a time, see finish_kernel)
-    cut.per_row = rows * cut.pieces <= cus ? cut.pieces : min(cut.pieces, max(1u, finish_grid / ((max(rows, 1u) + 7u) & ~7u)));
+    cut.per_row = rows * cut.pieces <= slots ? cut.pieces : min(cut.pieces, max(1u, finish_grid / ((max(rows, 1u) + 7u) & ~7u)));
     cut.busy = rows * cut.per_row;
     cut.rows = rows;
     return cut;
@@ -64,10 +66,18 @@ __device__ __forceinline__ SecondPassCut second_pass_cut(const mako_sample_desc&
 // batches the workgroups without work, which can only start once a CU is free, would lengthen the kernel instead.
 // (The rows of a large batch that are of another kind don't count: 97 of 512 rows, given four workgroups each for a grid of
 // 512, took one and a half rounds of them, 82 us; 60 to 68 with two each in one.)
-__host__ __device__ inline uint32_t second_pass_grid(uint32_t nucleus_rows, uint32_t cus)
+__host__ __device__ inline uint32_t second_pass_grid(uint32_t nucleus_rows, uint32_t cus, bool halves)
 {
-    const uint32_t rows8 = (nucleus_rows + 7u) & ~7u, rounds = 2u * nucleus_rows >= cus ? 2u : 1u;
-    return rows8 > rounds * cus ? rows8 : (rounds * cus + 7u) & ~7u;
+    const uint32_t rows8 = (nucleus_rows + 7u) & ~7u, slots = halves ? 2u * cus : cus, rounds = 2u * nucleus_rows >= cus ? 2u : 1u;
+    return rows8 > rounds * slots ? rows8 : (rounds * slots + 7u) & ~7u;
+}
+// Whether finish_kernel is the large batches' instance of half as many threads (k_finish_halves.hip).  Not with histories of more
+// than 2 048 entries, 16 a thread: those spill; nor where a row's pieces of 8 192 logits are more than its part_sum has room for; nor
+// beside rows of the whole-row class, whose workgroups in that launch take 16 384 logits each.  (On small batches, which have one
+// round of workgroups either way and a plan in each, two to a CU gained nothing: 19.0 us, 18.7 with one.)
+__host__ __device__ inline bool second_pass_halves(uint32_t n_vocab, int kh, bool unsorted)
+{
+    return unsorted && kh == 2 && n_vocab <= kMaxSlices * (kSliceMax / 2u);
 }
 
 // Which piece of work does workgroup `piece` of finish_kernel (per_nucleus = slices, per_other = 1) or of plan_kernel
