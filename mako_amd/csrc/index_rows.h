@@ -130,7 +130,8 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
             first_pivot(d, row, P, pen ? hl : 0u, m, sm);
     });
     const float inv_t = 1.0f / P.temperature;
-    const float floor_q = (1.0f < P.min_p) ? 1.0f : P.min_p;
+    // (a weight of zero is below either)
+    const float floor_p = (1.0f < P.min_p) ? 1.0f : P.min_p, floor_q = floor_p < 0x1p-149f ? 0x1p-149f : floor_p;
     NthFirst first = {0u, 0u, 0u, 0u}; // (in scalar registers)
     if (steps) {
         lds_barrier();
@@ -160,12 +161,12 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
             uint32_t k[4];
 #pragma unroll
             for (uint32_t c = 0; c < 4; ++c) {
-                const uint32_t at = elem_index(lo, tid, 4u * b + c);
+                // (what lies past the row's end is NaN, of which the weight is zero)
                 const float q = weight_of(wv[4u * b + c], m, inv_t, sm.tab);
-                const bool ok = at < hi && q >= floor_q && q > 0.0f; // src/gen/sampler.cpp:34-35
+                const bool ok = q >= floor_q; // src/gen/sampler.cpp:34-35
                 k[c] = ok ? __float_as_uint(q) : 0u;
                 is_cand |= (ok ? 1u : 0u) << (4u * b + c);
-                bsum[b] += ok ? (double)q : 0.0;
+                bsum[b] += (double)__uint_as_float(k[c]);
                 if (wide && ok)
                     atomicAdd(&bins[nth_bin(k[c])], 1u);
             }
