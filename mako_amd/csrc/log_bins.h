@@ -58,7 +58,8 @@ LOGBINS_HD uint32_t log_slot_in_frame(int32_t k, int32_t k_top, uint32_t spare_e
 {
     const uint32_t d = (uint32_t)k_top - (uint32_t)k;
     const uint32_t c = (uint32_t)(log_first_group(k_top) + (int32_t)kLogFine - log_group(k)); // kLogFine + coarse bin
-    return d < kLogFine ? d : (c < spare_end ? c : spare_end);
+    const uint32_t least = d < c ? d : c;
+    return least < spare_end ? least : spare_end;
 }
 
 // A unit of bin b of the frame of k_top (the bin's only one if the bin is fine, the lowest of its group otherwise):

@@ -7,14 +7,14 @@
 namespace mako {
 
 struct alignas(16) ScanShared {
+    float cw[kCap]; // (in front, where a candidate's address is its slot's number and nothing to add)
+    uint32_t ci[kCap];
     uint32_t wave_max[kWaves]; // order keys
     uint32_t wave_kth[kWaves];
     uint32_t wave_above[kWaves];
     uint32_t argidx;
     uint32_t emit_n;
     uint32_t emit_flags;
-    float cw[kCap];
-    uint32_t ci[kCap];
     uint32_t log_hist[kLogBins + kWave]; // top_k == 0 rows (and one slot per lane for what is not counted)
 };
 
@@ -208,8 +208,7 @@ __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(ALIGNE
 #pragma unroll
             for (uint32_t j = 0; j < 16; ++j) {
                 if (takes[j]) { // uniform
-                    const uint32_t pos =
-                        run + __builtin_amdgcn_mbcnt_hi((uint32_t)(takes[j] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)takes[j], 0u));
+                    const uint32_t pos = __builtin_amdgcn_mbcnt_hi((uint32_t)(takes[j] >> 32), __builtin_amdgcn_mbcnt_lo((uint32_t)takes[j], run));
                     const float w = wv[j];
                     if (w >= tau && pos < kCap) {
                         sm.cw[pos] = w;
