@@ -139,7 +139,8 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
                          uniform_u32((uint32_t)(sm.bs.u64[1] >> 32))};
     }
     // (~bits(q), at the token's own position)
-    uint32_t* key0 = sc.key[0] + (size_t)row * sc.vpad;
+    // (stores known to go to device memory: one that could go to LDS as well is waited for with the table's next read)
+    const global_ptr<uint32_t> key0 = as_global(sc.key[0]) + (size_t)row * sc.vpad;
     MAKO_CHECK(sc, kCheckStage, (uint64_t)hi <= sc.vpad);
     // (a wide row: its weights counted by value)
     const bool wide = STEPS && wide_row(P0) && nth_picks_for(d.n_vocab); // uniform
@@ -171,7 +172,7 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
                     atomicAdd(&bins[nth_bin(k[c])], 1u);
             }
             if (base + 3u < hi) {
-                *reinterpret_cast<uint4*>(key0 + base) = make_uint4(~k[0], ~k[1], ~k[2], ~k[3]);
+                *(global_ptr<u32x4>)(key0 + base) = u32x4{~k[0], ~k[1], ~k[2], ~k[3]};
             } else {
 #pragma unroll
                 for (uint32_t c = 0; c < 4; ++c)
@@ -196,9 +197,9 @@ __device__ __forceinline__ void index_weights_piece(const mako_sample_desc& d_ar
             } else if (!in_order) { // uniform
                 // the token ids as well: with them this is the whole-row path's list of candidates when every logit turns out
                 // to be one, as the pieces' counts will tell
-                uint32_t* li = sc.idx[0] + (size_t)row * sc.vpad;
+                const global_ptr<uint32_t> li = as_global(sc.idx[0]) + (size_t)row * sc.vpad;
                 if (base + 3u < hi) {
-                    *reinterpret_cast<uint4*>(li + base) = make_uint4(base, base + 1u, base + 2u, base + 3u);
+                    *(global_ptr<u32x4>)(li + base) = u32x4{base, base + 1u, base + 2u, base + 3u};
                 } else {
 #pragma unroll
                     for (uint32_t c = 0; c < 4; ++c)
