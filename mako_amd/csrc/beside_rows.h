@@ -24,7 +24,7 @@ __global__ __launch_bounds__(kThreads) void finish_beside_kernel(mako_sample_des
     __shared__ ArgsLds s_args;
     __shared__ CoarsePlan s_plan;
     if (blockIdx.y < finish_wgs) {
-        finish_body<ALIGNED, KH, UNSORTED, false>(d_arg, sc_val, slices, finish_wgs, s_dyn64, sm, s_args, s_plan);
+        finish_body<ALIGNED, KH, UNSORTED, false, kSortBesideWaves>(d_arg, sc_val, slices, finish_wgs, s_dyn64, sm, s_args, s_plan);
         return;
     }
     const uint32_t pieces = (d_arg.n_vocab + kSliceMax - 1u) / kSliceMax;

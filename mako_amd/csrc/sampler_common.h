@@ -139,17 +139,25 @@ constexpr uint32_t kOpaque = 1u << 25; // the record stands for a whole unsorted
 // The large batches' work lists of sort_kernel.  Workgroups are dispatched in the order of their numbers, to the XCDs
 // in turn, and the next one waits for a CU of ITS XCD: with entries of unequal cost in row order the XCDs fall out of
 // step and CUs idle (a quarter of the time on config 4).  So the costliest entries, the collectors of unsorted shares
-// (up to two per row, ~19 us), come first and together, then the workers that sort (~13 us) and the narrow rows
+// (up to three per row, ~19 us), come first and together, then the workers that sort (~13 us) and the narrow rows
 // (~10 us).  A workgroup without an entry costs nothing behind the last one with work, but between two of them it
 // waits for a CU like any other: the collectors' list is filled from its end backwards (work_n[3] of them, the last at
 // workgroup number sorted_at - 1), the others' forwards from sorted_at (work_n[0]), so that no gap lies between.
-constexpr uint32_t kSortItemsPerRow = kWorkers + 2u;
+// (a share a wave: with two for each of a collector's eight waves, in two collectors, 48 rows of 129 280 logits, half of them
+// flat, waited 34 us for them, and 23 for workgroups of sixteen waves before)
+constexpr uint32_t kSortWaves = 8u, kSortBesideWaves = 16u; // of sort_kernel_unsorted and sort_beside_kernel
+constexpr uint32_t kUnsortedMost = 24u; // shares of a row that its collectors have waves for; any beyond are a wave's second
+__host__ __device__ constexpr uint32_t collectors_per_row(uint32_t waves) { return (kUnsortedMost + waves - 1u) / waves; }
+__host__ __device__ constexpr uint32_t sort_items_per_row(uint32_t waves) { return kWorkers + collectors_per_row(waves); }
+constexpr uint32_t kSortItemsPerRow = sort_items_per_row(kSortWaves);
+static_assert(kSortItemsPerRow >= sort_items_per_row(kSortBesideWaves), "room for either kernel's lists");
 struct SortLists {
     uint32_t sorted_at; // first workgroup number (= entry of work_sort) of the workers that sort and the narrow rows
 };
-__host__ __device__ inline SortLists large_batch_lists(uint32_t nucleus_rows) // (Scratch::work_n[10])
+template <uint32_t WAVES>
+__device__ __forceinline__ SortLists large_batch_lists(uint32_t nucleus_rows) // (Scratch::work_n[10])
 {
-    return SortLists{2u * nucleus_rows};
+    return SortLists{collectors_per_row(WAVES) * nucleus_rows};
 }
 
 constexpr uint32_t kWorkWords = 12;        // of Scratch::work_n

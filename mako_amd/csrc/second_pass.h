@@ -22,7 +22,7 @@ namespace mako {
 // (`slices`: of scan_kernel, whose records give the row maximum)
 // (PLANNING: the workgroup's first piece, with which the plan is built; returns false when the row leaves for the
 // whole-row path and the pass has nothing more to do for it)
-template <bool ALIGNED, int KH, bool PEN, bool PLANNING, bool UNSORTED, bool AHEAD>
+template <bool ALIGNED, int KH, bool PEN, bool PLANNING, bool UNSORTED, bool AHEAD, uint32_t SORT_WAVES>
 __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t row, uint32_t slice, uint32_t slice_len,
                           const mako_sampling_params& P, uint32_t hl, uint32_t slices, const FinishLds& L, CoarsePlan& pl,
                           float& m, uint32_t& argidx, uint32_t opaque_first, SliceLoads<KH>& loads, uint32_t next)
@@ -81,12 +81,13 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
             const uint32_t unsorted = (UNSORTED && flag == 1) ? pl.opq_mask : 0u;
             plan->opq_mask = unsorted;
             if (flag == 1 || flag == 3) {
-                // sort_kernel's work: a workgroup per worker that sorts, and up to kCollectors whose waves take the row's
-                // unsorted shares, a share at a time (work items kWorkers + c)
-                const uint32_t n_unsorted = (uint32_t)__popc(unsorted), collectors = (n_unsorted + kCollected - 1u) / kCollected;
+                // sort_kernel's work: a workgroup per worker that sorts, and up to collectors_per_row() whose waves take the row's
+                // unsorted shares, a share each (work items kWorkers + c)
+                const uint32_t n_unsorted = (uint32_t)__popc(unsorted);
+                const uint32_t collectors = min((n_unsorted + SORT_WAVES - 1u) / SORT_WAVES, collectors_per_row(SORT_WAVES));
                 if constexpr (UNSORTED) {
                     // (two lists, the costly entries in front: large_batch_lists())
-                    const SortLists lists = large_batch_lists(pl.nucleus_rows);
+                    const SortLists lists = large_batch_lists<SORT_WAVES>(pl.nucleus_rows);
                     if (flag == 3) {
                         work_sort[lists.sorted_at + take(work_n + 0, 1u)] = row << 8;
                     } else {
@@ -298,7 +299,7 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
     return true;
 }
 
-template <bool ALIGNED, int KH, bool PEN, bool UNSORTED, bool AHEAD>
+template <bool ALIGNED, int KH, bool PEN, bool UNSORTED, bool AHEAD, uint32_t SORT_WAVES>
 __device__ void row_pieces(const mako_sample_desc& d, const Scratch& sc, uint32_t row, uint32_t first, uint32_t stride,
                            uint32_t n_pieces, uint32_t slice_len, const mako_sampling_params& P, uint32_t hl, uint32_t slices,
                            const FinishLds& L, CoarsePlan& pl, uint32_t opaque_first)
@@ -309,11 +310,11 @@ __device__ void row_pieces(const mako_sample_desc& d, const Scratch& sc, uint32_
     uint32_t argidx = 0;
     SliceLoads<KH> loads;
     auto behind = [&](uint32_t slice) { return slice + stride < n_pieces ? slice + stride : kNone; };
-    if (first >= n_pieces || !one_piece<ALIGNED, KH, PEN, true, UNSORTED, AHEAD>(d, sc, row, first, slice_len, P, hl, slices, L, pl, m, argidx, opaque_first, loads,
+    if (first >= n_pieces || !one_piece<ALIGNED, KH, PEN, true, UNSORTED, AHEAD, SORT_WAVES>(d, sc, row, first, slice_len, P, hl, slices, L, pl, m, argidx, opaque_first, loads,
                                                                          behind(first)))
         return;
     for (uint32_t slice = first + stride; slice < n_pieces; slice += stride)
-        one_piece<ALIGNED, KH, PEN, false, UNSORTED, AHEAD>(d, sc, row, slice, slice_len, P, hl, slices, L, pl, m, argidx, kNone, loads, behind(slice));
+        one_piece<ALIGNED, KH, PEN, false, UNSORTED, AHEAD, SORT_WAVES>(d, sc, row, slice, slice_len, P, hl, slices, L, pl, m, argidx, kNone, loads, behind(slice));
 }
 
 // Second pass over the top_k == 0 rows.  grid = (most pieces a row can have, rows) workgroups, of which workgroup i
@@ -321,8 +322,8 @@ __device__ void row_pieces(const mako_sample_desc& d, const Scratch& sc, uint32_
 // workgroups are then the first ones dispatched and land evenly on the XCDs, shader engines and CUs, whatever the
 // mix of rows.
 // (UNSORTED: the instance for batches of many such rows, whose plans leave shares unsorted: unsorted_shares.h)
-// (n_wgs: workgroups of the launch that are finish_kernel's)
-template <bool ALIGNED, int KH, bool UNSORTED, bool AHEAD>
+// (n_wgs: workgroups of the launch that are finish_kernel's.  SORT_WAVES: waves of a workgroup of the sort that follows)
+template <bool ALIGNED, int KH, bool UNSORTED, bool AHEAD, uint32_t SORT_WAVES>
 __device__ __forceinline__ void finish_body(const mako_sample_desc& d_arg, const Scratch& sc_arg, uint32_t slices, uint32_t n_wgs,
                                             unsigned long long* s_dyn64, FinishShared& sm, ArgsLds& s_args, CoarsePlan& s_plan)
 {
@@ -419,9 +420,9 @@ __device__ __forceinline__ void finish_body(const mako_sample_desc& d_arg, const
         s_plan.nucleus_rows = nucleus_rows; // (read behind the plan's barriers)
     const uint32_t opaque_first = (UNSORTED && !d.draft) ? max(kHeadGroups * kGroup, (d.out_cand_idx && d.out_cand_q) ? d.cand_cap : 0u) : kNone;
     if (d.hist_tokens && !penalties_neutral(P))
-        row_pieces<ALIGNED, KH, true, UNSORTED, AHEAD>(d, sc, row, piece, pieces, n_pieces, piece_len, P, hl, slices, L, s_plan, opaque_first);
+        row_pieces<ALIGNED, KH, true, UNSORTED, AHEAD, SORT_WAVES>(d, sc, row, piece, pieces, n_pieces, piece_len, P, hl, slices, L, s_plan, opaque_first);
     else
-        row_pieces<ALIGNED, KH, false, UNSORTED, AHEAD>(d, sc, row, piece, pieces, n_pieces, piece_len, P, hl, slices, L, s_plan, opaque_first);
+        row_pieces<ALIGNED, KH, false, UNSORTED, AHEAD, SORT_WAVES>(d, sc, row, piece, pieces, n_pieces, piece_len, P, hl, slices, L, s_plan, opaque_first);
 }
 
 // (its arguments by value: the cut is one trip to memory away, not two)
@@ -432,7 +433,7 @@ __global__ __launch_bounds__(THREADS) __attribute__((amdgpu_waves_per_eu(4))) vo
     __shared__ FinishShared sm;
     __shared__ ArgsLds s_args;
     __shared__ CoarsePlan s_plan;
-    finish_body<ALIGNED, KH, UNSORTED, UNSORTED && KH <= 2>(d_arg, sc_val, slices, gridDim.y, s_dyn64, sm, s_args, s_plan);
+    finish_body<ALIGNED, KH, UNSORTED, UNSORTED && KH <= 2, kSortWaves>(d_arg, sc_val, slices, gridDim.y, s_dyn64, sm, s_args, s_plan);
 }
 
 } // namespace mako

@@ -20,16 +20,13 @@ namespace mako {
 // path if it fails (the share's order would be needed then and does not exist).
 //
 // Only batches with many top_k == 0 rows do this (the host decides and launches the kernels' instances for it): there
-// sort_kernel is bound by the number of its workgroups, one per CU at a time, and a share that needs no sorting is summed
-// by one wave of a collector workgroup that takes sixteen of them; on a small batch every worker has a CU to itself and the batch waits for the slowest anyway.
+// sort_kernel is bound by the number of its workgroups, two to a CU, and a share that needs no sorting is summed by one
+// wave of a collector workgroup; on a small batch every worker has a CU to itself and the batch waits for the slowest anyway.
 
 // (A record with kOpaque set stands for a whole unsorted share: its increments are all there is.  Never among the first
 // kHeadGroups groups of a list, and the list's entries at its positions are not written.)
 constexpr int kOpaqueShift = 11;     // the share's largest weight lies at least this many binades below the sum and r
 constexpr uint32_t kOpaqueTies = 16; // exact ties a share may hold (expected: entries * 2^-kOpaqueShift <= 3)
-constexpr uint32_t kCollectors = 2;  // workgroups of sort_kernel that take a row's unsorted shares, a share per wave at a time (work items kWorkers + c)
-constexpr uint32_t kCollected = 16;  // shares that one of them takes
-static_assert(kCollectors * kCollected + 1u >= kWorkers, "every share but the last, which is never left unsorted");
 constexpr double kOpaqueMu = 0.01;   // what the estimates of the mass above a share are trusted to ...
 constexpr double kOpaqueMuCut = 0.03; // ... and of the mass below it
 

@@ -187,7 +187,7 @@ __device__ bool collect_run(const uint32_t* ks, const uint32_t* is, uint32_t key
 
 // ---- shares that need no sorting (unsorted_shares.h) ---------------------------------------------------------------
 //
-// The record of an unsorted share, by ONE wave (a collector workgroup's sixteen waves take a share each: no barrier,
+// The record of an unsorted share, by ONE wave (a collector workgroup's waves take a share each: no barrier,
 // nothing shared).  ks: the share's cnt weights as bits(q), in device memory, any order.  `lds`: kOpaqueLdsWords words
 // of LDS of the wave's own.  The share is streamed once (sixteen loads per lane in flight): its fp64 sum, its largest
 // weight, the sums of the increments of the weights that are no exact ties, and the ties themselves (kept apart, up
