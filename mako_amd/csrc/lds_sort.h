@@ -10,8 +10,8 @@ namespace mako {
 // the entries of its own bucket that precede it under (q desc, idx asc); they go to kout / iout as ~bits(q) and token id.
 // Returns false when a bucket is too crowded to be ranked by counting.  hist must be zero and sm.flag 0 on entry, behind a
 // barrier.
-// sorted_lds (optional, n words of LDS outside the sort's own): receives the sorted ~bits(q) as well, and the
-// function then returns behind a barrier that orders LDS only: the caller goes on from the copy instead of waiting
+// sorted_lds (optional, n words of LDS: outside the sort's own, or, of more than kSortedRoom entries, over A): receives the
+// sorted ~bits(q) as well, and the function then returns behind a barrier that orders LDS only: the caller goes on from the copy instead of waiting
 // for the stores to kout and reading them back.
 // (An entry moves as one 64-bit value, the weight above the complement of its token id, so that one comparison orders two of
 // them; and whoever counts may read past the bucket's end, where all there is is smaller.  With the two halves compared and the
@@ -71,6 +71,8 @@ __device__ bool lds_bucket_sort(const uint32_t (&k)[kSortPer], const uint32_t (&
     lds_barrier();
     MAKO_STAMP(15);
     // 2. rank inside the bucket, and out
+    const bool over = kSortedRoom < kSegCap && n > kSortedRoom; // uniform
+    uint32_t place[kSortPer];
 #pragma unroll
     for (uint32_t t = 0; t < kSortPer; ++t) {
         const uint32_t s = t * kThreads + tid;
@@ -91,9 +93,21 @@ __device__ bool lds_bucket_sort(const uint32_t (&k)[kSortPer], const uint32_t (&
             }
             kout[at] = ~(uint32_t)(me >> 32);
             iout[at] = ~(uint32_t)me;
-            if (sorted_lds)
+            if (sorted_lds && !over)
                 sorted_lds[at] = ~(uint32_t)(me >> 32);
+            place[t] = at;
         }
+    }
+    if (sorted_lds && over) { // (every entry has its place: the copy may go over them, once all weights are in registers)
+        uint32_t w[kSortPer];
+#pragma unroll
+        for (uint32_t t = 0; t < kSortPer; ++t)
+            w[t] = (uint32_t)(A[min(t * kThreads + tid, n - 1u)] >> 32);
+        lds_barrier();
+#pragma unroll
+        for (uint32_t t = 0; t < kSortPer; ++t)
+            if (t * kThreads + tid < n)
+                sorted_lds[place[t]] = ~w[t];
     }
     if (sorted_lds) // uniform
         lds_barrier();

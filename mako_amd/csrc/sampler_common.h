@@ -87,15 +87,20 @@ constexpr uint32_t kStageSlack = 64; // room a worker's share of the staging arr
                                      // promise (and 1/64 of that count); the rows' arrays are sized to hold it
 constexpr uint32_t kGroup = 256;      // a sorted list is processed in groups of one wave x four entries per lane
 constexpr uint32_t kMaxGroups = 1024; // groups per list
-constexpr uint32_t kSegCap = kThreads == 1024 ? 6144 : 5632; // entries a worker sorts in LDS (5 632: what two on a CU have room for)
+constexpr uint32_t kSegCap = 6144;    // entries a worker sorts in LDS
 constexpr uint32_t kFine = 2048;      // value buckets of that sort
 // dynamic LDS of sort_kernel: for the sort the entries in the order of their buckets (and four more), the buckets, and a copy of the
-// sorted weights for the group records, 81 968 bytes, or 75 824 for a workgroup of 512; for a narrow row the lists that its tail
-// works on, kTailLds, 90 112 bytes, which is what the launch asks for (with its 100 vector registers a workgroup of 1 024 has a CU to
-// itself either way), or kDynLds: two workgroups of 512 have 79 072 bytes each, of a CU's 163 840.
-constexpr uint32_t kSortedCopyAt = (kSegCap + 4u) * 8u + (kFine + 4u) * 4u; // byte offset of that copy
+// sorted weights for the group records, 81 968 bytes; for a narrow row the lists that its tail works on, kTailLds, 90 112 bytes,
+// which is what the launch asks for (with its 100 vector registers a workgroup of 1 024 has a CU to itself either way), or kDynLds.
+// Two workgroups of 512 have 81 920 bytes each, 3 248 of them static: room beside the sort for the copy of 5 120 entries.  A longer
+// share's goes over the entries once all have their places.  (With shares of up to 5 632 only, those beyond in two runs, four flat
+// rows of 151 552 logits took 85.5 us, the sort 23.6 of them; 77.2 so, and 75.3 in workgroups of 1 024.)
+constexpr uint32_t kSortedRoom = kThreads == 1024 ? kSegCap : 5120u;        // entries of the copy beside the sort
+constexpr uint32_t kSortedCopyAt = (kSegCap + 4u) * 8u + (kFine + 4u) * 4u; // its byte offset
+constexpr uint32_t kSortedOverAt = 16384u;                                  // and that of one over the entries (behind the groups' sums)
+static_assert(kSortedOverAt + kSegCap * 4u <= kSegCap * 8u, "a copy over the entries");
 constexpr uint32_t kSortNarrowLds = kThreads == 1024 ? kTailLds : kDynLds;
-constexpr uint32_t kSortLds = (kSortedCopyAt + kSegCap * 4u) > kSortNarrowLds ? (kSortedCopyAt + kSegCap * 4u) : kSortNarrowLds;
+constexpr uint32_t kSortLds = (kSortedCopyAt + kSortedRoom * 4u) > kSortNarrowLds ? (kSortedCopyAt + kSortedRoom * 4u) : kSortNarrowLds;
 
 // Work order for a top_k == 0 row, written by the second pass (every workgroup of the row derives the same one from
 // scan_kernel's coarse counts, see coarse_plan(); the row's first piece stores it): the weights with bits(q) >= thr

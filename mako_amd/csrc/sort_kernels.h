@@ -210,7 +210,7 @@ __device__ __forceinline__ void sort_body(const mako_sample_desc& d_arg, const S
         MAKO_STAMP(10);
         MAKO_COUNT(31, threadIdx.x == 0 && cnt > kSegCap ? 1 : 0);
         MAKO_COUNT(21, threadIdx.x == 0 ? cnt : 0);
-        uint32_t* sorted_copy = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(s_dyn64) + kSortedCopyAt);
+        uint32_t* sorted_copy = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(s_dyn64) + (cnt <= kSortedRoom ? kSortedCopyAt : kSortedOverAt));
         const FinishLds L = finish_lds_views(sm, s_dyn64);
         // (one sort of the share, or of one run of it after the other)
         const uint32_t runs = in_lds ? 1u : plan_runs(key1 + stage, key_lo, key_hi, cnt, s_dyn64, sm);
