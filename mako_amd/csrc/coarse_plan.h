@@ -11,6 +11,12 @@ constexpr uint32_t kBinsPer = kLogBins / (uint32_t)kThreads; // bins a thread: o
 static_assert(kBinsPer * (uint32_t)kThreads == kLogBins && kBinsPer <= 2u, "a thread's counts of a slice are one load");
 using BinCounts = std::conditional_t<kBinsPer == 1u, uint16_t, uint32_t>;
 
+// What the lane before holds of a wave's scan; 0 for the first.
+__device__ __forceinline__ float upto_neighbour(float scan)
+{
+    return __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(scan), 0x138 /* wave_shr:1 */, 0xf, 0xf, true));
+}
+
 // Every workgroup of a row builds the same plan (same inputs, same instructions); LDS of its own, beside the
 // penalty table that the logits' loads work on meanwhile.
 struct alignas(16) CoarsePlan {
@@ -107,6 +113,8 @@ __device__ void coarse_plan(const Scratch& sc, uint32_t row, uint32_t slices, ui
     // Running mass and count from the LOWEST bin up (thread t takes bin kLogBins - 1 - t, or the two from there down to
     // kLogBins - 2 - 2 t): the mass below a bin, which is what the threshold is about, is then a sum of small terms and as
     // accurate as they are, however close to one top_p is.  Wave scans, then one scan of the waves' totals by every wave for itself.
+    // (What is below is the sum up to the neighbour, never a sum less its last term: beside a heavy bin that difference is of its
+    // last places, and a top_p within some 2^-21 of one then lost the tail that its row needed.)
     uint32_t bin[kBinsPer], c[kBinsPer], c_all = 0;
     float mass[kBinsPer], mass_all = 0.0f;
     const float top_frac = fminf(fmaxf(m * scale, -1.0e9f), 1.0e9f) - (float)k_top; // the maximum inside its unit
@@ -134,7 +142,9 @@ __device__ void coarse_plan(const Scratch& sc, uint32_t row, uint32_t slices, ui
     const uint32_t all_c = (uint32_t)__builtin_amdgcn_readlane((int)wc_upto, kWaves - 1);
     float below_m[kBinsPer];     // mass under the bin
     uint32_t excl_c[kBinsPer];   // logits above it
-    below_m[0] = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wm_upto - wm), wave_id())) + mass_w - mass_all;
+    const uint32_t wave = (uint32_t)wave_id();
+    const float waves_below = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(wm_upto), max(wave, 1u) - 1u));
+    below_m[0] = (wave ? waves_below : 0.0f) + upto_neighbour(mass_w);
     excl_c[0] = all_c - ((uint32_t)__builtin_amdgcn_readlane((int)(wc_upto - wc), wave_id()) + cnt_w - c_all) - c[0];
 #pragma unroll
     for (uint32_t i = 1; i < kBinsPer; ++i) {
