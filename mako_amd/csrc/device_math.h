@@ -6,6 +6,8 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include "exp_form.h"
+
 namespace mako {
 
 // 2^(i/32) table of glibc 2.35 (sysdeps/ieee754/flt-32/e_exp2f_data.c):
@@ -30,28 +32,10 @@ __device__ const uint64_t k_exp2_tab[32] = {
 // nothing branches: with a branch per special case every call waited for its own table entry and its own chain, with none the
 // four calls side by side overlap (the second pass over 256 rows of 151 552
 // logits 123 -> 114 us, the weights of 64 rows in token order 19.7 -> 17.9).
-// The cubic by Horner's rule, scaled in its last multiply-add: an operation fewer than glibc's order, and the same float for
-// every argument (tests/cpu/exp_form.c).  With the scale put together as two words the kernels, bound by vector instructions,
-// have five fewer a weight: the weights of those 64 rows 18.7 -> 16.9 us, the second pass over 512 rows 57 -> 55.
 // (exp_moved(): NaN is moved to the lower bound.)
 __device__ __forceinline__ float exp_moved(float x, const uint64_t* tab)
 {
-    const double inv_ln2_n = 0x1.71547652b82fep+0 * 32.0;
-    const double shift = 0x1.8p+52;
-    const double c0 = 0x1.c6af84b912394p-5 / 32 / 32 / 32;
-    const double c1 = 0x1.ebfce50fac4f3p-3 / 32 / 32;
-    const double c2 = 0x1.62e42ff0c52d6p-1 / 32;
-    const double xd = (double)__builtin_amdgcn_fmed3f(x, -104.0f, 89.0f);
-    double kd = fma(inv_ln2_n, xd, shift);
-    const uint32_t ki = (uint32_t)__double_as_longlong(kd);
-    kd -= shift;
-    const double r = fma(inv_ln2_n, xd, -kd);
-    // (+ ki << 47, which the lower word has no part in.  As two words to the end: of a 64-bit sum the compiler makes five instructions)
-    typedef uint32_t u32x2_tab __attribute__((ext_vector_type(2)));
-    u32x2_tab t = __builtin_bit_cast(u32x2_tab, tab[ki & 31u]);
-    t.y += ki << 15;
-    const double s = __builtin_bit_cast(double, t);
-    return (float)fma(fma(r, fma(c0, r, c1), c2), r * s, s);
+    return exp_form(__builtin_amdgcn_fmed3f(x, kExpLow, kExpHigh), tab);
 }
 __device__ __forceinline__ float expf_glibc(float x, const uint64_t* tab)
 {
