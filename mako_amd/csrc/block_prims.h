@@ -20,7 +20,7 @@ extern "C" __device__ float __ockl_wfscan_add_f32(float, bool inclusive);
 
 namespace mako {
 
-// Threads of a workgroup: 1024, but for a translation unit that says otherwise (mako_amd/build.py).
+// Threads of a workgroup: 1024, but for a translation unit that says otherwise (k_sort.hip, k_sort_unsorted.hip, k_finish_halves.hip).
 #ifndef MAKO_THREADS
 #define MAKO_THREADS 1024
 #endif

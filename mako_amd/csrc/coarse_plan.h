@@ -66,7 +66,7 @@ __device__ __forceinline__ void issue_plan_loads(const mako_sample_desc& d, cons
 // estimated from the middle of the units it covers, and the threshold is put one bin below where the estimated mass
 // under it falls to 1 - top_p of the estimated total, less a few percent.  The list that results is checked by the
 // exact sums later: a plan that keeps too little costs a second look at the row, never a wrong answer.
-// (Every instruction here is latency of the whole pass: a workgroup's sixteen waves share four SIMDs.)
+// (Every instruction here is latency of the whole pass: a workgroup's waves share four SIMDs.)
 // share_min: entries a worker is given at least, if there are as many.
 // opaque_first: the first position of the list from which a share may be left unsorted (kNone: none may).
 __device__ void coarse_plan(const Scratch& sc, uint32_t row, uint32_t slices, uint32_t n_vocab, const mako_sampling_params& P,

@@ -1,6 +1,6 @@
 // finish_kernel for batches of many top_k == 0 rows: workgroups of 512 threads, two to a CU (79 680 bytes of LDS each).  A CU's vector
-// units were busy for 60 % of the kernel's time, its LDS for 40 %: what is between is barriers and trips to memory, which one
-// workgroup now fills for the other.  112 to 150 rows of 129 280 logits with histories of 1 024, in a batch of 512: 73.0 us with one
+// units were busy for 54 to 57 % of the kernel's time, its LDS for 16 to 37 %: what is between is barriers and trips to memory, which
+// one workgroup now fills for the other.  112 to 150 rows of 129 280 logits with histories of 1 024, in a batch of 512: 73.0 us with one
 // workgroup of 1 024, 66.4 so (the batch 187.2 -> 177.3); 256 rows of 151 552, half of them flat: 104.7 and 102.  With four history
 // entries a thread the next piece's loads ahead of the hand-over spill, and are worth nothing with a second workgroup on the CU
 // (68.3 us with them and 28 bytes of scratch memory, 66.4 without).

@@ -226,7 +226,7 @@ int mako_sampler_create(mako_sampler_ctx** out, int device, uint32_t max_rows, u
     (void)setup_static_scratch(device);
     (void)hipGetLastError();
     MAKO_HIP(ctx, hipDeviceSynchronize());
-    // the kernels overlay 64 to 128 KB of dynamic LDS (kDynLds, kTailLds, kSortLds) on a few KB of static LDS
+    // the kernels have 64 to 129 KB of dynamic LDS (kDynLds, kTailLds, kSortLds, kFinishLds) beside a few KB of static LDS
     MAKO_HIP(ctx, mako::init_scan_kernels());
     MAKO_HIP(ctx, mako::init_finish_kernels());
     MAKO_HIP(ctx, mako::init_plan_alone());
@@ -434,9 +434,11 @@ int run_batch(mako_sampler_ctx* ctx, const mako_sample_desc& d, const mako_sampl
     const uint32_t nth_steps = !any_nth ? 0u : (!any_rounds ? 1u : mako::nth_launches(d.n_vocab, least_top_k));
     const bool launch_sort = any_nucleus || any_late || beside;
     // Batches with many top_k == 0 rows leave the shares of their sorted lists that need no order unsorted
-    // (unsorted_shares.h): there sort_kernel is bound by the number of its workgroups, one per CU at a time, and not, as
-    // on a small batch, by its slowest worker.  More than four rounds of workers; without the caller's copy of the
-    // parameters, from twice as many rows.
+    // (unsorted_shares.h): there sort_kernel is bound by the number of its workgroups, and not, as on a small batch, by its
+    // slowest worker.  From 33 rows on a chip of 256 CUs, four workers a row and CU: sooner, flat rows gain 3 to 5 % (32 of
+    // 129 280 logits: 101.1 -> 96.0 us) and all others lose (32 of N(0, 3^2) 57.2 -> 63.1, 24 half flat ones 87.2 -> 90.9); later,
+    // flat ones lose 13 % (33: 104.6 -> 118.4) and the others gain 2 to 7 (33 of N(0, 3^2): 70.0 -> 68.6, of 32 000 logits 45.8 ->
+    // 42.7).  Without the caller's copy of the parameters, which may be of any kind, from twice as many rows.
     const bool unsorted = params_host ? (uint64_t)nucleus_rows * mako::kWorkers > 4ull * ctx->cus
                                       : (uint64_t)d.n_rows * mako::kWorkers > 8ull * ctx->cus;
     // (finish_kernel's grid: scan_kernel, which cuts the second pass up, is told of it)

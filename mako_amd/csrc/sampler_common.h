@@ -76,12 +76,19 @@ __device__ __forceinline__ int32_t log_unit(float logit, float scale)
 }
 
 constexpr uint32_t kWorkers = 32;  // workgroups that share the sort of one wide-nucleus row
-// Entries of a row's list that each of its workers is given at least, if there are as many (coarse_plan()).  A worker is a
-// workgroup with a CU to itself and takes 6.3 us for 90 entries, 9.7 for 4 400: on a large batch, which waits for all of
-// them, every row of some thousand entries cut into 32 shares costs its CUs ten times what one worker does (512 rows of a
-// decode batch: 1 820 workers, half of them with fewer than 94 entries; 225 us now, 255 in 32 shares, 240 with 5 000 entries
-// at least, which some shares overrun); on a small one the row waits for the slowest, but for more than one round of them too
-// (64 rows: 62.5 us, 65.4 in 32 shares).
+// Entries of a row's list that each of its workers is given at least, if there are as many (coarse_plan()).  Most of a worker's
+// time is what it costs whatever it sorts (6.3 us for 90 entries, 9.7 for 4 400, with a CU to itself): a large batch waits for
+// all of them, and every row of some thousand entries cut into 32 shares costs its CUs ten times what one worker does (512 rows
+// of a decode batch, 1 820 workers, half of them with fewer than 94 entries, when one had a CU: 225 us, 255 in 32 shares); on a small
+// one the row waits for the slowest, but for more than one round of them too.
+// With two workers to a CU (us):                    at least 2 048  3 072  4 096  5 120
+//   large: 256 rows of 151 552 logits, half flat             253.5  253.7  253.3  270.5
+//          200 of 129 280, half flat; of N(0, 3^2)    211.7, 152.1  211.5, 152.6  209.4, 148.7  221.5, 149.7
+//          40 of 129 280, half flat; of N(0, 3^2)      103.1, 67.7  104.1, 70.3  102.0, 70.9  108.7, 71.8
+//                                                     at least 256  512  1 024
+//   small: 32 rows of 151 552, N(0, 3^2); flat of 8 000  75.9, 61.6  68.9, 55.0  68.2, 52.9
+//          one row of 151 552, N(0, 3^2); flat of 8 000  41.5, 47.5  39.8, 47.4  39.8, 48.1
+//          64 rows of a decode batch of 129 280            59.2  58.0  58.6
 constexpr uint32_t kShareLarge = 4096, kShareSmall = 512;
 constexpr uint32_t kStageSlack = 64; // room a worker's share of the staging arrays gets beyond what the coarse counts
                                      // promise (and 1/64 of that count); the rows' arrays are sized to hold it
@@ -144,8 +151,8 @@ constexpr uint32_t kOpaque = 1u << 25; // the record stands for a whole unsorted
 // The large batches' work lists of sort_kernel.  Workgroups are dispatched in the order of their numbers, to the XCDs
 // in turn, and the next one waits for a CU of ITS XCD: with entries of unequal cost in row order the XCDs fall out of
 // step and CUs idle (a quarter of the time on config 4).  So the costliest entries, the collectors of unsorted shares
-// (up to three per row, ~19 us), come first and together, then the workers that sort (~13 us) and the narrow rows
-// (~10 us).  A workgroup without an entry costs nothing behind the last one with work, but between two of them it
+// (up to three per row), come first and together, then the workers that sort and the narrow rows (~19, ~13 and ~10 us with a CU
+// to themselves).  A workgroup without an entry costs nothing behind the last one with work, but between two of them it
 // waits for a CU like any other: the collectors' list is filled from its end backwards (work_n[3] of them, the last at
 // workgroup number sorted_at - 1), the others' forwards from sorted_at (work_n[0]), so that no gap lies between.
 // (a share a wave: with two for each of a collector's eight waves, in two collectors, 48 rows of 129 280 logits, half of them

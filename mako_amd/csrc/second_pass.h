@@ -190,7 +190,7 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
         __builtin_amdgcn_sched_barrier(0); // (not among the weights, whose registers these take)
     if (AHEAD && next != kNone) // uniform
         issue_slice<ALIGNED, KH>(d, row, next * slice_len, min(d.n_vocab, next * slice_len + slice_len), loads);
-    // the piece's sum: wave reductions, then the sixteen waves' results in order
+    // the piece's sum: wave reductions, then the waves' results in order
     {
         const double sw = __ockl_wfred_add_f64(sum);
         if (lane_id() == 0)
@@ -222,7 +222,7 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
     const global_ptr<uint32_t> kstage = as_global(sc.key[1]) + (size_t)row * sc.vpad;
     const global_ptr<uint32_t> istage = as_global(sc.idx[1]) + (size_t)row * sc.vpad;
     // (room for all a piece can hold: with half as much, a flat row's pieces, which keep nearly everything, went through
-    // it twice, 2 us more each, and the workgroup has its CU to itself anyway)
+    // it twice, 2 us more each; a workgroup of 1 024 has its CU to itself anyway, and two of 512 have room for all they can hold)
     uint2* buf = reinterpret_cast<uint2*>(L.cnt); // [kPieceMax + 3 kWorkers] (weight, token id)
     static_assert(kFinishLds >= (kPieceMax + 3u * kWorkers) * sizeof(uint2), "");
     const uint32_t kept = pl.lbase[kWorkers];

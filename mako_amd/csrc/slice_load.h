@@ -208,7 +208,7 @@ __device__ __forceinline__ void finish_slice(const RawSlice& r, uint32_t lo, uin
 
 // The thread's logits after the mask and the penalties (src/gen/sampler.cpp:22-28): wv[16] in the slice layout.
 //
-// KH > 0 (histories of at most KH * 1024 entries): thread t handles history entries t, t + 1024, ...  The
+// KH > 0 (histories of at most KH * kThreads entries): thread t handles history entries t, t + kThreads, ...  The
 // per-token counts are accumulated in LDS; for every distinct token of the slice the thread holding its first
 // entry (an election, so that each token is handled once) computes the penalised logit: one IEEE division per
 // history entry instead of one per logit slot.  The logit travels through the token's slot of the LDS table:

@@ -252,10 +252,12 @@ __device__ __forceinline__ void sort_body(const mako_sample_desc& d_arg, const S
 }
 #ifdef MAKO_EMIT_SORT_KERNELS // (not templates: defined by the one translation unit that launches them)
 // Workgroups of 512, two to a CU (four waves a SIMD: 128 registers).  A worker is three dependent trips to memory, some twenty
-// barriers and vector instructions for 40 % of the time in between: with 1 024 threads, alone on its CU, it leaves it idle for most of
+// barriers and vector instructions for 42 % of the time in between: with 1 024 threads, alone on its CU, it leaves it idle for most of
 // that, and two workgroups that have nothing to do with each other fill each other's gaps.  (256 rows of 151 552 logits, half of
-// them flat: the kernel 100 -> 66 us, the batch 289 -> 255; 97 nucleus rows of 512 189 -> 186.)  On a small batch, where a worker
-// has a CU to itself either way, half the waves start and meet sooner (one row 43.8 -> 42.9 us, 64 rows 58.0 -> 57.3).
+// them flat: the kernel 100 -> 66 us, the batch 289 -> 255; 16 flat rows of 129 280 90.5 -> 85.1.)  On a batch of up to eight rows, where
+// a worker has a CU to itself either way, half the waves start and meet sooner, and take longer over a full share: narrow rows gain
+// 4 %, one row of N(0, 3^2) 44.7 -> 43.8 us, flat rows of 129 280 logits and more lose 1 to 4 % (one 69.0 -> 69.3, eight 76.4 -> 77.1, of
+// 196 000 97.9 -> 101.5).
 // (sort_beside_kernel has 1 024, as the groups and steps in it want.)
 #ifdef MAKO_SORT_UNSORTED
 __global__ __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(4))) void sort_kernel_unsorted(mako_sample_desc d_arg, Scratch sc_val, uint32_t slices)

@@ -75,7 +75,7 @@ __device__ MAKO_RARE_CALL double reference_total(Get q_at, uint32_t n, FinishSha
 // Tail of every path that ends with a list sorted by (q desc, idx asc): kf[i] = ~bits(q_i), jf[i] = token id,
 // n1 entries (already cut to top_k).  Applies top-p (src/gen/sampler.cpp:44-61) against total64 (the fp64 sum over
 // the row's candidates; summed from the list when !have_total), then the exact fp32 total (:80-82) and walk
-// (:64-73).  All 1024 threads must call it.
+// (:64-73).  All threads of the workgroup must call it.
 //
 // When `need_cut` the list is only the heaviest part of the row's candidates and every candidate missing from
 // it weighs at most q_bound: the nucleus must then end inside the list, at an entry strictly heavier than

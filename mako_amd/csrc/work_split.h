@@ -7,7 +7,7 @@ namespace mako {
 
 // How finish_kernel cuts each top_k == 0 row into pieces, and how many workgroups share a row's pieces.  A piece is
 // one to four blocks of 4096 logits (a slice is four): as few blocks as keep all the pieces of the batch within one
-// round of workgroups (`cus` of them run at a time, one per CU), since the pass is bound by instruction issue and
+// round of workgroups (`cus` of them run at a time, one per CU, or two of 512 threads each), since the pass is bound by instruction issue and
 // more workgroups with less work each finish sooner.  A batch with more pieces than that takes whole slices, and as
 // many workgroups per row as keeps it to one round; each of them goes through its share of the row's pieces in turn
 // (and builds the row's plan once, not once per piece).  Worked out from the rows' parameters by one wave of

@@ -20,7 +20,7 @@ struct alignas(16) FinishShared {
 // Views into the first 64 KB of the dynamic LDS block; `cnt` (first pass) overlaps the two others (second pass).
 struct FinishLds {
     FinishShared* sm;
-    uint32_t* cnt;              // [kSliceMax]
+    uint32_t* cnt;              // [kPieceMax]
     unsigned long long* sortk;  // [kSortMax]
     uint32_t* wcount;           // [kWaves * 256]
 };
