@@ -8,7 +8,7 @@ void launch_sort_beside(hipStream_t st, const mako_sample_desc& d, const Scratch
                         uint32_t more, uint32_t cus)
 {
     static_assert(kSortBesideWaves == (uint32_t)kWaves, "");
-    const uint32_t x = unsorted ? sort_items_per_row(kSortBesideWaves) : kWorkers;
+    const uint32_t x = unsorted ? kSortItemsPerRow : kWorkers;
     const dim3 grid(x, grid_rows + (more + x - 1u) / x);
     if (unsorted)
         hipLaunchKernelGGL(sort_beside_kernel<true>, grid, dim3(kThreads), kSortLds, st, d, sc, slices, grid_rows, cus);

@@ -10,7 +10,7 @@ namespace mako {
 void launch_sort_unsorted(hipStream_t st, const mako_sample_desc& d, const Scratch& sc, uint32_t slices, uint32_t grid_rows)
 {
     static_assert(kSortWaves == (uint32_t)kWaves, "");
-    hipLaunchKernelGGL(sort_kernel_unsorted, dim3(sort_items_per_row(kSortWaves), grid_rows), dim3(kThreads), kSortLds, st, d, sc, slices);
+    hipLaunchKernelGGL(sort_kernel_unsorted, dim3(kSortItemsPerRow, grid_rows), dim3(kThreads), kSortLds, st, d, sc, slices);
 }
 
 hipError_t init_sort_unsorted()

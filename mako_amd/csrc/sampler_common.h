@@ -151,25 +151,31 @@ constexpr uint32_t kOpaque = 1u << 25; // the record stands for a whole unsorted
 // The large batches' work lists of sort_kernel.  Workgroups are dispatched in the order of their numbers, to the XCDs
 // in turn, and the next one waits for a CU of ITS XCD: with entries of unequal cost in row order the XCDs fall out of
 // step and CUs idle (a quarter of the time on config 4).  So the costliest entries, the collectors of unsorted shares
-// (up to three per row), come first and together, then the workers that sort and the narrow rows (~19, ~13 and ~10 us with a CU
+// (up to two per row), come first and together, then the workers that sort and the narrow rows (~19, ~13 and ~10 us with a CU
 // to themselves).  A workgroup without an entry costs nothing behind the last one with work, but between two of them it
 // waits for a CU like any other: the collectors' list is filled from its end backwards (work_n[3] of them, the last at
 // workgroup number sorted_at - 1), the others' forwards from sorted_at (work_n[0]), so that no gap lies between.
-// (a share a wave: with two for each of a collector's eight waves, in two collectors, 48 rows of 129 280 logits, half of them
-// flat, waited 34 us for them, and 23 for workgroups of sixteen waves before)
 constexpr uint32_t kSortWaves = 8u, kSortBesideWaves = 16u; // of sort_kernel_unsorted and sort_beside_kernel
-constexpr uint32_t kUnsortedMost = 24u; // shares of a row that its collectors have waves for; any beyond are a wave's second
-__host__ __device__ constexpr uint32_t collectors_per_row(uint32_t waves) { return (kUnsortedMost + waves - 1u) / waves; }
-__host__ __device__ constexpr uint32_t sort_items_per_row(uint32_t waves) { return kWorkers + collectors_per_row(waves); }
-constexpr uint32_t kSortItemsPerRow = sort_items_per_row(kSortWaves);
-static_assert(kSortItemsPerRow >= sort_items_per_row(kSortBesideWaves), "room for either kernel's lists");
+// Unsorted shares that a collector takes.  A workgroup of eight waves one each on batches of up to 80 top_k == 0 rows, which wait for
+// the slowest collector, and two each beyond, which wait for all of them (us, rows of 129 280 logits):
+//              33 rows: flat, half flat   64            80            96            128           256
+//   one each       104.5, 100.9  122.3, 109.3  140.8, 126.5  156.1, 133.2  183.6, 154.1  303.2, 241.2
+//   two            112.7, 108.1  124.4, 117.4  140.2, 131.3  153.0, 137.1  181.1, 153.5  300.0, 240.4
+// (A row's collectors beyond the second go where the workers are: with room for a third in front, 128 more workgroups without an
+// entry there, 128 rows without such shares took 1.7 us longer.)
+constexpr uint32_t kShareEachRows = 80u;
+__device__ __forceinline__ uint32_t shares_collected(uint32_t waves, uint32_t nucleus_rows)
+{
+    return waves == kSortWaves && nucleus_rows > kShareEachRows ? 2u * waves : waves;
+}
+constexpr uint32_t kCollectorsInFront = 2u;
+constexpr uint32_t kSortItemsPerRow = kWorkers + kCollectorsInFront;
 struct SortLists {
     uint32_t sorted_at; // first workgroup number (= entry of work_sort) of the workers that sort and the narrow rows
 };
-template <uint32_t WAVES>
-__device__ __forceinline__ SortLists large_batch_lists(uint32_t nucleus_rows) // (Scratch::work_n[10])
+__host__ __device__ inline SortLists large_batch_lists(uint32_t nucleus_rows) // (Scratch::work_n[10])
 {
-    return SortLists{collectors_per_row(WAVES) * nucleus_rows};
+    return SortLists{kCollectorsInFront * nucleus_rows};
 }
 
 constexpr uint32_t kWorkWords = 12;        // of Scratch::work_n

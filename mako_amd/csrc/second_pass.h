@@ -81,20 +81,23 @@ __device__ bool one_piece(const mako_sample_desc& d, const Scratch& sc, uint32_t
             const uint32_t unsorted = (UNSORTED && flag == 1) ? pl.opq_mask : 0u;
             plan->opq_mask = unsorted;
             if (flag == 1 || flag == 3) {
-                // sort_kernel's work: a workgroup per worker that sorts, and up to collectors_per_row() whose waves take the row's
-                // unsorted shares, a share each (work items kWorkers + c)
+                // sort_kernel's work: a workgroup per worker that sorts, and collectors whose waves take the row's unsorted
+                // shares, a share at a time (work items kWorkers + c)
                 const uint32_t n_unsorted = (uint32_t)__popc(unsorted);
-                const uint32_t collectors = min((n_unsorted + SORT_WAVES - 1u) / SORT_WAVES, collectors_per_row(SORT_WAVES));
+                const uint32_t each = shares_collected(SORT_WAVES, pl.nucleus_rows), collectors = (n_unsorted + each - 1u) / each;
                 if constexpr (UNSORTED) {
                     // (two lists, the costly entries in front: large_batch_lists())
-                    const SortLists lists = large_batch_lists<SORT_WAVES>(pl.nucleus_rows);
+                    const SortLists lists = large_batch_lists(pl.nucleus_rows);
                     if (flag == 3) {
                         work_sort[lists.sorted_at + take(work_n + 0, 1u)] = row << 8;
                     } else {
-                        uint32_t at = lists.sorted_at - take(work_n + 3, collectors) - collectors;
-                        for (uint32_t c = 0; c < collectors; ++c)
+                        const uint32_t in_front = min(collectors, kCollectorsInFront);
+                        uint32_t at = lists.sorted_at - take(work_n + 3, in_front) - in_front;
+                        for (uint32_t c = 0; c < in_front; ++c)
                             work_sort[at++] = (row << 8) | (kWorkers + c);
-                        at = lists.sorted_at + take(work_n + 0, pl.workers - n_unsorted);
+                        at = lists.sorted_at + take(work_n + 0, pl.workers - n_unsorted + collectors - in_front);
+                        for (uint32_t c = in_front; c < collectors; ++c)
+                            work_sort[at++] = (row << 8) | (kWorkers + c);
                         for (uint32_t w = 0; w < pl.workers; ++w)
                             if (!((unsorted >> w) & 1u))
                                 work_sort[at++] = (row << 8) | w;

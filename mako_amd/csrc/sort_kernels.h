@@ -50,7 +50,7 @@ __device__ __forceinline__ void sort_body(const mako_sample_desc& d_arg, const S
     if constexpr (UNSORTED) {
         // (two lists that meet at workgroup number sorted_at: large_batch_lists())
         const uint32_t n_collectors = first.n_collectors;
-        const SortLists lists = large_batch_lists<(uint32_t)kWaves>(first.nucleus_rows);
+        const SortLists lists = large_batch_lists(first.nucleus_rows);
         const bool with_work = piece < lists.sorted_at ? lists.sorted_at - piece <= n_collectors : piece - lists.sorted_at < n_work;
         if (!with_work)
             return;
@@ -169,20 +169,21 @@ __device__ __forceinline__ void sort_body(const mako_sample_desc& d_arg, const S
     const uint32_t gbase = (uint32_t)__builtin_amdgcn_readlane((int)(grp_upto - grp_l), (int)w);
     const size_t t_row = (size_t)row * sc.g_cap;
     if (UNSORTED && w >= kWorkers) {
-        // One of the row's collectors: each of its waves takes one of the shares that are left unsorted (and another one where
-        // there are more of them than waves) and leaves its record.  (The binades of the increments from the plan's estimates in
+        // One of the row's collectors: each of its waves takes one of the shares that are left unsorted, or two, and leaves its
+        // record.  (The binades of the increments from the plan's estimates in
         // the exact total's units; any guess is safe, the tail tests what it applies.  A verification row has no such
         // shares.)
         MAKO_WG_TAG(0xc0000000u);
         const double r0_raw = (double)u_row * ((double)s_args.P.top_p * total64);
         const double r0 = r0_raw == r0_raw ? r0_raw : 0.0, scale = mass_all > 0.0 ? total64 / mass_all : 0.0;
         uint32_t* wave_lds = reinterpret_cast<uint32_t*>(s_dyn64) + (uint32_t)wave_id() * (kOpaqueLdsWords + 2u);
-        uint32_t mine = (w - kWorkers) * (uint32_t)kWaves + (uint32_t)wave_id();
+        const uint32_t each = shares_collected((uint32_t)kWaves, first.nucleus_rows), end = (w - kWorkers + 1u) * each;
+        uint32_t mine = end - each + (uint32_t)wave_id();
         uint32_t rank = 0;
         for (uint32_t v = 0; v + 1u < kWorkers; ++v) { // (uniform)
-            if (!((opq_mask >> v) & 1u) || rank++ != mine)
+            if (!((opq_mask >> v) & 1u) || rank++ != mine || mine >= end)
                 continue;
-            mine += collectors_per_row((uint32_t)kWaves) * (uint32_t)kWaves;
+            mine += (uint32_t)kWaves;
             const uint32_t cnt_v = (uint32_t)__builtin_amdgcn_readlane((int)cnt_l, (int)v);
             const uint32_t stage_v = (uint32_t)__builtin_amdgcn_readlane((int)stage_l, (int)v);
             const uint32_t off_v = (uint32_t)__builtin_amdgcn_readlane((int)(cnt_upto - cnt_l), (int)v);

@@ -1,5 +1,5 @@
 """GPU parity of large batches whose flat rows leave from a few to some two dozen shares unsorted: the workgroups that take them
-have a wave for each, eight a workgroup (with the host copy of the parameters) or sixteen (without it)."""
+have eight waves with a share each or, from 81 rows, two (with the host copy of the parameters), or sixteen (without it)."""
 import pytest
 
 from mako_amd import api
@@ -9,8 +9,8 @@ pytestmark = pytest.mark.gpu
 
 
 @pytest.mark.parametrize("vocab", [41000, 74000, 107000, 129280, 196000, 262144])
-def test_one_to_three_workgroups_a_row(vocab):
-    rows = 66
+@pytest.mark.parametrize("rows", [66, 80, 81])
+def test_one_to_four_workgroups_a_row(vocab, rows):
     w = nucleus_batch(rows, vocab, vocab + 5, [0.05, 0.1, 0.4], [1.0], [0.9, 0.9995], us=[0.0, 0.3, 0.98, 1.0 - 2.0**-24, 0.6])
     w["params"]["top_k"][5::11] = 40
     ctx = api.SamplerContext(max_rows=rows, max_vocab=vocab)
