@@ -72,7 +72,7 @@ __device__ bool lds_bucket_sort(const uint32_t (&k)[kSortPer], const uint32_t (&
     MAKO_STAMP(15);
     // 2. rank inside the bucket, and out
     const bool over = kSortedRoom < kSegCap && n > kSortedRoom; // uniform
-    uint32_t place[kSortPer];
+    uint32_t place[(kSortPer + 1u) / 2u]; // (two to a word)
 #pragma unroll
     for (uint32_t t = 0; t < kSortPer; ++t) {
         const uint32_t s = t * kThreads + tid;
@@ -95,7 +95,7 @@ __device__ bool lds_bucket_sort(const uint32_t (&k)[kSortPer], const uint32_t (&
             iout[at] = ~(uint32_t)me;
             if (sorted_lds && !over)
                 sorted_lds[at] = ~(uint32_t)(me >> 32);
-            place[t] = at;
+            place[t / 2u] = t % 2u ? place[t / 2u] | (at << 16) : at;
         }
     }
     if (sorted_lds && over) { // (every entry has its place: the copy may go over them, once all weights are in registers)
@@ -107,7 +107,7 @@ __device__ bool lds_bucket_sort(const uint32_t (&k)[kSortPer], const uint32_t (&
 #pragma unroll
         for (uint32_t t = 0; t < kSortPer; ++t)
             if (t * kThreads + tid < n)
-                sorted_lds[place[t]] = ~w[t];
+                sorted_lds[t % 2u ? place[t / 2u] >> 16 : place[t / 2u] & 0xffffu] = ~w[t];
     }
     if (sorted_lds) // uniform
         lds_barrier();

@@ -95,6 +95,9 @@ constexpr uint32_t kStageSlack = 64; // room a worker's share of the staging arr
 constexpr uint32_t kGroup = 256;      // a sorted list is processed in groups of one wave x four entries per lane
 constexpr uint32_t kMaxGroups = 1024; // groups per list
 constexpr uint32_t kSegCap = 6144;    // entries a worker sorts in LDS
+// And of a longer share, in each of its runs (worker_sort.h): what is less has fewer in a bucket, and one share with a crowded
+// bucket among thousands is some 45 us of radix sort (64 flat rows of 262 144 logits: 250.5 us with runs of 6 144, 208.8 so).
+constexpr uint32_t kRunMost = kThreads == 1024 ? kSegCap : 5632;
 constexpr uint32_t kFine = 2048;      // value buckets of that sort
 // dynamic LDS of sort_kernel: for the sort the entries in the order of their buckets (and four more), the buckets, and a copy of the
 // sorted weights for the group records, 81 968 bytes; for a narrow row the lists that its tail works on, kTailLds, 90 112 bytes,

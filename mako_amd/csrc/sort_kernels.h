@@ -213,22 +213,50 @@ __device__ __forceinline__ void sort_body(const mako_sample_desc& d_arg, const S
         MAKO_COUNT(21, threadIdx.x == 0 ? cnt : 0);
         uint32_t* sorted_copy = reinterpret_cast<uint32_t*>(reinterpret_cast<char*>(s_dyn64) + (cnt <= kSortedRoom ? kSortedCopyAt : kSortedOverAt));
         const FinishLds L = finish_lds_views(sm, s_dyn64);
-        // (one sort of the share, or of one run of it after the other)
-        const uint32_t runs = in_lds ? 1u : plan_runs(key1 + stage, key_lo, key_hi, cnt, s_dyn64, sm);
-        bool sorted = runs != 0u;
-        for (uint32_t r = 0; sorted && r < runs; ++r) { // uniform
-            uint32_t lo_r = key_lo, hi_r = key_hi, at = 0, n = cnt;
-            if (!in_lds) {
-                // keys of buckets [b0, b1): (key_hi - 1 - k) >> shift in [b0, b1)
-                const uint32_t range = key_hi - key_lo, shift = range > kFine ? 32u - (uint32_t)__clz((range - 1u) >> 11) : 0u;
-                const uint32_t b0 = uniform_u32(sm.hist[r]), b1 = uniform_u32(sm.hist[64u + r]);
-                at = uniform_u32(sm.run[r]);
-                n = uniform_u32(sm.run[64u + r]);
-                hi_r = key_hi - (b0 << shift);
-                lo_r = ((unsigned long long)b1 << shift) >= range ? key_lo : key_hi - (b1 << shift);
-                sorted = collect_run(key1 + stage, idx1 + stage, key_lo, key_hi, cnt, lo_r, hi_r, n, s_dyn64, sm, share);
+        // one sort of the share, or of one run of it after the other
+        struct Run {
+            uint32_t key_lo, key_hi, at, n; // at: of the share's entries in order
+        };
+        auto run = [&](uint32_t r) {
+            // keys of buckets [b0, b1): (key_hi - 1 - k) >> shift in [b0, b1)
+            const uint32_t range = key_hi - key_lo, shift = range > kFine ? 32u - (uint32_t)__clz((range - 1u) >> 11) : 0u;
+            const uint32_t b0 = uniform_u32(sm.hist[r]), b1 = uniform_u32(sm.hist[64u + r]);
+            return Run{((unsigned long long)b1 << shift) >= range ? key_lo : key_hi - (b1 << shift), key_hi - (b0 << shift),
+                       uniform_u32(sm.run[r]), uniform_u32(sm.run[64u + r])};
+        };
+        auto collect = [&](const Run& x) {
+            return collect_run(key1 + stage, idx1 + stage, key_lo, key_hi, cnt, x.key_lo, x.key_hi, x.n, s_dyn64, sm, share);
+        };
+        auto sort = [&](const Run& x, uint32_t* copy) {
+            return lds_sort_staged(share, x.key_lo, x.key_hi, x.n, key0 + off + x.at, idx0 + off + x.at, s_dyn64, sm, copy);
+        };
+        const Run whole = {key_lo, key_hi, 0u, cnt};
+        bool sorted = false, copied = false; // (uniform)
+        if constexpr (kRunMost < kSegCap) {
+            // (a share that is longer than a run and too crowded at once is tried in runs, which are narrower: 32 flat rows of
+            // 196 000 logits, one of whose shares is, 198.9 -> 162.0 us)
+            if (in_lds)
+                sorted = copied = sort(whole, sorted_copy);
+            if (!sorted && cnt > kRunMost) {
+                const uint32_t runs = plan_runs(key1 + stage, key_lo, key_hi, cnt, s_dyn64, sm);
+                sorted = runs != 0u;
+                for (uint32_t r = 0; sorted && r < runs; ++r) {
+                    const Run x = run(r);
+                    sorted = collect(x) && sort(x, nullptr);
+                }
             }
-            sorted = sorted && lds_sort_staged(share, lo_r, hi_r, n, key0 + off + at, idx0 + off + at, s_dyn64, sm, in_lds ? sorted_copy : nullptr);
+        } else { // (the sort's code once: with two copies of it sort_beside_kernel is short of registers, and uses scratch memory)
+            const uint32_t runs = in_lds ? 1u : plan_runs(key1 + stage, key_lo, key_hi, cnt, s_dyn64, sm);
+            sorted = runs != 0u;
+            for (uint32_t r = 0; sorted && r < runs; ++r) {
+                Run x = whole;
+                if (!in_lds) {
+                    x = run(r);
+                    sorted = collect(x);
+                }
+                sorted = sorted && sort(x, in_lds ? sorted_copy : nullptr);
+            }
+            copied = in_lds && sorted;
         }
         if (cnt > kSegCap)
             MAKO_STAMP(18);
@@ -247,7 +275,7 @@ __device__ __forceinline__ void sort_body(const mako_sample_desc& d_arg, const S
             sort_segment(key0 + off, idx0 + off, key1 + stage, idx1 + stage, cnt, L);
         }
         MAKO_STAMP(11);
-        worker_groups(key0, off, cnt, sc.gt + t_row + gbase, before, L, (in_lds && sorted) ? sorted_copy : nullptr, r0);
+        worker_groups(key0, off, cnt, sc.gt + t_row + gbase, before, L, copied ? sorted_copy : nullptr, r0);
         MAKO_STAMP(12);
     }
 }

@@ -94,7 +94,7 @@ __device__ uint32_t plan_runs(const uint32_t* ks, uint32_t key_lo, uint32_t key_
         uint32_t runs = 0, b0 = 0;
         while (b0 < kFine && runs < 64u) {
             uint32_t b1 = b0 + 1u;
-            if (hist[b1] - hist[b0] > kSegCap) { // one bucket alone is too much
+            if (hist[b1] - hist[b0] > kRunMost) { // one bucket alone is too much
                 runs = 0;
                 b0 = kFine;
                 break;
@@ -103,7 +103,7 @@ __device__ uint32_t plan_runs(const uint32_t* ks, uint32_t key_lo, uint32_t key_
                 uint32_t lo = b1, hi = kFine;
                 while (lo < hi) {
                     const uint32_t mid = (lo + hi + 1u) / 2u;
-                    if (hist[mid] - hist[b0] <= kSegCap)
+                    if (hist[mid] - hist[b0] <= kRunMost)
                         lo = mid;
                     else
                         hi = mid - 1u;

@@ -23,3 +23,19 @@ def test_flat_rows(vocab, grid, rows):
         assert_parity(ctx, w, cap=min(vocab, 20000) if rows == 6 else 64, hinted=True)
     finally:
         ctx.close()
+
+
+@pytest.mark.parametrize("above", [0.5, 1.0, 2.0, 4.0, 8.0])
+@pytest.mark.parametrize("vocab", [182000, 188000, 194000, 230000])
+def test_crowded_shares(vocab, above):
+    """One token far above the others: the share it is in has a wide range of weights, nearly all of them at its lower end, in buckets
+    too crowded for one sort, for a run's, or for neither."""
+    for rows in (6, 36):
+        w = nucleus_batch(rows, vocab, vocab + int(above * 2), [0.1, 0.05, 0.3], [1.0], [0.9999], us=[0.3, 0.98, 0.0])
+        at = np.arange(rows) * 4099 % vocab
+        w["logits"][np.arange(rows), at] = w["logits"].max(axis=1) + np.float32(above)
+        ctx = api.SamplerContext(max_rows=rows, max_vocab=vocab)
+        try:
+            assert_parity(ctx, w, cap=12000, hinted=True)
+        finally:
+            ctx.close()
