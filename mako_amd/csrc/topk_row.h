@@ -6,6 +6,8 @@
 
 namespace mako {
 
+static_assert(kThreads == 1024, "the lists below and the whole-row path's sort have an entry of every 1 024 for each thread");
+
 // The row's candidates (all slices) weighted, sorted by (q desc, idx asc) and left in LDS as kf[i] = ~bits(q_i),
 // jf[i] = token id, invalid ones (q not a candidate) last.  Returns the number of valid candidates.
 template <int ITEMS>
